@@ -1,10 +1,10 @@
 // The plain product: 64x64 tiles through LDS, 32-bit FMA, k in ascending order.
-// With the 32-bit matrix-core tiles and the few-row kernel below it is the whole
+// With the 32-bit matrix-core tiles (here and in gemm_f32_tiles.hip) and the few-row kernels below it is the whole
 // 32-bit path (nothing here rounds its inputs) and the bfloat16 fallback for shapes
-// the bfloat16 MFMA kernels refuse.  Within each of the three kernels the order of
-// the sum for an output depends on K only, so a row's result does not depend on the
-// row's place in the batch or on its tile; which kernel runs depends on M (up to 8
-// rows, up to 16, more), so across those ranges results differ by rounding.
+// the bfloat16 MFMA kernels refuse.  Within each kernel the order of
+// the sum for an output depends on K only (and on the weight's shape), so a row's result does not depend on the
+// row's place in the batch or on its tile; which kernel runs depends on M and the shape, so across those
+// ranges results differ by rounding.
 // Reference: gemm_f32 accumulates in 32-bit the same way (shaders/ops.metal:1053-1079).
 #include "gemm.h"
 
@@ -65,7 +65,8 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(const T* __restrict__ 
     }
 }
 
-// 32-bit products on the matrix cores: v_mfma_f32_32x32x2_f32 multiplies and adds in 32-bit (no
+// 32-bit products on the matrix cores for rows that cannot be read in 16-byte pieces of whole 32-k blocks (gemm_f32_tiles.hip
+// and the few-row kernel below take the others): v_mfma_f32_32x32x2_f32 multiplies and adds in 32-bit (no
 // reduced-precision mode), k in ascending order, so an output's sum depends on K only here too.
 // 128 x 128 tiles of four waves (64 x 64 each), k in steps of 16 through two LDS buffers; the next
 // step's rows are on their way to registers while this step is multiplied.  Any M, N, K: rows and
@@ -236,82 +237,103 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const T* __restrict__ A,
     }
 }
 
-// Up to 16 tokens in 32-bit on the matrix cores: v_mfma_f32_16x16x4_f32 multiplies and adds in 32-bit (no
-// reduced-precision mode).  The weight's rows are the A operand, read once, 16 bytes a lane (lane l: feature
-// l % 16 of a tile, the four k-values 4 (l / 16) .. + 3 of a group of 16); the tokens' rows are the B operand, read
-// the same way once for all of a block's NT feature tiles, so that the tokens cost a load for every NT loads of
-// weights where the walk above asks for every token's row again for every two or four rows of the weight.  An MFMA
-// contracts the four k-values that the four lane groups hold in the same place of their loads.  A block's NW waves
+// Few tokens in 32-bit on the matrix cores: v_mfma_f32_16x16x4_f32 multiplies and adds in 32-bit (no
+// reduced-precision mode).  The weight's rows are the A operand, read once for every 16 MT tokens, 16 bytes a lane (lane
+// l: feature l % 16 of a tile, the four k-values 4 (l / 16) .. + 3 of a group of 16); the tokens' rows are the B
+// operand, read the same way once for all of a block's NT feature tiles, so that the tokens cost a load for every NT
+// loads of weights where the walk above asks for every token's row again for every two or four rows of the weight.  An
+// MFMA contracts the four k-values that the four lane groups hold in the same place of their loads.  A block's NW waves
 // take the 32-wide k-blocks in turn, U of them with all loads asked for before the first product, and add their sums
-// through LDS in wave order: an output's sum depends on K (and on the weight's shape, which chooses NW) only.
-// C: lane l holds token l % 16 and features 4 (l / 16) + r.  Needs K % 32 == 0 and 16-byte aligned rows.
+// through LDS in wave order.  C: lane l holds token l % 16 and features 4 (l / 16) + r.  Needs K % 32 == 0 and 16-byte
+// aligned rows.
+// Up to 16 tokens an output's sum depends on K and the weight's shape alone (which choose NW); with more tokens on the
+// form that launch_f32_few_rows picks as well.
+// LAST = 8 (NT = 1): a block takes half a tile of features; the other rows of the tile are never asked for.
+// rot_feats > 0: neighbouring groups of that many features begin their walk along k at different k-blocks and wrap
+// round.  Rows are a multiple of the memory channels' interleave apart, so blocks in step would all ask the same few
+// channels at once.  What bounds it: the weights' bytes, and beside them the tokens' rows, which every block reads again.
+// Measured at 8 rows, before -> with the walk staggered and these shapes of block (2048 features k 8192: half tiles):
+// 16384 x 2048 31.4 -> 27.5 us (4.9 TB/s of weights), 128256 x 2048 213 -> 184, 4096 x 4096 18.6 -> 15.8,
+// 6144 x 4096 30 -> 24, 2048 x 8192 27 -> 23, 28672 x 4096 88 -> 84.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-template <int NT, int NW, int U>
+template <int MT, int NT, int NW, int U, int LAST = 16>
 __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
-                                                                  void* __restrict__ out, int ldc, int M, int N, int K, int epi) {
-    extern __shared__ __attribute__((aligned(16))) float f32_skinny_red[];       // [NW][NT][4][64]
+                                                                  void* __restrict__ out, int ldc, int M, int N, int K, int epi, int rot_feats) {
+    extern __shared__ __attribute__((aligned(16))) float f32_skinny_red[];       // [NW][MT][NT][4][64]
     float* red = f32_skinny_red;
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int row = lane & 15, g = lane >> 4;
-    int n0 = blockIdx.x * NT * 16;
+    static_assert(LAST == 16 || (LAST == 8 && NT == 1), "whole tiles, or one half tile");
+    const bool asks = LAST == 16 || row < LAST;      // whether this lane's row of the weight is the block's
+    int n0 = blockIdx.x * (LAST == 16 ? NT * 16 : LAST), m0 = blockIdx.y * MT * 16;
     const float* wp[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) wp[nt] = W + (size_t)min(n0 + nt * 16 + row, N - 1) * K + 4 * g;
-    const float* xp = A + (size_t)min(row, M - 1) * lda + 4 * g;
-    f32x4_t acc[NT];
+    const float* xp[MT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; ++mt) xp[mt] = A + (size_t)min(m0 + mt * 16 + row, M - 1) * lda + 4 * g;
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const int nkb = K / 32;
-    auto products = [&](const f32x4_t (&w)[NT][2], const f32x4_t (&x)[2]) {
+    const int rot = rot_feats > 0 ? (int)((unsigned)(n0 / rot_feats) * 37u % (unsigned)nkb) : 0;
+    auto turn = [&](int j) { int x = j + rot; return (x >= nkb ? x - nkb : x) * 32; };
+    auto products = [&](const f32x4_t (&w)[NT][2], const f32x4_t (&x)[MT][2]) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int half = 0; half < 2; ++half)
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[nt][half][j], x[half][j], acc[nt], 0, 0, 0);
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[nt][half][j], x[mt][half][j], acc[mt][nt], 0, 0, 0);
+    };
+    auto ask = [&](f32x4_t (&w)[NT][2], f32x4_t (&x)[MT][2], int k) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            if (asks) { w[nt][0] = *(const f32x4_t*)(wp[nt] + k); w[nt][1] = *(const f32x4_t*)(wp[nt] + k + 16); }
+            else w[nt][0] = w[nt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) { x[mt][0] = *(const f32x4_t*)(xp[mt] + k); x[mt][1] = *(const f32x4_t*)(xp[mt] + k + 16); }
     };
     int kb = wave;
     for (; kb + (U - 1) * NW < nkb; kb += U * NW) {
-        f32x4_t w[U][NT][2], x[U][2];
+        f32x4_t w[U][NT][2], x[U][MT][2];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            int k = (kb + u * NW) * 32;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) { w[u][nt][0] = *(const f32x4_t*)(wp[nt] + k); w[u][nt][1] = *(const f32x4_t*)(wp[nt] + k + 16); }
-            x[u][0] = *(const f32x4_t*)(xp + k);
-            x[u][1] = *(const f32x4_t*)(xp + k + 16);
-        }
+        for (int u = 0; u < U; ++u) ask(w[u], x[u], turn(kb + u * NW));
         __builtin_amdgcn_sched_barrier(0);   // keep the round's loads together, ahead of its products
 #pragma unroll
         for (int u = 0; u < U; ++u) products(w[u], x[u]);
     }
     for (; kb < nkb; kb += NW) {
-        f32x4_t w[NT][2], x[2];
-        int k = kb * 32;
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) { w[nt][0] = *(const f32x4_t*)(wp[nt] + k); w[nt][1] = *(const f32x4_t*)(wp[nt] + k + 16); }
-        x[0] = *(const f32x4_t*)(xp + k);
-        x[1] = *(const f32x4_t*)(xp + k + 16);
+        f32x4_t w[NT][2], x[MT][2];
+        ask(w, x, turn(kb));
         products(w, x);
     }
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[((wave * NT + nt) * 4 + r) * 64 + lane] = acc[nt][r];
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[(((wave * MT + mt) * NT + nt) * 4 + r) * 64 + lane] = acc[mt][nt][r];
     __syncthreads();
-    // the block's feature tiles are shared out over its waves; each is summed over the waves in order
-    for (int nt = wave; nt < NT; nt += NW) {
+    // the block's tiles are shared out over its waves; each is summed over the waves in order
+    for (int tile = wave; tile < MT * NT; tile += NW) {
+        int mt = tile / NT, nt = tile % NT;
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             float s = 0.0f;
 #pragma unroll
-            for (int w2 = 0; w2 < NW; ++w2) s += red[((w2 * NT + nt) * 4 + r) * 64 + lane];
+            for (int w2 = 0; w2 < NW; ++w2) s += red[(((w2 * MT + mt) * NT + nt) * 4 + r) * 64 + lane];
             v[r] = s;
         }
-        int m = row, n = n0 + nt * 16 + 4 * g;
-        if (m >= M) continue;
+        int m = m0 + mt * 16 + row, n = n0 + nt * 16 + 4 * g;
+        if (m >= M || (LAST < 16 && 4 * g >= LAST)) continue;
         if (epi_gated(epi)) {
 #pragma unroll
             for (int r = 0; r < 4; r += 2)
@@ -324,16 +346,45 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const float* _
     }
 }
 
-template <int NT, int NW, int U>
-static void launch_f32_skinny(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi) {
-    size_t bytes = (size_t)NW * NT * 4 * 64 * sizeof(float);
-    static_assert((size_t)NW * NT * 4 * 64 * sizeof(float) <= 64 * 1024, "the waves' sums must fit in the LDS a block may ask for");
+template <int MT, int NT, int NW, int U, int LAST = 16>
+static void launch_f32_skinny(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi, int rot_feats = 0) {
+    constexpr size_t bytes = (size_t)NW * MT * NT * 4 * 64 * sizeof(float);
+    static_assert(bytes <= 64 * 1024, "the waves' sums must fit in the LDS a block may ask for");
     static bool configured = false;
     if (!configured) {
-        (void)hipFuncSetAttribute((const void*)gemm_f32_skinny_kernel<NT, NW, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        (void)hipFuncSetAttribute((const void*)gemm_f32_skinny_kernel<MT, NT, NW, U, LAST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         configured = true;
     }
-    gemm_f32_skinny_kernel<NT, NW, U><<<ceil_div(N, NT * 16), NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi);
+    gemm_f32_skinny_kernel<MT, NT, NW, U, LAST><<<dim3(ceil_div(N, LAST == 16 ? NT * 16 : LAST), ceil_div(M, MT * 16)), NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, rot_feats);
+}
+
+// The kernel above, in the form that the product's shape asks for; false: the tiles take it.
+static bool launch_f32_few_rows(hipStream_t stream, const float* a, int lda, const float* w, void* out, int ldc, int M, int N, int K, int epi) {
+    const int cus = llmrs_compute_units();
+    if (M <= 16) {
+        // (blocks of 7 tiles with one wave a SIMD took 92 us for the 8B shape's gate/up weight: a 32-bit MFMA is long, and
+        // the wave's loads and products took turns; two waves a SIMD)
+        if (N >= 16384) {
+            if (N % 112 == 0) launch_f32_skinny<1, 7, 8, 1>(stream, a, lda, w, out, ldc, M, N, K, epi, 112);
+            else launch_f32_skinny<1, 4, 4, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
+        } else if (K < 2048) launch_f32_skinny<1, 1, 4, 4>(stream, a, lda, w, out, ldc, M, N, K, epi);
+        // a weight so narrow that whole tiles would leave half of the compute units without a block: half tiles
+        else if (2 * ceil_div(N, 16) <= cus) launch_f32_skinny<1, 1, 8, 2, 8>(stream, a, lda, w, out, ldc, M, N, K, epi);
+        // between one and two blocks a unit: blocks of two tiles, one round of them
+        else if (ceil_div(N, 16) > cus && ceil_div(N, 32) <= cus) launch_f32_skinny<1, 2, 8, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 32);
+        else launch_f32_skinny<1, 1, 8, 4>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
+        return true;
+    }
+    // More rows: blocks of 32 tokens with the fewest features that still make one round of the compute units.  Where even
+    // 64 features to a block make more, the tiles take over, but for up to 32 tokens, whose weights are read once here.
+    // (us, 32-feature-tile form / tiles: 32 rows 2048 x 8192 45 / 168, 128256 x 2048 295 / 350; 64 rows 3072 x 2048 19 / 45,
+    // 16384 x 2048 66 / 48; 100 rows 2048 x 2048 19 / 45; 200 rows 2048 x 2048 29 / 45, 3072 x 2048 58 / 46)
+    const long rows = ceil_div(M, 32);
+    if (rows * ceil_div(N, 16) <= cus) launch_f32_skinny<2, 1, 4, 4>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
+    else if (rows * ceil_div(N, 32) <= cus) launch_f32_skinny<2, 2, 4, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
+    else if (rows * ceil_div(N, 64) <= cus || M <= 32) launch_f32_skinny<2, 4, 4, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
+    else return false;
+    return true;
 }
 
 // ---- the slots of the clamped gated epilogue's constants -------------------------------------------------------------
@@ -401,20 +452,9 @@ extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda,
     LLMRS_REQUIRE(scale_sumsq == nullptr && next_y == nullptr, "gemm: a deferred norm needs the bfloat16 matrix-core kernels (M=%d N=%d K=%d)", M, N, K);
     // (one or two tokens are better off with the walk below, which then asks for little beside the weights:
     // a decode step of the 8B shape at one request 7.1 against 7.8 ms)
-    if (dtype == LLMRS_F32 && allow_mfma && M > 2 && M <= 16 && K % 32 == 0 && lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0) {
-        // (the waves per block follow the weight's shape alone, so a row's sums do not depend on the batch)
-        const float* a = (const float*)A;
-        const float* w = (const float*)W;
-        // (blocks of 7 tiles with one wave a SIMD and one k-block in flight took 92 us for the 8B shape's gate/up
-        // weight: a 32-bit MFMA is long, and the wave's loads and products took turns; two waves a SIMD, two k-blocks each)
-        int cus = llmrs_compute_units();
-        if (N >= 16384) {
-            if (N % 112 == 0) launch_f32_skinny<7, 8, 2>(stream, a, lda, w, out, ldc, M, N, K, epi);
-            else launch_f32_skinny<4, 4, 2>(stream, a, lda, w, out, ldc, M, N, K, epi);
-        } else if (K >= 2048 && (ceil_div(N, 16) <= cus || ceil_div(N, 16) > 2 * cus)) launch_f32_skinny<1, 8, 4>(stream, a, lda, w, out, ldc, M, N, K, epi);
-        // between one and two blocks a unit: blocks of four waves, two of which a unit holds side by side, make it one round
-        else if (K >= 2048) launch_f32_skinny<1, 4, 8>(stream, a, lda, w, out, ldc, M, N, K, epi);
-        else launch_f32_skinny<1, 4, 4>(stream, a, lda, w, out, ldc, M, N, K, epi);
+    if (dtype == LLMRS_F32 && allow_mfma && M > 2 && K % 32 == 0 && lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0) {
+        if (!launch_f32_few_rows(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi) &&
+            llmrs_gemm_f32_tiles(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi) != 0) return -1;
         LLMRS_LAUNCH_CHECK("gemm");
         return 0;
     }

@@ -497,6 +497,29 @@ def test_gemm_float32_few_rows_on_the_matrix_cores(M, N, K):
         assert ((outs[0] - outs[1]).abs().double() <= 2 * out_tol(ref, torch.float32, floor)).all()
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # up to 16 rows: half tiles of a narrow weight with long rows, blocks of two tiles, the walk's start staggered over few k-blocks
+    (5, 1990, 2048), (16, 2048, 2080), (16, 5000, 2048), (3, 8190, 2048), (9, 16390, 64),
+    # 17 rows and more: blocks of 32 rows and 16, 32, 64 features, at the edges of a round of the compute units
+    (17, 4096, 64), (33, 2050, 96), (31, 4100, 96), (64, 4098, 32), (64, 8190, 32), (20, 16500, 64), (250, 2040, 32),
+    # the tiles: 64 x 64 alone on a unit and more to a unit, 128 x 128; cut by M and N
+    (40, 8200, 64), (65, 8200, 32), (130, 8300, 96), (1024, 16384, 32), (1000, 16300, 64), (129, 40, 320)])
+def test_gemm_float32_forms_by_shape(M, N, K):
+    """The 32-bit product's forms where one takes over from another, every epilogue, rows with a stride, against float64
+    (the bound of `test_gemm_float32_few_rows_on_the_matrix_cores`)."""
+    a_full = rnd((M, K + 8), torch.float32, 3)
+    a = a_full[:, :K]
+    w = rnd((N, K), torch.float32, 4, 0.1)
+    acc = a.double().cpu() @ w.double().cpu().T
+    for epi in (EPI_STORE, EPI_ACCUM_F32, EPI_SWIGLU):
+        out = rnd((M, N), torch.float32, 5) if epi == EPI_ACCUM_F32 else torch.zeros((M, N // 2 if epi == EPI_SWIGLU else N), dtype=torch.float32, device=DEV)
+        ref = out.double().cpu() + acc if epi == EPI_ACCUM_F32 else plain_silu(acc[:, 0::2]) * acc[:, 1::2] if epi == EPI_SWIGLU else acc
+        kernels().gemm(a, w, out, epi)
+        err = (out.double().cpu() - ref).abs()
+        floor = 2e-6 * math.sqrt(K) * (1 + 0.1 * math.sqrt(K) if epi == EPI_SWIGLU else 1)
+        assert (err <= out_tol(ref, torch.float32, floor)).all(), (epi, float(err.max()))
+
+
 def test_attention_chunk_rule_and_its_scratch():
     """The keys per wave that the split takes: a power of two from 64 to 1024 whatever the host says about the
     keys; never under what the scratch is sized by (the answer for one key); and the same results whichever chunk
