@@ -204,25 +204,34 @@ __global__ __launch_bounds__(256) void attn_f32_tiles_kernel(const float* __rest
         }
 }
 
-// Entries with one token: a wave for each (entry, kv head, chunk of F32_SPLIT_CHUNK keys, aligned to absolute positions):
+// Entries with one token: a block for each (entry, kv head, chunk of F32_SPLIT_CHUNK keys, aligned to absolute positions):
 // its columns are the heads of the kv head (the other columns of the 32 multiply zeros: the keys and values are read
-// once for all of them, 16 bytes a lane, which is what this step is bound by).  It leaves what the walk of
+// once for all of them, 16 bytes a lane).  It leaves what the walk of
 // attention_generic.hip leaves for such a chunk, where that file's merge finds it: the maximum (natural logarithm's
 // scale), the sum and the weighted values of each head, [entry][head][chunk][2 + head_dim].
-template <int HD, int MAPS>
-__global__ __launch_bounds__(64) void attn_f32_split_kernel(const float* __restrict__ q, float* __restrict__ partial,
+// WAVES 4: each wave takes 32 of the chunk's keys, and the waves' results are added in order through LDS.  What bounds this
+// step is neither bytes nor products but a wave's chain (a trip to memory, then 64 to 256 MFMAs of 64 cycles, for every 32 keys
+// one after the other): four waves side by side take a quarter of it.  (8 requests of 200 to 1800 keys, 8 kv heads of 64:
+// 22.2 -> 19.0 us; of 200 to 1000 keys, 4 kv heads of 128 with two maps: 32 -> 14.)  WAVES 1, one wave for all of the chunk's keys: where the columns' sums would not fit in LDS
+// (attn_f32_split_waves).
+static inline __host__ __device__ bool attn_f32_split_waves(int columns, int hd) { return columns * hd <= 2048; }
+template <int HD, int MAPS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_f32_split_kernel(const float* __restrict__ q, float* __restrict__ partial,
                                                             const float* __restrict__ kc, const float* __restrict__ vc,
                                                             const int* __restrict__ block_table,
                                                             const int* __restrict__ q_starts, const int* __restrict__ seq_lens,
                                                             int max_chunks, AttnArgs a, int G) {
-    int lane = threadIdx.x, c = lane & 31, h = lane >> 5;
-    int e = blockIdx.x, kvh = blockIdx.y, ch = blockIdx.z;
+    static_assert(WAVES == 1 || WAVES * 32 == F32_SPLIT_CHUNK, "a wave for every 32 keys of a chunk, or one for all");
+    __shared__ float others[WAVES > 1 ? (WAVES - 1) * 2048 : 1];              // [wave - 1][column][HD]
+    __shared__ float stats[WAVES][32][2];                                      // [wave][column]: maximum (base 2), sum
+    int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
+    int kvh = blockIdx.x, ch = blockIdx.y, e = blockIdx.z;
     int token = q_starts[e];
     if (q_starts[e + 1] - token != 1) return;
     int pos_t = seq_lens[e] - 1;                  // an entry with one token: its position is its length less one
     int lo = attn_window_lo(a, pos_t);
     int first = lo / F32_SPLIT_CHUNK;
-    if (ch > pos_t / F32_SPLIT_CHUNK - first) return;
+    if (ch > pos_t / F32_SPLIT_CHUNK - first) return;                         // (the same for all of a block's waves)
     int begin = max(lo, (first + ch) * F32_SPLIT_CHUNK), end = min(pos_t + 1, (first + ch + 1) * F32_SPLIT_CHUNK);
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS;         // (G: columns of a kv head; see the partial results' layout)
@@ -237,9 +246,52 @@ __global__ __launch_bounds__(64) void attn_f32_split_kernel(const float* __restr
         for (int i = 0; i < 16; ++i) O[dt][i] = 0.0f;
     float m = -INFINITY, l = 0.0f;
     const AttnFar far = attn_far_base2(a, head);
-    if (ch == 0 && a.keep_first > 0 && (begin & ~31) > 0)      // the first chunk's wave also takes the kept first keys
+    if (wave == 0 && ch == 0 && a.keep_first > 0 && (begin & ~31) > 0)      // the first chunk's (first) wave also takes the kept first keys
         f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, 0, min(a.keep_first, begin & ~31), O, m, l);
-    f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, begin & ~31, end, O, m, l);
+    if constexpr (WAVES == 1) f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, begin & ~31, end, O, m, l);
+    else {
+        int from = (first + ch) * F32_SPLIT_CHUNK + 32 * wave;
+        f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, max(from, begin & ~31), min(from + 32, end), O, m, l);
+        // this lane holds features dt * 32 + 8 g + 4 h + j of its column
+        if (h == 0) { stats[wave][c][0] = m; stats[wave][c][1] = l; }
+        if (wave > 0 && cvalid) {
+            float* mine = others + (size_t)(wave - 1) * 2048 + c * HD;
+#pragma unroll
+            for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *(f32x4*)(mine + dt * 32 + 8 * g + 4 * h) = f32x4{O[dt][4 * g], O[dt][4 * g + 1], O[dt][4 * g + 2], O[dt][4 * g + 3]};
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        float top = m, part[WAVES];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) top = fmaxf(top, stats[w][c][0]);
+        const float safe = top == -INFINITY ? 0.0f : top;                     // (a column that saw no key at all)
+        l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            part[w] = __builtin_amdgcn_exp2f(stats[w][c][0] - safe);            // (-inf - x: 0)
+            l = fmaf(stats[w][c][1], part[w], l);
+        }
+        m = top;
+        if (cvalid)
+#pragma unroll
+            for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    f32x4 v[WAVES - 1];
+#pragma unroll
+                    for (int w = 1; w < WAVES; ++w) v[w - 1] = *(const f32x4*)(others + (size_t)(w - 1) * 2048 + c * HD + dt * 32 + 8 * g + 4 * h);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float o = O[dt][4 * g + j] * part[0];
+#pragma unroll
+                        for (int w = 1; w < WAVES; ++w) o = fmaf(v[w - 1][j], part[w], o);
+                        O[dt][4 * g + j] = o;
+                    }
+                }
+    }
     if (!cvalid) return;
     float* pp = partial + ((size_t)(e * a.n_heads * MAPS + column) * max_chunks + ch) * (HD + 2);
     if (h == 0) { pp[0] = m * 0.69314718055994531f; pp[1] = l; }
@@ -297,10 +349,11 @@ int llmrs_attention_f32_mfma_split(hipStream_t stream, const float* q, float* pa
     if (a.q_stride % 4 || ((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)partial & 7))
         return 0;
     if (n_entries > 65535 || a.n_kv_heads > 65535 || max_chunks > 65535 || max_chunks < 1) return 0;
-    dim3 grid(n_entries, a.n_kv_heads, max_chunks);
+    dim3 grid(a.n_kv_heads, max_chunks, n_entries);      // (blocks go to the XCDs in turn: what all entries share alike comes first)
     switch (a.head_dim) {
-#define SPLIT(HD, MM) attn_f32_split_kernel<HD, MM><<<grid, 64, 0, stream>>>(q, partial, k_cache, v_cache, block_table, q_starts, seq_lens, max_chunks, a, G)
-#define CASE(HD) case HD: if (a.maps == 2) SPLIT(HD, 2); else SPLIT(HD, 1); break;
+#define SPLIT(HD, MM, WW) attn_f32_split_kernel<HD, MM, WW><<<grid, 64 * WW, 0, stream>>>(q, partial, k_cache, v_cache, block_table, q_starts, seq_lens, max_chunks, a, G)
+#define CASE(HD) case HD: if (attn_f32_split_waves(G, HD)) { if (a.maps == 2) SPLIT(HD, 2, 4); else SPLIT(HD, 1, 4); } \
+                          else { if (a.maps == 2) SPLIT(HD, 2, 1); else SPLIT(HD, 1, 1); } break;
         CASE(32) CASE(64) CASE(96) CASE(128) CASE(160) CASE(192) CASE(224) CASE(256)
 #undef CASE
 #undef SPLIT

@@ -661,7 +661,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 3
                                                         const int* __restrict__ seq_lens,
                                                         const int* __restrict__ q_starts, AttnArgs a, int G,
                                                         int max_chunks, int chunk, int plain) {
-    int e = blockIdx.x, kvh = blockIdx.y, ch = blockIdx.z;
+    int kvh = blockIdx.x, ch = blockIdx.y, e = blockIdx.z;
     int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -759,7 +759,7 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
                                                           const int* __restrict__ q_starts, AttnArgs a, int G,
                                                           int max_chunks, int chunk, int plain) {
     static_assert(KD % 32 == 0 && VD % 16 == 0, "the score products take 32 features at a time");
-    int e = blockIdx.x, kvh = blockIdx.y, ch = blockIdx.z;
+    int kvh = blockIdx.x, ch = blockIdx.y, e = blockIdx.z;
     int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -1246,7 +1246,10 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
         }
     }
     if (split) {
-        dim3 grid(n_entries, a.n_kv_heads, max_chunks);
+        // Blocks go to the eight XCDs in turn, so the grid's first dimension is one that all entries share alike: with the
+        // entries there, each XCD had every eighth entry whole, and one with a longer cache than the others kept its
+        // XCD busy alone (64 requests of 509 to 3585 keys: 114 -> 113 us; 160 of 128 to 4096, heads of 64: 158 -> 154).
+        dim3 grid(a.n_kv_heads, max_chunks, n_entries);
         int plain = only_single && attn_reach(a) == 0;
         if (G <= 16)
             attn_split16_kernel<KD, VD, MAPS><<<grid, 64, SPLIT16_LDS_BYTES, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain);
