@@ -968,7 +968,7 @@ static int launch_pingpong(hipStream_t stream, const bf16* A, int lda, const bf1
 }
 
 // ---------------------------------------------------------------------------
-// tiled, four waves: for K % 64 == 0, tiles of 256 x 256.
+// tiled, four waves: for K % 64 == 0, tiles of 256 x 256, 256 x 192 and 256 x 128.
 // One wave per SIMD with a tile of 128 x 128 outputs, all of them in the accumulation registers (256 of them):
 // a third fewer LDS reads per MFMA than the eight-wave tiles, and nothing shares the SIMD with the wave, so the
 // loop is written so that the wave itself always has work in flight.  A k-tile of 64 is four steps of 16; each
@@ -980,8 +980,9 @@ static int launch_pingpong(hipStream_t stream, const bf16* A, int lda, const bf1
 // registers read before it: the matrix cores work across the barrier.  Same LDS layout and order of sums as the
 // loops above: bitwise the same results.  The epilogue is a template argument: with all of them in one kernel the
 // compiler keeps a tile's 256 sums and every epilogue's temporaries alive together and spills.
-// (Measured on MI355X, 2048 x 4096 times 24576 features with the gate/up epilogue, inside a prompt step of the 8B
-// shape: 356 us against 372-376 for the eight waves in two groups and 367 with loads straight into LDS.)
+// (Measured on MI355X, 2048 x 4096 times 24576 features with the gate/up epilogue: 320 us, 1.29 PFLOP/s; the
+// eight waves in two groups 372-376.  The clock follows the power that the matrix cores draw: their MFMAs alone, on
+// random operands, would take 241.)
 // ---------------------------------------------------------------------------
 // What a wave of the four-wave tile does with its sums: one band of 32 rows at a time.  16-bit results go through
 // the wave's own part of LDS and leave as whole rows of the band, 16 bytes a lane; the 32-bit epilogues read and
@@ -1056,6 +1057,23 @@ __device__ __forceinline__ void band_epilogue(f32x16 (&acc)[BM / 64][BN / 64], u
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// A quarter of a wave's loads of a k-tile: of `groups` loads those from first_of(groups, q) up to first_of(groups, q + 1).
+constexpr int first_of(int groups, int q) { return q * groups / 4; }
+constexpr int quarter_of(int groups, int q) { return first_of(groups, q + 1) - first_of(groups, q); }
+
+// Which tile of the output a block works on.  Blocks go to the eight XCDs in turn; here an XCD gets a stretch of the tiles
+// that lie one after the other, eight rows of tiles at a time, column after column, so that the 32 blocks its units run at
+// once are eight rows of four columns: each brings its rows of the weight into one L2, once, and shares them with seven
+// others.  (Column after column over all XCDs, a grid of 224 columns gave an XCD 28 of them at once, each for one
+// block: 2048 x 8192 times 57344 features 1773 -> 1473 us, 24576 x 4096 the same.)
+__device__ __forceinline__ void tile_of_block(int& row, int& column) {
+    int columns = gridDim.x, rows = gridDim.y, id = blockIdx.y * columns + blockIdx.x, share = columns * rows / 8;
+    if (id < 8 * share) id = (id & 7) * share + (id >> 3);         // (what is left over when they do not divide by eight: as it comes)
+    int band = id / (8 * columns), within = id - band * 8 * columns, high = min(8, rows - 8 * band);
+    row = 8 * band + within % high;
+    column = within / high;
+}
+
 template <int BM, int BN, int EPI>
 __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
                                                             void* __restrict__ out, int ldc, int M, int N, int K, int epi) {
@@ -1064,13 +1082,13 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 32, FN = TN / 32;
     constexpr int STAGE_BYTES = (BM + BN) * 128;
     constexpr int A_GROUPS = BM / 8 / WAVES, W_GROUPS = BN / 8 / WAVES;   // 8-row groups per wave
-    constexpr int QA = A_GROUPS / 4, QW = W_GROUPS / 4, QL = QA + QW;     // a quarter of a wave's loads of a k-tile
     static_assert(BM == 256 && BN % 64 == 0 && FM * FN <= 16, "a wave's sums fill at most the 256 accumulation registers");
-    static_assert(A_GROUPS % 4 == 0 && W_GROUPS % 4 == 0, "a quarter of a k-tile's loads in each of its four steps");
     static_assert(32 * TN * 2 * WAVES <= 2 * STAGE_BYTES, "the waves' bands must fit in the tile buffers");
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int wm = wave / 2, wn = wave % 2;
-    int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    int tile_row, tile_column;
+    tile_of_block(tile_row, tile_column);
+    int m0 = tile_row * BM, n0 = tile_column * BN;
     int lrow = lane >> 3, lslot = lane & 7;
     // this lane's part of a tile: for each of its row groups, the byte offset of the chunk that belongs in the lane's
     // slot of the LDS image (the caller sees to it that both operands are under 4 GB: buffer descriptors)
@@ -1097,9 +1115,9 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         kt = min(kt, nk - 1);
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-        for (int i = q * QA; i < (q + 1) * QA; ++i) sa[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, oa[i], kt * 128, 0);
+        for (int i = first_of(A_GROUPS, q); i < first_of(A_GROUPS, q + 1); ++i) sa[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, oa[i], kt * 128, 0);
 #pragma unroll
-        for (int i = q * QW; i < (q + 1) * QW; ++i) sw_[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, ow[i], kt * 128, 0);
+        for (int i = first_of(W_GROUPS, q); i < first_of(W_GROUPS, q + 1); ++i) sw_[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, ow[i], kt * 128, 0);
 #endif
     };
     // quarter q of the registers into the LDS buffer of k-tile kt: a load's 64 lanes fill 1 KB in lane order
@@ -1107,9 +1125,9 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         constexpr int q = decltype(qc)::value;
         unsigned char* st = fw_smem + (kt & 1) * STAGE_BYTES;
 #pragma unroll
-        for (int i = q * QA; i < (q + 1) * QA; ++i) *(u32x4*)(st + (wave * A_GROUPS + i) * 1024 + lane * 16) = sa[i];
+        for (int i = first_of(A_GROUPS, q); i < first_of(A_GROUPS, q + 1); ++i) *(u32x4*)(st + (wave * A_GROUPS + i) * 1024 + lane * 16) = sa[i];
 #pragma unroll
-        for (int i = q * QW; i < (q + 1) * QW; ++i) *(u32x4*)(st + BM * 128 + (wave * W_GROUPS + i) * 1024 + lane * 16) = sw_[i];
+        for (int i = first_of(W_GROUPS, q); i < first_of(W_GROUPS, q + 1); ++i) *(u32x4*)(st + BM * 128 + (wave * W_GROUPS + i) * 1024 + lane * 16) = sw_[i];
     };
     f32x16 acc[FM][FN];
 #pragma unroll
@@ -1145,26 +1163,38 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
             for (int j = 0; j < FN; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[buf][i], fb[buf][j], acc[i][j], 0, 0, 0);
     };
-    // the order within a step: LDS reads, LDS writes and loads from memory each ahead of a group of the step's MFMAs
-    auto order = [] {
-        __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        __builtin_amdgcn_sched_group_barrier(0x200, QL, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        __builtin_amdgcn_sched_group_barrier(0x020, QL, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, FM * FN - 8, 0);
+    // The order within a step.  A SIMD has this one wave only, so whatever keeps it from issuing its next MFMA leaves the matrix
+    // cores idle: four loads asked for back to back wait for each other and the other waves' at the address unit (16 cycles
+    // each, 16 of them between the four waves) while an MFMA takes 32.  So LDS reads go out in pairs, and every LDS write
+    // and every load from memory by itself, with an MFMA after each.  Measured (2048 rows, back to back, before: all reads, 4
+    // MFMAs, all writes, 4 MFMAs, all loads): 24576 x 4096 350 -> 320 us, 4096 x 14336 232 -> 212, 4096 x 4096 77 -> 70;
+    // reads singly 331, in fours 324, writes and loads of a quarter as groups 331, loads first 357.
+    auto order = [](auto qc) {
+        constexpr int q = decltype(qc)::value, LOADS = quarter_of(A_GROUPS, q) + quarter_of(W_GROUPS, q);
+        static_for<0, (FM + FN) / 2>([](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        });
+        static_for<0, LOADS>([](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        });
+        __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);
     };
     // One step (a quarter of a k-tile).  While k-tile kt is multiplied, k-tile kt + 1 goes from registers into the
     // other LDS buffer and k-tile kt + 2 is asked for into the registers that frees.  A quarter written now was
-    // asked for a k-tile ago; loads complete in order, so it is there when all but the three quarters asked for
-    // since have completed.
+    // asked for a k-tile ago; loads complete in order, so it is there when all but the three other quarters, asked for
+    // since, have completed.
     auto step = [&](int kt, auto ksc, auto qc, auto rbuf, auto mbuf, auto multiply) {
         read(kt, ksc, rbuf);
-        wait_vmcnt<3 * QL>();
+        constexpr int q = decltype(qc)::value, others = A_GROUPS + W_GROUPS - quarter_of(A_GROUPS, q) - quarter_of(W_GROUPS, q);
+        wait_vmcnt<others>();
         put(kt + 1, qc);
         ask(kt + 2, qc);
         if constexpr (decltype(multiply)::value) mult(mbuf);
-        order();
+        order(qc);
         __builtin_amdgcn_sched_barrier(0);
     };
     using I0 = std::integral_constant<int, 0>;
@@ -1511,8 +1541,9 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             } else if (long t192 = m_tiles * ceil_div(N, 192); rest > 0 && t192 % cus == 0) {
                 // 256 x 192 tiles where they come to whole rounds of the device and the square ones do not: the
                 // q/k/v product of the 8B shape at 2048 rows is 192 square tiles on 256 units, or 256 of these
-                // (eight waves of 64 x 96: in a prompt step 103 us, against 107 for four waves of 128 x 96)
-                rc = small ? launch_pingpong<256, 192, 4, 2, true>(stream, A, lda, W, out, ldc, M, N, K, epi)
+                // (four waves of 128 x 96: 87 us, against 100 for the eight waves of 64 x 96)
+                rc = four ? launch_fourwave<256, 192>(stream, A, lda, W, out, ldc, M, N, K, epi)
+                   : small ? launch_pingpong<256, 192, 4, 2, true>(stream, A, lda, W, out, ldc, M, N, K, epi)
                            : launch_pingpong<256, 192, 4, 2, false>(stream, A, lda, W, out, ldc, M, N, K, epi);
             } else {
                 rc = four ? launch_fourwave<256, 256>(stream, A, lda, W, out, ldc, M, N, K, epi)

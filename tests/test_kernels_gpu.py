@@ -520,6 +520,21 @@ def test_gemm_float32_forms_by_shape(M, N, K):
         assert (err <= out_tol(ref, torch.float32, floor)).all(), (epi, float(err.max()))
 
 
+@pytest.mark.parametrize("M,N,K", [(2200, 6144, 64), (2816, 4352, 64), (4700, 8200, 64), (2048, 6160, 192), (1800, 6136, 64)])
+def test_gemm_large_tiles_of_many_rows(M, N, K):
+    """Grids of large tiles with more rows than an XCD takes at a time, numbers of tiles that eight does not divide, and 256 x 192
+    tiles cut by N: every tile of the output is written, once (a += shows a tile written twice)."""
+    a, w = rnd((M, K), torch.bfloat16, 3), rnd((N, K), torch.bfloat16, 4, 0.1)
+    acc = a.double().cpu() @ w.double().cpu().T
+    for epi in (EPI_STORE_F32, EPI_ACCUM_F32):
+        out = torch.zeros((M, N), dtype=torch.float32, device=DEV) if epi == EPI_STORE_F32 else rnd((M, N), torch.float32, 5)
+        ref = acc if epi == EPI_STORE_F32 else out.double().cpu() + acc
+        n_ws = kernels().gemm_workspace_floats(M, N, K)
+        kernels().gemm(a, w, out, epi, torch.empty(n_ws, dtype=torch.float32, device=DEV) if n_ws else None)
+        err = (out.double().cpu() - ref).abs()
+        assert (err <= out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))).all(), (epi, float(err.max()))
+
+
 def test_attention_chunk_rule_and_its_scratch():
     """The keys per wave that the split takes: a power of two from 64 to 1024 whatever the host says about the
     keys; never under what the scratch is sized by (the answer for one key); and the same results whichever chunk
