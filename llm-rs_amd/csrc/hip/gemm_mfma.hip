@@ -1103,7 +1103,17 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         int row = (wave * W_GROUPS + i) * 8 + lrow;
         ow[i] = (unsigned)(((size_t)min(n0 + row, N - 1) * K + ((lslot ^ ((row >> 1) & 7)) * 8)) * 2);
     }
-    const int nk = K / 64;
+    // With gridDim.z > 1 (the epilogue then is STORE_F32, `out` the partial sums [gridDim.z][M][N]) a block takes its share of
+    // the k-tiles, a contiguous range; no share is empty (the launcher sees to it).
+    const int share = (K / 64 + gridDim.z - 1) / gridDim.z, k_first = blockIdx.z * share;
+    const int nk = min(share, K / 64 - k_first);
+    if (gridDim.z > 1) {
+        out = (float*)out + (size_t)blockIdx.z * M * N;
+#pragma unroll
+        for (int i = 0; i < A_GROUPS; ++i) oa[i] += k_first * 128;
+#pragma unroll
+        for (int i = 0; i < W_GROUPS; ++i) ow[i] += k_first * 128;
+    }
 #if defined(__HIP_DEVICE_COMPILE__)
     __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)min((size_t)M * lda * 2, (size_t)0xffffffffu), 0x00020000);
     __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)min((size_t)N * K * 2, (size_t)0xffffffffu), 0x00020000);
@@ -1233,7 +1243,7 @@ static bool fourwave_takes(int epi, const void* out, int ldc, int N) {
     return false;
 }
 template <int BM, int BN, int EPI>
-static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi) {
+static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1) {
     static bool configured = false;
     size_t bytes = (size_t)2 * (BM + BN) * 128;
     if (!configured) {
@@ -1242,7 +1252,7 @@ static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const
         if (e != hipSuccess) return llmrs_fail("gemm: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
         configured = true;
     }
-    dim3 grid(ceil_div(N, BN), ceil_div(M, BM));
+    dim3 grid(ceil_div(N, BN), ceil_div(M, BM), splits);
     if (grid.y > 65535) return llmrs_fail("gemm: M=%d is too large for one launch", M);
     gemm_fourwave_kernel<BM, BN, EPI><<<grid, 256, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi);
     return 0;
@@ -1296,6 +1306,28 @@ static int launch_tiles_128(hipStream_t stream, const bf16* A, int lda, const bf
     if (deep_tiles(M, N, K)) return launch_dma<128, 128, 2, 4, 4>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, partial, next, finish);
     return launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, partial, next, finish);
 }
+// From 512 rows on, where square large tiles would not fill the device: tiles of 256 x 128 on four waves, a block to a unit, or
+// the 128 x 128 tiles above, two to a unit, by the time either takes: the k-tiles that a unit works through, round after
+// round, times what one takes there (measured: 1.0 us for a 256 x 128 k-tile of 64, 1.25 for two of 128 x 128, 1.05 for
+// one that is alone).  Both split k over blocks until the device is full.  Measured, 128 x 128 -> 256 x 128: 2032 rows
+// 2048 x 8192 in 2 parts 81 -> 71 us, 3072 x 2048 35 -> 29; 1024 rows 4096 x 14336 in 2 parts 140 -> 111; 512 rows in 4
+// parts 78 -> 64.  (The two operands' sizes, under 4 GB, are looked at where it is launched.)
+struct MidTiles {
+    bool four;
+    int splits;
+};
+static MidTiles mid_tiles(int M, int N, int K, bool may_split = true) {
+    if (M < 512 || K % 64) return MidTiles{false, may_split ? tiled_splits(M, N, K) : 1};
+    const int cus = llmrs_compute_units(), nk = K / 64;
+    const long tall = (long)ceil_div(M, 256) * ceil_div(N, 128), small = (long)ceil_div(M, 128) * ceil_div(N, 128);
+    int z = 1;
+    while (may_split && tall * z * 2 <= cus && z < 16 && nk / (z * 2) >= 8 && (z * 2 - 1) * ceil_div(nk, z * 2) < nk) z *= 2;
+    const int s = may_split ? tiled_splits(M, N, K) : 1;
+    const double tall_time = (double)ceil_div(tall * z, (long)cus) * ceil_div(nk, z);
+    const double small_time = (small * s <= cus ? 1.05 : 1.25 * ceil_div(small * s, 2L * cus)) * ceil_div(nk, s);
+    if (tall_time <= small_time) return MidTiles{true, z};
+    return MidTiles{false, s};
+}
 // 17..64 rows on a weight of middling width (more than 4096 features, fewer than the wide ones that
 // get blocks of many feature tiles): the 128 x 128 tiles with k split over blocks read the tokens'
 // rows less often than the few-row kernel's blocks of 32 features (measured at 64 rows:
@@ -1315,7 +1347,7 @@ extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
         return s > 1 ? (long)s * (M % 256) * N : 0;
     }
     if (M > 64 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160) {
-        int s = tiled_splits(M, N, K);
+        int s = mid_tiles(M, N, K).splits;
         long own = s > 1 ? (long)s * M * N : 0;
         // a few rows beyond whole 128-row tiles may go to the kernel for few rows, and the whole tiles be split then
         int over128 = M % 128;
@@ -1353,7 +1385,7 @@ extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
 extern "C" int llmrs_gemm_norms_whole(int M, int N, int K) {
     if (!(M > 16 && N >= 4 && N % 4 == 0 && N <= 16384 && K % 8 == 0)) return 0;
     if (M <= 256) return llmrs_gemm_workspace_floats(M, N, K) > 0;
-    return K % 64 == 0 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160 && tiled_splits(M, N, K) > 1;
+    return K % 64 == 0 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160 && mid_tiles(M, N, K).splits > 1;
 }
 
 // The product as parts of its sum over k, [parts][M][N] 32-bit in `workspace`, for a caller that adds them up itself
@@ -1531,9 +1563,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                      : small ? launch_pingpong<256, 256, 2, 4, true>(stream, A, lda, W, out, ldc, M, n_split, K, epi)
                              : launch_pingpong<256, 256, 2, 4, false>(stream, A, lda, W, out, ldc, M, n_split, K, epi);
                 if (rc == 0) {
-                    long wide_rest = m_tiles * ceil_div(N - n_split, 128);      // (256 x 128 tiles where they come to whole rounds, as below)
-                    if (four && M >= 1024 && fourwave_takes(epi, out_rest, ldc, N - n_split) &&
-                        10 * wide_rest >= 9 * (long)ceil_div(wide_rest, (long)cus) * cus)
+                    if (four && fourwave_takes(epi, out_rest, ldc, N - n_split) && mid_tiles(M, N - n_split, K, false).four)
                         rc = launch_fourwave<256, 128>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
                     else
                         rc = launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
@@ -1558,7 +1588,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             int over128 = M % 128;
             if (M >= 1024 && over128 > 0 && over128 <= 64 && !whole && next == nullptr && scale == nullptr) {
                 auto walk = [&](int rows) {
-                    int s = tiled_splits(rows, N, K);
+                    int s = mid_tiles(rows, N, K).splits;
                     if (s > 1 && (workspace == nullptr || workspace_bytes < (size_t)s * rows * N * sizeof(float))) s = 1;
                     long blocks = (long)ceil_div(rows, 128) * ceil_div(N, 128) * s;
                     return ceil_div(blocks, (long)cus * 2) * (K / 64 / s);
@@ -1572,17 +1602,18 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                                                 ldc, over128, N, K, epi, workspace, workspace_bytes, qkv);
                 }
             }
-            int splits = tiled_splits(M, N, K);
-            // Many rows on a weight too narrow for the square tiles: four waves on 256 x 128 (128 x 64 a wave, a block
-            // to a unit) where such tiles come to whole rounds of the device, or nearly: a k-step brings 48 KB into a
-            // unit for the work that two 128 x 128 blocks bring 64 KB for (the o and down products of the 8B shape at
-            // 2048 rows: a prompt step 31.55 -> 31.03 ms).
-            long wide_blocks = (long)ceil_div(M, 256) * ceil_div(N, 128);
+            // (a wider tile brings less into a unit for the same work: a k-step of 256 x 128 48 KB, of two 128 x 128 64 KB)
             const bool small4 = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
-            if (splits == 1 && !whole && next == nullptr && M >= 1024 && small4 && fourwave_takes(epi, out, ldc, N) &&
-                10 * wide_blocks >= 9 * (long)ceil_div(wide_blocks, (long)cus) * cus)
+            MidTiles plan = mid_tiles(M, N, K);
+            if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)))
+                plan = mid_tiles(M, N, K, false);
+            const int splits = plan.splits;
+            if (plan.four && small4 && splits > 1) {
+                rc = launch_fourwave_epi<256, 128, LLMRS_EPI_STORE_F32>(stream, A, lda, W, workspace, N, M, N, K, LLMRS_EPI_STORE_F32, splits);
+                if (rc == 0) launch_splitk_finish(stream, (const float*)workspace, splits, out, ldc, M, N, epi, next);
+            } else if (plan.four && small4 && !whole && next == nullptr && fourwave_takes(epi, out, ldc, N))
                 rc = launch_fourwave<256, 128>(stream, A, lda, W, out, ldc, M, N, K, epi);
-            else if (splits > 1 && workspace != nullptr && workspace_bytes >= (size_t)splits * M * N * sizeof(float))
+            else if (splits > 1)
                 rc = launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, splits, (float*)workspace, next);
             else if (whole) rc = llmrs_fail("gemm: M=%d N=%d K=%d is not split after all: the norm cannot be finished here", M, N, K);
             else

@@ -535,6 +535,30 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
         assert (err <= out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))).all(), (epi, float(err.max()))
 
 
+@pytest.mark.parametrize("M,N,K", [(512, 4096, 1024), (600, 4100, 1088), (1030, 2048, 2048), (530, 1000, 4160), (512, 130, 8256), (2032, 3072, 192),
+                                   (700, 16, 1024)])
+def test_gemm_tall_tiles_split_over_k(M, N, K):
+    """512 rows and more on a weight too narrow for square tiles: 256 x 128 tiles, k in parts of unequal length, with and without
+    the norm that follows, and without the room for parts."""
+    from llm_rs_amd.kernels import NextNorm
+    k = kernels()
+    a, w, h = rnd((M, K), torch.bfloat16, 3), rnd((N, K), torch.bfloat16, 4, 0.1), rnd((M, N), torch.float32, 5)
+    ref = h.double().cpu() + a.double().cpu() @ w.double().cpu().T
+    n_ws = k.gemm_workspace_floats(M, N, K)
+    tol = out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))
+    for room in ([True, False] if n_ws else [False]):
+        out = h.clone()
+        k.gemm(a, w, out, EPI_ACCUM_F32, torch.full((n_ws,), 7.0, dtype=torch.float32, device=DEV) if room else None)
+        assert ((out.double().cpu() - ref).abs() <= tol).all()
+    if k.gemm_norms_whole(M, N, K):
+        nw, y = rnd((N,), torch.float32, 6) * 0.1 + 1, torch.zeros((M, N), dtype=torch.bfloat16, device=DEV)
+        out = h.clone()
+        k.gemm(a, w, out, EPI_ACCUM_F32, torch.empty(n_ws, dtype=torch.float32, device=DEV), leave=NextNorm(y, None, nw, 1e-5))
+        assert ((out.double().cpu() - ref).abs() <= tol).all()
+        want = ref / torch.sqrt((ref * ref).mean(-1, keepdim=True) + 1e-5) * nw.double().cpu()
+        assert ((y.double().cpu() - want).abs() <= out_tol(want, torch.bfloat16, 1e-4)).all()
+
+
 def test_attention_chunk_rule_and_its_scratch():
     """The keys per wave that the split takes: a power of two from 64 to 1024 whatever the host says about the
     keys; never under what the scratch is sized by (the answer for one key); and the same results whichever chunk
