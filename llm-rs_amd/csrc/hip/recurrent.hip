@@ -382,6 +382,41 @@ __global__ __launch_bounds__(64) void selective_scan_kernel(const T* __restrict_
     }
 }
 
+// A step in which every entry brings one token (token e is entry e's): the scan above with nothing to walk.  All that a
+// thread needs is asked for at once, where the walk asks for the state, then for the B and C rows through LDS and
+// behind a barrier for the token's inputs.  Same sums in the same order.  (Before, 4 entries of 4096 channels, 16 states: 11.2 us.)
+template <class T, int NS>
+__global__ __launch_bounds__(64) void selective_step_kernel(const T* __restrict__ x, int ldx, const T* __restrict__ bc, int ldbc, int off_b,
+                                                            int off_c, const int* __restrict__ slots, T* __restrict__ out, int ldo, ScanArgs a) {
+    const int c = blockIdx.x * 64 + threadIdx.x, e = blockIdx.y;
+    if (c >= a.C) return;
+    const T* row = bc + (size_t)e * ldbc;
+    const float vdt = a.dt[(size_t)e * a.ld_dt + c] + (a.dt_bias ? a.dt_bias[c] : 0.0f), xv = to_f32(x[(size_t)e * ldx + c]);
+    const float vg = a.gate[(size_t)e * a.ld_gate + c], Dc = a.D[c];
+    float Ac[NS], B[NS], Cs[NS], S[NS];
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+        const int m = min(n, a.N - 1);
+        Ac[n] = a.A[(size_t)m * a.C + c];
+        B[n] = to_f32(row[off_b + m]);
+        Cs[n] = to_f32(row[off_c + m]);
+    }
+    float* sp = a.state + (size_t)slots[e] * a.state_stride + c;           // state n of this channel: sp[n * C]
+#pragma unroll
+    for (int n = 0; n < NS; ++n) S[n] = sp[(size_t)min(n, a.N - 1) * a.C];
+    const float step = softplus_f32(vdt), sx = step * xv;
+    float y = 0.0f;
+#pragma unroll
+    for (int n = 0; n < NS; ++n)
+        if (n < a.N) {
+            S[n] = fmaf(__builtin_amdgcn_exp2f(step * (Ac[n] * LOG2_E)), S[n], sx * B[n]);
+            y = fmaf(S[n], Cs[n], y);
+            sp[(size_t)n * a.C] = S[n];
+        }
+    y = fmaf(Dc, xv, y);
+    out[(size_t)e * ldo + c] = from_f32<T>(y * silu_f32(vg));
+}
+
 // One thread for each (entry, state, channel): what the chunks left becomes what each starts from.  Over a chunk
 // the decays multiply to exp(A[c, n] * the sum of its step sizes).  What SCAN_LOADS chunks left is fetched together.
 __global__ void selective_scan_carry_kernel(const int* __restrict__ q_starts, const int* __restrict__ slots, ScanArgs a) {
@@ -530,7 +565,7 @@ extern "C" int llmrs_conv_state_update(hipStream_t stream, const float* sums, in
 
 // x: [T, ldx] the convolution's output; bc: [T, ldbc] with B at column off_b and C at off_c, N wide each; both and
 // `out` in `dtype`.  ypart: [T, C] 32-bit, needed only when N > 64.  longest: the most tokens any entry brings (an
-// upper bound will do).  carry: [llmrs_scan_places][N + 1][C] floats, or null; with it, entries longer than a chunk
+// upper bound will do; 1 with as many tokens as entries: every entry brings one).  carry: [llmrs_scan_places][N + 1][C] floats, or null; with it, entries longer than a chunk
 // run in chunks.
 extern "C" int llmrs_selective_scan(hipStream_t stream, int dtype, const void* x, int ldx, const void* bc, int ldbc, int off_b,
                                     int off_c, const float* dt, int ld_dt, const float* dt_bias, const float* A, const float* D,
@@ -549,6 +584,15 @@ extern "C" int llmrs_selective_scan(hipStream_t stream, int dtype, const void* x
     // (the sums of the step sizes lie behind the states the chunks carry)
     ScanArgs a{dt, ld_dt, dt_bias, A, D, gate, ld_gate, state, state_stride, ypart, carry,
                cut ? carry + (size_t)llmrs_scan_places(n_tokens, n_entries) * N * C : nullptr, chunk, C, N};
+    if (longest == 1 && n_tokens == n_entries && N <= 16) {
+        dim3 each(ceil_div(C, 64), n_entries);
+#define STEP(T, NS) selective_step_kernel<T, NS><<<each, 64, 0, stream>>>((const T*)x, ldx, (const T*)bc, ldbc, off_b, off_c, slots, (T*)out, ldo, a)
+        if (dtype == LLMRS_F32) { if (N <= 8) STEP(float, 8); else STEP(float, 16); }
+        else { if (N <= 8) STEP(bf16, 8); else STEP(bf16, 16); }
+#undef STEP
+        LLMRS_LAUNCH_CHECK("selective_scan");
+        return 0;
+    }
     dim3 grid(ceil_div(C, 64), chunks, n_entries);
 #define SCAN(T, NS, LOCAL) selective_scan_kernel<T, NS, LOCAL><<<grid, 64, 0, stream>>>((const T*)x, ldx, (const T*)bc, ldbc, off_b, off_c, q_starts, slots, (T*)out, ldo, a)
 #define BY_STATES(T, LOCAL) do { if (N <= 8) SCAN(T, 8, LOCAL); else if (N <= 16) SCAN(T, 16, LOCAL); else if (N <= 32) SCAN(T, 32, LOCAL); else SCAN(T, 64, LOCAL); } while (0)

@@ -133,6 +133,92 @@ __global__ void group_rmsnorm_kernel(T* __restrict__ out, float* __restrict__ x,
     }
 }
 
+// The same with the row held in registers, four features a piece, for up to four streams and groups of whole 256 features (a
+// wave's piece of a row then lies in one group): everything the row needs is asked for at once, a group's squares are added by
+// waves side by side and meet behind one barrier, where the kernel above walks the groups one after the other between two
+// barriers each and puts the row through LDS.  What bounds it with few rows is its chain of trips; with many, the streams'
+// bytes.  (4 rows of 2048 in four streams, 4 groups: mix and norm as two launches 4.7 + 8.7 us, this one with the mix 6.4; 2048 rows 35 -> 30.)
+template <class T, bool MIX, int HELD>
+__global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__ out, float* __restrict__ x, size_t stream_stride, int n_streams,
+                                                                 const float* __restrict__ w_in, const float* __restrict__ weight,
+                                                                 const int* __restrict__ rows, int D, int groups, float eps,
+                                                                 float* zero, float* __restrict__ combined,
+                                                                 const float* __restrict__ mix, const float* __restrict__ w_out, const float* y) {
+    constexpr int SMAX = 4;
+    __shared__ float partial[64];                    // a sum of squares for every 256 features
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int n4 = D / 4, per_group = D / groups / 256;
+    const int r = rows ? rows[blockIdx.x] : blockIdx.x;
+    float* src = x + (size_t)r * D;
+    const bool plain = n_streams == 1 && w_in == nullptr;
+    float v[HELD][SMAX][4], yy[HELD][4], wt[HELD][4], u[HELD][4];
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        const int idx = i * blockDim.x + threadIdx.x;
+#pragma unroll
+        for (int s = 0; s < SMAX; ++s) {
+            v[i][s][0] = v[i][s][1] = v[i][s][2] = v[i][s][3] = 0.0f;
+            if (s < n_streams && idx < n4) load4(src + (size_t)s * stream_stride + 4 * idx, v[i][s]);
+        }
+        if (idx < n4) {
+            load4(weight + 4 * idx, wt[i]);
+            if (MIX) load4(y + (size_t)r * D + 4 * idx, yy[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        const int idx = i * blockDim.x + threadIdx.x;
+        if (MIX) {
+            float old[SMAX][4];
+#pragma unroll
+            for (int s = 0; s < SMAX; ++s)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) old[s][j] = v[i][s][j];
+#pragma unroll
+            for (int to = 0; to < SMAX; ++to) {
+                if (to < n_streams) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float nv = mix[to] * old[0][j];
+#pragma unroll
+                        for (int s = 1; s < SMAX; ++s)
+                            if (s < n_streams) nv = fmaf(mix[s * n_streams + to], old[s][j], nv);
+                        v[i][to][j] = fmaf(w_out[to], idx < n4 ? yy[i][j] : 0.0f, nv);
+                    }
+                    if (idx < n4) store4(src + (size_t)to * stream_stride + 4 * idx, v[i][to]);
+                }
+            }
+        }
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            u[i][j] = plain ? v[i][0][j] : (w_in ? w_in[0] : 1.0f) * v[i][0][j];
+#pragma unroll
+            for (int s = 1; s < SMAX; ++s)
+                if (s < n_streams) u[i][j] = fmaf(w_in ? w_in[s] : 1.0f, v[i][s][j], u[i][j]);
+            ss = fmaf(u[i][j], u[i][j], ss);
+        }
+        ss = wave_sum(ss);                            // (pieces past the row hold zeros)
+        const int part = i * waves + wave;
+        if (lane == 0 && part < D / 256) partial[part] = ss;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        const int idx = i * blockDim.x + threadIdx.x;
+        if (idx >= n4) continue;
+        const int first = (i * waves + wave) / per_group * per_group;
+        float total = 0.0f, o[4], z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int p = 0; p < per_group; ++p) total += partial[first + p];
+        const float inv = 1.0f / sqrtf(total / (float)(D / groups) + eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = u[i][j] * inv * wt[i][j];
+        store4(out + (size_t)blockIdx.x * D + 4 * idx, o);
+        if (zero) store4(zero + (size_t)blockIdx.x * D + 4 * idx, z);
+        if (combined) store4(combined + (size_t)blockIdx.x * D + 4 * idx, u[i]);
+    }
+}
+
 // X'[r] = sum_s mix[s][r] X[s] + w_out[r] y, in place: a thread reads one feature of every stream, then writes them.
 __global__ void streams_mix_kernel(float* __restrict__ x, size_t stream_stride, int n_streams, const float* __restrict__ mix,
                                    const float* __restrict__ w_out, const float* __restrict__ y, size_t n) {
@@ -184,6 +270,18 @@ extern "C" int llmrs_group_rmsnorm(hipStream_t stream, int dtype, void* out, flo
     if (dtype != LLMRS_F32 && dtype != LLMRS_BF16) return llmrs_fail("group_rmsnorm: unknown dtype %d", dtype);
     int wide = D % 4 == 0 && stream_stride % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)y & 15) == 0
                && ((uintptr_t)zero & 15) == 0 && ((uintptr_t)combined & 15) == 0;
+    if (wide && n_streams <= 4 && D / groups % 256 == 0 && D <= 8192 && ((uintptr_t)weight & 15) == 0) {
+        int held_threads = min(512, D / 4);           // (D is a multiple of 256: whole waves)
+#define HELD(T, MIX, N) group_rmsnorm_held_kernel<T, MIX, N><<<n_rows, held_threads, 0, stream>>>((T*)out, x, (size_t)stream_stride, n_streams, w_in, weight, \
+                                                                                                rows, D, groups, eps, zero, combined, mix, w_out, y)
+#define BY_WIDTH(T, MIX) do { if (D <= 2048) HELD(T, MIX, 1); else if (D <= 4096) HELD(T, MIX, 2); else HELD(T, MIX, 4); } while (0)
+        if (dtype == LLMRS_F32) { if (mix) BY_WIDTH(float, true); else BY_WIDTH(float, false); }
+        else { if (mix) BY_WIDTH(bf16, true); else BY_WIDTH(bf16, false); }
+#undef BY_WIDTH
+#undef HELD
+        LLMRS_LAUNCH_CHECK("group_rmsnorm");
+        return 0;
+    }
     int threads = D > 8192 ? 1024 : D > 2048 ? 512 : 256;
     size_t lds = (size_t)(D + groups + 16 + MAX_STREAMS * MAX_STREAMS + MAX_STREAMS) * sizeof(float);
 #define NORM(T, MIX, SMAX) group_rmsnorm_kernel<T, MIX, SMAX><<<n_rows, threads, lds, stream>>>((T*)out, x, (size_t)stream_stride, n_streams, w_in, weight, \

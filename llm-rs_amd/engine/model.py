@@ -205,7 +205,7 @@ class Model:
             x = ctx.workspace("model.head_in", (ctx.n_want, self.spec.hidden_size), self.dtype)
             if self.streamed:
                 # the stream is the sum of its copies: a norm that can reads them all at the wanted rows itself
-                if self.final_norm is None or not self.final_norm.forward_streams(ctx, h, None, x, ctx.want_rows):
+                if self.final_norm is None or not self.final_norm.forward_streams(ctx, h, None, x, None if ctx.wants_every_row else ctx.want_rows):
                     raise ValueError("a stream kept in several copies needs a final norm that reads them (forward_streams)")
             elif self.final_norm is not None:
                 self.final_norm.forward(ctx, h, x, ctx.want_rows)

@@ -268,7 +268,7 @@ class DeltaRule(Mixer):
         gate = ctx.workspace("delta.gate", (T, self.vw), torch.float32)
         k.gemm(low_g, self.w_g2, gate, EPI_STORE_F32, ctx.gemm_workspace(low_g, self.w_g2))
         qkv = ctx.workspace("delta.qkv", (T, C), torch.float32)
-        k.causal_conv_silu(sums, self.conv, None, cache.state[:, n_state:], ctx.q_starts, ctx.slots, ctx.token_entry, C, qkv)
+        k.causal_conv(sums, self.conv, None, cache.state[:, n_state:], ctx.q_starts, ctx.slots, ctx.token_entry, C, qkv, silu=True, longest=ctx.longest)
         beta = sums[:, C:]
         k.delta_prepare(qkv[:, :a], qkv[:, a:b], decay, beta, self.A_log, self.dt_bias, self.heads, self.kv_heads, self.dk, self.unit_eps)
         o = ctx.workspace("delta.o", (T, self.vw), torch.float32)

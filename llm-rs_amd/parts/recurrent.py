@@ -127,7 +127,7 @@ class Mamba1(Mixer):
         k.gemm(x, self.w_in, sums, EPI_STORE_F32, ctx.gemm_workspace(x, self.w_in))
         scan_state, conv_state = cache.state[:, :C * N], cache.state[:, C * N:]
         xc = ctx.workspace("mamba.x", (T, C), self.dtype)
-        k.causal_conv_silu(sums, self.conv, self.conv_bias, conv_state, ctx.q_starts, ctx.slots, ctx.token_entry, C, xc)
+        k.causal_conv(sums, self.conv, self.conv_bias, conv_state, ctx.q_starts, ctx.slots, ctx.token_entry, C, xc, silu=True, longest=ctx.longest)
         dbc = ctx.workspace("mamba.dbc", (T, R + 2 * N), self.dtype)
         k.gemm(xc, self.w_x, dbc, EPI_STORE, ctx.gemm_workspace(xc, self.w_x))
         dt = ctx.workspace("mamba.dt", (T, C), torch.float32)

@@ -316,6 +316,55 @@ def test_steps_of_many_rows_mix_the_streams_inside_the_next_norm(streams, width,
                 {"whole": whole(requests), "portions": portions(requests, (128, 2, 129, 41))})
 
 
+@pytest.mark.parametrize("rows,streams,width,groups", [(1, 4, 2048, 4), (5, 1, 256, 1), (3, 2, 768, 3), (130, 3, 3072, 2), (4, 4, 8192, 8), (2, 4, 2304, 9)])
+def test_rows_held_in_registers_are_mixed_and_normed_in_one_launch(rows, streams, width, groups):
+    """Up to four streams and groups of whole 256 features: mix and norm in one launch against the mix by itself (bit for bit) and
+    the norm in 64 bits; rows of fewer pieces than a block has threads, and of more."""
+    from llm_rs_amd import kernels
+    k, g = kernels(), torch.Generator(device="cuda").manual_seed(rows + width)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    x, y, mix, w_in, w_out, weight = rnd(streams, rows, width), rnd(rows, width), rnd(streams, streams), rnd(streams), rnd(streams), rnd(width)
+    mixed = x.clone()
+    k.streams_mix(mixed, mix, w_out, y)
+    u = (mixed.double() * w_in.double()[:, None, None]).sum(0)
+    want = plain_group_rmsnorm(u, weight.double(), 1e-5, groups)
+    size = u.abs().amax(-1, keepdim=True) / want.abs().amax(-1, keepdim=True)          # what a rounding of u is in the result
+    for dtype in (torch.float32, torch.bfloat16):
+        streams_now, room = x.clone(), y.clone()
+        out, combined = torch.empty((rows, width), dtype=dtype, device="cuda"), torch.empty((rows, width), device="cuda")
+        k.group_rmsnorm(out, streams_now, weight, 1e-5, groups, w_in=w_in, zero=room, combined=combined, mix=(mix, w_out, room))
+        assert torch.equal(streams_now, mixed) and not room.any()
+        # (a sum of S products in 32 bits: S roundings of its largest term; the norm's own few more)
+        assert ((combined.double() - u).abs() <= 2 ** -23 * (streams + 1) * (mixed.abs().double() * w_in.abs().double()[:, None, None]).sum(0)).all()
+        assert ((out.double() - want).abs() <= want.abs() * (2 ** -8 if dtype == torch.bfloat16 else 2 ** -20) + 2 ** -20 * u.abs().amax() / size).all()
+        last = torch.tensor([rows - 1], dtype=torch.int32, device="cuda")
+        one = torch.empty((1, width), dtype=dtype, device="cuda")
+        k.group_rmsnorm(one, mixed, weight, 1e-5, groups, last, w_in=w_in)
+        assert torch.equal(one[0], out[-1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("entries,channels,states", [(1, 64, 16), (4, 4096, 16), (3, 70, 5), (2, 100, 1), (5, 130, 9)])
+def test_single_tokens_through_the_scan_equal_the_walk(entries, channels, states, dtype):
+    """Where the caller says that every entry brings one token the scan and the convolution run in kernels of their own: the
+    same bits as the walk, the states too."""
+    from llm_rs_amd import kernels
+    k, g = kernels(), torch.Generator(device="cuda").manual_seed(channels)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    x, bc, dt, gate = rnd(entries, channels).to(dtype), rnd(entries, 2 * states + 3).to(dtype), rnd(entries, channels), rnd(entries, channels)
+    A, D, bias, taps = -torch.exp(rnd(states, channels)), rnd(channels), rnd(channels), rnd(channels, 4)
+    slots = torch.randperm(entries + 2, generator=torch.Generator().manual_seed(1))[:entries].int().cuda()
+    starts, entry = torch.arange(entries + 1, dtype=torch.int32, device="cuda"), torch.arange(entries, dtype=torch.int32, device="cuda")
+    before = rnd(entries + 2, channels * (states + 3))
+    got = []
+    for longest in (0, 1):
+        state, out, conv = before.clone(), torch.zeros((entries, channels), dtype=dtype, device="cuda"), torch.zeros((entries, channels), dtype=dtype, device="cuda")
+        k.causal_conv(gate, taps, bias, state[:, channels * states:], starts, slots, entry, channels, conv, silu=True, longest=longest)
+        k.selective_scan(x, bc, 3, 3 + states, dt, bias, A, D, gate, state, starts, slots, out, longest=longest)
+        got.append((state, out, conv))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and not torch.equal(got[0][0], before)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_step_of_more_than_a_thousand_tokens(dtype):
     """Steps this long take the convolution several tokens a block: a long portion beside a short one, both continued
