@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void attn_f32_tiles_kernel(const float* __rest
 // (attn_f32_split_waves).
 static inline __host__ __device__ bool attn_f32_split_waves(int columns, int hd) { return columns * hd <= 2048; }
 template <int HD, int MAPS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void attn_f32_split_kernel(const float* __restrict__ q, float* __restrict__ partial,
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 || HD > 96 ? 1 : HD <= 32 ? 4 : HD <= 64 ? 3 : 2))) void attn_f32_split_kernel(const float* __restrict__ q, float* __restrict__ partial,
                                                             const float* __restrict__ kc, const float* __restrict__ vc,
                                                             const int* __restrict__ block_table,
                                                             const int* __restrict__ q_starts, const int* __restrict__ seq_lens,

@@ -354,7 +354,8 @@ class HipKernels(Kernels):
 
     @staticmethod
     def _stream() -> int:
-        return torch.cuda.current_stream().cuda_stream
+        # (the raw handle: a stream object made for every launch cost as much host time as the launch)
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
     # out[t, :] = table[tokens[t], :] * scale as float32
     # (add: out[t, :] += the same, for a stream that is shown its tokens' embeddings again)
