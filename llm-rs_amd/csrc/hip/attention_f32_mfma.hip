@@ -5,7 +5,7 @@
 // the engine computes in float32: a 2,048-token prompt is then bound by its products again.
 //
 // One wave owns 32 columns (the heads of one kv head for a few consecutive tokens of one
-// request) and walks the keys it may see in tiles of 32, aligned to absolute positions:
+// request; up to head size 128 four waves share them, a quarter of the keys each) and walks the keys it may see in tiles of 32, aligned to absolute positions:
 //   S^T[key][col] = sum_d K[key][d] Q[col][d]        A operand = keys' rows, B = queries' rows
 //   online softmax down each column (a lane holds 16 of a column's 32 keys, its partner
 //   in the other half of the wave the other 16)
@@ -135,18 +135,79 @@ __device__ __forceinline__ void f32_query(f32x4 (&qf)[HD / 8], const float* qp, 
     }
 }
 
-template <int HD, int MAPS>
-__global__ __launch_bounds__(256) void attn_f32_tiles_kernel(const float* __restrict__ q, float* __restrict__ out,
+// What the waves of a block, each with the same columns and other keys, have come to is made one: the waves after the first leave
+// theirs in `others` ([wave - 1][column][HD], ROOM floats a wave) and return false; the first adds them in order to its own
+// maximum m (base 2), sum l and sums O, and returns true.
+template <int HD, int WAVES, int ROOM>
+__device__ __forceinline__ bool f32_meet(f32x16 (&O)[HD / 32], float& m, float& l, float* others, float (*stats)[32][2], int wave, int c, int h, bool cvalid) {
+    // a lane holds features dt * 32 + 8 g + 4 h + j of its column
+    if (h == 0) { stats[wave][c][0] = m; stats[wave][c][1] = l; }
+    if (wave > 0 && cvalid) {
+        float* mine = others + (size_t)(wave - 1) * ROOM + c * HD;
+#pragma unroll
+        for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *(f32x4*)(mine + dt * 32 + 8 * g + 4 * h) = f32x4{O[dt][4 * g], O[dt][4 * g + 1], O[dt][4 * g + 2], O[dt][4 * g + 3]};
+    }
+    __syncthreads();
+    if (wave > 0) return false;
+    float top = m, part[WAVES];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) top = fmaxf(top, stats[w][c][0]);
+    const float safe = top == -INFINITY ? 0.0f : top;                     // (a column that saw no key at all)
+    l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        part[w] = __builtin_amdgcn_exp2f(stats[w][c][0] - safe);            // (-inf - x: 0)
+        l = fmaf(stats[w][c][1], part[w], l);
+    }
+    m = top;
+    if (cvalid)
+#pragma unroll
+        for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                f32x4 v[WAVES - 1];
+#pragma unroll
+                for (int w = 1; w < WAVES; ++w) v[w - 1] = *(const f32x4*)(others + (size_t)(w - 1) * ROOM + c * HD + dt * 32 + 8 * g + 4 * h);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float o = O[dt][4 * g + j] * part[0];
+#pragma unroll
+                    for (int w = 1; w < WAVES; ++w) o = fmaf(v[w - 1][j], part[w], o);
+                    O[dt][4 * g + j] = o;
+                }
+            }
+    return true;
+}
+
+// SHARED: a block's four waves have the same columns and a quarter of the keys each, side by side, and meet at the end
+// (f32_meet); else four tiles of columns a block, a wave each, where the waves' sums would not fit in LDS (head sizes over
+// 128).  What bounds it is the longest wave: a trip to memory and 64 MFMAs of 64 cycles (head size 64) for every 32 keys, a wave
+// to a SIMD at 1023 tokens of 32 heads (128 us; shared 66).
+template <int HD, int MAPS, bool SHARED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHARED || HD > 96 ? 1 : HD <= 32 ? 4 : HD <= 64 ? 3 : 2))) void attn_f32_tiles_kernel(const float* __restrict__ q, float* __restrict__ out,
                                                              const float* __restrict__ kc, const float* __restrict__ vc,
                                                              const int* __restrict__ block_table,
                                                              const int* __restrict__ positions,
                                                              const int* __restrict__ q_starts, int n_entries,
                                                              AttnArgs a, int G, int tpt, int skip_single) {
+    __shared__ float others[SHARED ? 3 * 32 * HD : 1];
+    __shared__ float stats[SHARED ? 4 : 1][32][2];
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int c = lane & 31, h = lane >> 5;
-    int task = blockIdx.x * 4 + wave;
-    int kvh = (task >> 2) % a.n_kv_heads;
-    int tile = (task / (4 * a.n_kv_heads)) * 4 + (task & 3);
+    int kvh, tile;
+    if constexpr (SHARED) {        // (the last tiles, whose keys are most, first)
+        kvh = blockIdx.x % a.n_kv_heads;
+        int count = count_tiles(q_starts, n_entries, tpt, skip_single), g = blockIdx.x / a.n_kv_heads;
+        if (g >= count) return;
+        tile = count - 1 - g;
+    } else {
+        int task = blockIdx.x * 4 + wave;
+        kvh = (task >> 2) % a.n_kv_heads;
+        tile = (task / (4 * a.n_kv_heads)) * 4 + (task & 3);
+    }
     int e = 0, rem = 0;
     if (!locate_tile(q_starts, n_entries, tpt, skip_single, tile, e, rem)) return;
     int tok0 = q_starts[e] + rem * tpt;
@@ -174,8 +235,12 @@ __global__ __launch_bounds__(256) void attn_f32_tiles_kernel(const float* __rest
     const AttnFar far = attn_far_base2(a, head);
     // the first keys that stay visible, where they lie before the tiles of the window (those among the window's tiles
     // pass the mask there)
-    if (a.keep_first > 0 && t_begin > 0) f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, 0, min(a.keep_first, t_begin), O, m, l);
-    f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, t_begin, t_end, O, m, l);
+    if (a.keep_first > 0 && t_begin > 0 && (!SHARED || wave == 0)) f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, 0, min(a.keep_first, t_begin), O, m, l);
+    if constexpr (SHARED) {
+        int each = ((t_end - t_begin + 127) >> 7) * 32, from = t_begin + wave * each;
+        f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, from, min(from + each, t_end), O, m, l);
+        if (!f32_meet<HD, 4, 32 * HD>(O, m, l, others, stats, wave, c, h, cvalid)) return;
+    } else f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, t_begin, t_end, O, m, l);
     float inv = 1.0f / (l + attn_sink_term_base2(a, head, m));      // (the sum is complete here: the sink joins it once)
     if constexpr (MAPS == 2) {
         float ss = 0.0f;
@@ -212,8 +277,9 @@ __global__ __launch_bounds__(256) void attn_f32_tiles_kernel(const float* __rest
 // WAVES 4: each wave takes 32 of the chunk's keys, and the waves' results are added in order through LDS.  What bounds this
 // step is neither bytes nor products but a wave's chain (a trip to memory, then 64 to 256 MFMAs of 64 cycles, for every 32 keys
 // one after the other): four waves side by side take a quarter of it.  (8 requests of 200 to 1800 keys, 8 kv heads of 64:
-// 22.2 -> 19.0 us; of 200 to 1000 keys, 4 kv heads of 128 with two maps: 32 -> 14.)  WAVES 1, one wave for all of the chunk's keys: where the columns' sums would not fit in LDS
-// (attn_f32_split_waves).
+// 22.2 -> 14.9 us, with registers held to three blocks a unit (540 blocks here: two rounds of two to a unit took 19.0); of
+// 200 to 1000 keys, 4 kv heads of 128 with two maps: 32 -> 14.)  WAVES 1, one wave for all of the chunk's keys: where the
+// columns' sums would not fit in LDS (attn_f32_split_waves).
 static inline __host__ __device__ bool attn_f32_split_waves(int columns, int hd) { return columns * hd <= 2048; }
 template <int HD, int MAPS, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 || HD > 96 ? 1 : HD <= 32 ? 4 : HD <= 64 ? 3 : 2))) void attn_f32_split_kernel(const float* __restrict__ q, float* __restrict__ partial,
@@ -252,45 +318,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     else {
         int from = (first + ch) * F32_SPLIT_CHUNK + 32 * wave;
         f32_walk<HD>(qf, kc, vc, table, a, kvh, c, h, pos, lo, far, max(from, begin & ~31), min(from + 32, end), O, m, l);
-        // this lane holds features dt * 32 + 8 g + 4 h + j of its column
-        if (h == 0) { stats[wave][c][0] = m; stats[wave][c][1] = l; }
-        if (wave > 0 && cvalid) {
-            float* mine = others + (size_t)(wave - 1) * 2048 + c * HD;
-#pragma unroll
-            for (int dt = 0; dt < HD / 32; ++dt)
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *(f32x4*)(mine + dt * 32 + 8 * g + 4 * h) = f32x4{O[dt][4 * g], O[dt][4 * g + 1], O[dt][4 * g + 2], O[dt][4 * g + 3]};
-        }
-        __syncthreads();
-        if (wave > 0) return;
-        float top = m, part[WAVES];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w) top = fmaxf(top, stats[w][c][0]);
-        const float safe = top == -INFINITY ? 0.0f : top;                     // (a column that saw no key at all)
-        l = 0.0f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            part[w] = __builtin_amdgcn_exp2f(stats[w][c][0] - safe);            // (-inf - x: 0)
-            l = fmaf(stats[w][c][1], part[w], l);
-        }
-        m = top;
-        if (cvalid)
-#pragma unroll
-            for (int dt = 0; dt < HD / 32; ++dt)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    f32x4 v[WAVES - 1];
-#pragma unroll
-                    for (int w = 1; w < WAVES; ++w) v[w - 1] = *(const f32x4*)(others + (size_t)(w - 1) * 2048 + c * HD + dt * 32 + 8 * g + 4 * h);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        float o = O[dt][4 * g + j] * part[0];
-#pragma unroll
-                        for (int w = 1; w < WAVES; ++w) o = fmaf(v[w - 1][j], part[w], o);
-                        O[dt][4 * g + j] = o;
-                    }
-                }
+        if (!f32_meet<HD, WAVES, 2048>(O, m, l, others, stats, wave, c, h, cvalid)) return;
     }
     if (!cvalid) return;
     float* pp = partial + ((size_t)(e * a.n_heads * MAPS + column) * max_chunks + ch) * (HD + 2);
@@ -320,10 +348,11 @@ int llmrs_attention_f32_mfma(hipStream_t stream, const float* q, float* out, con
         return 0;
     int tpt = 32 / G;
     long tiles = a.n_tokens / tpt + n_entries;
-    long blocks = ((tiles + 3) / 4) * a.n_kv_heads;
+    const bool shared = a.head_dim <= 128;
+    long blocks = (shared ? tiles : (tiles + 3) / 4) * a.n_kv_heads;
     if (blocks > 0x7fffffffL) return 0;
     switch (a.head_dim) {
-#define TILES(HD, MM) attn_f32_tiles_kernel<HD, MM><<<(int)blocks, 256, 0, stream>>>(q, out, k_cache, v_cache, block_table, positions, q_starts, n_entries, a, G, tpt, skip_single)
+#define TILES(HD, MM) attn_f32_tiles_kernel<HD, MM, (HD <= 128)><<<(int)blocks, 256, 0, stream>>>(q, out, k_cache, v_cache, block_table, positions, q_starts, n_entries, a, G, tpt, skip_single)
 #define CASE(HD) case HD: if (a.maps == 2) TILES(HD, 2); else TILES(HD, 1); break;
         CASE(32) CASE(64) CASE(96) CASE(128) CASE(160) CASE(192) CASE(224) CASE(256)
 #undef CASE

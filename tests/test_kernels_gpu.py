@@ -590,6 +590,24 @@ def test_attention_chunk_rule_and_its_scratch():
     assert len(seen) >= 2, "the case itself: more than one chunk"
 
 
+@pytest.mark.parametrize("hd,n_heads,n_kv", [(32, 3, 1), (64, 8, 2), (128, 4, 4), (96, 6, 2), (160, 2, 1)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_attention_float32_portions_share_their_keys_over_waves(hd, n_heads, n_kv, window):
+    """Portions in 32-bit whose keys are fewer than four waves have tiles for, as many, one more, and many; beside each other and
+    with a cache before them."""
+    lens, starts = [1, 33, 128, 129, 260, 300, 200], [0, 0, 0, 0, 0, 268, 199]
+    case = PagedCase(torch.float32, lens, n_heads, n_kv, hd, 16, seed=51)
+    g = torch.Generator().manual_seed(6)
+    qs = [torch.randn((n - s, n_heads, hd), generator=g) for n, s in zip(lens, starts)]
+    pos = [list(range(s, n)) for n, s in zip(lens, starts)]
+    got, at = case.run(qs, pos, window=window), 0
+    for r in range(len(lens)):
+        some = sorted({0, len(pos[r]) - 1, *range(31, len(pos[r]), 48)})
+        ref = case.reference(r, qs[r][some], [pos[r][i] for i in some], window=window)
+        assert ((got[at:at + len(pos[r])][some].double() - ref).abs() <= out_tol(ref, torch.float32, 2e-6)).all(), (r, lens[r])
+        at += len(pos[r])
+
+
 def test_attention_chunk_rule_for_unequal_entries():
     """Unequal entries (a negative number of keys) get the same chunk as equal ones or a shorter one, never under what the scratch is
     sized by nor so short that a request has more than a quarter of the merge's chunks; and the same results."""
