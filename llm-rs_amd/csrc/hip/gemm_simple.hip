@@ -389,7 +389,7 @@ static bool launch_f32_few_rows(hipStream_t stream, const float* a, int lda, con
 
 // ---- the slots of the clamped gated epilogue's constants -------------------------------------------------------------
 // A set of constants (limit, alpha, cubic, up_add) gets a slot the first time a feed-forward asks for it on a device (when it takes its weights:
-// never inside a recording); the slot is written in both source files' tables and the stream is waited for, so every
+// never inside a recording); the slot is written in every source file's table and the stream is waited for, so every
 // later product on any stream finds it.  The same set on the same device gets the same slot again.
 #include <mutex>
 #include <vector>
@@ -413,6 +413,7 @@ extern "C" int llmrs_glu_clamp_slot(hipStream_t stream, float limit, float alpha
     GluClamp p{limit, alpha, cubic, up_add};
     glu_clamp_store_kernel<<<1, 1, 0, stream>>>(slot, p);
     llmrs_glu_clamp_store_mfma(stream, slot, p);
+    llmrs_glu_clamp_store_f32_tiles(stream, slot, p);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) { llmrs_fail("glu_clamp_slot: %s", hipGetErrorString(e)); return -1; }
