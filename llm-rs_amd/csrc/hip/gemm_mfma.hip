@@ -5,10 +5,10 @@
 //            memory into MFMA operands; a block owns 16 to 64 output features and
 //            its waves split K, so a layer's product has enough loads in flight to
 //            keep HBM busy.  v_mfma_f32_16x16x32_bf16, weights as the A operand.
-//   M  > 64  "tiled": prompts.  128x128 or 256x256 tiles of the output, K in steps
-//            of 64 through double-buffered LDS, v_mfma_f32_32x32x16_bf16; the tiles are
-//            loaded straight into LDS (global_load_lds) when K % 64 == 0; the large
-//            tiles' waves work as two groups out of step.
+//   M  > 64  "tiled": prompts.  Tiles of 128x128, 256x128, 256x192 or 256x256 outputs, K
+//            in steps of 64 through double-buffered LDS, v_mfma_f32_32x32x16_bf16; when
+//            K % 64 == 0 the tiles are loaded straight into LDS (global_load_lds), or, by
+//            the four waves of the large ones, through registers between the MFMAs.
 // Both need K % 8 == 0 and 16-byte aligned rows (16-byte loads); otherwise the
 // caller falls back to the plain kernel.
 //
