@@ -409,7 +409,9 @@ class StepRunner:
         # A decode step.  Everything the kernels take from the host must be the same for
         # every step of this key: sizes, addresses, and the bound on the context length.
         ctx.max_seq_len = min(w * g.page_size for w, g in zip(graph_widths, self.cache.groups)) if graph_widths else ctx.max_seq_len
-        key = (ctx.n_tokens, ctx.n_want, tuple(graph_widths), self._dev_words.data_ptr(), self.model.recording_key(ctx))
+        # (a step that wants every row leaves the gathering of rows out, which as many wanted rows do not say: a place may
+        # be wanted twice and another one not)
+        key = (ctx.n_tokens, ctx.n_want, ctx.wants_every_row, tuple(graph_widths), self._dev_words.data_ptr(), self.model.recording_key(ctx))
         hit = self._graphs.get(key)
         if hit is not None:
             self._graphs.move_to_end(key)

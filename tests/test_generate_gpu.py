@@ -271,6 +271,29 @@ def test_recorded_decode_steps_equal_eager_ones(folders, which, dtype):
     assert recorded.runner.graph_replays >= 30 and eager.runner.graph_replays == 0
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("which", ["llama", "tuvodra"])
+def test_a_row_wanted_twice_beside_one_not_wanted(folders, which, dtype):
+    """A step of two single tokens that wants the first's row twice has the sizes of a recorded step that wants each row once
+    (whose head takes the rows as they lie); it gets its own rows, before and after it is recorded itself."""
+    from tuvodra_cases import CONFIGS as TUVODRA, make_model
+    if which == "llama":
+        recorded, eager = (engine(folders["B"], "B", dtype) for _ in range(2))
+    else:
+        typed, tensors = make_model(TUVODRA["wide"], seed=3)
+        recorded, eager = (Engine(typed, tensors, dtype=dtype, page_size=16, num_pages=64, max_requests=4) for _ in range(2))
+    eager.runner.use_graphs = False
+    tokens = random_tokens(256, 60, seed=77)
+    slots = {e: [e.open_request() for _ in range(2)] for e in (recorded, eager)}
+    for i in range(24):
+        wants = ([0], [0]) if i % 8 < 4 else ([0, 0], []) if i % 8 < 7 else ([], [0, 0])
+        outs = [e.step([StepEntry(slots[e][r], i, [tokens[2 * i + r]], wants[r]) for r in range(2)]).clone() for e in (recorded, eager)]
+        torch.cuda.synchronize()
+        assert torch.equal(*outs), f"step {i}, wanted {wants}"
+        assert torch.equal(outs[0][0], outs[0][1]) == (wants[0] != [0])
+    assert recorded.runner.graph_replays >= 15
+
+
 def test_a_recording_is_kept_for_the_chunk_it_was_made_with():
     """The kernel library shares a decoding request's keys out over waves in chunks whose length it chooses by how
     many keys the step sees, and a recorded step holds the chunk it was recorded with.  Sixteen requests decode from

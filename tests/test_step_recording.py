@@ -115,3 +115,16 @@ def test_no_buffer_is_asked_to_grow_on_the_recording_pass(engine):
     for _ in range(4):
         _decode(engine, slots, pos)
     assert len(runner._graphs) == 1 and grown == []
+
+
+def test_a_step_that_wants_a_row_twice_is_not_another_steps_recording(engine):
+    """Two single tokens of which the first's row is wanted twice and the second's not: as many tokens and wanted rows as
+    a recorded step has that wants each row once, and no replay of it."""
+    runner = engine.runner
+    slots = [engine.open_request() for _ in range(2)]
+    pos = {s: 0 for s in slots}
+    for _ in range(4):
+        _decode(engine, slots, pos)
+    assert len(runner._graphs) == 1 and runner.graph_replays == 2
+    out = engine.step([StepEntry(slots[0], pos[slots[0]], [9], [0, 0]), StepEntry(slots[1], pos[slots[1]], [11], [])])
+    assert runner.graph_replays == 2 and torch.equal(out[0], out[1])
