@@ -291,7 +291,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     __shared__ float others[WAVES > 1 ? (WAVES - 1) * 2048 : 1];              // [wave - 1][column][HD]
     __shared__ float stats[WAVES][32][2];                                      // [wave][column]: maximum (base 2), sum
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
-    int kvh = blockIdx.x, ch = blockIdx.y, e = blockIdx.z;
+    int kvh = blockIdx.x, e = blockIdx.y, ch = blockIdx.z;
     int token = q_starts[e];
     if (q_starts[e + 1] - token != 1) return;
     int pos_t = seq_lens[e] - 1;                  // an entry with one token: its position is its length less one
@@ -378,7 +378,9 @@ int llmrs_attention_f32_mfma_split(hipStream_t stream, const float* q, float* pa
     if (a.q_stride % 4 || ((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)partial & 7))
         return 0;
     if (n_entries > 65535 || a.n_kv_heads > 65535 || max_chunks > 65535 || max_chunks < 1) return 0;
-    dim3 grid(a.n_kv_heads, max_chunks, n_entries);      // (blocks go to the XCDs in turn: what all entries share alike comes first)
+    // (blocks go to the XCDs in turn: what all entries share alike comes first; the chunk last, as short and empty ones are an
+    // entry's last: 32 requests of 200 keys under a bound of 1024, 8 kv heads of 64: 16.6 us, with the chunks before the entries 25)
+    dim3 grid(a.n_kv_heads, n_entries, max_chunks);
     switch (a.head_dim) {
 #define SPLIT(HD, MM, WW) attn_f32_split_kernel<HD, MM, WW><<<grid, 64 * WW, 0, stream>>>(q, partial, k_cache, v_cache, block_table, q_starts, seq_lens, max_chunks, a, G)
 #define CASE(HD) case HD: if (attn_f32_split_waves(G, HD)) { if (a.maps == 2) SPLIT(HD, 2, 4); else SPLIT(HD, 1, 4); } \

@@ -661,7 +661,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 3
                                                         const int* __restrict__ seq_lens,
                                                         const int* __restrict__ q_starts, AttnArgs a, int G,
                                                         int max_chunks, int chunk, int plain) {
-    int kvh = blockIdx.x, ch = blockIdx.y, e = blockIdx.z;
+    int kvh = blockIdx.x, e = blockIdx.y, ch = blockIdx.z;
     int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -759,7 +759,7 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
                                                           const int* __restrict__ q_starts, AttnArgs a, int G,
                                                           int max_chunks, int chunk, int plain) {
     static_assert(KD % 32 == 0 && VD % 16 == 0, "the score products take 32 features at a time");
-    int kvh = blockIdx.x, ch = blockIdx.y, e = blockIdx.z;
+    int kvh = blockIdx.x, e = blockIdx.y, ch = blockIdx.z;
     int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -1247,9 +1247,13 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
     }
     if (split) {
         // Blocks go to the eight XCDs in turn, so the grid's first dimension is one that all entries share alike: with the
-        // entries there, each XCD had every eighth entry whole, and one with a longer cache than the others kept its
-        // XCD busy alone (64 requests of 509 to 3585 keys: 114 -> 113 us; 160 of 128 to 4096, heads of 64: 158 -> 154).
-        dim3 grid(a.n_kv_heads, max_chunks, n_entries);
+        // entries there, each XCD had every eighth entry whole, and one with a longer cache than the others kept its XCD busy
+        // alone (24 requests of 800 to 8000 keys: 106 -> 102 us, 160 of 128 to 4096, heads of 64, in chunks of 1024: 165 -> 147).
+        // The chunk comes last: a recorded step's grid is as wide as its block table, and an entry's last chunk may hold a
+        // few keys, so with the chunks before the entries, whole, short and empty ones alternated, and the units that got
+        // the short ones first were left without work (64 requests of 2060 keys under a bound of 4096: 105 us, 132 that way;
+        // 256: 406, 506; without empty chunks the same either way).
+        dim3 grid(a.n_kv_heads, n_entries, max_chunks);
         int plain = only_single && attn_reach(a) == 0;
         if (G <= 16)
             attn_split16_kernel<KD, VD, MAPS><<<grid, 64, SPLIT16_LDS_BYTES, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain);
