@@ -149,7 +149,7 @@ int llmrs_attention_bf16_mfma(hipStream_t stream, const bf16* q, bf16* out, cons
                               size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, const AttnArgs& a);
 
 // Keys per wave when the matrix-core kernels split `singles` single-token entries of up to max_seq_len keys
-// that see single_keys keys together (0: unknown; negative: so many, and unequal numbers of them; 1 gives the smallest chunk any number of keys can give for these
+// that see single_keys keys together (0: unknown; 1 gives the smallest chunk any number of keys can give for these
 // entries and this bound, which is what the scratch is sized by).
 extern "C" int llmrs_attention_split_chunk(long singles, int n_kv_heads, int head_dim, int max_seq_len, long single_keys);
 

@@ -501,8 +501,7 @@ static int launch_generic(hipStream_t stream, const T* q, T* out, const T* k_cac
 // max_seq_len: an upper bound of seq_lens that the host knows (0: unknown, no split);
 // n_single: how many entries bring one token, if the host knows (-1: it does not); n_single == n_entries is the
 // caller's word that every entry brings exactly one token (then token t is entry t, and q_starts is not read);
-// single_keys: how many keys those entries see together (windows counted), if the host knows (0: it does not; negative: so
-// many, and unequal numbers of them):
+// single_keys: how many keys those entries see together (windows counted), if the host knows (0: it does not):
 // the matrix-core kernels choose the keys per wave by it.
 // v_dim: the width of a value (the cache's values are [page][kv_head][v_dim][slot], `out` has v_dim per head);
 // dist_r1, dist_r2: [n_heads] 32-bit, the distance penalty of AttnArgs (dist_r2 null: with the distance itself), or both null.

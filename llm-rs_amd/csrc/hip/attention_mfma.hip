@@ -62,7 +62,6 @@ static int split_waves_to_a_unit(int head_dim) {
 // record put this function's result into what they key their recordings by.  The scratch is sized by the smallest
 // chunk the entries and the bound allow, taken at an eighth of the bound for every entry; fewer keys than that get
 // that chunk too.
-// single_keys < 0: the entries see -single_keys together, unequal numbers of them (see below).
 // LLMRS_SPLIT_CHUNK in the environment (64 to 1024, a power of two) takes the choice away from the rule, for measuring it.
 extern "C" int llmrs_attention_split_chunk(long singles, int n_kv_heads, int head_dim, int max_seq_len, long single_keys) {
     if (const char* e = getenv("LLMRS_SPLIT_CHUNK")) {
@@ -98,18 +97,8 @@ extern "C" int llmrs_attention_split_chunk(long singles, int n_kv_heads, int hea
     };
     double bound_keys = (double)singles * max_seq_len;
     int least = pick(bound_keys / 8.0);
-    double keys = single_keys != 0 ? fmin(fabs((double)single_keys), bound_keys) : 0.75 * bound_keys;
-    int chunk = pick(keys);
-    // Unequal entries (a negative number of keys): with the longest chunks most waves are as long as the longest entry's and
-    // few, and the device waits for them; shorter ones share out.  Measured (four layers, 64 requests of 509 to
-    // 3585 keys at head size 128: 1330 us with chunks of 1024, 1291 with 512, 1293 with 256; 24 of 800 to 8000: 1020, 981, 995; at
-    // 64, 160 of 128 to 4096: 1226, 1164, 1158; 160 of 500 to 2000: 943, 943, 897; equal entries are as fast or 1 % faster
-    // with the longest: 64 of 4090 keys 1580, 1599, 1607).
-    if (single_keys < 0) {
-        const int most = head_dim <= 64 ? 2 * ATTN_CHUNK : 4 * ATTN_CHUNK;
-        while (chunk > most && (max_seq_len + chunk / 2 - 1) / (chunk / 2) <= MERGE_MAX_CHUNKS / 4) chunk /= 2;
-    }
-    return std::max(chunk, least);
+    double keys = single_keys > 0 ? fmin((double)single_keys, bound_keys) : 0.75 * bound_keys;
+    return std::max(pick(keys), least);
 }
 
 // Heads of two maps (attention_mfma_maps.hip).

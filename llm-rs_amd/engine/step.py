@@ -146,14 +146,6 @@ class StepContext:
             self._keys_seen[(window, mask_chunk)] = got
         return got
 
-    def keys_for_split(self, window: int = 0, mask_chunk: int = 0) -> int:
-        """The same for `kernels().attention`, which shares these keys out over waves: as a negative number where the entries
-        see unequal numbers of them (the longest a quarter more than the mean, or more)."""
-        keys = self.single_keys(window, mask_chunk)
-        sees = lambda n: (n - 1) % mask_chunk + 1 if mask_chunk > 0 else n if window <= 0 else min(n, window)
-        most = max(map(sees, self.single_lens), default=0)
-        return -keys if 4 * most * self.n_single >= 5 * keys else keys
-
     def room_for_next_norm(self, h: torch.Tensor, w: torch.Tensor):
         """For a part about to add a product with weight `w` into the stream `h`: a `kernels.NextNorm` for that
         product to fill (`kernels().gemm(..., leave=...)`; then `note_left(h, it)`), or None when the norm that

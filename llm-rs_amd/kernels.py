@@ -661,8 +661,7 @@ class HipKernels(Kernels):
         gate: float32 [T, n_heads * value_dim / gate_per] or None: every gate_per consecutive output features of a token
         are multiplied by the sigmoid of their number (32-bit, before the one rounding).
         sink: float32 [n_heads] or None: the softmax's denominator of head h also holds exp(sink[h]), once for every
-        query (a key without a value; not scaled).  single_keys: how many keys the single-token entries see together (windows counted), 0 if unknown,
-        negative where they see unequal numbers of them.
+        query (a key without a value; not scaled).  single_keys: how many keys the single-token entries see together (windows counted), 0 if unknown.
         value_dim: the width of a value where it is not a key's (0: the same).  distance: (r1, r2), float32 [n_heads]
         each: r1[h] * ln(1 + r2[h] * (i - j)) is taken off the scaled score of query i and key j; with r2 None r1[h] * (i - j).  softcap > 0: the
         scaled score s becomes softcap * tanh(s / softcap).  keep_first: with a window, the request's first so many

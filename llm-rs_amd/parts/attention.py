@@ -63,7 +63,7 @@ class KeyedBySplitChunk:
     and how much of it they see (the chunk may be left out: 0)."""
 
     # The kernel library shares the decoding requests' keys out over waves in chunks whose length it chooses by
-    # how many keys the step sees (`keys_for_split`).  A recorded step holds the chunk it was recorded with, so the
+    # how many keys the step sees (`single_keys`).  A recorded step holds the chunk it was recorded with, so the
     # chunk is part of what recordings are keyed by; and since recording a step again costs about as much as a step
     # while a chunk that is no longer the best one costs a few per cent of the attention, a batch keeps the figure
     # it was recorded with until the rule has asked for another chunk this many steps in a row.
@@ -73,7 +73,7 @@ class KeyedBySplitChunk:
         k = kernels()
         if not ctx.n_single:
             return 0
-        keys = ctx.keys_for_split(*self.recording_signature[3:])
+        keys = ctx.single_keys(*self.recording_signature[3:])
         want = k.attention_split_chunk(ctx.n_single, self.recording_signature[1], self.recording_signature[2], ctx.max_seq_len, keys)
         held = ctx.part_state.setdefault(self.recording_signature, {})
         at = (ctx.n_single, ctx.max_seq_len)
@@ -91,7 +91,7 @@ class KeyedBySplitChunk:
         now = ctx.part_state.get(self.recording_signature, {}).get((ctx.n_single, ctx.max_seq_len))
         if now is not None and now[3] == ctx.serial:      # this step was keyed by a chunk: the figure that gives it
             return now[1]
-        return ctx.keys_for_split(*self.recording_signature[3:])
+        return ctx.single_keys(*self.recording_signature[3:])
 
 
 class Attention(KeyedBySplitChunk, Mixer):

@@ -651,28 +651,6 @@ def test_attention_float32_portions_share_their_keys_over_waves(hd, n_heads, n_k
         at += len(pos[r])
 
 
-def test_attention_chunk_rule_for_unequal_entries():
-    """Unequal entries (a negative number of keys) get the same chunk as equal ones or a shorter one, never under what the scratch is
-    sized by nor so short that a request has more than a quarter of the merge's chunks; and the same results."""
-    k = kernels()
-    shorter = 0
-    for n, kv, hd, bound in ((1, 8, 128, 2048), (64, 8, 128, 4096), (160, 8, 64, 4096), (200, 4, 256, 8192), (48, 1, 32, 131072), (90, 8, 64, 300000)):
-        least = k.attention_split_chunk(n, kv, hd, bound, 1)
-        for keys in (1, n * bound // 16, n * bound // 3, n * bound, 10 * n * bound):
-            equal, c = k.attention_split_chunk(n, kv, hd, bound, keys), k.attention_split_chunk(n, kv, hd, bound, -keys)
-            assert c in (64, 128, 256, 512, 1024) and least <= c <= equal and (-(-bound // c) <= 256 or c == equal)
-            shorter += c < equal
-    assert shorter
-    lens = [1500, 40, 2047, 333, 900] * 30
-    case = PagedCase(torch.bfloat16, lens, 8, 8, 64, 16, seed=43)
-    g = torch.Generator().manual_seed(4)
-    qs, pos = [torch.randn((1, 8, 64), generator=g).to(torch.bfloat16) for _ in lens], [[n - 1] for n in lens]
-    assert k.attention_split_chunk(len(lens), 8, 64, 2048, -sum(lens)) < k.attention_split_chunk(len(lens), 8, 64, 2048, sum(lens))
-    got = case.run(qs, pos, scratch_floats=k.attention_scratch_floats(len(lens), 8, 64, 2048, 8, len(lens)), bound=2048, n_single=len(lens), single_keys=-sum(lens))
-    for r in range(0, len(lens), 7):
-        assert (got[r].float() - case.reference(r, qs[r], pos[r])[0].float()).abs().max() <= 2e-2, f"request {r}"
-
-
 @pytest.mark.parametrize("portion", [False, True])
 def test_attention_long_caches_with_a_window(portion):
     """Two decoding requests over long caches with a window of 8500 keys (more than 64 ranges to merge, the first of
