@@ -274,13 +274,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHARED || 
 // once for all of them, 16 bytes a lane).  It leaves what the walk of
 // attention_generic.hip leaves for such a chunk, where that file's merge finds it: the maximum (natural logarithm's
 // scale), the sum and the weighted values of each head, [entry][head][chunk][2 + head_dim].
-// WAVES 4: each wave takes 32 of the chunk's keys, and the waves' results are added in order through LDS.  What bounds this
-// step is neither bytes nor products but a wave's chain (a trip to memory, then 64 to 256 MFMAs of 64 cycles, for every 32 keys
-// one after the other): four waves side by side take a quarter of it.  (8 requests of 200 to 1800 keys, 8 kv heads of 64:
-// 22.2 -> 14.9 us, with registers held to three blocks a unit (540 blocks here: two rounds of two to a unit took 19.0); of
-// 200 to 1000 keys, 4 kv heads of 128 with two maps: 32 -> 14.)  WAVES 1, one wave for all of the chunk's keys: where the
-// columns' sums would not fit in LDS (attn_f32_split_waves).
-static inline __host__ __device__ bool attn_f32_split_waves(int columns, int hd) { return columns * hd <= 2048; }
+// WAVES 4: each wave takes 32 of the chunk's keys, and the waves' results are added in order through LDS.  With few blocks what
+// bounds this step is neither bytes nor products but a wave's chain (a trip to memory, then 64 to 256 MFMAs of 64 cycles, for
+// every 32 keys one after the other): four waves side by side take a quarter of it (8 requests of 200 to 1800 keys, 8 kv heads
+// of 64: 27.9 -> 21.8 us with the merge; 4 of 1800 keys, heads of 128: 43 -> 37).  WAVES 1, one wave for all of the chunk's
+// keys: where blocks are many, or the columns' sums would not fit in LDS (attn_f32_split_four).
 template <int HD, int MAPS, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 || HD > 96 ? 1 : HD <= 32 ? 4 : HD <= 64 ? 3 : 2))) void attn_f32_split_kernel(const float* __restrict__ q, float* __restrict__ partial,
                                                             const float* __restrict__ kc, const float* __restrict__ vc,
@@ -291,7 +289,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     __shared__ float others[WAVES > 1 ? (WAVES - 1) * 2048 : 1];              // [wave - 1][column][HD]
     __shared__ float stats[WAVES][32][2];                                      // [wave][column]: maximum (base 2), sum
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
-    int kvh = blockIdx.x, e = blockIdx.y, ch = blockIdx.z;
+    int kvh = WAVES > 1 ? blockIdx.x : blockIdx.y, e = WAVES > 1 ? blockIdx.y : blockIdx.x, ch = blockIdx.z;      // (see the launcher)
     int token = q_starts[e];
     if (q_starts[e + 1] - token != 1) return;
     int pos_t = seq_lens[e] - 1;                  // an entry with one token: its position is its length less one
@@ -367,6 +365,17 @@ int llmrs_attention_f32_mfma(hipStream_t stream, const float* q, float* out, con
     return 1;
 }
 
+// Whether four waves share a chunk.  A unit holds one such block of heads over 96, two or three of 96 and 64, four of 32, with the
+// registers they keep, and their meeting costs what a wave's shorter chain saves once the grid makes several rounds:
+// measured, four waves against one (grid in blocks to a unit): heads of 128 0.49-0.84 up to 1.5, 0.51-0.85 at 2, up to 1.07 at
+// 3, 1.24-1.91 at 64; of 64 0.53-0.93 up to 3, 0.55-0.94 at 6, up to 1.12 at 8; of 32 up to 0.88 at 6, 1.01 at 11, 1.11 at 16.
+// A bound of one chunk may hold 64 keys or fewer, which leaves two of the waves idle: 0.80 up to 1 block to a unit, 1.2-1.3 at
+// 1.5 to 4.  Counted over the grid, which a recorded step keeps, not over the keys of the moment.
+static bool attn_f32_split_four(int columns, int hd, long blocks, int max_chunks) {
+    const long to_a_unit = max_chunks == 1 ? 1 : hd <= 32 ? 12 : hd <= 96 ? 6 : 2;
+    return columns * hd <= 2048 && blocks <= to_a_unit * llmrs_compute_units();
+}
+
 // Takes the entries with one token, split by key range into `partial` (max_chunks chunks of F32_SPLIT_CHUNK keys an
 // entry; the caller merges them).  Returns 1 when it took them, 0 when the shape is not its own, -1 on error.
 int llmrs_attention_f32_mfma_split(hipStream_t stream, const float* q, float* partial, const float* k_cache, const float* v_cache,
@@ -378,12 +387,15 @@ int llmrs_attention_f32_mfma_split(hipStream_t stream, const float* q, float* pa
     if (a.q_stride % 4 || ((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)partial & 7))
         return 0;
     if (n_entries > 65535 || a.n_kv_heads > 65535 || max_chunks > 65535 || max_chunks < 1) return 0;
-    // (blocks go to the XCDs in turn: what all entries share alike comes first; the chunk last, as short and empty ones are an
-    // entry's last: 32 requests of 200 keys under a bound of 1024, 8 kv heads of 64: 16.6 us, with the chunks before the entries 25)
-    dim3 grid(a.n_kv_heads, n_entries, max_chunks);
+    const bool four = attn_f32_split_four(G, a.head_dim, (long)a.n_kv_heads * n_entries * max_chunks, max_chunks);
+    // The chunk last, as short and empty ones are an entry's last (32 requests of 200 keys under a bound of 1024, 8 kv heads of 64,
+    // four waves: 16.6 us, with the chunks before the entries 25).  Blocks go to the XCDs in turn: few blocks with the kv head
+    // first, so that every XCD gets a share of every entry; many with the entry first, as a first dimension of a few
+    // blocks hands thousands of empty ones out more slowly (64 requests of 200 keys under 8192, heads of 128: 47 against 51 us).
+    dim3 grid(four ? a.n_kv_heads : n_entries, four ? n_entries : a.n_kv_heads, max_chunks);
     switch (a.head_dim) {
 #define SPLIT(HD, MM, WW) attn_f32_split_kernel<HD, MM, WW><<<grid, 64 * WW, 0, stream>>>(q, partial, k_cache, v_cache, block_table, q_starts, seq_lens, max_chunks, a, G)
-#define CASE(HD) case HD: if (attn_f32_split_waves(G, HD)) { if (a.maps == 2) SPLIT(HD, 2, 4); else SPLIT(HD, 1, 4); } \
+#define CASE(HD) case HD: if (four) { if (a.maps == 2) SPLIT(HD, 2, 4); else SPLIT(HD, 1, 4); } \
                           else { if (a.maps == 2) SPLIT(HD, 2, 1); else SPLIT(HD, 1, 1); } break;
         CASE(32) CASE(64) CASE(96) CASE(128) CASE(160) CASE(192) CASE(224) CASE(256)
 #undef CASE

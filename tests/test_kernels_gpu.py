@@ -613,10 +613,11 @@ def replay_time(*calls):
 
 @pytest.mark.parametrize("dtype,n,length,n_heads,n_kv,hd,bounds", [(torch.bfloat16, 64, 2060, 32, 8, 128, (2064, 4096)),
                                                                    (torch.bfloat16, 32, 4200, 32, 8, 128, (4208, 8192)),
-                                                                   (torch.float32, 32, 200, 8, 2, 32, (256, 4096))])
+                                                                   (torch.float32, 32, 200, 8, 2, 32, (256, 4096)), (torch.float32, 64, 200, 32, 8, 128, (256, 8192))])
 def test_empty_chunks_of_a_wide_block_table_cost_little(dtype, n, length, n_heads, n_kv, hd, bounds):
     """A recorded decode step's grid is as wide as its block table: the chunks beyond the requests' keys, and their last chunks of a
-    few keys, come after the whole ones.  (Between them, they left units without work: 1.2, 1.2 and 1.6 times the time.)"""
+    few keys, come after the whole ones.  (Between them, they left units without work: 1.2, 1.2 and 1.6
+    times the time; blocks of four waves where one is enough: the last case 1.4.)"""
     g, k = torch.Generator(device=DEV).manual_seed(3), kernels()
     rand = lambda *shape: torch.randn(shape, generator=g, device=DEV).to(dtype)
     per = -(-length // 16)
@@ -631,6 +632,23 @@ def test_empty_chunks_of_a_wide_block_table_cost_little(dtype, n, length, n_head
                      k.attention(q, out, kc, vc, table, entry, pos, starts, lens, n_heads, n_kv, hd, 16, n * per, 0, hd ** -0.5, scratch, bound, n, n * length))
     # (the least of three comparisons: two timings of one case differ by 3 %)
     assert min(wide / exact for exact, wide in (replay_time(*calls) for _ in range(3))) <= 1.12
+
+
+@pytest.mark.parametrize("hd,n_heads,n_kv,n,bound", [
+    (32, 4, 4, 24, 4096), (32, 4, 4, 25, 4096), (96, 2, 2, 24, 4096), (96, 2, 2, 25, 4096), (128, 2, 2, 8, 4096), (128, 2, 2, 9, 4096),
+    (64, 4, 4, 64, 128), (64, 4, 4, 65, 128), (192, 4, 2, 9, 2048)])
+def test_attention_float32_single_tokens_by_number_of_blocks(hd, n_heads, n_kv, n, bound):
+    """Four waves or one for a chunk of keys, by how many blocks there are (256 units: 12, 6 and 2 to a unit, 1 where the bound is
+    one chunk): both sides of each line, requests of one key, of a wave's keys, a chunk's, and one more."""
+    lens = [(1, 32, 33, 96, 97, 128)[i % 6] if bound == 128 else (1, 33, 128, 129, 300, 257, 31)[i % 7] for i in range(n)]
+    case = PagedCase(torch.float32, lens, n_heads, n_kv, hd, 16, seed=61)
+    g = torch.Generator().manual_seed(8)
+    qs, pos = [torch.randn((1, n_heads, hd), generator=g) for _ in lens], [[m - 1] for m in lens]
+    case.tables = torch.cat([case.tables, torch.zeros((n, max(0, bound // 16 - case.width)), dtype=torch.int32)], 1).contiguous()
+    got = case.run(qs, pos, bound=bound, n_single=n, single_keys=sum(lens))
+    for r in range(n):
+        ref = case.reference(r, qs[r], pos[r])
+        assert ((got[r].double() - ref[0]).abs() <= out_tol(ref[0], torch.float32, 2e-6)).all(), (r, lens[r])
 
 
 @pytest.mark.parametrize("hd,n_heads,n_kv", [(32, 3, 1), (64, 8, 2), (128, 4, 4), (96, 6, 2), (160, 2, 1)])
