@@ -660,8 +660,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 3
                                                         const int* __restrict__ block_table,
                                                         const int* __restrict__ seq_lens,
                                                         const int* __restrict__ q_starts, AttnArgs a, int G,
-                                                        int max_chunks, int chunk, int plain) {
-    int kvh = blockIdx.x, e = blockIdx.y, ch = blockIdx.z;
+                                                        int max_chunks, int chunk, int plain, int entry_first) {
+    int kvh = entry_first ? blockIdx.y : blockIdx.x, e = entry_first ? blockIdx.x : blockIdx.y, ch = blockIdx.z;      // (see `launch`)
     int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -757,9 +757,9 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
                                                           const int* __restrict__ block_table,
                                                           const int* __restrict__ seq_lens,
                                                           const int* __restrict__ q_starts, AttnArgs a, int G,
-                                                          int max_chunks, int chunk, int plain) {
+                                                          int max_chunks, int chunk, int plain, int entry_first) {
     static_assert(KD % 32 == 0 && VD % 16 == 0, "the score products take 32 features at a time");
-    int kvh = blockIdx.x, e = blockIdx.y, ch = blockIdx.z;
+    int kvh = entry_first ? blockIdx.y : blockIdx.x, e = entry_first ? blockIdx.x : blockIdx.y, ch = blockIdx.z;      // (see `launch`)
     int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -1253,12 +1253,20 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
         // few keys, so with the chunks before the entries, whole, short and empty ones alternated, and the units that got
         // the short ones first were left without work (64 requests of 2060 keys under a bound of 4096: 105 us, 132 that way;
         // 256: 406, 506; without empty chunks the same either way).
-        dim3 grid(a.n_kv_heads, n_entries, max_chunks);
+        // With a grid of many more chunks than there are keys (one long cache under the same bound as many short ones) the entry
+        // comes first after all: a first dimension of a few blocks hands thousands of empty ones out more slowly (bound 4096, 32
+        // requests of 60 keys, heads of 64: 9.1 against 10.4 us; bound 32,768, 200 of 600: 66 against 74; of 13 to 14 times the
+        // keys neither is faster); and with no more than three waves to a unit, where nothing waits for a longer entry and the merge,
+        // whose blocks also go by entry, finds the parts in its XCD's L2 (8 requests of 600 keys: 10.4 against 10.9 us, 64 heads
+        // 11.0 against 11.7).
+        const int entry_first = single_keys <= 0 || (double)n_entries * max_chunks * chunk > 8.0 * single_keys ||
+                                (double)single_keys * a.n_kv_heads <= 3.0 * llmrs_compute_units() * chunk;
+        dim3 grid(entry_first ? n_entries : a.n_kv_heads, entry_first ? a.n_kv_heads : n_entries, max_chunks);
         int plain = only_single && attn_reach(a) == 0;
         if (G <= 16)
-            attn_split16_kernel<KD, VD, MAPS><<<grid, 64, SPLIT16_LDS_BYTES, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain);
+            attn_split16_kernel<KD, VD, MAPS><<<grid, 64, SPLIT16_LDS_BYTES, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain, entry_first);
         else
-            attn_split_kernel<KD, VD, MAPS><<<grid, 64, 0, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain);
+            attn_split_kernel<KD, VD, MAPS><<<grid, 64, 0, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain, entry_first);
         if constexpr (MAPS == 2)
             attn_merge_maps_kernel<<<dim3(n_entries, a.n_heads), MERGE_GROUP_THREADS, 0, single_stream>>>(scratch, out, seq_lens, q_starts, a, max_chunks, chunk, plain);
         else if (max_chunks > MERGE_ONE_WALK_CHUNKS && VD <= MERGE_GROUP_THREADS) {
