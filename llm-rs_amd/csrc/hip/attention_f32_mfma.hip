@@ -5,7 +5,7 @@
 // the engine computes in float32: a 2,048-token prompt is then bound by its products again.
 //
 // One wave owns 32 columns (the heads of one kv head for a few consecutive tokens of one
-// request; up to head size 128 four waves share them, a quarter of the keys each) and walks the keys it may see in tiles of 32, aligned to absolute positions:
+// request; four waves may share them, a quarter of the keys each) and walks the keys it may see in tiles of 32, aligned to absolute positions:
 //   S^T[key][col] = sum_d K[key][d] Q[col][d]        A operand = keys' rows, B = queries' rows
 //   online softmax down each column (a lane holds 16 of a column's 32 keys, its partner
 //   in the other half of the wave the other 16)
@@ -183,9 +183,10 @@ __device__ __forceinline__ bool f32_meet(f32x16 (&O)[HD / 32], float& m, float& 
 }
 
 // SHARED: a block's four waves have the same columns and a quarter of the keys each, side by side, and meet at the end
-// (f32_meet); else four tiles of columns a block, a wave each, where the waves' sums would not fit in LDS (head sizes over
-// 128).  What bounds it is the longest wave: a trip to memory and 64 MFMAs of 64 cycles (head size 64) for every 32 keys, a wave
-// to a SIMD at 1023 tokens of 32 heads (128 us; shared 66).
+// (f32_meet); else four tiles of columns a block, a wave each (and always where the waves' sums would not fit in LDS: head
+// sizes over 128).  What bounds either is the longest wave, a trip to memory and 64 MFMAs of 64 cycles (head size 64) for every 32
+// keys, where tiles are few; with many the bytes and products.  (A portion of 1023 tokens, 32 heads of 64 on 8 kv heads: a wave to
+// a tile 128 us, four 70; which of the two runs: attn_f32_shared.)
 template <int HD, int MAPS, bool SHARED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHARED || HD > 96 ? 1 : HD <= 32 ? 4 : HD <= 64 ? 3 : 2))) void attn_f32_tiles_kernel(const float* __restrict__ q, float* __restrict__ out,
                                                              const float* __restrict__ kc, const float* __restrict__ vc,
@@ -333,11 +334,26 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
             }
 }
 
-// Takes the entries with several tokens (all entries when skip_single is 0).  Returns 1 when it took them,
+// Whether four waves share a tile's keys, by `tiles` waves to a SIMD with a wave to a tile, and `reach`, how many keys a tile may
+// see.  With 32 keys or fewer three of the four would have none.  Measured, shared against a wave to a tile (1 to 128 portions of
+// 2 to 2048 tokens, at positions 0 to 2000): heads of 32 0.26-0.99 everywhere else; heads of 64, 96 and 128: 0.76-0.90 up to a
+// quarter of a wave and 64 keys (1.0-2.5 with more tiles); 0.40-0.93 up to half a wave and 256 keys (0.6-1.7 with more);
+// 0.30-0.9 up to one wave and any keys (heads of 128: three quarters; at one wave up to 1.1).  With more tiles than that the waves
+// of a device are even enough alone: heads of 128 0.9-1.3 unless the portions are long (512 tokens and more: 0.61-1.02), of 64
+// and 96 0.6-0.93 over 1100 keys, up to 1.13 under.
+static bool attn_f32_shared(int hd, double tiles, int reach, bool long_portions) {
+    if (hd > 128 || reach <= 32) return false;
+    if (hd <= 32) return true;
+    if (tiles <= (reach <= 64 ? 0.25 : reach <= 256 ? 0.5 : hd <= 96 ? 1.0 : 0.75)) return true;
+    return reach > 256 && (long_portions || (hd <= 96 && reach > 1100));
+}
+
+// Takes the entries with several tokens (all entries when skip_single is 0).  max_seq_len, n_single: what the host knows of the
+// entries (an upper bound of their lengths, how many bring one token), or 0 and -1.  Returns 1 when it took them,
 // 0 when the shape is not its own (the caller then walks), -1 on error.
 int llmrs_attention_f32_mfma(hipStream_t stream, const float* q, float* out, const float* k_cache, const float* v_cache,
                              const int* block_table, const int* positions, const int* q_starts, int n_entries,
-                             int skip_single, const AttnArgs& a) {
+                             int skip_single, int max_seq_len, int n_single, const AttnArgs& a) {
     int G = a.n_heads / a.n_kv_heads * a.maps;
     if (a.v_dim != a.head_dim || (a.dist_r1 != nullptr && a.dist_r2 != nullptr)) return 0;
     if (a.head_dim % 32 || a.head_dim > 256 || a.page_size % 4 || G > 32 || q_starts == nullptr) return 0;
@@ -346,15 +362,24 @@ int llmrs_attention_f32_mfma(hipStream_t stream, const float* q, float* out, con
         return 0;
     int tpt = 32 / G;
     long tiles = a.n_tokens / tpt + n_entries;
-    const bool shared = a.head_dim <= 128;
+    // The bound on the lengths holds for single tokens too, whose caches may be longer than the portions': beside them (or where
+    // the host does not say) a portion reaches as many keys as it has tokens, at least.
+    const int alone = skip_single && n_single > 0 ? min(n_single, n_entries - 1) : 0, mean = (a.n_tokens - alone) / max(1, n_entries - alone);
+    int reach = n_single == 0 && max_seq_len > 0 ? max_seq_len : mean;
+    if (a.window > 0) reach = min(reach, a.window + tpt + 31 + a.keep_first);
+    if (a.mask_chunk > 0) reach = min(reach, a.mask_chunk);
+    const double waves = (double)(a.n_tokens / tpt + n_entries) * a.n_kv_heads / (4.0 * llmrs_compute_units());
+    const bool shared = attn_f32_shared(a.head_dim, waves, reach, mean >= 512);
     long blocks = (shared ? tiles : (tiles + 3) / 4) * a.n_kv_heads;
     if (blocks > 0x7fffffffL) return 0;
     switch (a.head_dim) {
-#define TILES(HD, MM) attn_f32_tiles_kernel<HD, MM, (HD <= 128)><<<(int)blocks, 256, 0, stream>>>(q, out, k_cache, v_cache, block_table, positions, q_starts, n_entries, a, G, tpt, skip_single)
+#define TILES_(HD, MM, SS) attn_f32_tiles_kernel<HD, MM, SS><<<(int)blocks, 256, 0, stream>>>(q, out, k_cache, v_cache, block_table, positions, q_starts, n_entries, a, G, tpt, skip_single)
+#define TILES(HD, MM) do { if (shared) TILES_(HD, MM, (HD <= 128)); else TILES_(HD, MM, false); } while (0)
 #define CASE(HD) case HD: if (a.maps == 2) TILES(HD, 2); else TILES(HD, 1); break;
         CASE(32) CASE(64) CASE(96) CASE(128) CASE(160) CASE(192) CASE(224) CASE(256)
 #undef CASE
 #undef TILES
+#undef TILES_
         default: return 0;
     }
     hipError_t err = hipGetLastError();

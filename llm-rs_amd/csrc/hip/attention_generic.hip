@@ -433,7 +433,7 @@ static int launch_generic(hipStream_t stream, const T* q, T* out, const T* k_cac
         // 32-bit: entries with several tokens go to the matrix cores where the shape allows
         if (!only_single && allow_mfma) {
             int took = llmrs_attention_f32_mfma(stream, q, out, k_cache, v_cache, block_table, positions, q_starts, n_entries,
-                                                split ? 1 : 0, a);
+                                                split ? 1 : 0, max_seq_len, n_single, a);
             if (took < 0) return -1;
             tiles_took = took == 1;
         }

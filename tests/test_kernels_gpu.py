@@ -698,6 +698,43 @@ def test_attention_float32_portions_share_their_keys_over_waves(hd, n_heads, n_k
         at += len(pos[r])
 
 
+@pytest.mark.parametrize("hd,n_heads,n_kv,counts,start,window", [
+    # 32 keys or fewer, and more; up to a quarter of a wave to a SIMD and 64 keys, and beyond; half a wave and 256 keys, and beyond
+    (64, 32, 8, [30] * 3, 0, 0), (32, 32, 8, [33] * 9, 0, 0), (64, 32, 8, [40] * 5, 0, 0), (64, 32, 8, [40] * 6, 0, 0),
+    (128, 32, 8, [200] * 2, 0, 0), (128, 32, 8, [200] * 3, 0, 0), (96, 24, 8, [130] * 4, 20, 0), (96, 24, 8, [130] * 5, 20, 0),
+    # more keys: three quarters of a wave of heads of 128, one of 64; long portions; a window; single tokens beside a portion
+    (128, 32, 8, [300] * 2, 400, 0), (128, 32, 8, [300] * 3, 400, 0), (64, 32, 8, [240] * 4, 600, 0), (64, 32, 8, [260] * 4, 600, 0),
+    (128, 32, 8, [600, 520], 0, 0), (64, 32, 8, [1023], 100, 0), (64, 32, 8, [600], 100, 50), (128, 8, 2, [1, 1, 70, 1], 300, 0)])
+def test_attention_float32_portions_by_number_of_tiles(hd, n_heads, n_kv, counts, start, window):
+    """Four waves or one for a tile of columns, by how many tiles there are and how many keys they see: both sides of each line."""
+    lens = [start + c for c in counts]
+    case = PagedCase(torch.float32, lens, n_heads, n_kv, hd, 16, seed=81)
+    g = torch.Generator().manual_seed(12)
+    qs, pos = [torch.randn((c, n_heads, hd), generator=g) for c in counts], [list(range(start, n)) for n in lens]
+    got, at = case.run(qs, pos, window=window, n_single=counts.count(1)), 0
+    for r, c in enumerate(counts):
+        some = sorted({0, c - 1, min(c - 1, 31 + 7 * r), c // 2})
+        ref = case.reference(r, qs[r][some], [pos[r][i] for i in some], window=window)
+        assert ((got[at:at + c][some].double() - ref).abs() <= out_tol(ref, torch.float32, 2e-6)).all(), (r, c)
+        at += c
+
+
+def test_attention_float32_short_portions_do_not_wait_for_idle_waves():
+    """64 portions of 16 tokens take an eighth of the time of one of 1024, whose keys are 32 times as many (four waves to a tile,
+    three of them without a key, took 0.4 of it)."""
+    heads, kv, hd, k, calls = 32, 8, 128, kernels(), []
+    ints = lambda v: torch.tensor(list(v), dtype=torch.int32, device=DEV)
+    q, kc, vc = (rnd(shape, torch.float32, 1) for shape in ((1024, heads * hd), (64, kv, 16, hd), (64, kv, hd, 16)))
+    out = torch.empty_like(q)
+    for n in (64, 1):
+        each = 1024 // n
+        table, entry, pos = ints(range(64)).view(n, -1).contiguous(), ints(i // each for i in range(1024)), ints(i % each for i in range(1024))
+        starts, lens = ints(range(0, 1025, each)), ints([each] * n)
+        calls.append(lambda table=table, entry=entry, pos=pos, starts=starts, lens=lens, each=each:
+                     k.attention(q, out, kc, vc, table, entry, pos, starts, lens, heads, kv, hd, 16, 64, 0, hd ** -0.5, None, each, 0))
+    assert min(short / long for short, long in (replay_time(*calls) for _ in range(3))) <= 0.25
+
+
 @pytest.mark.parametrize("portion", [False, True])
 def test_attention_long_caches_with_a_window(portion):
     """Two decoding requests over long caches with a window of 8500 keys (more than 64 ranges to merge, the first of
