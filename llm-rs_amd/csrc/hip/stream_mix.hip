@@ -133,21 +133,24 @@ __global__ void group_rmsnorm_kernel(T* __restrict__ out, float* __restrict__ x,
     }
 }
 
-// The same with the row held in registers, four features a piece, for up to four streams and groups of whole 256 features (a
-// wave's piece of a row then lies in one group): everything the row needs is asked for at once, a group's squares are added by
-// waves side by side and meet behind one barrier, where the kernel above walks the groups one after the other between two
-// barriers each and puts the row through LDS.  What bounds it with few rows is its chain of trips; with many, the streams'
-// bytes.  (4 rows of 2048 in four streams, 4 groups: mix and norm as two launches 4.7 + 8.7 us, this one with the mix 6.4; 2048 rows 35 -> 30.)
+// The same with the row held in registers, four features a piece, for up to four streams and groups of whole 256 features:
+// everything the row needs is asked for at once, and the groups' squares are added by waves side by side, behind two barriers
+// in all, where the kernel above walks the groups one after the other between two barriers each.  `slots` is the other kernel's block
+// size at this width: a group's squares are added in its order (slot i takes features i, i + slots, ...; 64 slots at a time
+// across a wave; those sums in order), so the two give the same bits.  What bounds it with few rows is its chain of trips; with
+// many, the streams' bytes.  (4 rows of 2048 in four streams, 4 groups: mix and norm as two launches 11.7 us, this one with the mix
+// 6.4; 2048 rows 31 -> 29.)
 template <class T, bool MIX, int HELD>
 __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__ out, float* __restrict__ x, size_t stream_stride, int n_streams,
                                                                  const float* __restrict__ w_in, const float* __restrict__ weight,
                                                                  const int* __restrict__ rows, int D, int groups, float eps,
                                                                  float* zero, float* __restrict__ combined,
-                                                                 const float* __restrict__ mix, const float* __restrict__ w_out, const float* y) {
+                                                                 const float* __restrict__ mix, const float* __restrict__ w_out, const float* y, int slots) {
     constexpr int SMAX = 4;
-    __shared__ float partial[64];                    // a sum of squares for every 256 features
+    extern __shared__ __attribute__((aligned(16))) float row[];          // [D]
+    __shared__ float partial[HELD * 32];             // a sum of squares for every 64 slots of every group (D / 64 at most)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    const int n4 = D / 4, per_group = D / groups / 256;
+    const int n4 = D / 4, gs = D / groups, per_group = min(slots, gs) / 64;
     const int r = rows ? rows[blockIdx.x] : blockIdx.x;
     float* src = x + (size_t)r * D;
     const bool plain = n_streams == 1 && w_in == nullptr;
@@ -189,28 +192,32 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
                 }
             }
         }
-        float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             u[i][j] = plain ? v[i][0][j] : (w_in ? w_in[0] : 1.0f) * v[i][0][j];
 #pragma unroll
             for (int s = 1; s < SMAX; ++s)
                 if (s < n_streams) u[i][j] = fmaf(w_in ? w_in[s] : 1.0f, v[i][s][j], u[i][j]);
-            ss = fmaf(u[i][j], u[i][j], ss);
         }
-        ss = wave_sum(ss);                            // (pieces past the row hold zeros)
-        const int part = i * waves + wave;
-        if (lane == 0 && part < D / 256) partial[part] = ss;
+        if (idx < n4) store4(row + 4 * idx, u[i]);
+    }
+    __syncthreads();
+    for (int part = wave; part < groups * per_group; part += waves) {
+        const float* group = row + part / per_group * gs;
+        float ss = 0.0f;
+        for (int d = part % per_group * 64 + lane; d < gs; d += slots) ss = fmaf(group[d], group[d], ss);
+        ss = wave_sum(ss);
+        if (lane == 0) partial[part] = ss;
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
         const int idx = i * blockDim.x + threadIdx.x;
         if (idx >= n4) continue;
-        const int first = (i * waves + wave) / per_group * per_group;
+        const int first = 4 * idx / gs * per_group;          // (a piece lies in one group: their size is a multiple of four)
         float total = 0.0f, o[4], z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         for (int p = 0; p < per_group; ++p) total += partial[first + p];
-        const float inv = 1.0f / sqrtf(total / (float)(D / groups) + eps);
+        const float inv = 1.0f / sqrtf(total / (float)gs + eps);
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = u[i][j] * inv * wt[i][j];
         store4(out + (size_t)blockIdx.x * D + 4 * idx, o);
@@ -270,10 +277,11 @@ extern "C" int llmrs_group_rmsnorm(hipStream_t stream, int dtype, void* out, flo
     if (dtype != LLMRS_F32 && dtype != LLMRS_BF16) return llmrs_fail("group_rmsnorm: unknown dtype %d", dtype);
     int wide = D % 4 == 0 && stream_stride % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)y & 15) == 0
                && ((uintptr_t)zero & 15) == 0 && ((uintptr_t)combined & 15) == 0;
+    const int threads = D > 8192 ? 1024 : D > 2048 ? 512 : 256;
     if (wide && n_streams <= 4 && D / groups % 256 == 0 && D <= 8192 && ((uintptr_t)weight & 15) == 0) {
         int held_threads = min(512, D / 4);           // (D is a multiple of 256: whole waves)
-#define HELD(T, MIX, N) group_rmsnorm_held_kernel<T, MIX, N><<<n_rows, held_threads, 0, stream>>>((T*)out, x, (size_t)stream_stride, n_streams, w_in, weight, \
-                                                                                                rows, D, groups, eps, zero, combined, mix, w_out, y)
+#define HELD(T, MIX, N) group_rmsnorm_held_kernel<T, MIX, N><<<n_rows, held_threads, D * sizeof(float), stream>>>((T*)out, x, (size_t)stream_stride, n_streams, w_in, weight, \
+                                                                                                rows, D, groups, eps, zero, combined, mix, w_out, y, threads)
 #define BY_WIDTH(T, MIX) do { if (D <= 2048) HELD(T, MIX, 1); else if (D <= 4096) HELD(T, MIX, 2); else HELD(T, MIX, 4); } while (0)
         if (dtype == LLMRS_F32) { if (mix) BY_WIDTH(float, true); else BY_WIDTH(float, false); }
         else { if (mix) BY_WIDTH(bf16, true); else BY_WIDTH(bf16, false); }
@@ -282,7 +290,6 @@ extern "C" int llmrs_group_rmsnorm(hipStream_t stream, int dtype, void* out, flo
         LLMRS_LAUNCH_CHECK("group_rmsnorm");
         return 0;
     }
-    int threads = D > 8192 ? 1024 : D > 2048 ? 512 : 256;
     size_t lds = (size_t)(D + groups + 16 + MAX_STREAMS * MAX_STREAMS + MAX_STREAMS) * sizeof(float);
 #define NORM(T, MIX, SMAX) group_rmsnorm_kernel<T, MIX, SMAX><<<n_rows, threads, lds, stream>>>((T*)out, x, (size_t)stream_stride, n_streams, w_in, weight, \
                                                                                           rows, D, groups, eps, zero, combined, mix, w_out, y, wide)

@@ -343,6 +343,28 @@ def test_rows_held_in_registers_are_mixed_and_normed_in_one_launch(rows, streams
         assert torch.equal(one[0], out[-1])
 
 
+@pytest.mark.parametrize("rows,streams,width,groups", [(1, 4, 2048, 4), (5, 1, 256, 1), (3, 2, 768, 3), (130, 3, 3072, 2), (4, 4, 8192, 8), (3, 4, 8192, 32),
+                                                       (2, 4, 2304, 9), (2, 2, 2304, 1), (7, 4, 2048, 1), (3, 3, 4096, 2)])
+def test_rows_held_in_registers_get_the_bits_of_the_general_norm(rows, streams, width, groups):
+    """A group's squares are added in one order whether or not a block holds its row in registers (a weight whose rows do not begin
+    on 16 bytes is the general kernel's), with and without a mix: groups shorter and longer than a block, whole and cut."""
+    from llm_rs_amd import kernels
+    k, g = kernels(), torch.Generator(device="cuda").manual_seed(rows + width)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    x, y, mix, w_in, w_out = rnd(streams, rows, width), rnd(rows, width), rnd(streams, streams), rnd(streams), rnd(streams)
+    room = rnd(width + 1)
+    weights = room[1:], room[1:].clone()
+    assert weights[0].data_ptr() % 16 and weights[1].data_ptr() % 16 == 0
+    for dtype in (torch.float32, torch.bfloat16):
+        for with_mix in (False, True):
+            got = []
+            for weight in weights:
+                streams_now, out = x.clone(), torch.empty((rows, width), dtype=dtype, device="cuda")
+                k.group_rmsnorm(out, streams_now, weight, 1e-5, groups, w_in=w_in, mix=(mix, w_out, y) if with_mix else None)
+                got.append((out, streams_now))
+            assert all(torch.equal(a, b) for a, b in zip(*got)), (dtype, with_mix)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("entries,channels,states", [(1, 64, 16), (4, 4096, 16), (3, 70, 5), (2, 100, 1), (5, 130, 9)])
 def test_single_tokens_through_the_scan_equal_the_walk(entries, channels, states, dtype):
