@@ -586,7 +586,9 @@ def test_attention_chunk_rule_and_its_scratch():
         assert need >= len(lens) * n_heads * -(-2048 // c) * (hd + 2)
         got = case.run(qs, pos, scratch_floats=need, bound=2048, n_single=len(lens), single_keys=keys)
         for r in range(len(lens)):
-            assert (got[r].float() - refs[r]).abs().max() <= 2e-2, f"{keys} keys, request {r}"
+            # (a probability rounded to bfloat16 is off by 2^-9 of itself at most, so an element by some 2^-9 of the values' spread,
+            # 0.04 to 0.3 here; a tile of 32 keys left out of 1500 moves elements by 0.005 and the largest by 0.02)
+            assert ((got[r].float() - refs[r]).abs() <= out_tol(refs[r], torch.bfloat16, 2e-3)).all(), f"{keys} keys, request {r}"
     assert len(seen) >= 2, "the case itself: more than one chunk"
 
 
