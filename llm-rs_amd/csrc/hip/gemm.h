@@ -87,18 +87,19 @@ __device__ __forceinline__ void epilogue_store(int epi, void* out, int ldc, int 
     else if (epi == LLMRS_EPI_ACCUM_F32) ((float*)out)[(size_t)m * ldc + n] += v;
 }
 
+// 32-bit products on the matrix cores, tiles (gemm_f32_tiles.hip).  K % 32 == 0 and 16-byte aligned rows: the caller's to check.
+// 0, or -1 on error.
+int llmrs_gemm_f32_tiles(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi);
+// The product left as the parts of its sum over k, [parts][M][N] 32-bit in `workspace` (gemm_mfma.hip): the number of
+// parts, 0 when this product would not be split (nothing launched), -1 on error.
+int llmrs_gemm_bf16_split_parts(hipStream_t stream, const bf16* A, int lda, const bf16* W, int M, int N, int K,
+                                void* workspace, size_t workspace_bytes);
 // The 16-byte-load kernels on MFMA (gemm_mfma.hip).  Return 1 when they took the
 // product, 0 when its shape or alignment is not theirs, -1 on error.
 // workspace: device memory for the partial sums of products that split K over blocks (may be null).
 // qkv: needed when epi is LLMRS_EPI_QKV; such a call is taken only by the kernels that fuse it.
 // scale, next: see RowScale and NextNorm; both only where llmrs_gemm_defers_norm(M, N, K) holds (next: with
 // LLMRS_EPI_ACCUM_F32 only), or next with eps where llmrs_gemm_norms_whole(M, N, K) holds.
-// The product left as the parts of its sum over k, [parts][M][N] 32-bit in `workspace` (gemm_mfma.hip): the number of
-// parts, 0 when this product would not be split (nothing launched), -1 on error.
-// 32-bit products on the matrix cores, tiles (gemm_f32_tiles.hip).  K % 32 == 0 and 16-byte aligned rows: the caller's to check.
-int llmrs_gemm_f32_tiles(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi);
-int llmrs_gemm_bf16_split_parts(hipStream_t stream, const bf16* A, int lda, const bf16* W, int M, int N, int K,
-                                void* workspace, size_t workspace_bytes);
 int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc,
                          int M, int N, int K, int epi, void* workspace, size_t workspace_bytes,
                          const QkvEpilogue* qkv = nullptr, const RowScale* scale = nullptr, const NextNorm* next = nullptr);

@@ -1106,10 +1106,6 @@ class HipKernels(Kernels):
                   _p(state), state.stride(0), _p(q_starts), _p(slots), _p(token_entry), slots.numel(), T, channels, K, int(silu), _p(out), out.stride(0),
                   _p(out32), 0 if out32 is None else out32.stride(0), int(longest))
 
-    def causal_conv_silu(self, sums: torch.Tensor, taps: torch.Tensor, bias, state: torch.Tensor, q_starts, slots, token_entry,
-                         channels: int, out: torch.Tensor) -> None:
-        self.causal_conv(sums, taps, bias, state, q_starts, slots, token_entry, channels, out, silu=True)
-
     def gated_unit_scan(self, u: torch.Tensor, gates: torch.Tensor, size: int, bias_r, bias_i, rate: torch.Tensor, y: torch.Tensor, bias_y,
                         state: torch.Tensor, q_starts, slots, out: torch.Tensor, longest: int = 0, carry: Optional[torch.Tensor] = None) -> None:
         """A real-gated linear recurrent unit, per channel: log a = rate sigmoid(gate_r + bias_r); s <- a s + sqrt(1 - a^2)

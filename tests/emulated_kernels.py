@@ -346,9 +346,6 @@ class EmulatedKernels(Kernels):
     def add_bias_rows(self, rows, bias):
         rows.add_(bias)
 
-    def causal_conv_silu(self, sums, taps, bias, state, q_starts, slots, token_entry, channels, out):
-        self.causal_conv(sums, taps, bias, state, q_starts, slots, token_entry, channels, out, silu=True)
-
     def causal_conv(self, sums, taps, bias, state, q_starts, slots, token_entry, channels, out, in_bias=None, silu=False, out32=None, longest=0):
         sums = sums[:, :channels] + (in_bias if in_bias is not None else 0.0)
         K = taps.shape[1]
