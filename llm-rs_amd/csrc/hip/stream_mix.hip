@@ -202,12 +202,25 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
         if (idx < n4) store4(row + 4 * idx, u[i]);
     }
     __syncthreads();
-    for (int part = wave; part < groups * per_group; part += waves) {
-        const float* group = row + part / per_group * gs;
-        float ss = 0.0f;
-        for (int d = part % per_group * 64 + lane; d < gs; d += slots) ss = fmaf(group[d], group[d], ss);
-        ss = wave_sum(ss);
-        if (lane == 0) partial[part] = ss;
+    for (int part = wave; part < groups * per_group; part += 2 * waves) {      // (two at a time: a sum across a wave is a chain)
+        float ss[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int p = part + t * waves;
+            const float* group = row + p / per_group * gs;
+            if (p < groups * per_group)
+                for (int d = p % per_group * 64 + lane; d < gs; d += slots) ss[t] = fmaf(group[d], group[d], ss[t]);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const float other[2] = {__shfl_xor(ss[0], off, 64), __shfl_xor(ss[1], off, 64)};
+            ss[0] += other[0];
+            ss[1] += other[1];
+        }
+        if (lane == 0) {
+            partial[part] = ss[0];
+            if (part + waves < groups * per_group) partial[part + waves] = ss[1];
+        }
     }
     __syncthreads();
 #pragma unroll
@@ -278,7 +291,14 @@ extern "C" int llmrs_group_rmsnorm(hipStream_t stream, int dtype, void* out, flo
     int wide = D % 4 == 0 && stream_stride % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)y & 15) == 0
                && ((uintptr_t)zero & 15) == 0 && ((uintptr_t)combined & 15) == 0;
     const int threads = D > 8192 ? 1024 : D > 2048 ? 512 : 256;
-    if (wide && n_streams <= 4 && D / groups % 256 == 0 && D <= 8192 && ((uintptr_t)weight & 15) == 0) {
+    // The row in registers from 1024 features on (a row of 256 leaves a block one wave, which adds the groups' squares alone: 4.4
+    // against 4.1 us), and with a mix of more than 2048 up to one block to a unit: the registers that the old and the
+    // new streams take leave a unit one block of 8192 features, and three of 4096, where the general kernel has four (held against
+    // general, bfloat16, four streams: 128 rows of 8192 in 8 groups 18.8 against 21.1 us, 300 38.0 against 29.4, 1000 85 against 57,
+    // 2048 178 against 124; 1000 of 3072 24.8 against 24.0; 1000 of 2048 16.1 against 20.9).
+    const bool in_registers = wide && n_streams <= 4 && D / groups % 256 == 0 && D >= 1024 && D <= 8192 && ((uintptr_t)weight & 15) == 0 &&
+                              (mix == nullptr || D <= 2048 || n_rows <= llmrs_compute_units());
+    if (in_registers) {
         int held_threads = min(512, D / 4);           // (D is a multiple of 256: whole waves)
 #define HELD(T, MIX, N) group_rmsnorm_held_kernel<T, MIX, N><<<n_rows, held_threads, D * sizeof(float), stream>>>((T*)out, x, (size_t)stream_stride, n_streams, w_in, weight, \
                                                                                                 rows, D, groups, eps, zero, combined, mix, w_out, y, threads)

@@ -104,8 +104,8 @@ class GroupRMSNorm(Norm):
     def forward_streams(self, ctx, hs, w_in, out, rows=None, zero=None):
         # A mix of these streams that is still to be done runs in the norm's launch, when the norm reads every row
         # and there are rows enough to fill the device with one block a row (the mix alone spreads a row over blocks),
-        # or a block holds its row in registers (up to four streams, groups of whole 256 features).
-        held = hs.shape[0] <= 4 and self.size <= 8192 and self.size // self.groups % 256 == 0
+        # or a block holds its row in registers (up to four streams, rows of 1024 features and more in groups of whole 256).
+        held = hs.shape[0] <= 4 and 1024 <= self.size <= 8192 and self.size // self.groups % 256 == 0
         mix = ctx.take_streams_mix(hs) if rows is None and (held or hs.shape[1] >= self.FUSE_MIX_FROM_ROWS) else None
         if mix is None:
             ctx.flush_streams()
