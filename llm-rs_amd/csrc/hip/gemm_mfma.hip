@@ -1308,25 +1308,32 @@ static int launch_tiles_128(hipStream_t stream, const bf16* A, int lda, const bf
 }
 // From 512 rows on, where square large tiles would not fill the device: tiles of 256 x 128 on four waves, a block to a unit, or
 // the 128 x 128 tiles above, two to a unit, by the time either takes: the k-tiles that a unit works through, round after
-// round, times what one takes there (measured: 1.0 us for a 256 x 128 k-tile of 64, 1.25 for two of 128 x 128, 1.05 for
-// one that is alone).  Both split k over blocks until the device is full.  Measured, 128 x 128 -> 256 x 128: 2032 rows
-// 2048 x 8192 in 2 parts 81 -> 71 us, 3072 x 2048 35 -> 29; 1024 rows 4096 x 14336 in 2 parts 140 -> 111; 512 rows in 4
-// parts 78 -> 64.  (The two operands' sizes, under 4 GB, are looked at where it is launched.)
+// round, times what one takes there (measured, us: 1.0 for a 256 x 128 k-tile of 64, 1.25 for two of 128 x 128, 1.05 for
+// one that is alone), and for a block of the first what its way in and out takes beyond what two blocks of a unit hide from each other:
+// 1.5 where it stores 16-bit results, none where 32-bit ones, 0.8 where gated halves, 6 where it adds to 32-bit ones, and 3.5 where it leaves
+// a part of the sum, 5 of a weight of fewer than 2048 features (each XCD then reads all rows).  Both split k over blocks until
+// the device is full.  Measured, 128 x 128 -> 256 x 128: 2032 rows 2048 x 8192 in 2 parts 81 -> 71 us, 3072 x 2048
+// 35 -> 29; 1024 rows 4096 x 14336 in 2 parts 140 -> 111; 512 rows in 4 parts 78 -> 64; but 600 rows 4096 x 128
+// added to 32-bit 7.5 -> 12 us, 2049 rows 4096 x 1024 40 -> 48, 640 rows 512 x 2048 in 4 parts 15.2 -> 17.7.  (512 to 6000 rows of 160 to 8192
+// features, k from 64 to 4096, every epilogue, against 128 x 128 alone: none slower by more than 3 %.  Both sum in one
+// order.  The two operands' sizes, under 4 GB, are looked at where it is launched.)
 struct MidTiles {
     bool four;
     int splits;
+    double time;
 };
-static MidTiles mid_tiles(int M, int N, int K, bool may_split = true) {
-    if (M < 512 || K % 64) return MidTiles{false, may_split ? tiled_splits(M, N, K) : 1};
-    const int cus = llmrs_compute_units(), nk = K / 64;
-    const long tall = (long)ceil_div(M, 256) * ceil_div(N, 128), small = (long)ceil_div(M, 128) * ceil_div(N, 128);
+static MidTiles mid_tiles(int M, int N, int K, int epi, bool may_split = true) {
+    const int cus = llmrs_compute_units(), nk = K / 64, s = may_split ? tiled_splits(M, N, K) : 1;
+    const long tall = (long)ceil_div(M, 256) * ceil_div(N, 128), small = (long)ceil_div(M, 128) * ceil_div(N, 128) * s;
+    const long last = small % (2L * cus);
+    const double small_time = (1.25 * (double)(small / (2L * cus)) + (last == 0 ? 0.0 : last <= cus ? 1.05 : 1.25)) * ceil_div(nk, s);
+    if (M < 512 || K % 64) return MidTiles{false, s, small_time};
     int z = 1;
     while (may_split && tall * z * 2 <= cus && z < 16 && nk / (z * 2) >= 8 && (z * 2 - 1) * ceil_div(nk, z * 2) < nk) z *= 2;
-    const int s = may_split ? tiled_splits(M, N, K) : 1;
-    const double tall_time = (double)ceil_div(tall * z, (long)cus) * ceil_div(nk, z);
-    const double small_time = (small * s <= cus ? 1.05 : 1.25 * ceil_div(small * s, 2L * cus)) * ceil_div(nk, s);
-    if (tall_time <= small_time) return MidTiles{true, z};
-    return MidTiles{false, s};
+    const double in_and_out = z > 1 ? (N >= 2048 ? 3.5 : 5.0) : epi == LLMRS_EPI_ACCUM_F32 ? 6.0 : epi == LLMRS_EPI_STORE_F32 ? 0.0 : epi_gated(epi) ? 0.8 : 1.5;
+    const double tall_time = (double)ceil_div(tall * z, (long)cus) * (ceil_div(nk, z) + in_and_out);
+    if (tall_time <= small_time) return MidTiles{true, z, tall_time};
+    return MidTiles{false, s, small_time};
 }
 // 17..64 rows on a weight of middling width (more than 4096 features, fewer than the wide ones that
 // get blocks of many feature tiles): the 128 x 128 tiles with k split over blocks read the tokens'
@@ -1347,7 +1354,7 @@ extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
         return s > 1 ? (long)s * (M % 256) * N : 0;
     }
     if (M > 64 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160) {
-        int s = mid_tiles(M, N, K).splits;
+        int s = mid_tiles(M, N, K, LLMRS_EPI_ACCUM_F32).splits;      // (no epilogue's plan has more parts)
         long own = s > 1 ? (long)s * M * N : 0;
         // a few rows beyond whole 128-row tiles may go to the kernel for few rows, and the whole tiles be split then
         int over128 = M % 128;
@@ -1385,7 +1392,7 @@ extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
 extern "C" int llmrs_gemm_norms_whole(int M, int N, int K) {
     if (!(M > 16 && N >= 4 && N % 4 == 0 && N <= 16384 && K % 8 == 0)) return 0;
     if (M <= 256) return llmrs_gemm_workspace_floats(M, N, K) > 0;
-    return K % 64 == 0 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160 && mid_tiles(M, N, K).splits > 1;
+    return K % 64 == 0 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160 && mid_tiles(M, N, K, LLMRS_EPI_ACCUM_F32).splits > 1;
 }
 
 // The product as parts of its sum over k, [parts][M][N] 32-bit in `workspace`, for a caller that adds them up itself
@@ -1563,7 +1570,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                      : small ? launch_pingpong<256, 256, 2, 4, true>(stream, A, lda, W, out, ldc, M, n_split, K, epi)
                              : launch_pingpong<256, 256, 2, 4, false>(stream, A, lda, W, out, ldc, M, n_split, K, epi);
                 if (rc == 0) {
-                    if (four && fourwave_takes(epi, out_rest, ldc, N - n_split) && mid_tiles(M, N - n_split, K, false).four)
+                    if (four && fourwave_takes(epi, out_rest, ldc, N - n_split) && mid_tiles(M, N - n_split, K, epi, false).four)
                         rc = launch_fourwave<256, 128>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
                     else
                         rc = launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
@@ -1584,16 +1591,16 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             // The same for the 128 x 128 tiles, whose blocks run two to a compute unit: a few rows beyond whole
             // tiles that cost them another round of the device, or the split of k that filled it, go to the kernel
             // for few rows (the o and down products of the 8B shape: 2049 rows 526 -> about 350 us, 1025 rows 287 -> 240).
-            // Counted in k-tiles that a place works through, round after round.
+            // By the time of the plans for all rows and for the whole tiles' (us, mid_tiles).
             int over128 = M % 128;
             if (M >= 1024 && over128 > 0 && over128 <= 64 && !whole && next == nullptr && scale == nullptr) {
                 auto walk = [&](int rows) {
-                    int s = mid_tiles(rows, N, K).splits;
-                    if (s > 1 && (workspace == nullptr || workspace_bytes < (size_t)s * rows * N * sizeof(float))) s = 1;
-                    long blocks = (long)ceil_div(rows, 128) * ceil_div(N, 128) * s;
-                    return ceil_div(blocks, (long)cus * 2) * (K / 64 / s);
+                    MidTiles plan = mid_tiles(rows, N, K, epi);
+                    if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < (size_t)plan.splits * rows * N * sizeof(float)))
+                        plan = mid_tiles(rows, N, K, epi, false);
+                    return plan.time;
                 };
-                if (walk(M) - walk(M - over128) >= 32) {
+                if (walk(M) - walk(M - over128) >= 30.0) {
                     size_t elt = (epi == LLMRS_EPI_STORE_F32 || epi == LLMRS_EPI_ACCUM_F32) ? sizeof(float) : sizeof(bf16);
                     int whole_rows = M - over128;
                     rc = llmrs_gemm_bf16_mfma(stream, A, lda, W, out, ldc, whole_rows, N, K, epi, workspace, workspace_bytes, qkv);
@@ -1604,9 +1611,9 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             }
             // (a wider tile brings less into a unit for the same work: a k-step of 256 x 128 48 KB, of two 128 x 128 64 KB)
             const bool small4 = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
-            MidTiles plan = mid_tiles(M, N, K);
+            MidTiles plan = mid_tiles(M, N, K, epi);
             if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)))
-                plan = mid_tiles(M, N, K, false);
+                plan = mid_tiles(M, N, K, epi, false);
             const int splits = plan.splits;
             if (plan.four && small4 && splits > 1) {
                 rc = launch_fourwave_epi<256, 128, LLMRS_EPI_STORE_F32>(stream, A, lda, W, workspace, N, M, N, K, LLMRS_EPI_STORE_F32, splits);
