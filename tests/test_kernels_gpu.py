@@ -520,7 +520,8 @@ def test_gemm_float32_forms_by_shape(M, N, K):
         assert (err <= out_tol(ref, torch.float32, floor)).all(), (epi, float(err.max()))
 
 
-@pytest.mark.parametrize("M,N,K", [(2200, 6144, 64), (2816, 4352, 64), (4700, 8200, 64), (2048, 6160, 192), (1800, 6136, 64)])
+@pytest.mark.parametrize("M,N,K", [(2200, 6144, 64), (2816, 4352, 64), (4700, 8200, 64), (2048, 6160, 192), (1800, 6136, 64),
+                                   (2200, 6144, 1024), (2816, 4352, 1024), (2048, 6160, 1088)])
 def test_gemm_large_tiles_of_many_rows(M, N, K):
     """Grids of large tiles with more rows than an XCD takes at a time, numbers of tiles that eight does not divide, and 256 x 192
     tiles cut by N: every tile of the output is written, once (a += shows a tile written twice)."""
