@@ -21,17 +21,22 @@ enum LlmrsEpilogue {
 // The constants of the gated epilogue with constants lie in a table in device memory, a slot for each set of them that a
 // model has (llmrs_glu_clamp_slot, called when a feed-forward takes its weights, writes a slot once and for all); the
 // epilogue's number says which slot, so no kernel's argument list holds them and a recorded step finds them as any
-// other does.  Each source file with such kernels has the table for itself (the variable is static) and a function that
-// writes a slot of it, which llmrs_glu_clamp_slot calls.
+// other does.  Each source file that includes this has the table for itself (the variable is static), and by including
+// it puts it on the list that llmrs_glu_clamp_slot writes through: no file can read a table that nothing writes.
 #define LLMRS_GLU_SLOTS 256
 struct GluClamp {
     float limit, alpha, cubic, up_add;
 };
 static __device__ GluClamp llmrs_glu_clamp[LLMRS_GLU_SLOTS];
 static __global__ void glu_clamp_store_kernel(int slot, GluClamp p) { llmrs_glu_clamp[slot] = p; }
-// (gemm_mfma.hip, gemm_f32_tiles.hip: the same slot of that file's table)
-void llmrs_glu_clamp_store_mfma(hipStream_t stream, int slot, GluClamp p);
-void llmrs_glu_clamp_store_f32_tiles(hipStream_t stream, int slot, GluClamp p);
+struct GluClampTable {
+    void (*store)(hipStream_t stream, int slot, GluClamp p);
+    GluClampTable* next;
+};
+extern GluClampTable* llmrs_glu_clamp_tables;        // gemm_simple.hip
+static void glu_clamp_store(hipStream_t stream, int slot, GluClamp p) { glu_clamp_store_kernel<<<1, 1, 0, stream>>>(slot, p); }
+static GluClampTable llmrs_glu_clamp_table = {glu_clamp_store, nullptr};
+static const bool llmrs_glu_clamp_listed = (llmrs_glu_clamp_table.next = llmrs_glu_clamp_tables, llmrs_glu_clamp_tables = &llmrs_glu_clamp_table, true);
 
 __host__ __device__ __forceinline__ bool epi_gated(int epi) { return epi == LLMRS_EPI_SWIGLU || epi >= LLMRS_EPI_GLU_CLAMP; }
 // act(gate, up) of the gated epilogues, on 32-bit sums

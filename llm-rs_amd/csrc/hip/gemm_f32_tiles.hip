@@ -12,9 +12,6 @@
 // 3072 x 2048 194 -> 126, 16384 x 2048 660 -> 591 (116 TFLOP/s of 157 nominal).
 #include "gemm_tile.h"
 
-// (the constants of the gated epilogue that this file's products read: see gemm.h)
-void llmrs_glu_clamp_store_f32_tiles(hipStream_t stream, int slot, GluClamp p) { glu_clamp_store_kernel<<<1, 1, 0, stream>>>(slot, p); }
-
 template <int BM, int BN, int WGM, int WGN, int STAGES>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_f32_dma_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
                                                                       void* __restrict__ out, int ldc, int M, int N, int K, int epi) {

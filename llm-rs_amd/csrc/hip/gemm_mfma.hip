@@ -50,7 +50,6 @@ __device__ __forceinline__ float gated_act_fast(const GatedAct& a, float g, floa
     u = fminf(fmaxf(u, -a.limit), a.limit);
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(a.cubic * g * g, g, g) * a.alpha2)) * (u + a.up_add);
 }
-void llmrs_glu_clamp_store_mfma(hipStream_t stream, int slot, GluClamp p) { glu_clamp_store_kernel<<<1, 1, 0, stream>>>(slot, p); }
 
 // ---------------------------------------------------------------------------
 // skinny: C^T[n, m] = sum_k W[n, k] X[m, k]

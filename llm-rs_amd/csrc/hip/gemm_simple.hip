@@ -393,6 +393,12 @@ static bool launch_f32_few_rows(hipStream_t stream, const float* a, int lda, con
 // later product on any stream finds it.  The same set on the same device gets the same slot again.
 #include <mutex>
 #include <vector>
+GluClampTable* llmrs_glu_clamp_tables;               // (null before the first file's table is put on it: no constructor runs for it)
+extern "C" int llmrs_glu_clamp_table_count() {
+    int n = 0;
+    for (const GluClampTable* table = llmrs_glu_clamp_tables; table != nullptr; table = table->next) ++n;
+    return n;
+}
 struct GluSlot { int device; GluClamp p; };
 static std::mutex glu_mutex;
 static std::vector<GluSlot> glu_slots;
@@ -411,9 +417,7 @@ extern "C" int llmrs_glu_clamp_slot(hipStream_t stream, float limit, float alpha
     if (glu_slots.size() >= LLMRS_GLU_SLOTS) { llmrs_fail("glu_clamp_slot: more than %d different sets of constants", LLMRS_GLU_SLOTS); return -1; }
     int slot = (int)glu_slots.size();
     GluClamp p{limit, alpha, cubic, up_add};
-    glu_clamp_store_kernel<<<1, 1, 0, stream>>>(slot, p);
-    llmrs_glu_clamp_store_mfma(stream, slot, p);
-    llmrs_glu_clamp_store_f32_tiles(stream, slot, p);
+    for (const GluClampTable* table = llmrs_glu_clamp_tables; table != nullptr; table = table->next) table->store(stream, slot, p);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) { llmrs_fail("glu_clamp_slot: %s", hipGetErrorString(e)); return -1; }

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import copy
 import math
+import os
 
 import pytest
 import torch
@@ -299,3 +300,17 @@ def test_a_layer_of_each_kind_alone_on_the_host_logic():
         exact = reference(cfg, tensors, requests)
         for name, steps in {"whole": whole(requests), "portions": portions(requests, (2, 5, 3)), "mixed": mixed(requests, live=2)}.items():
             check_rows(replay_cpu(typed, tensors, "float32", 4, steps), exact, requests, 3e-5, f"{layer['type']} {name}")
+
+
+def test_every_kernel_file_with_a_table_of_clamped_constants_is_written_to():
+    """Each file that includes gemm.h has a table of the clamped gated products' constants for itself; all of them are on the list
+    that a slot is written through."""
+    from llm_rs_amd.csrc import build as native
+    folder = os.path.join(native.CSRC, "hip")
+    text = {name: open(os.path.join(folder, name)).read() for name in os.listdir(folder) if name.endswith((".h", ".hip"))}
+    has = {"gemm.h"}
+    while more := {name for name, source in text.items() if name not in has and any(f'#include "{h}"' in source for h in has)}:
+        has |= more
+    files = sorted(name for name in has if name.endswith(".hip"))
+    assert {"gemm_simple.hip", "gemm_mfma.hip", "gemm_f32_tiles.hip"} <= set(files)
+    assert native.load_hip().llmrs_glu_clamp_table_count() == len(files)
