@@ -1110,9 +1110,10 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
     }
     // With gridDim.z > 1 (the epilogue then is STORE_F32, `out` the partial sums [gridDim.z][M][N]) a block takes its share of
     // the k-tiles, a contiguous range; no share is empty (the launcher sees to it).
-    const int share = (K / 64 + gridDim.z - 1) / gridDim.z, k_first = blockIdx.z * share;
-    const int nk = min(share, K / 64 - k_first);
+    int nk = K / 64;
     if (gridDim.z > 1) {
+        const int share = (nk + gridDim.z - 1) / gridDim.z, k_first = blockIdx.z * share;
+        nk = min(share, nk - k_first);
         out = (float*)out + (size_t)blockIdx.z * M * N;
 #pragma unroll
         for (int i = 0; i < A_GROUPS; ++i) oa[i] += k_first * 128;
