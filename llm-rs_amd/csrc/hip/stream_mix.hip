@@ -139,7 +139,7 @@ __global__ void group_rmsnorm_kernel(T* __restrict__ out, float* __restrict__ x,
 // size at this width: a group's squares are added in its order (slot i takes features i, i + slots, ...; 64 slots at a time
 // across a wave; those sums in order), so the two give the same bits.  What bounds it with few rows is its chain of trips; with
 // many, the streams' bytes.  (4 rows of 2048 in four streams, 4 groups: mix and norm as two launches 11.7 us, this one with the mix
-// 6.4; 2048 rows 31 -> 29.)
+// 6.2; 2048 rows 31 -> 28.5.)
 template <class T, bool MIX, int HELD>
 __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__ out, float* __restrict__ x, size_t stream_stride, int n_streams,
                                                                  const float* __restrict__ w_in, const float* __restrict__ weight,
@@ -150,11 +150,12 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
     extern __shared__ __attribute__((aligned(16))) float row[];          // [D]
     __shared__ float partial[HELD * 32];             // a sum of squares for every 64 slots of every group (D / 64 at most)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    const int n4 = D / 4, gs = D / groups, per_group = min(slots, gs) / 64;
+    const int n4 = D / 4, gs = D / groups, log_per = slots >= 512 && gs >= 512 ? 3 : 2, per_group = 1 << log_per;      // (min(slots, gs) / 64: 4 or 8)
     const int r = rows ? rows[blockIdx.x] : blockIdx.x;
     float* src = x + (size_t)r * D;
     const bool plain = n_streams == 1 && w_in == nullptr;
     float v[HELD][SMAX][4], yy[HELD][4], wt[HELD][4], u[HELD][4];
+    int first[HELD];                                 // where a piece's group has its sums (a piece lies in one group: their size is a multiple of four)
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
         const int idx = i * blockDim.x + threadIdx.x;
@@ -165,6 +166,7 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
         }
         if (idx < n4) {
             load4(weight + 4 * idx, wt[i]);
+            first[i] = 4 * idx / gs << log_per;
             if (MIX) load4(y + (size_t)r * D + 4 * idx, yy[i]);
         }
     }
@@ -207,9 +209,9 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int p = part + t * waves;
-            const float* group = row + p / per_group * gs;
+            const float* group = row + (p >> log_per) * gs;
             if (p < groups * per_group)
-                for (int d = p % per_group * 64 + lane; d < gs; d += slots) ss[t] = fmaf(group[d], group[d], ss[t]);
+                for (int d = (p & (per_group - 1)) * 64 + lane; d < gs; d += slots) ss[t] = fmaf(group[d], group[d], ss[t]);
         }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
@@ -227,9 +229,8 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
     for (int i = 0; i < HELD; ++i) {
         const int idx = i * blockDim.x + threadIdx.x;
         if (idx >= n4) continue;
-        const int first = 4 * idx / gs * per_group;          // (a piece lies in one group: their size is a multiple of four)
         float total = 0.0f, o[4], z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int p = 0; p < per_group; ++p) total += partial[first + p];
+        for (int p = 0; p < per_group; ++p) total += partial[first[i] + p];
         const float inv = 1.0f / sqrtf(total / (float)gs + eps);
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = u[i][j] * inv * wt[i][j];
