@@ -53,20 +53,20 @@ struct QkvEpilogue {
     const int* positions;     // [M]
     const int* slot_map;      // [M] page * page_size + slot
     const float* inv_freq;    // [rotary_dim / 2]
-    bf16* k_cache;
-    bf16* v_cache;
+    void* k_cache;            // in the activation type, as the rows
+    void* v_cache;
     int n_heads, n_kv_heads, head_dim, rotary_dim;
     int page_size, num_pages, write_kv;
 };
 
 // RMSNorm without a kernel of its own, for steps of up to 16 tokens.  The product that adds into the
 // 32-bit stream (its last writer before a norm) also leaves, for the norm that follows,
-//   y[m, n]     = bfloat16(h[m, n] * weight[n])        the new row times the norm's weight, rounded once
+//   y[m, n]     = h[m, n] * weight[n]                  the new row times the norm's weight, rounded once (to bfloat16; 32-bit stays)
 //   sumsq[m, p] = sum of h[m, n]^2 over the 16 (for some shapes 8) features n of group p
 // (NextNorm); the product that follows takes y as its rows and multiplies each of its 32-bit sums by
 //   inv[m] = 1 / sqrt(sum_p sumsq[m, p] / K + eps)       (RowScale; the groups are added in a fixed order)
 // before its epilogue.  x W^T with x = h inv weight is the same number as inv (h weight) W^T; what
-// differs from the norm kernel's output is where the one rounding to bfloat16 falls (on h weight
+// differs from the norm kernel's output is where the one rounding to the activation type falls (on h weight
 // instead of on h inv weight), not how many there are.
 // With more rows, a product whose sums are split over blocks (k ranges) has a kernel that adds the parts up, and
 // that kernel sees whole rows: with eps > 0 it finishes the following norm itself,
@@ -74,7 +74,7 @@ struct QkvEpilogue {
 // which any product takes as plain rows (sumsq is not used then).
 struct NextNorm {
     float* sumsq;          // [M, llmrs_gemm_next_parts(M, N, K)]: a part per 16 features, or per 8 (not used with eps > 0)
-    bf16* y;               // [M, N], row stride ldy; null: nothing is left
+    void* y;               // [M, N] in the activation type, row stride ldy; null: nothing is left
     int ldy;
     const float* weight;   // [N]
     float eps;             // > 0: the norm is finished here (llmrs_gemm_norms_whole), else left to the next product
@@ -92,6 +92,14 @@ __device__ __forceinline__ void epilogue_store(int epi, void* out, int ldc, int 
     else if (epi == LLMRS_EPI_ACCUM_F32) ((float*)out)[(size_t)m * ldc + n] += v;
 }
 
+// Up to 16 rows (gemm_few.hip): 16-byte aligned rows, K % 8 == 0 (32-bit: K % 32 == 0), the caller's to check.  1, 0 where the q/k/v
+// epilogue's shape or alignment is not the kernel's, -1 on error (a deferred norm that cannot be taken); a launch's own
+// error is the caller's to ask for.
+int llmrs_gemm_few_bf16(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi,
+                        const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next);
+int llmrs_gemm_few_f32(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi,
+                       const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next);
+bool llmrs_half_tile_blocks(int N, int whole, int cus);
 // 32-bit products on the matrix cores, tiles (gemm_f32_tiles.hip).  K % 32 == 0 and 16-byte aligned rows: the caller's to check.
 // 0, or -1 on error.
 int llmrs_gemm_f32_tiles(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi);
@@ -108,8 +116,9 @@ int llmrs_gemm_bf16_split_parts(hipStream_t stream, const bf16* A, int lda, cons
 int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc,
                          int M, int N, int K, int epi, void* workspace, size_t workspace_bytes,
                          const QkvEpilogue* qkv = nullptr, const RowScale* scale = nullptr, const NextNorm* next = nullptr);
-// Whether the bfloat16 product of this shape goes to the kernel that can scale its rows' sums and leave a NextNorm.
+// Whether the product of this shape, in bfloat16 or in 32-bit, goes to the kernel that can scale its rows' sums and leave a NextNorm.
 extern "C" int llmrs_gemm_defers_norm(int M, int N, int K);
+extern "C" int llmrs_gemm_f32_defers_norm(int M, int N, int K);
 // The parts per row of the sums of squares that such a product leaves (NextNorm): what the caller sizes sumsq by.
 extern "C" int llmrs_gemm_next_parts(int M, int N, int K);
 // Whether the bfloat16 product of this shape, adding into the stream and given the workspace that

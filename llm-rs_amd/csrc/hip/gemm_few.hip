@@ -1,0 +1,454 @@
+// Products of up to 16 rows (decoding), bfloat16 and 32-bit, on the matrix cores with 32-bit sums.
+//
+// What bounds them: the weight's bytes, each read once, and how many of them are on their way at a time.  A block owns
+// 8 NG output features; its NW waves take the k-blocks (128 bytes of a row: 64 bfloat16 or 32 32-bit numbers) in turn, U
+// of them a round with all loads of a round asked for before its first product, and add their sums through LDS in wave order.
+//
+// v_mfma_f32_16x16x32_bf16 and v_mfma_f32_16x16x4_f32 multiply 16 rows of the weight (operand A) by 16 tokens (operand B).
+//   Up to 8 tokens (FOLD) half of that would be work for rows that are not there, so the operands are folded: their 16 rows are
+//   8 features, and 8 tokens, in each of the two halves of a k-block.  A load instruction then brings whole 128-byte lines of
+//   8 rows of the weight and every lane has a piece of them (with 16 features to an operand it brings 64 bytes of
+//   each, and in a block of 8 features half of the lanes idle), one MFMA contracts the whole k-block, and of
+//   its 16 x 16 results the two 8 x 8 blocks on the diagonal are the halves' sums.
+//   9 to 16 tokens: an operand is 16 features, or 16 tokens, of one half of a k-block, and the two halves have sums of their own.
+// Either way an output is the sum, in wave order, of each wave's (first halves' sum + second halves' sum): in bfloat16 its
+// bits depend on K and on the weight's shape, which choose NW and where a block's walk along k begins, never on M.
+// (In 32-bit they differ between up to 8 and more rows, and on the widest weights with the form that M picks, by rounding.)
+// Measured, 16 features an operand for any M -> as here (MI355X, weights from memory, us): bfloat16 at 1 row 2048 x 8192
+// 12.2 -> 8.2, 2048 x 2048 5.3 -> 4.1, 16384 x 2048 15.1 -> 12.6 (5.3 TB/s); at 8 rows 4096 x 4096 11.0 -> 8.4, 4096 x 14336
+// 27.9 -> 24.5, 28672 x 4096 44.4 -> 42.6; 32-bit at 8 rows 2048 x 8192 25.5 -> 18.1, 2048 x 32768 88 -> 61,
+// 16384 x 2048 29.1 -> 25.6.  (A 32-bit MFMA is long: of the 25.5 us some 7 were products for rows that were not there.)
+#include "cache_layout.h"
+#include "gemm_tile.h"
+
+template <class T> struct Few;
+template <> struct Few<bf16> { typedef bf16x8 Piece; typedef bf16x4 Four; };
+template <> struct Few<float> { typedef f32x4 Piece; typedef f32x4 Four; };
+
+// The sums of a tile: a 32-bit piece is four MFMAs, whose products go to SUMS sums of their own, added pairwise at the end
+// (a quarter of the products one after the other in a sum, and an error against 64 bits to match).
+template <class T, int SUMS>
+struct FewSums {
+    f32x4 s[SUMS];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < SUMS; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __device__ __forceinline__ void add(const typename Few<T>::Piece& w, const typename Few<T>::Piece& x) {
+        if constexpr (sizeof(T) == 2) s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, s[0], 0, 0, 0);
+        else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j % SUMS] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], s[j % SUMS], 0, 0, 0);
+        }
+    }
+    __device__ __forceinline__ f32x4 total() const {
+        if constexpr (SUMS == 4) return (s[0] + s[1]) + (s[2] + s[3]);
+        else if constexpr (SUMS == 2) return s[0] + s[1];
+        else return s[0];
+    }
+};
+// In lanes 0..7 and 16..23: the sum with the lane 40 further on (the other half of the k-blocks, see above).
+__device__ __forceinline__ float with_other_half(float x) {
+    unsigned u = __float_as_uint(x);
+    auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);       // [1]: in the low lanes the values of the high ones
+    int far = (int)sw[1];
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(far, far, 0x128, 0xf, 0xf, true));     // row_ror:8
+}
+
+// What a call brings beyond its operands, a kernel for each kind: an argument's trip from memory in front of the first load
+// costs a product of few microseconds a tenth of its time (1 row of 2048 x 2048 bfloat16, with all of them 5.1 us, with none 4.45).
+struct FewPlain {};
+struct FewScaled { RowScale scale; };
+struct FewNext { RowScale scale; NextNorm next; };
+struct FewQkv { RowScale scale; QkvEpilogue qkv; };
+template <class T, bool FOLD, int NG, int NW, int U, int ROT, int SUMS, class Extra>
+__global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ W, void* __restrict__ out, int lda,
+                                                           int ldc, int M, int N, int K, int epi, unsigned inv_full, Extra extra) {
+    constexpr bool NEXT = std::is_same<Extra, FewNext>::value, QKV = std::is_same<Extra, FewQkv>::value;
+    RowScale rs{};
+    NextNorm nn{};
+    QkvEpilogue qe{};
+    if constexpr (!std::is_same<Extra, FewPlain>::value) rs = extra.scale;
+    if constexpr (NEXT) nn = extra.next;
+    if constexpr (QKV) qe = extra.qkv;
+    typedef typename Few<T>::Piece Piece;
+    typedef typename Few<T>::Four Four;
+    constexpr int PER = 16 / (int)sizeof(T), KB = 8 * PER;         // numbers in a lane's piece, in a k-block
+    constexpr int TILES = (NG + 1) / 2;                            // tiles of 16 features (the last one half, where NG is odd)
+    constexpr int TOK = FOLD ? 8 : 16;
+    constexpr int WL = FOLD ? NG : TILES * 2, XL = FOLD ? 1 : 2;   // a lane's pieces of a k-block: weight, tokens
+    extern __shared__ __attribute__((aligned(16))) unsigned char few_smem[];
+    f32x4* red = (f32x4*)few_smem;                                 // [NW][NG][2: four features each][TOK]
+    float* scale_red = (float*)(red + NW * NG * 2 * TOK);          // [NW][16]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * NG * 8;
+    // where a lane's pieces lie within a k-block, and its rows
+    const int first = (FOLD ? (row >> 3) * 4 + g : g) * PER;
+    const T* wp[FOLD ? NG : TILES];
+    const bool last_asks = FOLD || NG % 2 == 0 || row < 8;         // whether this lane's row of the last tile is the block's
+#pragma unroll
+    for (int i = 0; i < (FOLD ? NG : TILES); ++i)
+        wp[i] = W + (size_t)min(n0 + (FOLD ? i * 8 + (row & 7) : i * 16 + row), N - 1) * K + first;
+    const T* xp = A + (size_t)min(FOLD ? row & 7 : row, M - 1) * lda + first;
+    FewSums<T, SUMS> acc[WL];
+#pragma unroll
+    for (int i = 0; i < WL; ++i) acc[i].clear();
+
+    // A norm left to this product (RowScale): its partial sums of squares are shared out over the waves and asked for before
+    // the weights, so that their trip to memory (they were written on other XCDs) costs nothing beside the weights'.
+    // (Asked for after the walk along k it was a trip in front of every result: 0.9 us of the product.)
+    constexpr int AHEAD = 4;
+    const bool scaled = !std::is_same<Extra, FewPlain>::value && rs.sumsq != nullptr, by_four = rs.nparts % 16 == 0 && ((uintptr_t)rs.sumsq & 15) == 0;
+    const float* sp = rs.sumsq + (size_t)min(row, M - 1) * rs.nparts;
+    f32x4 part[AHEAD];
+    if (scaled && by_four) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            int at = 16 * (wave + NW * i) + 4 * g;
+            part[i] = at < rs.nparts ? *(const f32x4*)(sp + at) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    // out += sum: the old values of the tile this wave will finish, and the next norm's weight for them, likewise
+    float old[4] = {0.0f, 0.0f, 0.0f, 0.0f}, next_w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const bool old_ahead = !QKV && epi == LLMRS_EPI_ACCUM_F32 && wave < TILES;
+    if (old_ahead && row < M) {
+        int n = n0 + wave * 16 + 4 * g;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (n + r < N && 4 * g < 8 * NG - 16 * wave) {
+                old[r] = ((const float*)out)[(size_t)row * ldc + n + r];
+                if (NEXT) next_w[r] = nn.weight[n + r];
+            }
+    }
+
+    const int full = (unsigned)K / KB;
+    // A block's walk along k begins at a k-block of its own and wraps round: rows are a multiple of the memory channels'
+    // interleave apart, so blocks in step would all ask the same few channels at once.  The start depends on the group of ROT
+    // features alone that the block's lie in, not on how many it takes: STEP times the group's number, modulo the k-blocks
+    // (by a product with `inv_full`, 2^32 / full rounded up: exact for what fits in 16 bits, and any start will do).
+    int rot = 0;
+    if constexpr (ROT > 0) {
+        constexpr unsigned STEP = ROT == 112 && sizeof(T) == 2 ? 1u : 37u;      // (28672 x 4096 bfloat16 at 1 row: 40.3 us with 1, 46.5 with 37; 6144 x 4096 13.9 and 12.6)
+        unsigned start = (unsigned)n0 / ROT * STEP & 0xffffu;
+        rot = full > 1 ? (int)(start - __umulhi(start, inv_full) * (unsigned)full) : 0;
+    }
+    auto turn = [&](int j) { int x = j + rot; return (x >= full ? x - full : x) * KB; };
+    auto ask = [&](Piece (&w)[WL], Piece (&x)[XL], int k) {
+        if constexpr (FOLD) {
+#pragma unroll
+            for (int i = 0; i < NG; ++i) w[i] = *(const Piece*)(wp[i] + k);
+            x[0] = *(const Piece*)(xp + k);
+        } else {
+#pragma unroll
+            for (int i = 0; i < TILES; ++i) {
+                if (i < TILES - 1 || last_asks) { w[2 * i] = *(const Piece*)(wp[i] + k); w[2 * i + 1] = *(const Piece*)(wp[i] + k + KB / 2); }
+                else w[2 * i] = w[2 * i + 1] = Piece{};
+            }
+            x[0] = *(const Piece*)(xp + k);
+            x[1] = *(const Piece*)(xp + k + KB / 2);
+        }
+    };
+    auto products = [&](const Piece (&w)[WL], const Piece (&x)[XL]) {
+#pragma unroll
+        for (int i = 0; i < WL; ++i) acc[i].add(w[i], x[FOLD ? 0 : i & 1]);
+    };
+    int j = wave;
+    for (; j + (U - 1) * NW < full; j += U * NW) {
+        Piece w[U][WL], x[U][XL];
+#pragma unroll
+        for (int u = 0; u < U; ++u) ask(w[u], x[u], turn(j + u * NW));
+        __builtin_amdgcn_sched_barrier(0);       // keep the round's loads together, ahead of its products
+#pragma unroll
+        for (int u = 0; u < U; ++u) products(w[u], x[u]);
+    }
+    if (U > 1 && j < full) {                     // what is left of this wave's turns: a round too
+        Piece w[U][WL], x[U][XL];
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (j + u * NW < full) ask(w[u], x[u], turn(j + u * NW));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (j + u * NW < full) products(w[u], x[u]);
+    }
+    if (K % KB != 0 && wave == full % NW) {      // the k-block that K cuts
+        const int k = full * KB;
+        const bool v0 = k + first < K, v1 = !FOLD && k + KB / 2 + first < K;
+        Piece w[WL], x[XL];
+#pragma unroll
+        for (int i = 0; i < WL; ++i) {
+            const int t = FOLD ? i : i / 2;
+            const bool asks = (FOLD || t < TILES - 1 || last_asks) && (FOLD || i % 2 == 0 ? v0 : v1);
+            w[i] = asks ? *(const Piece*)(wp[t] + k + (FOLD ? 0 : (i % 2) * (KB / 2))) : Piece{};
+        }
+        x[0] = v0 ? *(const Piece*)(xp + k) : Piece{};
+        if constexpr (!FOLD) x[1] = v1 ? *(const Piece*)(xp + k + KB / 2) : Piece{};
+        products(w, x);
+    }
+    if (scaled) {
+        float ss = 0.0f;
+        if (by_four) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) ss += (part[i][0] + part[i][1]) + (part[i][2] + part[i][3]);
+            for (int at = 16 * (wave + NW * AHEAD) + 4 * g; at < rs.nparts; at += 16 * NW) {
+                f32x4 p = *(const f32x4*)(sp + at);
+                ss += (p[0] + p[1]) + (p[2] + p[3]);
+            }
+        } else {
+            for (int at = 4 * wave + g; at < rs.nparts; at += 4 * NW) ss += sp[at];
+        }
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        if (g == 0) scale_red[wave * 16 + row] = ss;
+    }
+    if constexpr (FOLD) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            f32x4 s = acc[i].total();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] = with_other_half(s[r]);
+            if (row < 8 && g < 2) red[((wave * NG + i) * 2 + g) * TOK + row] = s;
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+            if (2 * t + (g >> 1) < NG) red[((wave * NG + 2 * t) * 2 + g) * TOK + row] = acc[2 * t].total() + acc[2 * t + 1].total();
+    }
+    __syncthreads();
+    // the tiles are shared out over the waves: lane l finishes token l % 16 and features 4 (l / 16) + r
+    const int m = row;
+    if (wave >= TILES || m >= M) return;
+    float inv = 1.0f;
+    if (scaled) {
+        float total = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) total += scale_red[w * 16 + m];
+        inv = 1.0f / sqrtf(total / (float)K + rs.eps);
+    }
+    for (int tile = wave; tile < TILES; tile += NW) {
+        if (2 * tile + (g >> 1) >= NG) continue;                   // the half of the last tile that is the next block's
+        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += red[((w * NG + 2 * tile) * 2 + g) * TOK + m];
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = s[r] * inv;
+        const int n = n0 + tile * 16 + 4 * g;
+        if (!NEXT && !QKV && epi_gated(epi)) {
+#pragma unroll
+            for (int r = 0; r < 4; r += 2)
+                if (n + r + 1 < N) ((T*)out)[(size_t)m * ldc + (n + r) / 2] = from_f32<T>(gated_act(epi, v[r], v[r + 1]));
+        } else if (QKV) {
+            // four consecutive features of one head: two rotation pairs (2i, 2i+1); the rotation is applied to the 32-bit
+            // sums, which are rounded once
+            if (n >= N) continue;
+            int hd = qe.head_dim, head = n / hd, d = n % hd;
+            bool is_q = head < qe.n_heads, is_k = !is_q && head < qe.n_heads + qe.n_kv_heads;
+            if (is_q || is_k) {
+                float pos = (float)qe.positions[m];
+#pragma unroll
+                for (int r = 0; r < 4; r += 2)
+                    if (d + r < qe.rotary_dim) {
+                        float sn, cs;
+                        sincosf(pos * qe.inv_freq[(d + r) >> 1], &sn, &cs);
+                        float a = v[r], b = v[r + 1];
+                        v[r] = a * cs - b * sn;
+                        v[r + 1] = a * sn + b * cs;
+                    }
+            }
+            Four o4;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o4[r] = from_f32<T>(v[r]);
+            if (is_q) {
+                *(Four*)((T*)out + (size_t)m * ldc + n) = o4;
+            } else if (qe.write_kv) {
+                int slot = qe.slot_map[m];
+                if (slot < 0 || slot >= qe.num_pages * qe.page_size) continue;   // never write outside the cache
+                int page = slot / qe.page_size, off = slot % qe.page_size;
+                int kvh = head - qe.n_heads - (is_k ? 0 : qe.n_kv_heads);
+                if (is_k) {
+                    *(Four*)((T*)qe.k_cache + k_cache_index(page, kvh, off, d, qe.n_kv_heads, qe.page_size, hd)) = o4;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        ((T*)qe.v_cache)[v_cache_index(page, kvh, off, d + r, qe.n_kv_heads, qe.page_size, hd)] = o4[r];
+                }
+            }
+        } else if (old_ahead && tile == wave) {
+            float ss = 0.0f;
+            Four y4;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float nv = 0.0f;
+                if (n + r < N) {
+                    nv = old[r] + v[r];
+                    ((float*)out)[(size_t)m * ldc + n + r] = nv;
+                    ss = fmaf(nv, nv, ss);
+                    nv *= next_w[r];
+                }
+                y4[r] = from_f32<T>(nv);
+            }
+            if (NEXT) {
+                // for the norm that follows (NextNorm).  The row's lanes hold four features each; they are all here: a row is
+                // in the batch for all of them or for none.
+                T* y = (T*)nn.y + (size_t)m * nn.ldy + n;
+                if (n + 3 < N) *(Four*)y = y4;
+                else
+                    for (int r = 0; r < 4; ++r)
+                        if (n + r < N) y[r] = y4[r];
+                ss += __shfl_xor(ss, 16, 64);
+                if constexpr (NG == 1) {
+                    if (g == 0) nn.sumsq[(size_t)m * ((N + 7) / 8) + n0 / 8] = ss;        // a part is the block's 8 features
+                } else {
+                    ss += __shfl_xor(ss, 32, 64);
+                    if (g == 0) nn.sumsq[(size_t)m * ((N + 15) / 16) + (n0 / 16 + tile)] = ss;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < N) epilogue_store<T>(epi, out, ldc, m, n + r, v[r]);
+        }
+    }
+}
+
+struct FewCall {
+    hipStream_t stream;
+    const void* A;
+    int lda;
+    const void* W;
+    void* out;
+    int ldc, M, N, K, epi;
+    QkvEpilogue qkv;
+    RowScale scale;
+    NextNorm next;
+};
+template <class T, bool FOLD, int NG, int NW, int U, int ROT, int SUMS = 1>
+static void launch_few(const FewCall& c) {
+    static_assert(ROT % (NG * 8) == 0, "a block's features lie in one group");
+    const unsigned full = c.K * sizeof(T) / 128, inv_full = full > 1 ? (unsigned)(((1ull << 32) + full - 1) / full) : 0;
+    constexpr size_t bytes = (size_t)NW * NG * 2 * (FOLD ? 8 : 16) * 16 + NW * 16 * sizeof(float);
+    static_assert(bytes <= 64 * 1024, "the waves' sums must fit in the LDS that a block may ask for");
+    auto launch = [&](auto extra) {
+        gemm_few_kernel<T, FOLD, NG, NW, U, ROT, SUMS><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
+            (const T*)c.A, (const T*)c.W, c.out, c.lda, c.ldc, c.M, c.N, c.K, c.epi, inv_full, extra);
+    };
+    if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
+    else if (c.next.y != nullptr) launch(FewNext{c.scale, c.next});
+    else if (c.scale.sumsq != nullptr) launch(FewScaled{c.scale});
+    else launch(FewPlain{});
+}
+// bfloat16.  Up to 8 rows: blocks of 8 NG features, U k-blocks a round; 9 to 16 rows: of 8 NG16, U16.  NW and ROT are the same on both sides.
+template <int NW, int ROT, int NG, int U, int NG16, int U16>
+static void launch_few_by_rows(const FewCall& c) {
+    if (c.M <= 8) launch_few<bf16, true, NG, NW, U, ROT>(c);
+    else launch_few<bf16, false, NG16, NW, U16, ROT>(c);
+}
+
+// Whether blocks of 24 features (a tile and a half) share a weight of N features out over the device's units more
+// evenly, by a tenth of a round or more, than blocks of `whole` features (16 or 32) do.
+bool llmrs_half_tile_blocks(int N, int whole, int cus) {
+    auto even = [&](int b) { return (double)b / ((double)ceil_div(b, cus) * cus); };
+    return N % 8 == 0 && even(ceil_div(N, 24)) > even(ceil_div(N, whole)) + 0.1;
+}
+// A narrow weight with long rows (16-feature blocks would leave half of the compute units without one): blocks of 8 features.
+static bool half_blocks_for_narrow(int N, int K) {
+    return N < 16384 && K >= 2048 && N % 8 == 0 && ceil_div(N, 16) * 2 <= llmrs_compute_units();
+}
+// A wide weight's blocks of 9 to 16 rows take 7 or 4 tiles of 16 features, whichever number of blocks fills the device's
+// units more evenly (28672 features are 256 blocks of 7 tiles).
+static int wide_tiles(int N, int cus) {
+    auto evenness = [&](int nt) { int b = ceil_div(N, 16 * nt); return (double)b / ((double)ceil_div(b, cus) * cus); };
+    return evenness(7) >= evenness(4) ? 7 : 4;
+}
+extern "C" int llmrs_gemm_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 8 == 0; }
+extern "C" int llmrs_gemm_f32_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 32 == 0; }
+extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
+    return M <= 16 && half_blocks_for_narrow(N, K) ? ceil_div(N, 8) : ceil_div(N, 16);
+}
+
+// In bfloat16 waves per block and the walk's start come from the weight's shape alone (see above).  With fewer features a block, more
+// blocks ask at once but each reads the tokens' rows again.
+static void few_rows(const FewCall& c, bf16) {
+    const int N = c.N, K = c.K, cus = llmrs_compute_units();
+    if (N >= 16384) {
+        if (wide_tiles(N, cus) == 7) {
+            // (28672 x 4096 at 1, 4, 8 rows: blocks of 16 features 40.3, 40.7, 44, of 112 41.5, 42.3, 43.4)
+            if (c.M <= 4) launch_few<bf16, true, 2, 4, 8, 112>(c);
+            else launch_few<bf16, false, 14, 4, 1, 112>(c);
+        }
+        // (16384 x 2048 at 1, 4, 8 rows: blocks of 16 features 14.4, 14.7, 15.9, of 32 15.0, 15.0, 15.2; 128256 at 1 row 92.7 and 88.4)
+        else if (c.M <= 4 && N < 32768) launch_few<bf16, true, 2, 4, 8, 64>(c);
+        else launch_few_by_rows<4, 64, 4, 8, 8, 2>(c);
+    }
+    else if (K < 2048) launch_few_by_rows<4, 0, 2, 4, 2, 4>(c);
+    else if (K >= 16384 && N >= 8192) launch_few_by_rows<8, 64, 4, 4, 4, 4>(c);      // 8192 x 28672 at 16 rows: 90 -> 83 us
+    else if (half_blocks_for_narrow(N, K)) {
+        if (K >= 4096) launch_few_by_rows<8, 64, 1, 8, 1, 4>(c);
+        else launch_few_by_rows<8, 0, 1, 4, 1, 4>(c);
+    }
+    // (nothing is to be left for a norm, which counts its sums by 16 features; 6144 x 4096 at 8 rows 12.6 against 16.0 in
+    // blocks of 16, 10240 x 8192 at 2 rows 34.9 against 37.1)
+    else if (c.next.y == nullptr && (llmrs_half_tile_blocks(N, 16, cus) || ceil_div(N, 16) > 2 * cus)) {
+        if (K >= 4096) launch_few_by_rows<8, 96, 3, 8, 3, 4>(c);
+        else launch_few_by_rows<8, 96, 3, 4, 3, 4>(c);
+    }
+    else if (K >= 4096) launch_few_by_rows<8, 64, 2, 8, 2, 4>(c);
+    else launch_few_by_rows<8, 0, 2, 4, 2, 4>(c);
+}
+// 32-bit: up to 8 rows four sums a tile (two in blocks of 56 features, which have no registers for four), more rows one: in each
+// the error against 64 bits is no larger than it was with one sum for whole k-blocks (K = 2048: 1.25e-7 up to 8 rows, 2.1e-7 from
+// 9 on, against 2.9e-7; one and two rows as in gemm_rows_kernel, 1.2e-7).
+static void few_rows(const FewCall& c, float) {
+    const int N = c.N, K = c.K, cus = llmrs_compute_units();
+    const bool fold = c.M <= 8;
+    if (N >= 16384) {
+        if (N % 112 == 0) {
+            // (28672 x 4096 at 1 row: blocks of 16 features 83.2, of 56 86.8; at 8 rows 90 and 86.5)
+            if (c.M <= 4) launch_few<float, true, 2, 8, 4, 112, 4>(c);
+            else if (fold) launch_few<float, true, 7, 8, 2, 112, 2>(c);
+            else launch_few<float, false, 14, 8, 1, 112>(c);
+        }
+        else if (fold) launch_few<float, true, 4, 8, 2, 64, 4>(c);
+        else launch_few<float, false, 8, 8, 1, 64>(c);
+    } else if (K < 512) {
+        launch_few<float, false, 2, 4, 2, 0, 2>(c);
+    } else if (K < 2048) {
+        if (fold) launch_few<float, true, 2, 4, 4, 0, 4>(c);
+        else launch_few<float, false, 2, 4, 4, 0>(c);
+    } else if (half_blocks_for_narrow(N, K)) {
+        if (!fold) launch_few<float, false, 1, 8, 4, 64>(c);
+        else if (K >= 4096) launch_few<float, true, 1, 8, 8, 64, 4>(c);
+        else launch_few<float, true, 1, 8, 4, 0, 4>(c);
+    } else if (c.next.y == nullptr && llmrs_half_tile_blocks(N, 16, cus)) {
+        if (fold) launch_few<float, true, 3, 8, 4, 96, 4>(c);
+        else launch_few<float, false, 3, 8, 2, 96>(c);
+    }
+    else if (fold) launch_few<float, true, 2, 16, 4, 0, 4>(c);           // (sixteen waves: 4096 x 4096 at 8 rows 17.0 us, eight 19.4)
+    else launch_few<float, false, 2, 8, 4, 64>(c);
+}
+
+template <class T>
+static int gemm_few(hipStream_t stream, const T* A, int lda, const T* W, void* out, int ldc, int M, int N, int K, int epi,
+                    const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next) {
+    constexpr int FOUR = 4 * (int)sizeof(T);
+    if (scale != nullptr || next != nullptr) {
+        bool ok = (scale == nullptr || (scale->sumsq != nullptr && scale->nparts >= 1 && scale->eps > 0.0f)) &&
+                  (next == nullptr || (epi == LLMRS_EPI_ACCUM_F32 && N < 16384 && next->sumsq != nullptr && next->y != nullptr &&
+                                       next->weight != nullptr && next->ldy >= N && next->ldy % 4 == 0 && (uintptr_t)next->y % FOUR == 0));
+        if (!ok) { llmrs_fail("gemm: a deferred norm is taken for up to 16 rows (what is left for the next one: with the += epilogue, under 16384 features), got M=%d N=%d K=%d epilogue %d", M, N, K, epi); return -1; }
+    }
+    if (epi == LLMRS_EPI_QKV && (qkv == nullptr || qkv->head_dim % 4 || ldc % 4 || (uintptr_t)out % FOUR || (uintptr_t)qkv->k_cache % FOUR || qkv->rotary_dim % 4))
+        return 0;           // (four features of a head are stored at once)
+    few_rows(FewCall{stream, A, lda, W, out, ldc, M, N, K, epi, qkv ? *qkv : QkvEpilogue{}, scale ? *scale : RowScale{}, next ? *next : NextNorm{}}, T{});
+    return 1;
+}
+int llmrs_gemm_few_bf16(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi,
+                        const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next) {
+    return gemm_few<bf16>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, scale, next);
+}
+int llmrs_gemm_few_f32(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi,
+                       const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next) {
+    return gemm_few<float>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, scale, next);
+}

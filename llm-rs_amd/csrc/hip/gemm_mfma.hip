@@ -1,6 +1,6 @@
 // bfloat16 products on the matrix cores, 32-bit accumulation.
 //
-// Two kernels, chosen by M (the number of tokens in the step):
+// Two kernels, chosen by M (the number of tokens in the step); up to 16 rows go to gemm_few.hip:
 //   M <= 64  "skinny": decoding.  Every weight is read once, straight from
 //            memory into MFMA operands; a block owns 16 to 64 output features and
 //            its waves split K, so a layer's product has enough loads in flight to
@@ -77,8 +77,7 @@ template <int MT, int NT, int NW, int U, int LAST = 16>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __restrict__ A, int lda,
                                                               const bf16* __restrict__ W, void* __restrict__ out,
                                                               int ldc, int M, int N, int K, int epi,
-                                                              float* __restrict__ partial, QkvEpilogue qe, int rot_feats,
-                                                              RowScale rs, NextNorm nn) {
+                                                              float* __restrict__ partial, QkvEpilogue qe, int rot_feats) {
     extern __shared__ __attribute__((aligned(16))) unsigned char skinny_smem[];
     float* red = (float*)skinny_smem;          // [NW][MT][NT][4][64]
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -115,17 +114,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
     // out += sum: the old values of the tile this wave will finish are asked for now, so that
     // their trip to memory runs beside the weights' instead of after the sums are ready
     float old[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float next_w[4] = {0.0f, 0.0f, 0.0f, 0.0f};     // the next norm's weight for the same features, if something is left for it
     const bool old_ahead = epi == LLMRS_EPI_ACCUM_F32 && partial == nullptr && wave < MT * NT;
     if (old_ahead) {
         int m = (wave / NT) * 16 + row, n = n0 + (wave % NT) * 16 + 4 * g;
         if (m < M)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (n + r < N) {
-                    old[r] = ((const float*)out)[(size_t)m * ldc + n + r];
-                    if (nn.sumsq != nullptr) next_w[r] = nn.weight[n + r];
-                }
+                if (n + r < N) old[r] = ((const float*)out)[(size_t)m * ldc + n + r];
     }
     int j = wave;
     for (; j + (U - 1) * NW < cnt; j += U * NW) {
@@ -176,35 +171,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
         }
         if (partial_turn) break;
     }
-    // A norm left to this product (RowScale, up to 16 rows, so MT = 1): the waves that will finish tiles find their
-    // row's scale now, so that the trip for the partial sums of squares runs beside the other waves' last rounds and
-    // the barrier.  The row's four lanes take every fourth group of four parts in ascending order and add their sums
-    // pairwise; every lane of a row, in every block, ends with the same bits.
-    float inv_row = 1.0f;
-    if (rs.sumsq != nullptr && wave < MT * NT) {
-        const float* sp = rs.sumsq + (size_t)min(row, M - 1) * rs.nparts;
-        float ss = 0.0f;
-        if (rs.nparts % 16 == 0 && ((uintptr_t)rs.sumsq & 15) == 0) {
-            // up to sixteen loads on their way at a time (the sums were written on other XCDs and come from memory);
-            // a group past the row's parts adds zeros
-            for (int base = 4 * g; base < rs.nparts; base += 256) {
-                f32x4 p[16];
-#pragma unroll
-                for (int t = 0; t < 16; ++t)
-                    p[t] = base + 16 * t < rs.nparts ? *(const f32x4*)(sp + base + 16 * t) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < 16; ++t) { ss += p[t][0]; ss += p[t][1]; ss += p[t][2]; ss += p[t][3]; }
-            }
-        } else {
-            for (int i = 4 * g; i < rs.nparts; i += 16)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (i + q < rs.nparts) ss += sp[i + q];
-        }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
-        inv_row = 1.0f / sqrtf(ss / (float)K + rs.eps);
-    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -221,7 +187,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
             float s = 0.0f;
 #pragma unroll
             for (int w = 0; w < NW; ++w) s += red[(((w * MT + mt) * NT + nt) * 4 + r) * 64 + lane];
-            v[r] = s * inv_row;      // (1 without a norm left to this product; with one, MT = 1 and the lane's row is `row`)
+            v[r] = s;
         }
         int m = mt * 16 + row;
         int n = n0 + nt * 16 + 4 * g;
@@ -264,44 +230,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
                 int page = slot / qe.page_size, off = slot % qe.page_size;
                 if (is_k) {
                     int kvh = head - qe.n_heads;
-                    *(bf16x4*)(qe.k_cache + k_cache_index(page, kvh, off, d, qe.n_kv_heads, qe.page_size, hd)) = o4;
+                    *(bf16x4*)((bf16*)qe.k_cache + k_cache_index(page, kvh, off, d, qe.n_kv_heads, qe.page_size, hd)) = o4;
                 } else {
                     int kvh = head - qe.n_heads - qe.n_kv_heads;
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        qe.v_cache[v_cache_index(page, kvh, off, d + r, qe.n_kv_heads, qe.page_size, hd)] = o4[r];
+                        ((bf16*)qe.v_cache)[v_cache_index(page, kvh, off, d + r, qe.n_kv_heads, qe.page_size, hd)] = o4[r];
                 }
             }
         } else if (old_ahead && tile == wave) {
-            float ss = 0.0f;
-            bf16x4 y4;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float nv = 0.0f;
-                if (n + r < N) {
-                    nv = old[r] + v[r];
-                    ((float*)out)[(size_t)m * ldc + n + r] = nv;
-                    ss = fmaf(nv, nv, ss);
-                    nv *= next_w[r];
-                }
-                y4[r] = (bf16)nv;
-            }
-            if (nn.sumsq != nullptr) {
-                // for the norm that follows (NextNorm).  The row's four lanes hold four features each of this tile's
-                // sixteen; they are all here: a row is in the batch for all of them or for none.
-                if (n + 3 < N) *(bf16x4*)(nn.y + (size_t)m * nn.ldy + n) = y4;
-                else
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < N) nn.y[(size_t)m * nn.ldy + n + r] = y4[r];
-                ss += __shfl_xor(ss, 16, 64);
-                if constexpr (LAST == 16) {
-                    ss += __shfl_xor(ss, 32, 64);
-                    if (g == 0) nn.sumsq[(size_t)m * ((N + 15) / 16) + (n0 / 16 + nt)] = ss;
-                } else {
-                    // blocks of 8 features (NT = 1: the launcher sees to it): a part is the block's 8, held by two lanes
-                    if (g == 0) nn.sumsq[(size_t)m * ((N + 7) / 8) + n0 / 8] = ss;
-                }
-            }
+            for (int r = 0; r < 4; ++r)
+                if (n + r < N) ((float*)out)[(size_t)m * ldc + n + r] = old[r] + v[r];
         } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -372,7 +312,7 @@ __global__ __launch_bounds__(1024) void gemm_splitk_finish_norm_kernel(const flo
             bf16x4 y;
 #pragma unroll
             for (int r = 0; r < 4; ++r) y[r] = (bf16)(h[i][r] * inv * w[r]);
-            *(bf16x4*)(nn.y + (size_t)m * nn.ldy + n) = y;
+            *(bf16x4*)((bf16*)nn.y + (size_t)m * nn.ldy + n) = y;
         }
     }
 }
@@ -391,8 +331,7 @@ static void launch_splitk_finish(hipStream_t stream, const float* partial, int s
 template <int MT, int NT, int NW, int U, int LAST = 16>
 static void launch_skinny(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc,
                           int M, int N, int K, int epi, const QkvEpilogue* qkv, int splits = 1,
-                          float* partial = nullptr, int rot_feats = 0, const RowScale* scale = nullptr,
-                          const NextNorm* next = nullptr) {
+                          float* partial = nullptr, int rot_feats = 0, const NextNorm* next = nullptr) {
     size_t bytes = (size_t)NW * MT * NT * 4 * 64 * sizeof(float);
     static bool configured = false;
     if (!configured) {
@@ -403,9 +342,7 @@ static void launch_skinny(hipStream_t stream, const bf16* A, int lda, const bf16
     dim3 grid(ceil_div(N, (NT - 1) * 16 + LAST), splits);
     gemm_skinny_kernel<MT, NT, NW, U, LAST><<<grid, NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi,
                                                                           splits > 1 ? partial : nullptr,
-                                                                          qkv ? *qkv : QkvEpilogue{}, rot_feats,
-                                                                          scale ? *scale : RowScale{},
-                                                                          next && splits == 1 ? *next : NextNorm{});
+                                                                          qkv ? *qkv : QkvEpilogue{}, rot_feats);
     if (splits > 1) launch_splitk_finish(stream, partial, splits, out, ldc, M, N, epi, next);
 }
 
@@ -1371,27 +1308,6 @@ extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
     return 0;
 }
 
-// Up to 16 rows a bfloat16 product goes to the kernel for few rows with every tile of a block finished by a wave
-// of its own (not the widest weights, whose blocks take seven tiles): that kernel scales its rows' sums by a
-// norm left to it and leaves what the next norm needs.
-// Whether blocks of 24 features (a tile and a half) share a weight of N features out over the device's units more
-// evenly, by a tenth of a round or more, than blocks of `whole` features (16 or 32) do.
-static bool half_tile_blocks(int N, int whole, int cus) {
-    auto even = [&](int b) { return (double)b / ((double)ceil_div(b, cus) * cus); };
-    return N % 8 == 0 && even(ceil_div(N, 24)) > even(ceil_div(N, whole)) + 0.1;
-}
-
-extern "C" int llmrs_gemm_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 8 == 0; }
-// Up to 16 rows on a narrow weight with long rows (16-feature blocks would leave half of the compute units without
-// one): blocks of 8 features, half a tile each (the tile's other rows are never asked for).  Measured at 1 row:
-// 2048 x 8192 14.8 -> 12.3 us, 2048 x 2048 6.1 -> 5.6 us.
-static bool half_blocks_for_narrow(int N, int K) {
-    return N < 16384 && K >= 2048 && N % 8 == 0 && ceil_div(N, 16) * 2 <= llmrs_compute_units();
-}
-// How many partial sums of squares per row such a product leaves for the norm that follows (NextNorm without eps).
-extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
-    return M <= 16 && half_blocks_for_narrow(N, K) ? ceil_div(N, 8) : ceil_div(N, 16);
-}
 // 17 rows or more whose sums are split over blocks: the kernel that adds the parts up can finish the following norm.
 // (Beyond 256 rows that is where the 128 x 128 tiles take all rows with k split: a narrow weight whose tiles leave
 // half of the device's places empty, as the o and down products of a small model do beside a prompt portion.)
@@ -1431,11 +1347,9 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                   next->weight != nullptr && next->ldy >= N && next->ldy % 4 == 0 && ((uintptr_t)next->y & 7) == 0 &&
                   ((uintptr_t)next->weight & 15) == 0 && ldc % 4 == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)workspace & 15) == 0;
         if (!ok) { llmrs_fail("gemm: a norm finished by a split product needs the += epilogue, 17 rows or more of a shape that is split, its workspace and aligned rows, got M=%d N=%d K=%d epilogue %d", M, N, K, epi); return -1; }
-    } else if (scale != nullptr || next != nullptr) {
-        bool ok = llmrs_gemm_defers_norm(M, N, K) && (scale == nullptr || (scale->sumsq != nullptr && scale->nparts >= 1 && scale->eps > 0.0f)) &&
-                  (next == nullptr || (epi == LLMRS_EPI_ACCUM_F32 && N < 16384 && next->sumsq != nullptr && next->y != nullptr &&
-                                       next->weight != nullptr && next->ldy >= N && next->ldy % 4 == 0 && ((uintptr_t)next->y & 7) == 0));
-        if (!ok) { llmrs_fail("gemm: a deferred norm is taken for up to 16 rows (what is left for the next one: with the += epilogue, under 16384 features), got M=%d N=%d K=%d epilogue %d", M, N, K, epi); return -1; }
+    } else if ((scale != nullptr || next != nullptr) && !llmrs_gemm_defers_norm(M, N, K)) {
+        llmrs_fail("gemm: a deferred norm is taken for up to 16 rows, got M=%d N=%d K=%d epilogue %d", M, N, K, epi);
+        return -1;
     }
     if (epi == LLMRS_EPI_QKV) {   // only the skinny kernel fuses it; its 8-byte stores need aligned rows
         if (M > 64 || qkv == nullptr || qkv->head_dim % 4 || ldc % 4 || ((uintptr_t)out & 7) ||
@@ -1448,6 +1362,13 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         if (M > 32 && K >= 8192 && few_rows_take_tiles(M, N, K)) return 0;
     }
     int rc = 0;
+    if (M <= 16) {
+        int took = llmrs_gemm_few_bf16(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, scale, next);
+        if (took <= 0) return took;
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) { llmrs_fail("gemm (mfma): launch failed: %s", hipGetErrorString(e)); return -1; }
+        return 1;
+    }
     bool tiles_for_few = false;
     if (epi != LLMRS_EPI_QKV && few_rows_take_tiles(M, N, K)) {
         int splits = tiled_splits(M, N, K);
@@ -1456,10 +1377,6 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
     if (tiles_for_few) {
         rc = launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, tiled_splits(M, N, K), (float*)workspace, next);
     } else if (M <= 64) {
-        // Waves per block (NW) come from the weight's shape alone: k-blocks go to the
-        // waves in turn and their sums are added in wave order, so for a given weight an
-        // output's sum has one order whatever M, MT, NT and U are (up to 16 rows; with more, a
-        // weight with few rows may have its k-blocks shared out over blocks as well).
         // Features per block (NT*16) grow with N and M: a block reads its tokens' rows
         // again for every 16*NT features, which costs L2 bandwidth once M is large, but
         // a weight with few rows needs small blocks to have enough of them.
@@ -1476,33 +1393,15 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         // Other weights with long rows (measured at 8192 x 8192: 32.6 -> 28.6 us; nothing at K = 4096):
         // by groups of 64 features, which hold the features of any block that these weights get.
         int rot = wide ? 16 * wide_nt : (K >= 8192 ? 64 : 0);
-#define SKINNY(MT, NT, NW, U) launch_skinny<MT, NT, NW, U>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot, scale, next)
-        if (M <= 16) {
-            if (wide) {
-                // up to 4 rows blocks of 16 features (a decode step of eight 8B layers: 1.100 -> 1.086 ms at 3 rows,
-                // 1.121 -> 1.116 at 4, slower from 6 on: every block reads the tokens' rows again)
-                if (M <= 4) SKINNY(1, 1, 4, 8); else if (wide_nt == 7) SKINNY(1, 7, 4, 1); else SKINNY(1, 4, 4, 2);
-            }
-            else if (eight) {
-                // Blocks of 16 features, unless they come to a round and a half of the device's units (6144 features on
-                // 256: 384 blocks) and blocks of 24 to whole rounds: those, when nothing is to be left for a norm (which
-                // counts its sums by 16 features)
-                if (K >= 16384 && N >= 8192) SKINNY(1, 2, 8, 4);   // 8192 x 28672: 90 -> 83 us
-                else if (half_blocks_for_narrow(N, K))
-                    launch_skinny<1, 1, 8, 4, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot, scale, next);
-                else if (next == nullptr && half_tile_blocks(N, 16, cus))
-                    launch_skinny<1, 2, 8, 4, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot, scale, nullptr);
-                else SKINNY(1, 1, 8, 4);
-            }
-            else SKINNY(1, 1, 4, 4);
-        } else if (M <= 32) {
+#define SKINNY(MT, NT, NW, U) launch_skinny<MT, NT, NW, U>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot)
+        if (M <= 32) {
             int splits = skinny_splits(N, K);
             if (splits > 1 && epi != LLMRS_EPI_QKV && workspace != nullptr &&
                 workspace_bytes >= (size_t)splits * M * N * sizeof(float)) {
-                launch_skinny<2, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, nullptr, next);
+                launch_skinny<2, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, next);
             } else if (wide) { if (wide_nt == 7) SKINNY(2, 7, 4, 1); else SKINNY(2, 4, 4, 2); }
             else if (N > 4096) {
-                if (eight && half_tile_blocks(N, 32, cus)) launch_skinny<2, 2, 8, 2, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot);
+                if (eight && llmrs_half_tile_blocks(N, 32, cus)) launch_skinny<2, 2, 8, 2, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot);
                 else if (eight) SKINNY(2, 2, 8, 2);
                 else SKINNY(2, 2, 4, 2);
             }
@@ -1516,10 +1415,10 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                 int splits = skinny_splits(N, K);
                 if (splits > 1 && epi != LLMRS_EPI_QKV && workspace != nullptr &&
                     workspace_bytes >= (size_t)splits * M * N * sizeof(float)) {
-                    launch_skinny<MT, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, nullptr, next);
+                    launch_skinny<MT, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, next);
                 } else if (wide) { if (wide_nt == 7) SKINNY(MT, 7, 4, 1); else SKINNY(MT, 4, 4, 2); }
                 else if (N > 4096) {
-                    if (eight && half_tile_blocks(N, 32, cus)) launch_skinny<MT, 2, 8, 1, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot);
+                    if (eight && llmrs_half_tile_blocks(N, 32, cus)) launch_skinny<MT, 2, 8, 1, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot);
                     else if (eight) SKINNY(MT, 2, 8, 1);
                     else SKINNY(MT, 2, 4, 2);
                 }

@@ -237,35 +237,25 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const T* __restrict__ A,
     }
 }
 
-// Few tokens in 32-bit on the matrix cores: v_mfma_f32_16x16x4_f32 multiplies and adds in 32-bit (no
-// reduced-precision mode).  The weight's rows are the A operand, read once for every 16 MT tokens, 16 bytes a lane (lane
-// l: feature l % 16 of a tile, the four k-values 4 (l / 16) .. + 3 of a group of 16); the tokens' rows are the B
-// operand, read the same way once for all of a block's NT feature tiles, so that the tokens cost a load for every NT
-// loads of weights where the walk above asks for every token's row again for every two or four rows of the weight.  An
-// MFMA contracts the four k-values that the four lane groups hold in the same place of their loads.  A block's NW waves
-// take the 32-wide k-blocks in turn, U of them with all loads asked for before the first product, and add their sums
-// through LDS in wave order.  C: lane l holds token l % 16 and features 4 (l / 16) + r.  Needs K % 32 == 0 and 16-byte
-// aligned rows.
-// Up to 16 tokens an output's sum depends on K and the weight's shape alone (which choose NW); with more tokens on the
-// form that launch_f32_few_rows picks as well.
-// LAST = 8 (NT = 1): a block takes half a tile of features; the other rows of the tile are never asked for.
+// 17 tokens and more in 32-bit on the matrix cores (up to 16: gemm_few.hip): v_mfma_f32_16x16x4_f32 multiplies and adds in
+// 32-bit (no reduced-precision mode).  The weight's rows are the A operand, read once for every 16 MT tokens, 16 bytes a
+// lane (lane l: feature l % 16 of a tile, the four k-values 4 (l / 16) .. + 3 of a group of 16); the tokens' rows are the B
+// operand, read the same way once for all of a block's NT feature tiles.  An MFMA contracts the four k-values that the
+// four lane groups hold in the same place of their loads.  A block's NW waves take the 32-wide k-blocks in turn, U of them
+// with all loads asked for before the first product, and add their sums through LDS in wave order.  C: lane l holds token
+// l % 16 and features 4 (l / 16) + r.  Needs K % 32 == 0 and 16-byte aligned rows.
 // rot_feats > 0: neighbouring groups of that many features begin their walk along k at different k-blocks and wrap
 // round.  Rows are a multiple of the memory channels' interleave apart, so blocks in step would all ask the same few
 // channels at once.  What bounds it: the weights' bytes, and beside them the tokens' rows, which every block reads again.
-// Measured at 8 rows, before -> with the walk staggered and these shapes of block (2048 features k 8192: half tiles):
-// 16384 x 2048 31.4 -> 27.5 us (4.9 TB/s of weights), 128256 x 2048 213 -> 184, 4096 x 4096 18.6 -> 15.8,
-// 6144 x 4096 30 -> 24, 2048 x 8192 27 -> 23, 28672 x 4096 88 -> 84.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-template <int MT, int NT, int NW, int U, int LAST = 16>
+template <int MT, int NT, int NW, int U>
 __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
                                                                   void* __restrict__ out, int ldc, int M, int N, int K, int epi, int rot_feats) {
     extern __shared__ __attribute__((aligned(16))) float f32_skinny_red[];       // [NW][MT][NT][4][64]
     float* red = f32_skinny_red;
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int row = lane & 15, g = lane >> 4;
-    static_assert(LAST == 16 || (LAST == 8 && NT == 1), "whole tiles, or one half tile");
-    const bool asks = LAST == 16 || row < LAST;      // whether this lane's row of the weight is the block's
-    int n0 = blockIdx.x * (LAST == 16 ? NT * 16 : LAST), m0 = blockIdx.y * MT * 16;
+    int n0 = blockIdx.x * NT * 16, m0 = blockIdx.y * MT * 16;
     const float* wp[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) wp[nt] = W + (size_t)min(n0 + nt * 16 + row, N - 1) * K + 4 * g;
@@ -293,10 +283,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const float* _
     };
     auto ask = [&](f32x4_t (&w)[NT][2], f32x4_t (&x)[MT][2], int k) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            if (asks) { w[nt][0] = *(const f32x4_t*)(wp[nt] + k); w[nt][1] = *(const f32x4_t*)(wp[nt] + k + 16); }
-            else w[nt][0] = w[nt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
+        for (int nt = 0; nt < NT; ++nt) { w[nt][0] = *(const f32x4_t*)(wp[nt] + k); w[nt][1] = *(const f32x4_t*)(wp[nt] + k + 16); }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) { x[mt][0] = *(const f32x4_t*)(xp[mt] + k); x[mt][1] = *(const f32x4_t*)(xp[mt] + k + 16); }
     };
@@ -333,7 +320,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const float* _
             v[r] = s;
         }
         int m = m0 + mt * 16 + row, n = n0 + nt * 16 + 4 * g;
-        if (m >= M || (LAST < 16 && 4 * g >= LAST)) continue;
+        if (m >= M) continue;
         if (epi_gated(epi)) {
 #pragma unroll
             for (int r = 0; r < 4; r += 2)
@@ -346,36 +333,22 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const float* _
     }
 }
 
-template <int MT, int NT, int NW, int U, int LAST = 16>
+template <int MT, int NT, int NW, int U>
 static void launch_f32_skinny(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi, int rot_feats = 0) {
     constexpr size_t bytes = (size_t)NW * MT * NT * 4 * 64 * sizeof(float);
     static_assert(bytes <= 64 * 1024, "the waves' sums must fit in the LDS a block may ask for");
     static bool configured = false;
     if (!configured) {
-        (void)hipFuncSetAttribute((const void*)gemm_f32_skinny_kernel<MT, NT, NW, U, LAST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        (void)hipFuncSetAttribute((const void*)gemm_f32_skinny_kernel<MT, NT, NW, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         configured = true;
     }
-    gemm_f32_skinny_kernel<MT, NT, NW, U, LAST><<<dim3(ceil_div(N, LAST == 16 ? NT * 16 : LAST), ceil_div(M, MT * 16)), NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, rot_feats);
+    gemm_f32_skinny_kernel<MT, NT, NW, U><<<dim3(ceil_div(N, NT * 16), ceil_div(M, MT * 16)), NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, rot_feats);
 }
 
 // The kernel above, in the form that the product's shape asks for; false: the tiles take it.
 static bool launch_f32_few_rows(hipStream_t stream, const float* a, int lda, const float* w, void* out, int ldc, int M, int N, int K, int epi) {
     const int cus = llmrs_compute_units();
-    if (M <= 16) {
-        // (blocks of 7 tiles with one wave a SIMD took 92 us for the 8B shape's gate/up weight: a 32-bit MFMA is long, and
-        // the wave's loads and products took turns; two waves a SIMD)
-        if (N >= 16384) {
-            if (N % 112 == 0) launch_f32_skinny<1, 7, 8, 1>(stream, a, lda, w, out, ldc, M, N, K, epi, 112);
-            else launch_f32_skinny<1, 4, 4, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
-        } else if (K < 2048) launch_f32_skinny<1, 1, 4, 4>(stream, a, lda, w, out, ldc, M, N, K, epi);
-        // a weight so narrow that whole tiles would leave half of the compute units without a block: half tiles
-        else if (2 * ceil_div(N, 16) <= cus) launch_f32_skinny<1, 1, 8, 2, 8>(stream, a, lda, w, out, ldc, M, N, K, epi);
-        // between one and two blocks a unit: blocks of two tiles, one round of them
-        else if (ceil_div(N, 16) > cus && ceil_div(N, 32) <= cus) launch_f32_skinny<1, 2, 8, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 32);
-        else launch_f32_skinny<1, 1, 8, 4>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
-        return true;
-    }
-    // More rows: blocks of 32 tokens with the fewest features that still make one round of the compute units.  Where even
+    // Blocks of 32 tokens with the fewest features that still make one round of the compute units.  Where even
     // 64 features to a block make more, the tiles take over, but for up to 32 tokens, whose weights are read once here.
     // (us, 32-feature-tile form / tiles: 32 rows 2048 x 8192 45 / 168, 128256 x 2048 295 / 350; 64 rows 3072 x 2048 19 / 45,
     // 16384 x 2048 66 / 48; 100 rows 2048 x 2048 19 / 45; 200 rows 2048 x 2048 29 / 45, 3072 x 2048 58 / 46)
@@ -431,7 +404,7 @@ extern "C" int llmrs_glu_clamp_slot(hipStream_t stream, float limit, float alpha
 // scale_sumsq (with its parts and eps): a norm left to this product, see RowScale in gemm.h.  next_sumsq (with next_y,
 // its row stride and the next norm's weight): what the += epilogue leaves for the norm that follows, see NextNorm.
 // Both null in the ordinary case; otherwise the product must be one llmrs_gemm_defers_norm(M, N, K) accepts, in
-// bfloat16 on the matrix cores, or the call fails.
+// bfloat16 or (llmrs_gemm_f32_defers_norm) in 32-bit on the matrix cores, or the call fails.
 extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda, const void* W, void* out, int ldc,
                           int M, int N, int K, int epi, void* workspace, size_t workspace_bytes, int allow_mfma,
                           const float* scale_sumsq, int scale_parts, float scale_eps, float* next_sumsq, void* next_y,
@@ -449,15 +422,23 @@ extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda,
     if (M == 0) return 0;
     if (dtype == LLMRS_BF16 && allow_mfma) {
         RowScale rs{scale_sumsq, scale_parts, scale_eps};
-        NextNorm nn{next_sumsq, (bf16*)next_y, next_ldy, next_weight, next_eps};
+        NextNorm nn{next_sumsq, next_y, next_ldy, next_weight, next_eps};
         int took = llmrs_gemm_bf16_mfma(stream, (const bf16*)A, lda, (const bf16*)W, out, ldc, M, N, K, epi, workspace,
                                         workspace_bytes, nullptr, scale_sumsq ? &rs : nullptr, next_y ? &nn : nullptr);
         if (took != 0) return took < 0 ? -1 : 0;
     }
-    LLMRS_REQUIRE(scale_sumsq == nullptr && next_y == nullptr, "gemm: a deferred norm needs the bfloat16 matrix-core kernels (M=%d N=%d K=%d)", M, N, K);
-    // (one or two tokens are better off with the walk below, which then asks for little beside the weights:
-    // a decode step of the 8B shape at one request 7.1 against 7.8 ms)
-    if (dtype == LLMRS_F32 && allow_mfma && M > 2 && K % 32 == 0 && lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0) {
+    const bool f32_cores = dtype == LLMRS_F32 && allow_mfma && K % 32 == 0 && lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
+    // (one or two tokens on the widest weights are better off with the walk below: 128256 x 2048 173 against 177 us)
+    if (f32_cores && M <= 16 && !(M <= 2 && N >= 65536 && scale_sumsq == nullptr && next_y == nullptr)) {
+        RowScale rs{scale_sumsq, scale_parts, scale_eps};
+        NextNorm nn{next_sumsq, next_y, next_ldy, next_weight, 0.0f};
+        if (llmrs_gemm_few_f32(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi, nullptr, scale_sumsq ? &rs : nullptr,
+                               next_y ? &nn : nullptr) < 0) return -1;
+        LLMRS_LAUNCH_CHECK("gemm");
+        return 0;
+    }
+    LLMRS_REQUIRE(scale_sumsq == nullptr && next_y == nullptr, "gemm: a deferred norm needs the matrix-core kernels for few rows (M=%d N=%d K=%d)", M, N, K);
+    if (f32_cores && M > 2) {
         if (!launch_f32_few_rows(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi) &&
             llmrs_gemm_f32_tiles(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi) != 0) return -1;
         LLMRS_LAUNCH_CHECK("gemm");

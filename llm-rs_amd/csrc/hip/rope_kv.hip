@@ -262,10 +262,19 @@ extern "C" int llmrs_qkv_rope_cache(hipStream_t stream, int dtype, const void* x
                   "qkv_rope_cache: rotary_dim %d does not fit head_dim %d", rotary_dim, head_dim);
     LLMRS_REQUIRE(page_size > 0 && num_pages > 0, "qkv_rope_cache: bad cache geometry");
     if (M == 0) return 0;
+    const QkvEpilogue qe{positions, slot_map, inv_freq, k_cache, v_cache, n_heads, n_kv_heads, head_dim,
+                         rotary_dim, page_size, num_pages, write_kv};
+    const RowScale rs{scale_sumsq, scale_parts, scale_eps};
+    if (dtype == LLMRS_F32 && allow_mfma && M <= 16 && K % 32 == 0 && lda % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
+        int took = llmrs_gemm_few_f32(stream, (const float*)x, lda, (const float*)w, qkv, row_stride, M, N, K, LLMRS_EPI_QKV, &qe,
+                                      scale_sumsq ? &rs : nullptr, nullptr);
+        if (took < 0) return -1;
+        if (took > 0) {
+            LLMRS_LAUNCH_CHECK("qkv_rope_cache");
+            return 0;
+        }
+    }
     if (dtype == LLMRS_BF16 && allow_mfma) {
-        QkvEpilogue qe{positions, slot_map, inv_freq, (bf16*)k_cache, (bf16*)v_cache, n_heads, n_kv_heads, head_dim,
-                       rotary_dim, page_size, num_pages, write_kv};
-        RowScale rs{scale_sumsq, scale_parts, scale_eps};
         int took = llmrs_gemm_bf16_mfma(stream, (const bf16*)x, lda, (const bf16*)w, qkv, row_stride, M, N, K,
                                         LLMRS_EPI_QKV, nullptr, 0, &qe, scale_sumsq ? &rs : nullptr);
         if (took != 0) return took < 0 ? -1 : 0;
@@ -284,7 +293,7 @@ extern "C" int llmrs_qkv_rope_cache(hipStream_t stream, int dtype, const void* x
             }
         }
     }
-    LLMRS_REQUIRE(scale_sumsq == nullptr, "qkv_rope_cache: a deferred norm needs the fused bfloat16 kernel (M=%d K=%d)", M, K);
+    LLMRS_REQUIRE(scale_sumsq == nullptr, "qkv_rope_cache: a deferred norm needs the fused kernel (M=%d K=%d)", M, K);
     int rc = llmrs_gemm(stream, dtype, x, lda, w, qkv, row_stride, M, N, K, LLMRS_EPI_STORE, workspace, workspace_bytes,
                         allow_mfma, nullptr, 0, 0.0f, nullptr, nullptr, 0, nullptr, 0.0f);
     if (rc != 0) return rc;

@@ -201,6 +201,8 @@ class Model:
         # (A step of few single tokens that wants them all: the last product has prepared the final norm, and the
         # output matrix's product finishes it; no norm kernel runs.)
         x = self.final_norm.deferred(ctx, h) if ctx.wants_every_row and self.final_norm is not None and not self.streamed else None
+        if x is not None and not isinstance(x, torch.Tensor) and not k.product_norms_its_rows(T, self.head.shape[0], self.head.shape[1], self.dtype):
+            x = None            # (rows that the output matrix's product cannot scale: the norm runs)
         if x is None:
             x = ctx.workspace("model.head_in", (ctx.n_want, self.spec.hidden_size), self.dtype)
             if self.streamed:

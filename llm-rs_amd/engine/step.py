@@ -160,16 +160,16 @@ class StepContext:
         if plan is None:
             return None
         if not plan.whole:
-            return NextNorm(self._prenormed(T, N), self.workspace("model.sumsq", (T, plan.parts), torch.float32), weight)
+            return NextNorm(self._prenormed(T, N, w.dtype), self.workspace("model.sumsq", (T, plan.parts), torch.float32), weight)
         eps = norm.deferred_eps()
-        return NextNorm(self._prenormed(T, N), None, weight, eps) if eps is not None and eps > 0 else None
+        return NextNorm(self._prenormed(T, N, w.dtype), None, weight, eps) if eps is not None and eps > 0 else None
 
-    def _prenormed(self, T: int, N: int) -> torch.Tensor:
+    def _prenormed(self, T: int, N: int, dtype: torch.dtype) -> torch.Tensor:
         """Room for the rows a product leaves: not the rows that were left last, which the part at work may
         still be reading as its input."""
-        y = self.workspace("model.prenormed", (T, N), torch.bfloat16)
+        y = self.workspace("model.prenormed", (T, N), dtype)
         if self._last_y == y.data_ptr():
-            y = self.workspace("model.prenormed.other", (T, N), torch.bfloat16)
+            y = self.workspace("model.prenormed.other", (T, N), dtype)
         return y
 
     def note_left(self, h: torch.Tensor, left) -> None:

@@ -38,7 +38,7 @@ class KernelError(RuntimeError):
 
 class NormedRows:
     """Rows whose norm is left to the product that takes them (steps of a few tokens; no norm kernel runs).
-    `y` [rows, K] holds the stream's rows times the norm's weight, rounded once to the activation type, and
+    `y` [rows, K] holds the stream's rows times the norm's weight, rounded once to the activation type (32-bit: not at all), and
     `sumsq` [rows, parts] the sums of squares of each 16 consecutive features of the stream's rows: both left
     by the product that added into the stream last.  The product multiplies each of its 32-bit sums by the row's
     1 / sqrt(sum(sumsq) / K + eps): x W^T with x = h inv weight equals inv (h weight) W^T."""
@@ -230,6 +230,7 @@ class HipKernels(Kernels):
             "llmrs_gemm": [V, I, V, I, V, V, I, I, I, I, I, V, c_size_t, I, V, I, F, V, V, I, V, F],
             "llmrs_glu_clamp_slot": [V, F, F, F, F],
             "llmrs_gemm_defers_norm": [I, I, I],
+            "llmrs_gemm_f32_defers_norm": [I, I, I],
             "llmrs_gemm_norms_whole": [I, I, I],
             "llmrs_gemm_next_parts": [I, I, I],
             "llmrs_rope_kv_write": [V, I, V, I, V, V, V, I, I, V, V, I, I, I, I, I, I, I],
@@ -300,26 +301,25 @@ class HipKernels(Kernels):
         return int(self.lib.llmrs_gemm_workspace_floats(int(M), int(N), int(K)))
 
     def product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype) -> bool:
-        return dtype == torch.bfloat16 and self.gemm_defers_norm(M, N, K)
+        return self.gemm_defers_norm(M, N, K, dtype)
 
     def norm_left_by_product(self, M: int, N: int, K: int, dtype: torch.dtype) -> Optional[NormPlan]:
-        if dtype != torch.bfloat16:
-            return None
         # up to a few rows: partial sums of squares, for the next product to finish (the kernels keep at most 1024
         # of them a row); more rows: a product that is split over blocks finishes the norm where its parts are added up
-        if N < 16384 and self.gemm_defers_norm(M, N, K):
+        if N < 16384 and self.gemm_defers_norm(M, N, K, dtype):
             return NormPlan(False, self.gemm_next_parts(M, N, K))
-        if self.gemm_norms_whole(M, N, K):
+        if dtype == torch.bfloat16 and self.gemm_norms_whole(M, N, K):
             return NormPlan(True, 0)
         return None
 
     def grouped_experts_take(self, hidden: int, ff: int, dtype: torch.dtype) -> bool:
         return dtype == torch.bfloat16 and self.allow_mfma and bool(self.lib.llmrs_expert_gemm_takes(int(hidden), int(ff)))
 
-    def gemm_defers_norm(self, M: int, N: int, K: int) -> bool:
-        """Whether the bfloat16 product of M rows with an [N, K] weight takes `NormedRows` as its rows and, adding
+    def gemm_defers_norm(self, M: int, N: int, K: int, dtype: torch.dtype = torch.bfloat16) -> bool:
+        """Whether the product of M rows with an [N, K] weight takes `NormedRows` as its rows and, adding
         into the stream, leaves a `NextNorm` (that: for fewer than 16384 features)."""
-        return self.allow_mfma and bool(self.lib.llmrs_gemm_defers_norm(int(M), int(N), int(K)))
+        asked = self.lib.llmrs_gemm_defers_norm if dtype == torch.bfloat16 else self.lib.llmrs_gemm_f32_defers_norm
+        return self.allow_mfma and bool(asked(int(M), int(N), int(K)))
 
     def gemm_next_parts(self, M: int, N: int, K: int) -> int:
         """Partial sums of squares per row that a product leaving a `NextNorm` writes (one per 16 features, for some
@@ -574,14 +574,14 @@ class HipKernels(Kernels):
         whole = leave is not None and leave.whole
         if leave is not None:
             assert epilogue == EPI_ACCUM_F32 and tuple(leave.y.shape) == (M, N) and leave.y.stride(1) == 1
-            assert leave.y.dtype == torch.bfloat16 and leave.weight.dtype == torch.float32 and leave.weight.shape[0] == N
+            assert leave.y.dtype == a.dtype and leave.weight.dtype == torch.float32 and leave.weight.shape[0] == N
             if not whole:
                 assert N < 16384 and leave.sumsq.dtype == torch.float32 and leave.sumsq.is_contiguous()
                 assert tuple(leave.sumsq.shape) == (M, self.gemm_next_parts(M, N, K))
         if whole:
             assert a.dtype == torch.bfloat16 and scale is None and self.gemm_norms_whole(M, N, K) and workspace is not None
         elif scale is not None or leave is not None:
-            assert a.dtype == torch.bfloat16 and self.gemm_defers_norm(M, N, K)
+            assert self.gemm_defers_norm(M, N, K, a.dtype)
         want = torch.float32 if epilogue in (EPI_STORE_F32, EPI_ACCUM_F32) else a.dtype
         assert out.dtype == want and out.shape[0] == M and out.shape[1] == (N // 2 if epilogue in _EPI_GATED else N)
         moved = (M * K + N * K) * a.element_size() + out.numel() * out.element_size() * (2 if epilogue == EPI_ACCUM_F32 else 1)
@@ -628,7 +628,7 @@ class HipKernels(Kernels):
         if isinstance(x, NormedRows):
             scale, x = x, x.y
             assert scale.sumsq.dtype == torch.float32 and scale.sumsq.is_contiguous() and scale.sumsq.shape[0] == x.shape[0]
-            assert x.dtype == torch.bfloat16 and self.gemm_defers_norm(x.shape[0], w.shape[0], x.shape[1])
+            assert self.gemm_defers_norm(x.shape[0], w.shape[0], x.shape[1], x.dtype)
         assert x.stride(1) == 1 and qkv.stride(1) == 1 and w.is_contiguous() and x.dtype == w.dtype == qkv.dtype
         assert rotary_dim == 0 or (inv_freq.dtype == torch.float32 and inv_freq.shape[0] == rotary_dim // 2)
         if write_kv:

@@ -1443,6 +1443,36 @@ def test_a_norm_left_by_one_product_and_finished_by_the_next(M, hidden, inter):
     assert float((got.double().cpu() - exact).abs().max()) <= 2e-2 * scale
 
 
+@pytest.mark.parametrize("M,hidden,inter", [(1, 2048, 2048), (8, 2048, 8192), (9, 2048, 4096), (16, 96, 320), (5, 4096, 640), (3, 3072, 2048)])
+def test_float32_products_hand_a_norm_over(M, hidden, inter):
+    """The same in 32-bit, up to 16 rows: the stream bit for bit as without, the rows of the stream times the weight, and a q/k/v
+    product with its rotation and cache write on such rows against 64 bits (the bound of the 32-bit products; a deferred scale
+    adds roundings of 2^-24 of a result)."""
+    from llm_rs_amd.kernels import NextNorm, NormedRows
+    k, eps, heads, kv, hd = kernels(), 1e-5, 6, 2, 32
+    assert k.gemm_defers_norm(M, hidden, inter, torch.float32) and k.gemm_defers_norm(M, (heads + 2 * kv) * hd, hidden, torch.float32)
+    a, w_down, w_qkv = rnd((M, inter), torch.float32, 60), rnd((hidden, inter), torch.float32, 61, 0.05), rnd(((heads + 2 * kv) * hd, hidden), torch.float32, 62, 0.1)
+    nw, h = rnd((hidden,), torch.float32, 63) * 0.1 + 1, rnd((M, hidden), torch.float32, 64, 2.0)
+    plain = h.clone()
+    k.gemm(a, w_down, plain, EPI_ACCUM_F32)
+    left = NextNorm(torch.zeros((M, hidden), device=DEV), torch.full((M, k.gemm_next_parts(M, hidden, inter)), -1.0, device=DEV), nw)
+    k.gemm(a, w_down, h, EPI_ACCUM_F32, None, leave=left)
+    assert torch.equal(h, plain) and torch.equal(left.y, h * nw)
+    hd64 = h.double().cpu()
+    assert float((left.sumsq.double().cpu().sum(-1) / (hd64 * hd64).sum(-1) - 1).abs().max()) <= 1e-5
+    x = hd64 / torch.sqrt((hd64 * hd64).mean(-1, keepdim=True) + eps) * nw.double().cpu()
+    acc = x @ w_qkv.double().cpu().T
+    positions, slots = torch.arange(3, 3 + M, dtype=torch.int32, device=DEV), torch.arange(M, dtype=torch.int32, device=DEV)
+    inv_freq = plain_inv_freq(hd, 10000.0, None).to(DEV)
+    qkv, kc, vc = torch.zeros((M, w_qkv.shape[0]), device=DEV), torch.zeros((1, kv, 16, hd), device=DEV), torch.zeros((1, kv, hd, 16), device=DEV)
+    k.qkv_rope_cache(NormedRows(left.y, left.sumsq, eps), w_qkv, qkv, positions, slots, inv_freq, hd, kc, vc, heads, kv, hd, 16, 1, True)
+    split = [acc[:, i * hd:j * hd].view(M, -1, hd) for i, j in ((0, heads), (heads, heads + kv), (heads + kv, heads + 2 * kv))]
+    want = [plain_rope(t, positions.cpu(), inv_freq.cpu(), "interleaved") for t in split[:2]] + split[2:]
+    got = [qkv[:, :heads * hd].double().cpu().view(M, heads, hd), kc[0].double().cpu().permute(1, 0, 2)[:M], vc[0].double().cpu().permute(2, 0, 1)[:M]]
+    for g, r in zip(got, want):
+        assert float((g - r).abs().max()) <= 2e-6 * math.sqrt(hidden) + 1e-5 * float(r.abs().max())
+
+
 @pytest.mark.parametrize("M,N,K", [(64, 4096, 4096), (17, 4096, 14336), (24, 1024, 2048), (33, 2048, 8192), (200, 512, 4096),
                                    (128, 4096, 4096), (256, 1000, 2048), (40, 6144, 4096), (64, 8192, 8192), (45, 4096, 4096),
                                    (2030, 2048, 2048), (1900, 2048, 8192), (700, 4096, 4096), (300, 1000, 2048)])
