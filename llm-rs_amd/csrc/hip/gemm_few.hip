@@ -18,7 +18,6 @@
 // 12.2 -> 8.2, 2048 x 2048 5.3 -> 4.1, 16384 x 2048 15.1 -> 12.6 (5.3 TB/s); at 8 rows 4096 x 4096 11.0 -> 8.4, 4096 x 14336
 // 27.9 -> 24.5, 28672 x 4096 44.4 -> 42.6; 32-bit at 8 rows 2048 x 8192 25.5 -> 18.1, 2048 x 32768 88 -> 61,
 // 16384 x 2048 29.1 -> 25.6.  (A 32-bit MFMA is long: of the 25.5 us some 7 were products for rows that were not there.)
-#include "cache_layout.h"
 #include "gemm_tile.h"
 
 template <class T> struct Few;
@@ -240,41 +239,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
             for (int r = 0; r < 4; r += 2)
                 if (n + r + 1 < N) ((T*)out)[(size_t)m * ldc + (n + r) / 2] = from_f32<T>(gated_act(epi, v[r], v[r + 1]));
         } else if (QKV) {
-            // four consecutive features of one head: two rotation pairs (2i, 2i+1); the rotation is applied to the 32-bit
-            // sums, which are rounded once
-            if (n >= N) continue;
-            int hd = qe.head_dim, head = n / hd, d = n % hd;
-            bool is_q = head < qe.n_heads, is_k = !is_q && head < qe.n_heads + qe.n_kv_heads;
-            if (is_q || is_k) {
-                float pos = (float)qe.positions[m];
-#pragma unroll
-                for (int r = 0; r < 4; r += 2)
-                    if (d + r < qe.rotary_dim) {
-                        float sn, cs;
-                        sincosf(pos * qe.inv_freq[(d + r) >> 1], &sn, &cs);
-                        float a = v[r], b = v[r + 1];
-                        v[r] = a * cs - b * sn;
-                        v[r + 1] = a * sn + b * cs;
-                    }
-            }
-            Four o4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o4[r] = from_f32<T>(v[r]);
-            if (is_q) {
-                *(Four*)((T*)out + (size_t)m * ldc + n) = o4;
-            } else if (qe.write_kv) {
-                int slot = qe.slot_map[m];
-                if (slot < 0 || slot >= qe.num_pages * qe.page_size) continue;   // never write outside the cache
-                int page = slot / qe.page_size, off = slot % qe.page_size;
-                int kvh = head - qe.n_heads - (is_k ? 0 : qe.n_kv_heads);
-                if (is_k) {
-                    *(Four*)((T*)qe.k_cache + k_cache_index(page, kvh, off, d, qe.n_kv_heads, qe.page_size, hd)) = o4;
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        ((T*)qe.v_cache)[v_cache_index(page, kvh, off, d + r, qe.n_kv_heads, qe.page_size, hd)] = o4[r];
-                }
-            }
+            if (n < N) store_qkv4<T>(qe, out, ldc, m, n, v);
         } else if (old_ahead && tile == wave) {
             float ss = 0.0f;
             Four y4;

@@ -1,10 +1,9 @@
 // bfloat16 products on the matrix cores, 32-bit accumulation.
 //
 // Two kernels, chosen by M (the number of tokens in the step); up to 16 rows go to gemm_few.hip:
-//   M <= 64  "skinny": decoding.  Every weight is read once, straight from
-//            memory into MFMA operands; a block owns 16 to 64 output features and
-//            its waves split K, so a layer's product has enough loads in flight to
-//            keep HBM busy.  v_mfma_f32_16x16x32_bf16, weights as the A operand.
+//   M <= 64  many requests decoding.  K % 64 == 0: gemm_ring.h.  Other K "skinny": every
+//            weight is read once, straight from memory into MFMA operands; a block owns 32 or
+//            64 output features and its waves split K.
 //   M  > 64  "tiled": prompts.  Tiles of 128x128, 256x128, 256x192 or 256x256 outputs, K
 //            in steps of 64 through double-buffered LDS, v_mfma_f32_32x32x16_bf16; when
 //            K % 64 == 0 the tiles are loaded straight into LDS (global_load_lds), or, by
@@ -16,7 +15,7 @@
 // kernel, never on M, the row's place in the batch or the tile it falls in.
 // Replaces the reference's matvec_bf16_simd / gemm_bf16 (shaders/ops.metal:52-159,
 // :1090-1143); unlike gemm_bf16 (:1107) the accumulator is 32-bit.
-#include "cache_layout.h"
+#include "gemm_ring.h"
 #include "gemm_tile.h"
 
 __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *(const bf16x8*)p; }
@@ -69,23 +68,18 @@ __device__ __forceinline__ float gated_act_fast(const GatedAct& a, float g, floa
 // the epilogue.  That is for weights with few rows and many tokens (17..64),
 // where blocks of 64 features are needed to keep the tokens' rows from being
 // read too often, and would otherwise be too few to fill the device.
+// (For rows that are no whole k-blocks; gemm_ring.h takes the others.)
 // ---------------------------------------------------------------------------
-// LAST < 16: the last of a block's feature tiles has only LAST features (a block of 24 features is a tile and a
-// half): the rows beyond are never asked for (their lanes load nothing and multiply zeros), so a weight whose
-// 16-feature blocks would be one and a half rounds of the device can be shared out evenly.
-template <int MT, int NT, int NW, int U, int LAST = 16>
+template <int MT, int NT, int NW, int U>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __restrict__ A, int lda,
                                                               const bf16* __restrict__ W, void* __restrict__ out,
                                                               int ldc, int M, int N, int K, int epi,
-                                                              float* __restrict__ partial, QkvEpilogue qe, int rot_feats) {
+                                                              float* __restrict__ partial, QkvEpilogue qe) {
     extern __shared__ __attribute__((aligned(16))) unsigned char skinny_smem[];
     float* red = (float*)skinny_smem;          // [NW][MT][NT][4][64]
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int row = lane & 15, g = lane >> 4;
-    constexpr int BF = (NT - 1) * 16 + LAST;       // features of a block
-    static_assert(LAST == 16 || LAST == 8, "a whole last tile, or half of one");
-    int n0 = blockIdx.x * BF;
-    const bool last_asks = LAST == 16 || row < LAST;   // whether this lane's row of the last tile exists
+    int n0 = blockIdx.x * NT * 16;
     const bf16* wp[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) wp[nt] = W + (size_t)min(n0 + nt * 16 + row, N - 1) * K;
@@ -104,13 +98,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
     int lo = blockIdx.y * per;
     int kb_hi = min(nkb, lo + per);                        // this block's k-blocks: [lo, kb_hi)
     int cnt = max(min(full, kb_hi) - lo, 0);               // the full ones among them
-    // The block walks its full k-blocks starting at `rot` and wraps round: with rot_feats > 0,
-    // neighbouring groups of rot_feats features are at different places of their rows at any
-    // moment.  Rows are a multiple of the memory channels' interleave apart, so blocks in step
-    // would all ask the same few channels at once.  The start depends on the features alone
-    // (a block's features lie within one group), not on how many of them a block takes.
-    int rot = (cnt > 0 && rot_feats > 0) ? (n0 / rot_feats) % cnt : 0;
-    auto turn = [&](int j) { int x = j + rot; return lo + (x >= cnt ? x - cnt : x); };
     // out += sum: the old values of the tile this wave will finish are asked for now, so that
     // their trip to memory runs beside the weights' instead of after the sums are ready
     float old[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -127,12 +114,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
         bf16x8 w[U][NT][2], x[U][MT][2];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            int k = turn(j + u * NW) * 64 + g * 8;
+            int k = (lo + j + u * NW) * 64 + g * 8;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                if (LAST == 16 || nt < NT - 1 || last_asks) { w[u][nt][0] = load8(wp[nt] + k); w[u][nt][1] = load8(wp[nt] + k + 32); }
-                else { w[u][nt][0] = zero8(); w[u][nt][1] = zero8(); }
-            }
+            for (int nt = 0; nt < NT; ++nt) { w[u][nt][0] = load8(wp[nt] + k); w[u][nt][1] = load8(wp[nt] + k + 32); }
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) { x[u][mt][0] = load8(xp[mt] + k); x[u][mt][1] = load8(xp[mt] + k + 32); }
         }
@@ -151,14 +135,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
     for (;; j += NW) {
         bool partial_turn = j == cnt && kb_hi > lo + cnt;   // one k-block past the full ones, cut by K
         if (j >= cnt && !partial_turn) break;
-        int k = (partial_turn ? lo + cnt : turn(j)) * 64 + g * 8;
+        int k = (lo + j) * 64 + g * 8;
         bool v0 = k < K, v1 = k + 32 < K;
         bf16x8 w0[NT], w1[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            bool asks = LAST == 16 || nt < NT - 1 || last_asks;
-            w0[nt] = v0 && asks ? load8(wp[nt] + k) : zero8();
-            w1[nt] = v1 && asks ? load8(wp[nt] + k + 32) : zero8();
+            w0[nt] = v0 ? load8(wp[nt] + k) : zero8();
+            w1[nt] = v1 ? load8(wp[nt] + k + 32) : zero8();
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -192,7 +175,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
         int m = mt * 16 + row;
         int n = n0 + nt * 16 + 4 * g;
         if (m >= M) continue;
-        if (LAST < 16 && nt == NT - 1 && 4 * g >= LAST) continue;     // the half of the last tile that is the next block's
         if (partial != nullptr) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -202,42 +184,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
             for (int r = 0; r < 4; r += 2)
                 if (n + r + 1 < N) ((bf16*)out)[(size_t)m * ldc + (n + r) / 2] = (bf16)gated_act(epi, v[r], v[r + 1]);
         } else if (epi == LLMRS_EPI_QKV) {
-            // four consecutive features of one head: two rotation pairs (2i, 2i+1); the
-            // rotation is applied to the 32-bit sums, which are rounded once
-            if (n >= N) continue;
-            int hd = qe.head_dim, head = n / hd, d = n % hd;
-            bool is_q = head < qe.n_heads, is_k = !is_q && head < qe.n_heads + qe.n_kv_heads;
-            if (is_q || is_k) {
-                float pos = (float)qe.positions[m];
-#pragma unroll
-                for (int r = 0; r < 4; r += 2)
-                    if (d + r < qe.rotary_dim) {
-                        float sn, cs;
-                        sincosf(pos * qe.inv_freq[(d + r) >> 1], &sn, &cs);
-                        float a = v[r], b = v[r + 1];
-                        v[r] = a * cs - b * sn;
-                        v[r + 1] = a * sn + b * cs;
-                    }
-            }
-            bf16x4 o4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o4[r] = (bf16)v[r];
-            if (is_q) {
-                *(bf16x4*)((bf16*)out + (size_t)m * ldc + n) = o4;
-            } else if (qe.write_kv) {
-                int slot = qe.slot_map[m];
-                if (slot < 0 || slot >= qe.num_pages * qe.page_size) continue;   // never write outside the cache
-                int page = slot / qe.page_size, off = slot % qe.page_size;
-                if (is_k) {
-                    int kvh = head - qe.n_heads;
-                    *(bf16x4*)((bf16*)qe.k_cache + k_cache_index(page, kvh, off, d, qe.n_kv_heads, qe.page_size, hd)) = o4;
-                } else {
-                    int kvh = head - qe.n_heads - qe.n_kv_heads;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        ((bf16*)qe.v_cache)[v_cache_index(page, kvh, off, d + r, qe.n_kv_heads, qe.page_size, hd)] = o4[r];
-                }
-            }
+            if (n < N) store_qkv4<bf16>(qe, out, ldc, m, n, v);
         } else if (old_ahead && tile == wave) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -328,21 +275,40 @@ static void launch_splitk_finish(hipStream_t stream, const float* partial, int s
     gemm_splitk_finish_kernel<<<ceil_div(pairs, 256), 256, 0, stream>>>(partial, splits, out, ldc, M, N, epi);
 }
 
-template <int MT, int NT, int NW, int U, int LAST = 16>
+template <int MT, int NT, int NW, int U>
 static void launch_skinny(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc,
-                          int M, int N, int K, int epi, const QkvEpilogue* qkv, int splits = 1,
-                          float* partial = nullptr, int rot_feats = 0, const NextNorm* next = nullptr) {
+                          int M, int N, int K, int epi, const QkvEpilogue* qkv, int splits = 1, float* partial = nullptr, const NextNorm* next = nullptr) {
     size_t bytes = (size_t)NW * MT * NT * 4 * 64 * sizeof(float);
     static bool configured = false;
     if (!configured) {
-        (void)hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, NT, NW, U, LAST>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        (void)hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, NT, NW, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         configured = true;
     }
-    dim3 grid(ceil_div(N, (NT - 1) * 16 + LAST), splits);
-    gemm_skinny_kernel<MT, NT, NW, U, LAST><<<grid, NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi,
-                                                                          splits > 1 ? partial : nullptr,
-                                                                          qkv ? *qkv : QkvEpilogue{}, rot_feats);
+    gemm_skinny_kernel<MT, NT, NW, U><<<dim3(ceil_div(N, NT * 16), splits), NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi,
+                                                                                                    splits > 1 ? partial : nullptr, qkv ? *qkv : QkvEpilogue{});
+    if (splits > 1) launch_splitk_finish(stream, partial, splits, out, ldc, M, N, epi, next);
+}
+
+// Stages: what fits in half of a unit's LDS, three to twelve.  (All of it, twice as many on their way, is no faster where a
+// unit has one block, 64 rows of 28672 x 4096 46.6 against 46.0 us, and keeps a second block off where there are more, 16384 x 2048
+// 20.4 against 19.2.)
+template <int MT, int NT, int LAST, int KSUB>
+constexpr int ring_stages() {
+    constexpr int room = 75 * 1024 / ring_stage_bytes<MT, NT, LAST>(KSUB);
+    return room > 12 ? 12 : room;
+}
+template <int MT, int NT, int LAST, int KSUB>
+static void launch_ring(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi,
+                        const QkvEpilogue* qkv, int splits = 1, float* partial = nullptr, int rot_feats = 0, const NextNorm* next = nullptr) {
+    constexpr int STAGES = ring_stages<MT, NT, LAST, KSUB>();
+    constexpr size_t bytes = (size_t)STAGES * ring_stage_bytes<MT, NT, LAST>(KSUB);
+    static bool configured = false;
+    if (!configured) {
+        (void)hipFuncSetAttribute((const void*)gemm_ring_kernel<MT, NT, LAST, KSUB, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        configured = true;
+    }
+    gemm_ring_kernel<MT, NT, LAST, KSUB, STAGES><<<dim3(ceil_div(N, (NT - 1) * 16 + LAST), splits), 64 * ring_waves<MT>(), bytes, stream>>>(
+        A, W, out, lda, ldc, M, N, K, epi, splits > 1 ? partial : nullptr, rot_feats, qkv ? *qkv : QkvEpilogue{});
     if (splits > 1) launch_splitk_finish(stream, partial, splits, out, ldc, M, N, epi, next);
 }
 
@@ -1377,56 +1343,38 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
     if (tiles_for_few) {
         rc = launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, tiled_splits(M, N, K), (float*)workspace, next);
     } else if (M <= 64) {
-        // Features per block (NT*16) grow with N and M: a block reads its tokens' rows
-        // again for every 16*NT features, which costs L2 bandwidth once M is large, but
-        // a weight with few rows needs small blocks to have enough of them.
-        // (Measured on MI355X at the 8B shapes.)
-        bool wide = N >= 16384;
-        bool eight = !wide && K >= 2048;
+        // Features per block grow with N: a block reads its tokens' rows again, which costs once M is large, but a weight
+        // with few rows needs small blocks to have enough of them; the narrowest ones have their k-blocks shared out over blocks
+        // as well.  (Measured on MI355X at the 1B and 8B shapes.)
+        const bool wide = N >= 16384;
+        const int cus = llmrs_compute_units(), splits = skinny_splits(N, K);
+        const bool split = splits > 1 && epi != LLMRS_EPI_QKV && workspace != nullptr && workspace_bytes >= (size_t)splits * M * N * sizeof(float);
+        if (whole && splits <= 1) { llmrs_fail("gemm: M=%d N=%d K=%d is not split after all: the norm cannot be finished here", M, N, K); return -1; }
         // A wide weight's blocks take 7 or 4 feature tiles: whichever number of blocks fills the
-        // device's compute units more evenly (28672 features are 256 blocks of 7 tiles).  Its blocks
-        // start their walk along k at staggered places, by groups of that many features.
-        if (whole && skinny_splits(N, K) <= 1) { llmrs_fail("gemm: M=%d N=%d K=%d is not split after all: the norm cannot be finished here", M, N, K); return -1; }
-        int cus = llmrs_compute_units();
+        // device's compute units more evenly (28672 features are 256 blocks of 7 tiles).
         auto evenness = [&](int nt) { int b = ceil_div(N, 16 * nt); return (double)b / ((double)ceil_div(b, cus) * cus); };
-        int wide_nt = (wide && evenness(7) >= evenness(4)) ? 7 : 4;
-        // Other weights with long rows (measured at 8192 x 8192: 32.6 -> 28.6 us; nothing at K = 4096):
-        // by groups of 64 features, which hold the features of any block that these weights get.
-        int rot = wide ? 16 * wide_nt : (K >= 8192 ? 64 : 0);
-#define SKINNY(MT, NT, NW, U) launch_skinny<MT, NT, NW, U>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot)
-        if (M <= 32) {
-            int splits = skinny_splits(N, K);
-            if (splits > 1 && epi != LLMRS_EPI_QKV && workspace != nullptr &&
-                workspace_bytes >= (size_t)splits * M * N * sizeof(float)) {
-                launch_skinny<2, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, next);
-            } else if (wide) { if (wide_nt == 7) SKINNY(2, 7, 4, 1); else SKINNY(2, 4, 4, 2); }
-            else if (N > 4096) {
-                if (eight && llmrs_half_tile_blocks(N, 32, cus)) launch_skinny<2, 2, 8, 2, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot);
-                else if (eight) SKINNY(2, 2, 8, 2);
-                else SKINNY(2, 2, 4, 2);
+        auto rows_of = [&](auto tiles) {
+            constexpr int MT = decltype(tiles)::value;
+            if (K % 64) {
+                if (split) launch_skinny<MT, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, next);
+                else if (wide) launch_skinny<MT, 4, 4, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv);
+                else launch_skinny<MT, 2, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv);
+                return;
             }
-            else { if (eight) SKINNY(2, 1, 8, 4); else SKINNY(2, 1, 4, 4); }
-        } else {
-            // 48 or 64 tokens and 64 features per block; when that leaves no more than 64 blocks, K is split
-            // over blocks too, if the caller gave room for the partial sums (measured: it
-            // pays for N = 4096, K = 14336, and no longer for N = 6144).
-            auto rows_of = [&](auto tiles) {
-                constexpr int MT = decltype(tiles)::value;
-                int splits = skinny_splits(N, K);
-                if (splits > 1 && epi != LLMRS_EPI_QKV && workspace != nullptr &&
-                    workspace_bytes >= (size_t)splits * M * N * sizeof(float)) {
-                    launch_skinny<MT, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, next);
-                } else if (wide) { if (wide_nt == 7) SKINNY(MT, 7, 4, 1); else SKINNY(MT, 4, 4, 2); }
-                else if (N > 4096) {
-                    if (eight && llmrs_half_tile_blocks(N, 32, cus)) launch_skinny<MT, 2, 8, 1, 8>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot);
-                    else if (eight) SKINNY(MT, 2, 8, 1);
-                    else SKINNY(MT, 2, 4, 2);
-                }
-                else { if (eight) SKINNY(MT, 1, 8, 2); else SKINNY(MT, 1, 4, 2); }
-            };
-            if (M <= 48) rows_of(std::integral_constant<int, 3>{}); else rows_of(std::integral_constant<int, 4>{});
-        }
-#undef SKINNY
+#define RING(NT, LAST, KSUB, ROT) launch_ring<MT, NT, LAST, KSUB>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, ROT)
+#define RING_SPLIT(NT, KSUB) launch_ring<MT, NT, 16, KSUB>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, next)
+            // (64 rows: 2048 x 2048, 128 blocks of 64 features with their shares of k, 12.0 us, 256 of 32 10.4; 2048 x 8192 16.6 and 18.5)
+            if (split) { if (ceil_div(N, 64) * splits >= cus) RING_SPLIT(4, 1); else RING_SPLIT(2, 2); }
+            else if (wide) { if (evenness(7) >= evenness(4)) RING(7, 16, 1, 112); else RING(4, 16, 1, 64); }
+            // 6144 features are 256 blocks of 24 (a tile and a half), 3072 192 of 16
+            else if (N > 4096) { if (llmrs_half_tile_blocks(N, 32, cus)) RING(2, 8, 1, 0); else RING(2, 16, 1, 0); }
+            else RING(1, 16, 2, 0);
+#undef RING
+#undef RING_SPLIT
+        };
+        if (M <= 32) rows_of(std::integral_constant<int, 2>{});
+        else if (M <= 48) rows_of(std::integral_constant<int, 3>{});
+        else rows_of(std::integral_constant<int, 4>{});
     } else {
         // K % 64 == 0: tiles loaded straight into LDS, two k-tiles of 64 there.  Other K: through
         // registers, with zero-filled tails.

@@ -536,6 +536,29 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
         assert (err <= out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))).all(), (epi, float(err.max()))
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 40, 64), (33, 250, 128), (48, 4090, 192), (49, 3000, 704), (64, 16, 1344), (20, 6140, 64), (64, 8200, 320),
+                                   (40, 16400, 64), (64, 28672, 192), (31, 16500, 576), (64, 4000, 1088), (18, 2040, 2112), (48, 1000, 8256), (64, 2048, 1984)])
+def test_gemm_ring_of_k_blocks(M, N, K):
+    """17 to 64 rows, k-blocks through a ring in LDS: fewer and more k-blocks than the ring has stages, odd numbers of them where a
+    stage holds two, unequal shares of a split k, blocks of 16, 24, 32, 64 and 112 features cut by N; every epilogue, rows with a stride."""
+    k = kernels()
+    a, w = rnd((M, K + 16), torch.bfloat16, 3)[:, :K], rnd((N, K), torch.bfloat16, 4, 0.1)
+    acc = a.double().cpu() @ w.double().cpu().T
+    n_ws = k.gemm_workspace_floats(M, N, K)
+    for epi in (EPI_STORE, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU):
+        if epi == EPI_SWIGLU:
+            out, ref = torch.zeros((M, N // 2), dtype=torch.bfloat16, device=DEV), plain_silu(acc[:, 0::2]) * acc[:, 1::2]
+        else:
+            out = rnd((M, N), torch.float32, 5) if epi == EPI_ACCUM_F32 else torch.zeros((M, N), dtype=torch.bfloat16 if epi == EPI_STORE else torch.float32, device=DEV)
+            ref = out.double().cpu() + acc if epi == EPI_ACCUM_F32 else acc
+        for room in ([False, True] if n_ws else [False]):
+            got = out.clone()
+            k.gemm(a, w, got, epi, torch.full((n_ws,), 7.0, device=DEV) if room else None)
+            err = (got.double().cpu() - ref).abs()
+            floor = 1e-5 * math.sqrt(K) * (1 + 0.1 * math.sqrt(K) if epi == EPI_SWIGLU else 1)
+            assert (err <= out_tol(ref, out.dtype, floor)).all(), (epi, room, float(err.max()))
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 4096, 1024), (600, 4100, 1088), (1030, 2048, 2048), (530, 1000, 4160), (512, 130, 8256), (2032, 3072, 192),
                                    (700, 16, 1024)])
 def test_gemm_tall_tiles_split_over_k(M, N, K):
