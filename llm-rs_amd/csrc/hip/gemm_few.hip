@@ -1,23 +1,26 @@
 // Products of up to 16 rows (decoding), bfloat16 and 32-bit, on the matrix cores with 32-bit sums.
 //
-// What bounds them: the weight's bytes, each read once, and how many of them are on their way at a time.  A block owns
-// 8 NG output features; its NW waves take the k-blocks (128 bytes of a row: 64 bfloat16 or 32 32-bit numbers) in turn, U
-// of them a round with all loads of a round asked for before its first product, and add their sums through LDS in wave order.
+// What bounds them: the weight's bytes, each read once, how many of them are on their way at a time, and the address unit in
+// front of the vector cache, which takes a line a clock.  A block owns 8 NG output features; its NW waves take the k-blocks
+// (128 bytes of a row: 64 bfloat16 or 32 32-bit numbers) in turn and add their sums through LDS in wave order.  Every wave has
+// a ring of R k-blocks in LDS to itself: loads straight into LDS bring whole lines, eight rows of 128 bytes to an
+// instruction (an operand read straight from memory is 16 rows to 16 lanes, 64 lines to an instruction; in a block of 8 features
+// with 8 tokens that was 33,000 clocks of 2048 x 8192 32-bit numbers' 48,000), no barrier stands between them, and the
+// next ones are on their way while this one is multiplied.  Chunk c of row r lies in slot c ^ (r & 7) of its row: eight lanes' reads
+// hit eight bank groups.
 //
 // v_mfma_f32_16x16x32_bf16 and v_mfma_f32_16x16x4_f32 multiply 16 rows of the weight (operand A) by 16 tokens (operand B).
 //   Up to 8 tokens (FOLD) half of that would be work for rows that are not there, so the operands are folded: their 16 rows are
-//   8 features, and 8 tokens, in each of the two halves of a k-block.  A load instruction then brings whole 128-byte lines of
-//   8 rows of the weight and every lane has a piece of them (with 16 features to an operand it brings 64 bytes of
-//   each, and in a block of 8 features half of the lanes idle), one MFMA contracts the whole k-block, and of
-//   its 16 x 16 results the two 8 x 8 blocks on the diagonal are the halves' sums.
+//   8 features, and 8 tokens, in each of the two halves of a k-block.  One MFMA (four in 32-bit) contracts the whole
+//   k-block, and of its 16 x 16 results the two 8 x 8 blocks on the diagonal are the halves' sums.
 //   9 to 16 tokens: an operand is 16 features, or 16 tokens, of one half of a k-block, and the two halves have sums of their own.
 // Either way an output is the sum, in wave order, of each wave's (first halves' sum + second halves' sum): in bfloat16 its
 // bits depend on K and on the weight's shape, which choose NW and where a block's walk along k begins, never on M.
-// (In 32-bit they differ between up to 8 and more rows, and on the widest weights with the form that M picks, by rounding.)
-// Measured, 16 features an operand for any M -> as here (MI355X, weights from memory, us): bfloat16 at 1 row 2048 x 8192
-// 12.2 -> 8.2, 2048 x 2048 5.3 -> 4.1, 16384 x 2048 15.1 -> 12.6 (5.3 TB/s); at 8 rows 4096 x 4096 11.0 -> 8.4, 4096 x 14336
-// 27.9 -> 24.5, 28672 x 4096 44.4 -> 42.6; 32-bit at 8 rows 2048 x 8192 25.5 -> 18.1, 2048 x 32768 88 -> 61,
-// 16384 x 2048 29.1 -> 25.6.  (A 32-bit MFMA is long: of the 25.5 us some 7 were products for rows that were not there.)
+// (In 32-bit they differ between up to 8 and more rows by rounding.)
+// Measured, 16 features an operand and operands from memory -> as here (MI355X, weights from memory, us): bfloat16 at 1 row
+// 2048 x 8192 12.3 -> 8.6, 2048 x 2048 5.7 -> 4.3, 128256 x 2048 90 -> 83 (6.3 TB/s); at 8 rows 4096 x 4096 11.4 -> 8.6, 4096 x 14336
+// 28.5 -> 23.2, 28672 x 4096 44.2 -> 42.0; at 16 rows 4096 x 4096 13.3 -> 8.5, 4096 x 14336 35 -> 24.7, 10240 x 8192 49.5 -> 34.6;
+// 32-bit at 8 rows 2048 x 8192 26.1 -> 15.5, 2048 x 32768 88 -> 52, 16384 x 2048 28.8 -> 25.9, 128256 x 2048 187 -> 174.
 #include "gemm_tile.h"
 
 template <class T> struct Few;
@@ -60,7 +63,7 @@ struct FewPlain {};
 struct FewScaled { RowScale scale; };
 struct FewNext { RowScale scale; NextNorm next; };
 struct FewQkv { RowScale scale; QkvEpilogue qkv; };
-template <class T, bool FOLD, int NG, int NW, int U, int ROT, int SUMS, class Extra>
+template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS, class Extra>
 __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ W, void* __restrict__ out, int lda,
                                                            int ldc, int M, int N, int K, int epi, unsigned inv_full, Extra extra) {
     constexpr bool NEXT = std::is_same<Extra, FewNext>::value, QKV = std::is_same<Extra, FewQkv>::value;
@@ -76,20 +79,23 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     constexpr int TILES = (NG + 1) / 2;                            // tiles of 16 features (the last one half, where NG is odd)
     constexpr int TOK = FOLD ? 8 : 16;
     constexpr int WL = FOLD ? NG : TILES * 2, XL = FOLD ? 1 : 2;   // a lane's pieces of a k-block: weight, tokens
-    extern __shared__ __attribute__((aligned(16))) unsigned char few_smem[];
-    f32x4* red = (f32x4*)few_smem;                                 // [NW][NG][2: four features each][TOK]
+    constexpr int LOADS = NG + XL, BLOCK = LOADS * 1024;           // a k-block in LDS: eight rows of 128 bytes to a load
+    static_assert((R - 2) * LOADS < 64 && R >= 2, "vmcnt counts to 63");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char few_smem[];
+    f32x4* red = (f32x4*)(few_smem + NW * R * BLOCK);              // [NW][NG][2: four features each][TOK]
     float* scale_red = (float*)(red + NW * NG * 2 * TOK);          // [NW][16]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * NG * 8;
-    // where a lane's pieces lie within a k-block, and its rows
-    const int first = (FOLD ? (row >> 3) * 4 + g : g) * PER;
-    const T* wp[FOLD ? NG : TILES];
-    const bool last_asks = FOLD || NG % 2 == 0 || row < 8;         // whether this lane's row of the last tile is the block's
+    // the rows that this lane's part of a load is of, at the chunk that belongs in the lane's slot
+    const T* src[LOADS];
+    {
+        const int lrow = lane >> 3, chunk = ((lane & 7) ^ lrow) * PER;
 #pragma unroll
-    for (int i = 0; i < (FOLD ? NG : TILES); ++i)
-        wp[i] = W + (size_t)min(n0 + (FOLD ? i * 8 + (row & 7) : i * 16 + row), N - 1) * K + first;
-    const T* xp = A + (size_t)min(FOLD ? row & 7 : row, M - 1) * lda + first;
+        for (int i = 0; i < NG; ++i) src[i] = W + (size_t)min(n0 + i * 8 + lrow, N - 1) * K + chunk;
+#pragma unroll
+        for (int i = 0; i < XL; ++i) src[NG + i] = A + (size_t)min(i * 8 + lrow, M - 1) * lda + chunk;
+    }
     FewSums<T, SUMS> acc[WL];
 #pragma unroll
     for (int i = 0; i < WL; ++i) acc[i].clear();
@@ -132,57 +138,66 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
         unsigned start = (unsigned)n0 / ROT * STEP & 0xffffu;
         rot = full > 1 ? (int)(start - __umulhi(start, inv_full) * (unsigned)full) : 0;
     }
-    auto turn = [&](int j) { int x = j + rot; return (x >= full ? x - full : x) * KB; };
-    auto ask = [&](Piece (&w)[WL], Piece (&x)[XL], int k) {
-        if constexpr (FOLD) {
+    // This wave's k-blocks, the wave + NW i'th of the walk, through a ring of R places of its own: R - 1 of them on their way.
+    // Loads complete in order, so a k-block has landed when all but the loads behind its own have; the place that the next
+    // one goes into was read for the products before.
+    unsigned char* ring = few_smem + wave * (R * BLOCK);
+    const int mine = (full - wave + NW - 1) / NW;
+    int at = wave + rot, put = 0;                                  // of the next k-block asked for: its place in the row, and in the ring
+    auto ask = [&] {
+        const size_t k = (size_t)(at >= full ? at - full : at) * KB;
 #pragma unroll
-            for (int i = 0; i < NG; ++i) w[i] = *(const Piece*)(wp[i] + k);
-            x[0] = *(const Piece*)(xp + k);
-        } else {
-#pragma unroll
-            for (int i = 0; i < TILES; ++i) {
-                if (i < TILES - 1 || last_asks) { w[2 * i] = *(const Piece*)(wp[i] + k); w[2 * i + 1] = *(const Piece*)(wp[i] + k + KB / 2); }
-                else w[2 * i] = w[2 * i + 1] = Piece{};
-            }
-            x[0] = *(const Piece*)(xp + k);
-            x[1] = *(const Piece*)(xp + k + KB / 2);
-        }
+        for (int i = 0; i < LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + k),
+                                             (__attribute__((address_space(3))) void*)(ring + __builtin_amdgcn_readfirstlane(put * BLOCK + i * 1024)), 16, 0, 0);
+        at += NW;
+        put = put + 1 == R ? 0 : put + 1;
     };
     auto products = [&](const Piece (&w)[WL], const Piece (&x)[XL]) {
 #pragma unroll
         for (int i = 0; i < WL; ++i) acc[i].add(w[i], x[FOLD ? 0 : i & 1]);
     };
-    int j = wave;
-    for (; j + (U - 1) * NW < full; j += U * NW) {
-        Piece w[U][WL], x[U][XL];
 #pragma unroll
-        for (int u = 0; u < U; ++u) ask(w[u], x[u], turn(j + u * NW));
-        __builtin_amdgcn_sched_barrier(0);       // keep the round's loads together, ahead of its products
+    for (int i = 0; i < R - 1; ++i)
+        if (i < mine) ask();
+    const int f = row & 7;
+    const int off0 = f * 128 + (((FOLD ? (row >> 3) * 4 + g : g) ^ f) * 16), off1 = f * 128 + (((4 + g) ^ f) * 16);      // a lane's pieces of eight rows
+    for (int i = 0, get = 0; i < mine; ++i, get = get + 1 == R ? 0 : get + 1) {
+        if (i + R - 1 <= mine) wait_vmcnt<(R - 2) * LOADS>(); else wait_vmcnt<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // (the place about to be filled has been read)
+        if (i + R - 1 < mine) ask();
+        const unsigned char* b = ring + get * BLOCK;
+        Piece w[WL], x[XL];
+        if constexpr (FOLD) {
+            x[0] = *(const Piece*)(b + NG * 1024 + off0);
 #pragma unroll
-        for (int u = 0; u < U; ++u) products(w[u], x[u]);
+            for (int t = 0; t < NG; ++t) w[t] = *(const Piece*)(b + t * 1024 + off0);
+        } else {
+            const int half = (row >> 3) * 1024;
+            x[0] = *(const Piece*)(b + NG * 1024 + half + off0);
+            x[1] = *(const Piece*)(b + NG * 1024 + half + off1);
+            // (with an odd number of groups the last tile's other half reads the tokens' rows: its sums are not used)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+                w[2 * t] = *(const Piece*)(b + t * 2048 + half + off0);
+                w[2 * t + 1] = *(const Piece*)(b + t * 2048 + half + off1);
+            }
+        }
+        products(w, x);
     }
-    if (U > 1 && j < full) {                     // what is left of this wave's turns: a round too
-        Piece w[U][WL], x[U][XL];
-#pragma unroll
-        for (int u = 0; u < U - 1; ++u)
-            if (j + u * NW < full) ask(w[u], x[u], turn(j + u * NW));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < U - 1; ++u)
-            if (j + u * NW < full) products(w[u], x[u]);
-    }
-    if (K % KB != 0 && wave == full % NW) {      // the k-block that K cuts
-        const int k = full * KB;
-        const bool v0 = k + first < K, v1 = !FOLD && k + KB / 2 + first < K;
+    if (K % KB != 0 && wave == full % NW) {      // the k-block that K cuts, straight from memory
+        const int k = full * KB, first = (FOLD ? (row >> 3) * 4 + g : g) * PER;
         Piece w[WL], x[XL];
 #pragma unroll
         for (int i = 0; i < WL; ++i) {
-            const int t = FOLD ? i : i / 2;
-            const bool asks = (FOLD || t < TILES - 1 || last_asks) && (FOLD || i % 2 == 0 ? v0 : v1);
-            w[i] = asks ? *(const Piece*)(wp[t] + k + (FOLD ? 0 : (i % 2) * (KB / 2))) : Piece{};
+            const int n = n0 + (FOLD ? i * 8 + f : (i / 2) * 16 + row), from = k + first + (FOLD ? 0 : (i % 2) * (KB / 2));
+            w[i] = from < K ? *(const Piece*)(W + (size_t)min(n, N - 1) * K + from) : Piece{};
         }
-        x[0] = v0 ? *(const Piece*)(xp + k) : Piece{};
-        if constexpr (!FOLD) x[1] = v1 ? *(const Piece*)(xp + k + KB / 2) : Piece{};
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const int from = k + first + i * (KB / 2);
+            x[i] = from < K ? *(const Piece*)(A + (size_t)min(FOLD ? f : row, M - 1) * lda + from) : Piece{};
+        }
         products(w, x);
     }
     if (scaled) {
@@ -289,14 +304,19 @@ struct FewCall {
     RowScale scale;
     NextNorm next;
 };
-template <class T, bool FOLD, int NG, int NW, int U, int ROT, int SUMS = 1>
+template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS = 1>
 static void launch_few(const FewCall& c) {
     static_assert(ROT % (NG * 8) == 0, "a block's features lie in one group");
     const unsigned full = c.K * sizeof(T) / 128, inv_full = full > 1 ? (unsigned)(((1ull << 32) + full - 1) / full) : 0;
-    constexpr size_t bytes = (size_t)NW * NG * 2 * (FOLD ? 8 : 16) * 16 + NW * 16 * sizeof(float);
-    static_assert(bytes <= 64 * 1024, "the waves' sums must fit in the LDS that a block may ask for");
+    constexpr size_t bytes = (size_t)NW * R * (NG + (FOLD ? 1 : 2)) * 1024 + (size_t)NW * NG * 2 * (FOLD ? 8 : 16) * 16 + NW * 16 * sizeof(float);
+    static_assert(bytes <= 160 * 1024, "the rings and the waves' sums must fit in a unit's LDS");
     auto launch = [&](auto extra) {
-        gemm_few_kernel<T, FOLD, NG, NW, U, ROT, SUMS><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
+        static bool configured = false;
+        if (!configured) {
+            (void)hipFuncSetAttribute((const void*)gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS, decltype(extra)>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+            configured = true;
+        }
+        gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
             (const T*)c.A, (const T*)c.W, c.out, c.lda, c.ldc, c.M, c.N, c.K, c.epi, inv_full, extra);
     };
     if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
@@ -304,13 +324,6 @@ static void launch_few(const FewCall& c) {
     else if (c.scale.sumsq != nullptr) launch(FewScaled{c.scale});
     else launch(FewPlain{});
 }
-// bfloat16.  Up to 8 rows: blocks of 8 NG features, U k-blocks a round; 9 to 16 rows: of 8 NG16, U16.  NW and ROT are the same on both sides.
-template <int NW, int ROT, int NG, int U, int NG16, int U16>
-static void launch_few_by_rows(const FewCall& c) {
-    if (c.M <= 8) launch_few<bf16, true, NG, NW, U, ROT>(c);
-    else launch_few<bf16, false, NG16, NW, U16, ROT>(c);
-}
-
 // Whether blocks of 24 features (a tile and a half) share a weight of N features out over the device's units more
 // evenly, by a tenth of a round or more, than blocks of `whole` features (16 or 32) do.
 bool llmrs_half_tile_blocks(int N, int whole, int cus) {
@@ -321,8 +334,8 @@ bool llmrs_half_tile_blocks(int N, int whole, int cus) {
 static bool half_blocks_for_narrow(int N, int K) {
     return N < 16384 && K >= 2048 && N % 8 == 0 && ceil_div(N, 16) * 2 <= llmrs_compute_units();
 }
-// A wide weight's blocks of 9 to 16 rows take 7 or 4 tiles of 16 features, whichever number of blocks fills the device's
-// units more evenly (28672 features are 256 blocks of 7 tiles).
+// Whether a wide weight's blocks fill the device's units more evenly by 7 or by 4 tiles of 16 features
+// (28672 features are 256 blocks of 7 tiles).
 static int wide_tiles(int N, int cus) {
     auto evenness = [&](int nt) { int b = ceil_div(N, 16 * nt); return (double)b / ((double)ceil_div(b, cus) * cus); };
     return evenness(7) >= evenness(4) ? 7 : 4;
@@ -333,65 +346,37 @@ extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
     return M <= 16 && half_blocks_for_narrow(N, K) ? ceil_div(N, 8) : ceil_div(N, 16);
 }
 
-// In bfloat16 waves per block and the walk's start come from the weight's shape alone (see above).  With fewer features a block, more
-// blocks ask at once but each reads the tokens' rows again.
-static void few_rows(const FewCall& c, bf16) {
-    const int N = c.N, K = c.K, cus = llmrs_compute_units();
-    if (N >= 16384) {
-        if (wide_tiles(N, cus) == 7) {
-            // (28672 x 4096 at 1, 4, 8 rows: blocks of 16 features 40.3, 40.7, 44, of 112 41.5, 42.3, 43.4)
-            if (c.M <= 4) launch_few<bf16, true, 2, 4, 8, 112>(c);
-            else launch_few<bf16, false, 14, 4, 1, 112>(c);
-        }
-        // (16384 x 2048 at 1, 4, 8 rows: blocks of 16 features 14.4, 14.7, 15.9, of 32 15.0, 15.0, 15.2; 128256 at 1 row 92.7 and 88.4)
-        else if (c.M <= 4 && N < 32768) launch_few<bf16, true, 2, 4, 8, 64>(c);
-        else launch_few_by_rows<4, 64, 4, 8, 8, 2>(c);
-    }
-    else if (K < 2048) launch_few_by_rows<4, 0, 2, 4, 2, 4>(c);
-    else if (K >= 16384 && N >= 8192) launch_few_by_rows<8, 64, 4, 4, 4, 4>(c);      // 8192 x 28672 at 16 rows: 90 -> 83 us
-    else if (half_blocks_for_narrow(N, K)) {
-        if (K >= 4096) launch_few_by_rows<8, 64, 1, 8, 1, 4>(c);
-        else launch_few_by_rows<8, 0, 1, 4, 1, 4>(c);
-    }
-    // (nothing is to be left for a norm, which counts its sums by 16 features; 6144 x 4096 at 8 rows 12.6 against 16.0 in
-    // blocks of 16, 10240 x 8192 at 2 rows 34.9 against 37.1)
-    else if (c.next.y == nullptr && (llmrs_half_tile_blocks(N, 16, cus) || ceil_div(N, 16) > 2 * cus)) {
-        if (K >= 4096) launch_few_by_rows<8, 96, 3, 8, 3, 4>(c);
-        else launch_few_by_rows<8, 96, 3, 4, 3, 4>(c);
-    }
-    else if (K >= 4096) launch_few_by_rows<8, 64, 2, 8, 2, 4>(c);
-    else launch_few_by_rows<8, 0, 2, 4, 2, 4>(c);
+// Up to 8 rows: blocks of 8 NG features, rings of R k-blocks, in 32-bit four sums a tile; 9 to 16 rows: of 8 NG16, R16, one sum: the
+// error of the 32-bit products against 64 bits is then no larger than it was with one sum for whole k-blocks (K = 2048: 1.25e-7
+// up to 8 rows, 2.1e-7 from 9 on, against 2.9e-7; one and two rows as in gemm_rows_kernel, 1.2e-7).
+template <class T, int NW, int ROT, int NG, int R, int NG16, int R16>
+static void launch_few_by_rows(const FewCall& c) {
+    if (c.M <= 8) launch_few<T, true, NG, NW, R, ROT, sizeof(T) == 4 ? 4 : 1>(c);
+    else launch_few<T, false, NG16, NW, R16, ROT>(c);
 }
-// 32-bit: up to 8 rows four sums a tile (two in blocks of 56 features, which have no registers for four), more rows one: in each
-// the error against 64 bits is no larger than it was with one sum for whole k-blocks (K = 2048: 1.25e-7 up to 8 rows, 2.1e-7 from
-// 9 on, against 2.9e-7; one and two rows as in gemm_rows_kernel, 1.2e-7).
-static void few_rows(const FewCall& c, float) {
+// Waves per block and the walk's start come from the weight's shape alone (see above).  With fewer features a block, more blocks
+// ask at once but each reads the tokens' rows again.  Rings of three k-blocks do nearly as well as any: what is on its way
+// is then some 32 KB of the weight a unit.
+template <class T>
+static void few_rows(const FewCall& c) {
     const int N = c.N, K = c.K, cus = llmrs_compute_units();
-    const bool fold = c.M <= 8;
     if (N >= 16384) {
-        if (N % 112 == 0) {
-            // (28672 x 4096 at 1 row: blocks of 16 features 83.2, of 56 86.8; at 8 rows 90 and 86.5)
-            if (c.M <= 4) launch_few<float, true, 2, 8, 4, 112, 4>(c);
-            else if (fold) launch_few<float, true, 7, 8, 2, 112, 2>(c);
-            else launch_few<float, false, 14, 8, 1, 112>(c);
-        }
-        else if (fold) launch_few<float, true, 4, 8, 2, 64, 4>(c);
-        else launch_few<float, false, 8, 8, 1, 64>(c);
-    } else if (K < 512) {
-        launch_few<float, false, 2, 4, 2, 0, 2>(c);
-    } else if (K < 2048) {
-        if (fold) launch_few<float, true, 2, 4, 4, 0, 4>(c);
-        else launch_few<float, false, 2, 4, 4, 0>(c);
-    } else if (half_blocks_for_narrow(N, K)) {
-        if (!fold) launch_few<float, false, 1, 8, 4, 64>(c);
-        else if (K >= 4096) launch_few<float, true, 1, 8, 8, 64, 4>(c);
-        else launch_few<float, true, 1, 8, 4, 0, 4>(c);
-    } else if (c.next.y == nullptr && llmrs_half_tile_blocks(N, 16, cus)) {
-        if (fold) launch_few<float, true, 3, 8, 4, 96, 4>(c);
-        else launch_few<float, false, 3, 8, 2, 96>(c);
+        // (28672 x 4096 bfloat16 at 8 rows: blocks of 16 features 42.0 us, of 56 43.7, of 112 47; at 16 rows of 56 41.8, of 112 42.4)
+        if (wide_tiles(N, cus) == 7) launch_few_by_rows<T, 4, 112, 2, 4, 7, 3>(c);
+        // (at 16 rows 16384 x 2048: blocks of 64 features 14.5, of 16 15.1; in 32-bit, where a k-block is more MFMAs, 27.4 and 26.0)
+        else if (c.M > 8 && sizeof(T) == 2) launch_few<T, false, 8, 4, 3, 64>(c);
+        // (one and two rows in 32-bit: eight waves, and so sums half as long: the error of gemm_rows_kernel's)
+        else if (c.M <= 2 && sizeof(T) == 4) launch_few<T, true, 2, 8, 3, 64, 4>(c);
+        // (deeper rings let fewer blocks share a unit: 16384 x 2048 at 8 rows 14.3 with three, 14.9 with five; 128256 x 2048 93.2 and 90.9)
+        else if (N < 32768) launch_few_by_rows<T, 4, 64, 2, 3, 2, 4>(c);
+        else launch_few_by_rows<T, 4, 64, 2, 5, 2, 4>(c);
     }
-    else if (fold) launch_few<float, true, 2, 16, 4, 0, 4>(c);           // (sixteen waves: 4096 x 4096 at 8 rows 17.0 us, eight 19.4)
-    else launch_few<float, false, 2, 8, 4, 64>(c);
+    else if (K < 2048) launch_few_by_rows<T, 4, 0, 2, 4, 2, 4>(c);
+    else if (K >= 16384 && N >= 8192) launch_few_by_rows<T, 8, 64, 4, 2, 4, 2>(c);      // 8192 x 28672 at 16 rows: 80.8 us, in blocks of 16 features 89.9
+    else if (half_blocks_for_narrow(N, K)) launch_few_by_rows<T, 8, 64, 1, 5, 1, 4>(c);
+    // (nothing is to be left for a norm, which counts its sums by 16 features; 6144 x 4096 at 8 rows 11.6 us, in blocks of 16 13.5)
+    else if (c.next.y == nullptr && (llmrs_half_tile_blocks(N, 16, cus) || ceil_div(N, 16) > 2 * cus)) launch_few_by_rows<T, 8, 96, 3, 3, 3, 3>(c);
+    else launch_few_by_rows<T, 8, 64, 2, 3, 2, 3>(c);
 }
 
 template <class T>
@@ -406,7 +391,7 @@ static int gemm_few(hipStream_t stream, const T* A, int lda, const T* W, void* o
     }
     if (epi == LLMRS_EPI_QKV && (qkv == nullptr || qkv->head_dim % 4 || ldc % 4 || (uintptr_t)out % FOUR || (uintptr_t)qkv->k_cache % FOUR || qkv->rotary_dim % 4))
         return 0;           // (four features of a head are stored at once)
-    few_rows(FewCall{stream, A, lda, W, out, ldc, M, N, K, epi, qkv ? *qkv : QkvEpilogue{}, scale ? *scale : RowScale{}, next ? *next : NextNorm{}}, T{});
+    few_rows<T>(FewCall{stream, A, lda, W, out, ldc, M, N, K, epi, qkv ? *qkv : QkvEpilogue{}, scale ? *scale : RowScale{}, next ? *next : NextNorm{}});
     return 1;
 }
 int llmrs_gemm_few_bf16(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi,

@@ -536,6 +536,27 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
         assert (err <= out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))).all(), (epi, float(err.max()))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(1, 40, 64), (8, 24, 96), (9, 250, 544), (16, 1990, 2048), (7, 2040, 2080), (16, 2048, 2592), (8, 3000, 2304), (13, 3080, 2176),
+                                   (8, 6136, 2112), (16, 6150, 2048), (3, 16390, 288), (10, 16400, 2048), (8, 33000, 160), (5, 28650, 352), (11, 28672, 64), (8, 8200, 16448)])
+def test_gemm_few_rows_and_their_rings(dtype, M, N, K):
+    """Up to 16 rows: waves with no k-block, fewer than their ring has places, as many and more; blocks of 8, 16, 24, 32, 56 and 64
+    features cut by N, a k-block cut by K; both sides of 8 rows; every epilogue, rows with a stride."""
+    k = kernels()
+    a, w = rnd((M, K + 24), dtype, 3)[:, :K], rnd((N, K), dtype, 4, 0.1)
+    acc = a.double().cpu() @ w.double().cpu().T
+    for epi in (EPI_STORE, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU):
+        if epi == EPI_SWIGLU:
+            out, ref = torch.zeros((M, N // 2), dtype=dtype, device=DEV), plain_silu(acc[:, 0::2]) * acc[:, 1::2]
+        else:
+            out = rnd((M, N), torch.float32, 5) if epi == EPI_ACCUM_F32 else torch.zeros((M, N), dtype=dtype if epi == EPI_STORE else torch.float32, device=DEV)
+            ref = out.double().cpu() + acc if epi == EPI_ACCUM_F32 else acc
+        k.gemm(a, w, out, epi)
+        err = (out.double().cpu() - ref).abs()
+        floor = (2e-6 if dtype == torch.float32 else 1e-5) * math.sqrt(K) * (1 + 0.1 * math.sqrt(K) if epi == EPI_SWIGLU else 1)
+        assert (err <= out_tol(ref, out.dtype, floor)).all(), (epi, float(err.max()))
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 40, 64), (33, 250, 128), (48, 4090, 192), (49, 3000, 704), (64, 16, 1344), (20, 6140, 64), (64, 8200, 320),
                                    (40, 16400, 64), (64, 28672, 192), (31, 16500, 576), (64, 4000, 1088), (18, 2040, 2112), (48, 1000, 8256), (64, 2048, 1984)])
 def test_gemm_ring_of_k_blocks(M, N, K):
