@@ -337,67 +337,75 @@ __global__ __launch_bounds__(64) void attention_generic_group_kernel(
     }
 }
 
-// One wave for each (entry, head) adds the chunks up.  The chunks' maxima and sums are read 64 at a time, a lane
-// each; the weighted values are added chunk by chunk in ascending order, four chunks' rows asked for at a time.
-template <class T, int MAPS>
+// One wave for each (entry, head) adds the chunks up, in ascending order; VALS: values of a row that a lane holds.  The
+// kernel is a chain of trips to memory and little else, so the first one brings all that most requests need: the entry's length,
+// the maxima and sums of up to 64 chunks, a lane each, and the rows of the first chunks, of both maps, asked for before
+// the length is known (they lie within the scratch; what is beyond the entry's chunks is not used).  Further rows come as many at a time.
+// (32-bit, 8 requests of 200 to 1800 keys, heads of 64: 6.6 us with lengths, maxima and rows one after the other, rows four at
+// a time; now 4.9.  Of up to 1000 keys, two maps and values of 128: 11.3, now 6.0.)
+template <class T, int MAPS, int VALS>
 __global__ __launch_bounds__(64) void attention_generic_merge_kernel(
     const float* __restrict__ partial, T* __restrict__ out, const int* __restrict__ q_starts,
     const int* __restrict__ seq_lens, int max_chunks, AttnArgs a) {
+    constexpr int AHEAD = VALS == 1 ? 16 : VALS == 2 ? 8 : 4;
     int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, hd = a.v_dim;     // (the rows added up are values)
-    int t = q_starts[e];
-    if (q_starts[e + 1] - t != 1) return;
-    int pos = seq_lens[e] - 1;
+    const size_t stride = hd + 2;
+    int t = q_starts[e], next = q_starts[e + 1], pos = seq_lens[e] - 1;
+    float m_first[MAPS], l_first[MAPS], rows[MAPS][AHEAD][VALS];
+    auto ask = [&](float (&v)[AHEAD][VALS], const float* pp, int first, int n) {       // rows first .. of n
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+            for (int i = 0; i < VALS; ++i) {
+                int d = lane + 64 * i;
+                v[u][i] = first + u < n && d < hd ? pp[(size_t)(first + u) * stride + 2 + d] : 0.0f;
+            }
+    };
+#pragma unroll
+    for (int map = 0; map < MAPS; ++map) {
+        const float* pp = partial + (size_t)((e * a.n_heads + h) * MAPS + map) * max_chunks * stride;
+        m_first[map] = lane < max_chunks ? pp[(size_t)lane * stride] : -INFINITY;
+        l_first[map] = lane < max_chunks ? pp[(size_t)lane * stride + 1] : 0.0f;
+        ask(rows[map], pp, 0, max_chunks);
+    }
+    if (next - t != 1) return;
     int lo = attn_window_lo(a, pos);
     int n_chunks = pos / GENERIC_CHUNK - lo / GENERIC_CHUNK + 1;
-    const size_t stride = hd + 2;
     float o[MAPS][MAX_HEAD_DIM / 64] = {};
 #pragma unroll
     for (int map = 0; map < MAPS; ++map) {
         const float* pp = partial + (size_t)((e * a.n_heads + h) * MAPS + map) * max_chunks * stride;
-        float M = -INFINITY;
-        for (int ch = lane; ch < n_chunks; ch += 64) M = fmaxf(M, pp[(size_t)ch * stride]);
+        float M = lane < n_chunks ? m_first[map] : -INFINITY;
+        for (int ch = lane + 64; ch < n_chunks; ch += 64) M = fmaxf(M, pp[(size_t)ch * stride]);
         M = wave_max(M);
         float L = 0.0f;
         for (int base = 0; base < n_chunks; base += 64) {
             int mine = base + lane;
-            float w_mine = mine < n_chunks ? expf(pp[(size_t)mine * stride] - M) : 0.0f;
-            float l_mine = mine < n_chunks ? pp[(size_t)mine * stride + 1] * w_mine : 0.0f;
+            float m_mine = base == 0 ? m_first[map] : mine < n_chunks ? pp[(size_t)mine * stride] : 0.0f;
+            float l_mine = base == 0 ? l_first[map] : mine < n_chunks ? pp[(size_t)mine * stride + 1] : 0.0f;
+            float w_mine = mine < n_chunks ? expf(m_mine - M) : 0.0f;
+            l_mine = mine < n_chunks ? l_mine * w_mine : 0.0f;
             L += wave_sum(l_mine);
             int n = min(64, n_chunks - base);
-            int j = 0;
-            for (; j + 4 <= n; j += 4) {
-                float v[4][MAX_HEAD_DIM / 64];
+            for (int j = 0; j < n; j += AHEAD) {
+                if (base + j > 0) ask(rows[map], pp, base + j, n_chunks);
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int i = 0; i < MAX_HEAD_DIM / 64; ++i) {
-                        int d = lane + 64 * i;
-                        v[u][i] = d < hd ? pp[(size_t)(base + j + u) * stride + 2 + d] : 0.0f;
-                    }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < AHEAD; ++u) {
+                    if (j + u >= n) break;                       // (the same in all lanes)
                     float w = __shfl(w_mine, j + u, 64);
 #pragma unroll
-                    for (int i = 0; i < MAX_HEAD_DIM / 64; ++i) o[map][i] = fmaf(v[u][i], w, o[map][i]);
-                }
-            }
-            for (; j < n; ++j) {
-                float w = __shfl(w_mine, j, 64);
-#pragma unroll
-                for (int i = 0; i < MAX_HEAD_DIM / 64; ++i) {
-                    int d = lane + 64 * i;
-                    if (d < hd) o[map][i] = fmaf(pp[(size_t)(base + j) * stride + 2 + d], w, o[map][i]);
+                    for (int i = 0; i < VALS; ++i) o[map][i] = fmaf(rows[map][u][i], w, o[map][i]);
                 }
             }
         }
         L += attn_sink_term(a, h, M);
 #pragma unroll
-        for (int i = 0; i < MAX_HEAD_DIM / 64; ++i) o[map][i] /= L;
+        for (int i = 0; i < VALS; ++i) o[map][i] /= L;
     }
     combine_maps<MAPS>(o, a);
     T* orow = out + (size_t)t * a.out_stride + (size_t)h * hd;
 #pragma unroll
-    for (int i = 0; i < MAX_HEAD_DIM / 64; ++i) {
+    for (int i = 0; i < VALS; ++i) {
         int d = lane + 64 * i;
         if (d < hd) orow[d] = from_f32<T>(o[0][i] * attn_gate(a, t, h, d));
     }
@@ -487,8 +495,10 @@ static int launch_generic(hipStream_t stream, const T* q, T* out, const T* k_cac
 #undef SPLIT
         }
         dim3 heads(n_entries, a.n_heads);
-        if (a.maps == 2) attention_generic_merge_kernel<T, 2><<<heads, 64, 0, stream>>>(scratch, out, q_starts, seq_lens, max_chunks, a);
-        else attention_generic_merge_kernel<T, 1><<<heads, 64, 0, stream>>>(scratch, out, q_starts, seq_lens, max_chunks, a);
+#define MERGE(MM, VALS) attention_generic_merge_kernel<T, MM, VALS><<<heads, 64, 0, stream>>>(scratch, out, q_starts, seq_lens, max_chunks, a)
+        if (a.maps == 2) { if (a.v_dim <= 64) MERGE(2, 1); else if (a.v_dim <= 128) MERGE(2, 2); else MERGE(2, MAX_HEAD_DIM / 64); }
+        else { if (a.v_dim <= 64) MERGE(1, 1); else if (a.v_dim <= 128) MERGE(1, 2); else MERGE(1, MAX_HEAD_DIM / 64); }
+#undef MERGE
     }
     return 0;
 }

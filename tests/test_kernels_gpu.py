@@ -460,6 +460,23 @@ def test_attention_float32_decoding_requests(n_heads, n_kv, hd, ps, window):
         assert (err <= out_tol(ref, torch.float32, 2e-6)).all(), f"request of length {lens[r]}: {float(err.max())}"
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (2, 1, 128), (1, 1, 160)])
+def test_attention_float32_merges_many_chunks(n_heads, n_kv, hd):
+    """Requests of as many chunks as the merge asks for at once (16, 8 and 4 rows), one more, and more than a lane has chunks (64):
+    the largest weight lies in the first, the last and a middle chunk in turn, beside an entry of several tokens."""
+    lens = [512, 513, 1024, 1025, 2048, 2049, 8300, 40]
+    case = PagedCase(torch.float32, lens, n_heads, n_kv, hd, 16, seed=37)
+    g = torch.Generator().manual_seed(5)
+    for where in (0, -1, 300):
+        qs = [case.k[r][where].repeat_interleave(n_heads // n_kv, dim=0).unsqueeze(0) * 0.5 + torch.randn((1, n_heads, hd), generator=g) for r in range(7)]
+        qs.append(torch.randn((3, n_heads, hd), generator=g))
+        pos = [[n - 1] for n in lens[:7]] + [[37, 38, 39]]
+        got = case.run(qs, pos, n_single=7, single_keys=sum(lens[:7]))
+        for r in range(7):
+            ref = case.reference(r, qs[r], pos[r])[0]
+            assert ((got[r].double() - ref).abs() <= out_tol(ref, torch.float32, 2e-6)).all(), (lens[r], where)
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 48, 64), (8, 4096, 4096), (16, 6144, 2048), (5, 130, 96), (9, 28672, 256), (12, 16400, 128),
                                    (16, 2048, 8192), (7, 5000, 1024), (4, 100, 32)])
 def test_gemm_float32_few_rows_on_the_matrix_cores(M, N, K):
