@@ -732,8 +732,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // sixteen to a compute unit the scattered pages come slower than with eight once the device is full (decode steps
 // of the 8B shape, eight waves against twelve: 64 requests over 8128 keys 15.9 against 16.9 ms, 256 over 2048 18.3
 // against 20.7; the 1B serving run 3.03 against 3.10 s with sixteen).  Every block asks for an eighth of a
-// unit's LDS, which it does not use, and that keeps a unit to eight.
+// unit's LDS, and that keeps a unit to eight.
 #define SPLIT16_LDS_BYTES (160 * 1024 / 8)
+// Heads of 64: a step's keys and values (8 KB) go straight into the LDS that a block asks for anyway, two steps' places of it, the
+// next step's while this one is multiplied.  Operands straight from memory are 16 rows to 16 lanes, 64 lines an instruction
+// in front of the vector cache, and a step waits for its values after its scores.  (160 requests of 128 to 4096 keys, heads of
+// 64: eight layers 2.141 -> 2.120 ms; beside a prompt portion, the 1B serving step, 7.96 -> 7.80.  Three or four places leave a
+// unit six or five of these waves: 2.08 for the 160, but 32 requests of 500 to 3000 keys 0.837 -> 0.847.  Heads of 128, whose
+// steps are 16 KB, are slower that way: 64 requests 2.00 -> 2.07.)
+constexpr int split16_ring(int kd, int vd) { return kd == 64 && vd <= 64 ? 2 : 0; }
 
 // The value of the lane 16 further on or back (the partner in the neighbouring row of 16 lanes), by the register
 // swap of gfx950: of {x, x} it makes {rows 0, 0, 2, 2 of x; rows 1, 1, 3, 3 of x}.
@@ -759,6 +766,10 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
                                                           const int* __restrict__ q_starts, AttnArgs a, int G,
                                                           int max_chunks, int chunk, int plain, int entry_first) {
     static_assert(KD % 32 == 0 && VD % 16 == 0, "the score products take 32 features at a time");
+    constexpr int RING = split16_ring(KD, VD);      // steps in LDS (0: operands straight from memory)
+    constexpr int PAGE_K = KD * 32, PAGE_V = VD * 32, STEP = 2 * (PAGE_K + PAGE_V), LOADS = STEP / 1024;
+    static_assert(RING * STEP <= SPLIT16_LDS_BYTES, "the steps lie in what a block asks for");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char split16_smem[];
     int kvh = entry_first ? blockIdx.y : blockIdx.x, e = entry_first ? blockIdx.x : blockIdx.y, ch = blockIdx.z;      // (see `launch`)
     int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     bool cvalid = c < G;
@@ -812,9 +823,9 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
     float m = -INFINITY, l = 0.0f;                    // m: the same in a column's four lanes; l: this lane's share of the sum
     // the keys of tile t that this lane's operand row holds, within a 32-key step: 8 * (row / 4) + row % 4 + 4t
     int krow = 8 * (c >> 2) + (c & 3);
-    // A unit holds eight of these waves whatever they take (see SPLIT16_LDS_BYTES), so up to head size 128 a wave has
-    // the registers for a second set of key operands: the next step's keys are asked for before this step's products.
-    constexpr bool KEYS_AHEAD = KD <= 128;
+    // Without a ring a wave has the registers for a second set of key operands up to head size 128: the next step's keys are asked
+    // for before this step's products.
+    constexpr bool KEYS_AHEAD = RING == 0 && KD <= 128;
     auto pages_of = [&](int t0, int& a0, int& a1) {
         int lp = t0 >> 4;
         if (lp + 1 - pv_base >= 64) { pv_base = lp; pv = load_pages(lp); }
@@ -830,8 +841,31 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
             for (int j = 0; j < KD / 32; ++j) k[t][j] = *(const bf16x8*)(kp + j * 32);
         }
     };
+    // A step's two pages of keys and two of values straight into LDS, whole lines at a time.  Chunk x of a key's row lies in
+    // slot x ^ f of it, f made of the bits of the key that differ between eight lanes of an operand read (0, 1 and 3).
+    auto bring = [&](int t0, int place) {
+        int a0, a1;
+        pages_of(t0, a0, a1);
+        unsigned char* to = split16_smem + place * STEP;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const bf16* kp = kc + ((size_t)(p ? a1 : a0) * a.n_kv_heads + kvh) * (16 * KD);
+            const bf16* vp = vc + ((size_t)(p ? a1 : a0) * a.n_kv_heads + kvh) * (16 * VD);
+#pragma unroll
+            for (int i = 0; i < PAGE_K / 1024; ++i) {
+                constexpr int PER_ROW = KD / 8;                        // 16-byte chunks of a key
+                int at = i * 64 + lane, key = at / PER_ROW, slot = at % PER_ROW, f = (key & 3) | ((key >> 1) & 4);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kp + key * KD + (slot ^ f) * 8),
+                                                 (__attribute__((address_space(3))) void*)(to + __builtin_amdgcn_readfirstlane(p * PAGE_K + i * 1024)), 16, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < PAGE_V / 1024; ++i)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vp + i * 512 + lane * 8),
+                                                 (__attribute__((address_space(3))) void*)(to + __builtin_amdgcn_readfirstlane(2 * PAGE_K + p * PAGE_V + i * 1024)), 16, 0, 0);
+        }
+    };
     bf16x8 kf[2][KD / 32];
-    int p0 = 0, p1 = 0;
+    int p0 = 0, p1 = 0, put = 0, get = 0;
     for (int walk = kept_end > 0 ? 0 : 1; walk < 2; ++walk) {
     if (kept_end > 0) {                                // (the same in all lanes) this walk's keys and their page numbers
         t_begin = walk == 0 ? 0 : chunk_begin;
@@ -843,24 +877,48 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
         pages_of(t_begin, p0, p1);
         load_keys(kf, p0, p1);
     }
+    if constexpr (RING > 0) {
+        put = get = 0;
+#pragma unroll
+        for (int i = 0; i < RING - 1; ++i)
+            if (t_begin + 32 * i < t_end) { bring(t_begin + 32 * i, put); put = put + 1 == RING ? 0 : put + 1; }
+    }
     for (int t0 = t_begin; t0 < t_end; t0 += 32) {
         bf16x8 kn[2][KD / 32];
         int n0 = 0, n1 = 0;
         const bool more = t0 + 32 < t_end;                            // (the same in all lanes)
-        if constexpr (KEYS_AHEAD) {
-            if (more) {
-                pages_of(t0 + 32, n0, n1);
-                load_keys(kn, n0, n1);
-            }
-        } else {
-            pages_of(t0, p0, p1);
-            load_keys(kf, p0, p1);
-        }
-        // values: lane (feature row c, g) takes keys 8g .. 8g + 7 of the step: page g / 2, keys 8 * (g % 2) .. of it
         bf16x8 vf[VD / 16];
-        const bf16* vp = vc + (((size_t)(g < 2 ? p0 : p1) * a.n_kv_heads + kvh) * VD + c) * 16 + (g & 1) * 8;
+        if constexpr (RING > 0) {
+            // this step has landed when all but the loads of the steps behind it have; the place that the next one goes into was
+            // read for the products before
+            if (t0 + 32 * (RING - 2) < t_end) wait_vmcnt_n<(RING - 2) * LOADS>(); else wait_vmcnt_all();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (t0 + 32 * (RING - 1) < t_end) { bring(t0 + 32 * (RING - 1), put); put = put + 1 == RING ? 0 : put + 1; }
+            const unsigned char* from = split16_smem + get * STEP;
+            get = get + 1 == RING ? 0 : get + 1;
 #pragma unroll
-        for (int dt = 0; dt < VD / 16; ++dt) vf[dt] = *(const bf16x8*)(vp + dt * 16 * 16);
+            for (int t = 0; t < 2; ++t) {
+                const int key = krow + 4 * t, f = (key & 3) | ((key >> 1) & 4);
+#pragma unroll
+                for (int j = 0; j < KD / 32; ++j) kf[t][j] = *(const bf16x8*)(from + key * (KD * 2) + (((j * 4 + g) ^ f) * 16));
+            }
+            // values: lane (feature row c, g) takes keys 8g .. 8g + 7 of the step: page g / 2, keys 8 * (g % 2) .. of it
+#pragma unroll
+            for (int dt = 0; dt < VD / 16; ++dt) vf[dt] = *(const bf16x8*)(from + 2 * PAGE_K + (g >> 1) * PAGE_V + (dt * 16 + c) * 32 + (g & 1) * 16);
+        } else {
+            if constexpr (KEYS_AHEAD) {
+                if (more) {
+                    pages_of(t0 + 32, n0, n1);
+                    load_keys(kn, n0, n1);
+                }
+            } else {
+                pages_of(t0, p0, p1);
+                load_keys(kf, p0, p1);
+            }
+            const bf16* vp = vc + (((size_t)(g < 2 ? p0 : p1) * a.n_kv_heads + kvh) * VD + c) * 16 + (g & 1) * 8;
+#pragma unroll
+            for (int dt = 0; dt < VD / 16; ++dt) vf[dt] = *(const bf16x8*)(vp + dt * 16 * 16);
+        }
         f32x4 S[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {

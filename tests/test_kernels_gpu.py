@@ -460,6 +460,21 @@ def test_attention_float32_decoding_requests(n_heads, n_kv, hd, ps, window):
         assert (err <= out_tol(ref, torch.float32, 2e-6)).all(), f"request of length {lens[r]}: {float(err.max())}"
 
 
+@pytest.mark.parametrize("n_heads,n_kv,window", [(8, 2, 0), (8, 2, 40), (3, 3, 0), (32, 2, 0), (16, 1, 70)])
+def test_attention_single_tokens_of_heads_of_64(n_heads, n_kv, window):
+    """Steps of 32 keys through LDS: requests of one key, of a page, of less and more than a step, of one step, two and three, and of
+    chunks' lengths, with and without a window that cuts a step."""
+    lens = [1, 15, 16, 17, 32, 33, 48, 64, 65, 96, 97, 128, 513, 1100]
+    case = PagedCase(torch.bfloat16, lens, n_heads, n_kv, 64, 16, seed=91)
+    g = torch.Generator().manual_seed(2)
+    qs, pos = [torch.randn((1, n_heads, 64), generator=g).to(torch.bfloat16) for _ in lens], [[n - 1] for n in lens]
+    got = case.run(qs, pos, window=window, n_single=len(lens), single_keys=sum(lens))
+    for r in range(len(lens)):
+        # (probabilities are rounded to bfloat16, 2^-9 of a value at most: of values of size 1 to 4, averaged)
+        ref = case.reference(r, qs[r], pos[r], window=window)[0]
+        assert ((got[r].double() - ref).abs() <= out_tol(ref, torch.bfloat16, 8e-3)).all(), lens[r]
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (2, 1, 128), (1, 1, 160)])
 def test_attention_float32_merges_many_chunks(n_heads, n_kv, hd):
     """Requests of as many chunks as the merge asks for at once (16, 8 and 4 rows), one more, and more than a lane has chunks (64):
