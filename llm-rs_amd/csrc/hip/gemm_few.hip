@@ -1,4 +1,4 @@
-// Products of up to 16 rows (decoding), bfloat16 and 32-bit, on the matrix cores with 32-bit sums.
+// Products of up to 16 rows (decoding), in 32-bit up to 32, bfloat16 and 32-bit, on the matrix cores with 32-bit sums.
 //
 // What bounds them: the weight's bytes, each read once, how many of them are on their way at a time, and the address unit in
 // front of the vector cache, which takes a line a clock.  A block owns 8 NG output features; its NW waves take the k-blocks
@@ -13,7 +13,8 @@
 //   Up to 8 tokens (FOLD) half of that would be work for rows that are not there, so the operands are folded: their 16 rows are
 //   8 features, and 8 tokens, in each of the two halves of a k-block.  One MFMA (four in 32-bit) contracts the whole
 //   k-block, and of its 16 x 16 results the two 8 x 8 blocks on the diagonal are the halves' sums.
-//   9 to 16 tokens: an operand is 16 features, or 16 tokens, of one half of a k-block, and the two halves have sums of their own.
+//   9 to 16 tokens: an operand is 16 features, or 16 tokens, of one half of a k-block, and the two halves have sums of their own;
+//   17 to 32: the same with TT = 2 tiles of tokens.
 // Either way an output is the sum, in wave order, of each wave's (first halves' sum + second halves' sum): in bfloat16 its
 // bits depend on K and on the weight's shape, which choose NW and where a block's walk along k begins, never on M.
 // (In 32-bit they differ between up to 8 and more rows by rounding.)
@@ -63,7 +64,7 @@ struct FewPlain {};
 struct FewScaled { RowScale scale; };
 struct FewNext { RowScale scale; NextNorm next; };
 struct FewQkv { RowScale scale; QkvEpilogue qkv; };
-template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS, class Extra>
+template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS, int TT, class Extra>
 __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ W, void* __restrict__ out, int lda,
                                                            int ldc, int M, int N, int K, int epi, unsigned inv_full, Extra extra) {
     constexpr bool NEXT = std::is_same<Extra, FewNext>::value, QKV = std::is_same<Extra, FewQkv>::value;
@@ -78,12 +79,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     constexpr int PER = 16 / (int)sizeof(T), KB = 8 * PER;         // numbers in a lane's piece, in a k-block
     constexpr int TILES = (NG + 1) / 2;                            // tiles of 16 features (the last one half, where NG is odd)
     constexpr int TOK = FOLD ? 8 : 16;
-    constexpr int WL = FOLD ? NG : TILES * 2, XL = FOLD ? 1 : 2;   // a lane's pieces of a k-block: weight, tokens
+    constexpr int WL = FOLD ? NG : TILES * 2, XL = FOLD ? 1 : 2 * TT;   // a lane's pieces of a k-block: weight, tokens (TT tiles of them)
+    static_assert(TT == 1 || !FOLD, "folded operands are of eight tokens");
     constexpr int LOADS = NG + XL, BLOCK = LOADS * 1024;           // a k-block in LDS: eight rows of 128 bytes to a load
     static_assert((R - 2) * LOADS < 64 && R >= 2, "vmcnt counts to 63");
     extern __shared__ __attribute__((aligned(1024))) unsigned char few_smem[];
-    f32x4* red = (f32x4*)(few_smem + NW * R * BLOCK);              // [NW][NG][2: four features each][TOK]
-    float* scale_red = (float*)(red + NW * NG * 2 * TOK);          // [NW][16]
+    f32x4* red = (f32x4*)(few_smem + NW * R * BLOCK);              // [NW][TT][NG][2: four features each][TOK]
+    float* scale_red = (float*)(red + NW * TT * NG * 2 * TOK);     // [NW][16]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * NG * 8;
@@ -96,15 +98,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
 #pragma unroll
         for (int i = 0; i < XL; ++i) src[NG + i] = A + (size_t)min(i * 8 + lrow, M - 1) * lda + chunk;
     }
-    FewSums<T, SUMS> acc[WL];
+    FewSums<T, SUMS> acc[TT][WL];
 #pragma unroll
-    for (int i = 0; i < WL; ++i) acc[i].clear();
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int i = 0; i < WL; ++i) acc[tt][i].clear();
 
     // A norm left to this product (RowScale): its partial sums of squares are shared out over the waves and asked for before
     // the weights, so that their trip to memory (they were written on other XCDs) costs nothing beside the weights'.
     // (Asked for after the walk along k it was a trip in front of every result: 0.9 us of the product.)
     constexpr int AHEAD = 4;
-    const bool scaled = !std::is_same<Extra, FewPlain>::value && rs.sumsq != nullptr, by_four = rs.nparts % 16 == 0 && ((uintptr_t)rs.sumsq & 15) == 0;
+    const bool scaled = TT == 1 && !std::is_same<Extra, FewPlain>::value && rs.sumsq != nullptr, by_four = rs.nparts % 16 == 0 && ((uintptr_t)rs.sumsq & 15) == 0;
     const float* sp = rs.sumsq + (size_t)min(row, M - 1) * rs.nparts;
     f32x4 part[AHEAD];
     if (scaled && by_four) {
@@ -116,13 +120,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     }
     // out += sum: the old values of the tile this wave will finish, and the next norm's weight for them, likewise
     float old[4] = {0.0f, 0.0f, 0.0f, 0.0f}, next_w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const bool old_ahead = !QKV && epi == LLMRS_EPI_ACCUM_F32 && wave < TILES;
-    if (old_ahead && row < M) {
-        int n = n0 + wave * 16 + 4 * g;
+    const bool old_ahead = !QKV && epi == LLMRS_EPI_ACCUM_F32 && wave < TILES * TT;
+    const int own = wave % TILES, own_m = wave / TILES * 16 + row;          // that tile, and this lane's token of it
+    if (old_ahead && own_m < M) {
+        int n = n0 + own * 16 + 4 * g;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (n + r < N && 4 * g < 8 * NG - 16 * wave) {
-                old[r] = ((const float*)out)[(size_t)row * ldc + n + r];
+            if (n + r < N && 4 * g < 8 * NG - 16 * own) {
+                old[r] = ((const float*)out)[(size_t)own_m * ldc + n + r];
                 if (NEXT) next_w[r] = nn.weight[n + r];
             }
     }
@@ -155,7 +160,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     };
     auto products = [&](const Piece (&w)[WL], const Piece (&x)[XL]) {
 #pragma unroll
-        for (int i = 0; i < WL; ++i) acc[i].add(w[i], x[FOLD ? 0 : i & 1]);
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int i = 0; i < WL; ++i) acc[tt][i].add(w[i], x[FOLD ? 0 : 2 * tt + (i & 1)]);
     };
 #pragma unroll
     for (int i = 0; i < R - 1; ++i)
@@ -174,8 +181,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
             for (int t = 0; t < NG; ++t) w[t] = *(const Piece*)(b + t * 1024 + off0);
         } else {
             const int half = (row >> 3) * 1024;
-            x[0] = *(const Piece*)(b + NG * 1024 + half + off0);
-            x[1] = *(const Piece*)(b + NG * 1024 + half + off1);
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                x[2 * tt] = *(const Piece*)(b + (NG + 2 * tt) * 1024 + half + off0);
+                x[2 * tt + 1] = *(const Piece*)(b + (NG + 2 * tt) * 1024 + half + off1);
+            }
             // (with an odd number of groups the last tile's other half reads the tokens' rows: its sums are not used)
 #pragma unroll
             for (int t = 0; t < TILES; ++t) {
@@ -195,8 +205,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
         }
 #pragma unroll
         for (int i = 0; i < XL; ++i) {
-            const int from = k + first + i * (KB / 2);
-            x[i] = from < K ? *(const Piece*)(A + (size_t)min(FOLD ? f : row, M - 1) * lda + from) : Piece{};
+            const int from = k + first + (i & 1) * (KB / 2);
+            x[i] = from < K ? *(const Piece*)(A + (size_t)min(FOLD ? f : i / 2 * 16 + row, M - 1) * lda + from) : Piece{};
         }
         products(w, x);
     }
@@ -219,32 +229,34 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     if constexpr (FOLD) {
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
-            f32x4 s = acc[i].total();
+            f32x4 s = acc[0][i].total();
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[r] = with_other_half(s[r]);
             if (row < 8 && g < 2) red[((wave * NG + i) * 2 + g) * TOK + row] = s;
         }
     } else {
 #pragma unroll
-        for (int t = 0; t < TILES; ++t)
-            if (2 * t + (g >> 1) < NG) red[((wave * NG + 2 * t) * 2 + g) * TOK + row] = acc[2 * t].total() + acc[2 * t + 1].total();
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+                if (2 * t + (g >> 1) < NG) red[(((wave * TT + tt) * NG + 2 * t) * 2 + g) * TOK + row] = acc[tt][2 * t].total() + acc[tt][2 * t + 1].total();
     }
     __syncthreads();
     // the tiles are shared out over the waves: lane l finishes token l % 16 and features 4 (l / 16) + r
-    const int m = row;
-    if (wave >= TILES || m >= M) return;
+    if (wave >= TILES * TT || (TT == 1 && row >= M)) return;
     float inv = 1.0f;
     if (scaled) {
         float total = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) total += scale_red[w * 16 + m];
+        for (int w = 0; w < NW; ++w) total += scale_red[w * 16 + row];
         inv = 1.0f / sqrtf(total / (float)K + rs.eps);
     }
-    for (int tile = wave; tile < TILES; tile += NW) {
-        if (2 * tile + (g >> 1) >= NG) continue;                   // the half of the last tile that is the next block's
+    for (int which = wave; which < TILES * TT; which += NW) {
+        const int tile = which % TILES, tt = which / TILES, m = tt * 16 + row;
+        if (m >= M || 2 * tile + (g >> 1) >= NG) continue;         // (the half of the last tile is the next block's)
         f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < NW; ++w) s += red[((w * NG + 2 * tile) * 2 + g) * TOK + m];
+        for (int w = 0; w < NW; ++w) s += red[(((w * TT + tt) * NG + 2 * tile) * 2 + g) * TOK + row];
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = s[r] * inv;
@@ -255,7 +267,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
                 if (n + r + 1 < N) ((T*)out)[(size_t)m * ldc + (n + r) / 2] = from_f32<T>(gated_act(epi, v[r], v[r + 1]));
         } else if (QKV) {
             if (n < N) store_qkv4<T>(qe, out, ldc, m, n, v);
-        } else if (old_ahead && tile == wave) {
+        } else if (old_ahead && which == wave) {
             float ss = 0.0f;
             Four y4;
 #pragma unroll
@@ -304,22 +316,23 @@ struct FewCall {
     RowScale scale;
     NextNorm next;
 };
-template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS = 1>
+template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS = 1, int TT = 1>
 static void launch_few(const FewCall& c) {
     static_assert(ROT % (NG * 8) == 0, "a block's features lie in one group");
     const unsigned full = c.K * sizeof(T) / 128, inv_full = full > 1 ? (unsigned)(((1ull << 32) + full - 1) / full) : 0;
-    constexpr size_t bytes = (size_t)NW * R * (NG + (FOLD ? 1 : 2)) * 1024 + (size_t)NW * NG * 2 * (FOLD ? 8 : 16) * 16 + NW * 16 * sizeof(float);
+    constexpr size_t bytes = (size_t)NW * R * (NG + (FOLD ? 1 : 2 * TT)) * 1024 + (size_t)NW * TT * NG * 2 * (FOLD ? 8 : 16) * 16 + NW * 16 * sizeof(float);
     static_assert(bytes <= 160 * 1024, "the rings and the waves' sums must fit in a unit's LDS");
     auto launch = [&](auto extra) {
         static bool configured = false;
         if (!configured) {
-            (void)hipFuncSetAttribute((const void*)gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS, decltype(extra)>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+            (void)hipFuncSetAttribute((const void*)gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS, TT, decltype(extra)>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
             configured = true;
         }
-        gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
+        gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS, TT><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
             (const T*)c.A, (const T*)c.W, c.out, c.lda, c.ldc, c.M, c.N, c.K, c.epi, inv_full, extra);
     };
     if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
+    else if constexpr (TT > 1) launch(FewPlain{});        // (no norm is left to a product of more than 16 rows)
     else if (c.next.y != nullptr) launch(FewNext{c.scale, c.next});
     else if (c.scale.sumsq != nullptr) launch(FewScaled{c.scale});
     else launch(FewPlain{});
@@ -357,9 +370,23 @@ static void launch_few_by_rows(const FewCall& c) {
 // Waves per block and the walk's start come from the weight's shape alone (see above).  With fewer features a block, more blocks
 // ask at once but each reads the tokens' rows again.  Rings of three k-blocks do nearly as well as any: what is on its way
 // is then some 32 KB of the weight a unit.
+// 17 to 32 rows in 32-bit: two tiles of tokens for every piece of the weight, which is read once.  (us at 32 rows against
+// gemm_f32_skinny_kernel, whose operands come straight from memory and touch eight times the cache lines: 2048 x 2048 15.1 -> 9.4,
+// 2048 x 8192 46.2 -> 27.7, 3072 x 2048 14.4 -> 10.7, 16384 x 2048 33.4 -> 29.9, 28672 x 4096 148 -> 90, 128256 x 2048 312 -> 206;
+// 8192 x 28672 239 -> 191.)  The shares of k are half as long and two sums run beside each other: the error against 64 bits is smaller.
+// The widest weights want many features a block, as each block reads the tokens' rows again (128256 x 2048: 64 features 206, 32
+// 230-245, 16 285); the narrow ones enough blocks (3072 x 2048: 16 features 10.7, 8 16.9).
+static void few_rows_two_tiles(const FewCall& c) {
+    if (c.N >= 16384) launch_few<float, false, 8, 4, 2, 64, 1, 2>(c);
+    else if (c.K < 2048) launch_few<float, false, 2, 4, 2, 0, 1, 2>(c);
+    else if (c.N >= 8192) launch_few<float, false, 4, 4, 3, 64, 1, 2>(c);
+    else if (half_blocks_for_narrow(c.N, c.K)) launch_few<float, false, 1, 8, 2, 64, 1, 2>(c);
+    else launch_few<float, false, 2, 8, 2, 0, 1, 2>(c);
+}
 template <class T>
 static void few_rows(const FewCall& c) {
     const int N = c.N, K = c.K, cus = llmrs_compute_units();
+    if (sizeof(T) == 4 && c.M > 16) { few_rows_two_tiles(c); return; }
     if (N >= 16384) {
         // (28672 x 4096 bfloat16 at 8 rows: blocks of 16 features 42.0 us, of 56 43.7, of 112 47; at 16 rows of 56 41.8, of 112 42.4)
         if (wide_tiles(N, cus) == 7) launch_few_by_rows<T, 4, 112, 2, 4, 7, 3>(c);

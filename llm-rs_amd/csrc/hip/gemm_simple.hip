@@ -1,6 +1,6 @@
 // The plain product: 64x64 tiles through LDS, 32-bit FMA, k in ascending order.
-// With the 32-bit matrix-core tiles (here and in gemm_f32_tiles.hip) and the few-row kernels below it is the whole
-// 32-bit path (nothing here rounds its inputs) and the bfloat16 fallback for shapes
+// With the 32-bit matrix-core tiles (here and in gemm_f32_tiles.hip), the products of few rows (gemm_few.hip) and the kernels
+// of some more below it is the whole 32-bit path (nothing here rounds its inputs) and the bfloat16 fallback for shapes
 // the bfloat16 MFMA kernels refuse.  Within each kernel the order of
 // the sum for an output depends on K only (and on the weight's shape), so a row's result does not depend on the
 // row's place in the batch or on its tile; which kernel runs depends on M and the shape, so across those
@@ -350,7 +350,7 @@ static bool launch_f32_few_rows(hipStream_t stream, const float* a, int lda, con
     const int cus = llmrs_compute_units();
     // Blocks of 32 tokens with the fewest features that still make one round of the compute units.  Where even
     // 64 features to a block make more, the tiles take over, but for up to 32 tokens, whose weights are read once here.
-    // (us, 32-feature-tile form / tiles: 32 rows 2048 x 8192 45 / 168, 128256 x 2048 295 / 350; 64 rows 3072 x 2048 19 / 45,
+    // (us, this kernel / tiles: 64 rows 3072 x 2048 19 / 45,
     // 16384 x 2048 66 / 48; 100 rows 2048 x 2048 19 / 45; 200 rows 2048 x 2048 29 / 45, 3072 x 2048 58 / 46)
     const long rows = ceil_div(M, 32);
     if (rows * ceil_div(N, 16) <= cus) launch_f32_skinny<2, 1, 4, 4>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
@@ -429,7 +429,11 @@ extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda,
     }
     const bool f32_cores = dtype == LLMRS_F32 && allow_mfma && K % 32 == 0 && lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
     // (one or two tokens on the widest weights are better off with the walk below: 128256 x 2048 173 against 177 us)
-    if (f32_cores && M <= 16 && !(M <= 2 && N >= 65536 && scale_sumsq == nullptr && next_y == nullptr)) {
+    // (17 to 32 on wide weights with the shortest rows with gemm_f32_skinny_kernel: 65536 x 128 16.1 against 19.8 us; from rows of 256 on there is
+    // no difference, and the longer ones gain)
+    const bool plain = scale_sumsq == nullptr && next_y == nullptr;
+    if (f32_cores && M <= 32 && !(plain && M <= 2 && N >= 65536) && !(plain && M > 16 && N >= 16384 && K < 256)) {
+        LLMRS_REQUIRE(plain || M <= 16, "gemm: a deferred norm needs the matrix-core kernels for few rows (M=%d N=%d K=%d)", M, N, K);
         RowScale rs{scale_sumsq, scale_parts, scale_eps};
         NextNorm nn{next_sumsq, next_y, next_ldy, next_weight, 0.0f};
         if (llmrs_gemm_few_f32(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi, nullptr, scale_sumsq ? &rs : nullptr,
@@ -437,7 +441,7 @@ extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda,
         LLMRS_LAUNCH_CHECK("gemm");
         return 0;
     }
-    LLMRS_REQUIRE(scale_sumsq == nullptr && next_y == nullptr, "gemm: a deferred norm needs the matrix-core kernels for few rows (M=%d N=%d K=%d)", M, N, K);
+    LLMRS_REQUIRE(plain, "gemm: a deferred norm needs the matrix-core kernels for few rows (M=%d N=%d K=%d)", M, N, K);
     if (f32_cores && M > 2) {
         if (!launch_f32_few_rows(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi) &&
             llmrs_gemm_f32_tiles(stream, (const float*)A, lda, (const float*)W, out, ldc, M, N, K, epi) != 0) return -1;

@@ -589,6 +589,14 @@ def test_gemm_few_rows_and_their_rings(dtype, M, N, K):
         assert (err <= out_tol(ref, out.dtype, floor)).all(), (epi, float(err.max()))
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 8, 32), (32, 250, 544), (20, 1990, 2048), (31, 2040, 2080), (32, 3080, 2592), (18, 9000, 96), (29, 8200, 2080),
+                                   (32, 16390, 288), (17, 20000, 128), (24, 16400, 2048)])
+def test_gemm_float32_two_tiles_of_tokens(M, N, K):
+    """17 to 32 rows in 32-bit: the second tile of tokens nearly empty and full, waves with no k-block, fewer than their ring has
+    places and more; blocks of 8, 16, 32 and 64 features cut by N; every epilogue, rows with a stride; the bound is that of up to 16 rows."""
+    test_gemm_few_rows_and_their_rings(torch.float32, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 40, 64), (33, 250, 128), (48, 4090, 192), (49, 3000, 704), (64, 16, 1344), (20, 6140, 64), (64, 8200, 320),
                                    (40, 16400, 64), (64, 28672, 192), (31, 16500, 576), (64, 4000, 1088), (18, 2040, 2112), (48, 1000, 8256), (64, 2048, 1984)])
 def test_gemm_ring_of_k_blocks(M, N, K):
