@@ -1245,13 +1245,17 @@ static MidTiles mid_tiles(int M, int N, int K, int epi, bool may_split = true) {
     return MidTiles{false, s, small_time};
 }
 // 17..64 rows on a weight of middling width (more than 4096 features, fewer than the wide ones that
-// get blocks of many feature tiles): the 128 x 128 tiles with k split over blocks read the tokens'
-// rows less often than the few-row kernel's blocks of 32 features (measured at 64 rows:
-// 10240 x 8192 90 -> 51 us, 8192 x 8192 49 -> 38, 8192 x 28672 160 -> 99, 6144 x 4096 31 -> 21;
-// at 32 rows: 10240 x 8192 63 -> 48, 8192 x 28672 110 -> 90).
+// get blocks of many feature tiles): the 128 x 128 tiles with k split over blocks.  Where they add to the stream their finish also
+// does the norm that follows; their tokens' rows are read less often than the ring's blocks of 32 features read them, which pays at
+// long rows and many tokens (ring against tiles, us: 8192 x 28672 111 / 90 at 20 rows, 133 / 99 at 64; 10240 x 8192 60 / 52 at 64,
+// 12288 x 4096 35.6 / 34.3 at 64).
 static bool few_rows_take_tiles(int M, int N, int K) {
     return M > 16 && M <= 64 && N > 4096 && N < 16384 && K % 64 == 0 && tiled_splits(M, N, K) > 1;
 }
+// Of those the products with short rows that store their results or gate them are better off with the ring (tiles with their finish -> ring, us:
+// 17 rows 8192 x 2048 15.3 -> 11.3, 10240 x 4096 27.8 -> 22.0; over 4608 to 16000 features a ratio of 0.67 at K = 1024 whatever
+// the rows, 0.81-0.96 at 2048 to 4096 and up to 48 rows; with more rows or longer ones some gain and some lose up to 22 %).
+static bool ring_stores_faster(int M, int K) { return K <= (M <= 48 ? 4096 : 1024); }
 // Room (in floats) for the partial sums of a product that would be split: what the caller should bring.
 extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
     if (M > 16 && M <= 64) {
@@ -1322,7 +1326,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             ((uintptr_t)qkv->k_cache & 7) || qkv->rotary_dim % 4)
             return 0;
         // long rows and many tokens: the tiles with k split over blocks are so much faster that
-        // the separate rotation kernel is paid for (10240 x 8192 at 64 rows: 90 us fused, 51 + 6)
+        // the separate rotation kernel is paid for (10240 x 8192 at 64 rows: 60 us in the ring, 52 + 6; the tiles' parts are added by the rotation)
         // (with rows of 4096 the same route gains nothing: a decode step of the 8B shape at 64 requests 7.60 -> 7.55 ms,
         // at 40 and 48 requests none or a loss)
         if (M > 32 && K >= 8192 && few_rows_take_tiles(M, N, K)) return 0;
@@ -1336,7 +1340,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         return 1;
     }
     bool tiles_for_few = false;
-    if (epi != LLMRS_EPI_QKV && few_rows_take_tiles(M, N, K)) {
+    if (epi != LLMRS_EPI_QKV && few_rows_take_tiles(M, N, K) && (epi == LLMRS_EPI_ACCUM_F32 || !ring_stores_faster(M, K))) {
         int splits = tiled_splits(M, N, K);
         tiles_for_few = workspace != nullptr && workspace_bytes >= (size_t)splits * M * N * sizeof(float);
     }

@@ -598,7 +598,8 @@ def test_gemm_float32_two_tiles_of_tokens(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 40, 64), (33, 250, 128), (48, 4090, 192), (49, 3000, 704), (64, 16, 1344), (20, 6140, 64), (64, 8200, 320),
-                                   (40, 16400, 64), (64, 28672, 192), (31, 16500, 576), (64, 4000, 1088), (18, 2040, 2112), (48, 1000, 8256), (64, 2048, 1984)])
+                                   (40, 16400, 64), (64, 28672, 192), (31, 16500, 576), (64, 4000, 1088), (18, 2040, 2112), (48, 1000, 8256), (64, 2048, 1984),
+                                   (40, 6140, 1088), (64, 8200, 1024), (17, 4600, 4096)])
 def test_gemm_ring_of_k_blocks(M, N, K):
     """17 to 64 rows, k-blocks through a ring in LDS: fewer and more k-blocks than the ring has stages, odd numbers of them where a
     stage holds two, unequal shares of a split k, blocks of 16, 24, 32, 64 and 112 features cut by N; every epilogue, rows with a stride."""
