@@ -342,7 +342,9 @@ __global__ __launch_bounds__(64) void attention_generic_group_kernel(
 // the maxima and sums of up to 64 chunks, a lane each, and the rows of the first chunks, of both maps, asked for before
 // the length is known (they lie within the scratch; what is beyond the entry's chunks is not used).  Further rows come as many at a time.
 // (32-bit, 8 requests of 200 to 1800 keys, heads of 64: 6.6 us with lengths, maxima and rows one after the other, rows four at
-// a time; now 4.9.  Of up to 1000 keys, two maps and values of 128: 11.3, now 6.0.)
+// a time; now 4.9.  Of up to 1000 keys, two maps and values of 128: 11.3, now 6.0.)  With more than 1024 waves (four to a compute unit)
+// it is bound by what it reads and no longer by the trips, and a recorded step's table may be far wider than its keys: then
+// the length comes first (64 requests of 200 keys, 32 heads of 128, a table for 8192: the call 1.14 times that of a table for 256 otherwise).
 template <class T, int MAPS, int VALS>
 __global__ __launch_bounds__(64) void attention_generic_merge_kernel(
     const float* __restrict__ partial, T* __restrict__ out, const int* __restrict__ q_starts,
@@ -352,6 +354,7 @@ __global__ __launch_bounds__(64) void attention_generic_merge_kernel(
     const size_t stride = hd + 2;
     int t = q_starts[e], next = q_starts[e + 1], pos = seq_lens[e] - 1;
     float m_first[MAPS], l_first[MAPS], rows[MAPS][AHEAD][VALS];
+    const bool length_first = gridDim.x * gridDim.y > 1024;
     auto ask = [&](float (&v)[AHEAD][VALS], const float* pp, int first, int n) {       // rows first .. of n
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u)
@@ -361,16 +364,20 @@ __global__ __launch_bounds__(64) void attention_generic_merge_kernel(
                 v[u][i] = first + u < n && d < hd ? pp[(size_t)(first + u) * stride + 2 + d] : 0.0f;
             }
     };
+    auto first_trip = [&](int n) {
 #pragma unroll
-    for (int map = 0; map < MAPS; ++map) {
-        const float* pp = partial + (size_t)((e * a.n_heads + h) * MAPS + map) * max_chunks * stride;
-        m_first[map] = lane < max_chunks ? pp[(size_t)lane * stride] : -INFINITY;
-        l_first[map] = lane < max_chunks ? pp[(size_t)lane * stride + 1] : 0.0f;
-        ask(rows[map], pp, 0, max_chunks);
-    }
+        for (int map = 0; map < MAPS; ++map) {
+            const float* pp = partial + (size_t)((e * a.n_heads + h) * MAPS + map) * max_chunks * stride;
+            m_first[map] = lane < n ? pp[(size_t)lane * stride] : -INFINITY;
+            l_first[map] = lane < n ? pp[(size_t)lane * stride + 1] : 0.0f;
+            ask(rows[map], pp, 0, n);
+        }
+    };
+    if (!length_first) first_trip(max_chunks);
     if (next - t != 1) return;
     int lo = attn_window_lo(a, pos);
     int n_chunks = pos / GENERIC_CHUNK - lo / GENERIC_CHUNK + 1;
+    if (length_first) first_trip(n_chunks);
     float o[MAPS][MAX_HEAD_DIM / 64] = {};
 #pragma unroll
     for (int map = 0; map < MAPS; ++map) {

@@ -475,10 +475,10 @@ def test_attention_single_tokens_of_heads_of_64(n_heads, n_kv, window):
         assert ((got[r].double() - ref).abs() <= out_tol(ref, torch.bfloat16, 8e-3)).all(), lens[r]
 
 
-@pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (2, 1, 128), (1, 1, 160)])
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (2, 1, 128), (1, 1, 160), (160, 5, 64)])
 def test_attention_float32_merges_many_chunks(n_heads, n_kv, hd):
-    """Requests of as many chunks as the merge asks for at once (16, 8 and 4 rows), one more, and more than a lane has chunks (64):
-    the largest weight lies in the first, the last and a middle chunk in turn, beside an entry of several tokens."""
+    """Requests of as many chunks as the merge asks for at once (16, 8 and 4 rows), one more, and more than a lane has chunks (64),
+    in a merge of few waves and of many (which reads the lengths first): the largest weight lies in the first, the last and a middle chunk in turn, beside an entry of several tokens."""
     lens = [512, 513, 1024, 1025, 2048, 2049, 8300, 40]
     case = PagedCase(torch.float32, lens, n_heads, n_kv, hd, 16, seed=37)
     g = torch.Generator().manual_seed(5)
