@@ -119,6 +119,12 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
 // Whether the product of this shape, in bfloat16 or in 32-bit, goes to the kernel that can scale its rows' sums and leave a NextNorm.
 extern "C" int llmrs_gemm_defers_norm(int M, int N, int K);
 extern "C" int llmrs_gemm_f32_defers_norm(int M, int N, int K);
+// Whether a product of that kind with N features can leave a NextNorm (the rows left are stored four features at once, and the widest
+// weights' blocks take more tiles than they have waves).
+extern "C" int llmrs_gemm_leaves_norm(int N);
+// Whether the q/k/v epilogue, which stores four consecutive features of a head at once, takes heads of this geometry.  A product
+// whose norm was left to it has no other way to its caches: who leaves the norm to it asks first.
+extern "C" int llmrs_qkv_by_fours(int head_dim, int rotary_dim);
 // The parts per row of the sums of squares that such a product leaves (NextNorm): what the caller sizes sumsq by.
 extern "C" int llmrs_gemm_next_parts(int M, int N, int K);
 // Whether the bfloat16 product of this shape, adding into the stream and given the workspace that

@@ -355,6 +355,8 @@ static int wide_tiles(int N, int cus) {
 }
 extern "C" int llmrs_gemm_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 8 == 0; }
 extern "C" int llmrs_gemm_f32_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 32 == 0; }
+extern "C" int llmrs_gemm_leaves_norm(int N) { return N < 16384 && N % 4 == 0; }
+extern "C" int llmrs_qkv_by_fours(int head_dim, int rotary_dim) { return head_dim % 4 == 0 && rotary_dim % 4 == 0; }
 extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
     return M <= 16 && half_blocks_for_narrow(N, K) ? ceil_div(N, 8) : ceil_div(N, 16);
 }
@@ -412,12 +414,12 @@ static int gemm_few(hipStream_t stream, const T* A, int lda, const T* W, void* o
     constexpr int FOUR = 4 * (int)sizeof(T);
     if (scale != nullptr || next != nullptr) {
         bool ok = (scale == nullptr || (scale->sumsq != nullptr && scale->nparts >= 1 && scale->eps > 0.0f)) &&
-                  (next == nullptr || (epi == LLMRS_EPI_ACCUM_F32 && N < 16384 && next->sumsq != nullptr && next->y != nullptr &&
+                  (next == nullptr || (epi == LLMRS_EPI_ACCUM_F32 && llmrs_gemm_leaves_norm(N) && next->sumsq != nullptr && next->y != nullptr &&
                                        next->weight != nullptr && next->ldy >= N && next->ldy % 4 == 0 && (uintptr_t)next->y % FOUR == 0));
-        if (!ok) { llmrs_fail("gemm: a deferred norm is taken for up to 16 rows (what is left for the next one: with the += epilogue, under 16384 features), got M=%d N=%d K=%d epilogue %d", M, N, K, epi); return -1; }
+        if (!ok) { llmrs_fail("gemm: a deferred norm is taken for up to 16 rows (what is left for the next one: with the += epilogue, a multiple of 4 and under 16384 features), got M=%d N=%d K=%d epilogue %d", M, N, K, epi); return -1; }
     }
-    if (epi == LLMRS_EPI_QKV && (qkv == nullptr || qkv->head_dim % 4 || ldc % 4 || (uintptr_t)out % FOUR || (uintptr_t)qkv->k_cache % FOUR || qkv->rotary_dim % 4))
-        return 0;           // (four features of a head are stored at once)
+    if (epi == LLMRS_EPI_QKV && (qkv == nullptr || !llmrs_qkv_by_fours(qkv->head_dim, qkv->rotary_dim) || ldc % 4 || (uintptr_t)out % FOUR || (uintptr_t)qkv->k_cache % FOUR))
+        return 0;
     few_rows<T>(FewCall{stream, A, lda, W, out, ldc, M, N, K, epi, qkv ? *qkv : QkvEpilogue{}, scale ? *scale : RowScale{}, next ? *next : NextNorm{}});
     return 1;
 }

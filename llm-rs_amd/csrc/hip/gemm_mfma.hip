@@ -1322,8 +1322,8 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         return -1;
     }
     if (epi == LLMRS_EPI_QKV) {   // only the skinny kernel fuses it; its 8-byte stores need aligned rows
-        if (M > 64 || qkv == nullptr || qkv->head_dim % 4 || ldc % 4 || ((uintptr_t)out & 7) ||
-            ((uintptr_t)qkv->k_cache & 7) || qkv->rotary_dim % 4)
+        if (M > 64 || qkv == nullptr || !llmrs_qkv_by_fours(qkv->head_dim, qkv->rotary_dim) || ldc % 4 || ((uintptr_t)out & 7) ||
+            ((uintptr_t)qkv->k_cache & 7))
             return 0;
         // long rows and many tokens: the tiles with k split over blocks are so much faster that
         // the separate rotation kernel is paid for (10240 x 8192 at 64 rows: 60 us in the ring, 52 + 6; the tiles' parts are added by the rotation)

@@ -169,6 +169,10 @@ class Kernels:
         their norm) in place of normed rows."""
         return False
 
+    def qkv_product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype, head_dim: int, rotary_dim: int) -> bool:
+        """The same of the q/k/v product, which rotates `rotary_dim` features of every head and writes the cache."""
+        return self.product_norms_its_rows(M, N, K, dtype)
+
     def norm_left_by_product(self, M: int, N: int, K: int, dtype: torch.dtype) -> Optional[NormPlan]:
         """What the product of M rows with an [N, K] weight, adding into the stream, can leave for the norm that
         reads the stream next (`NextNorm`), or None: then a norm kernel runs."""
@@ -231,6 +235,8 @@ class HipKernels(Kernels):
             "llmrs_glu_clamp_slot": [V, F, F, F, F],
             "llmrs_gemm_defers_norm": [I, I, I],
             "llmrs_gemm_f32_defers_norm": [I, I, I],
+            "llmrs_gemm_leaves_norm": [I],
+            "llmrs_qkv_by_fours": [I, I],
             "llmrs_gemm_norms_whole": [I, I, I],
             "llmrs_gemm_next_parts": [I, I, I],
             "llmrs_rope_kv_write": [V, I, V, I, V, V, V, I, I, V, V, I, I, I, I, I, I, I],
@@ -303,10 +309,13 @@ class HipKernels(Kernels):
     def product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype) -> bool:
         return self.gemm_defers_norm(M, N, K, dtype)
 
+    def qkv_product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype, head_dim: int, rotary_dim: int) -> bool:
+        return bool(self.lib.llmrs_qkv_by_fours(int(head_dim), int(rotary_dim))) and self.gemm_defers_norm(M, N, K, dtype)
+
     def norm_left_by_product(self, M: int, N: int, K: int, dtype: torch.dtype) -> Optional[NormPlan]:
         # up to a few rows: partial sums of squares, for the next product to finish (the kernels keep at most 1024
         # of them a row); more rows: a product that is split over blocks finishes the norm where its parts are added up
-        if N < 16384 and self.gemm_defers_norm(M, N, K, dtype):
+        if self.lib.llmrs_gemm_leaves_norm(int(N)) and self.gemm_defers_norm(M, N, K, dtype):
             return NormPlan(False, self.gemm_next_parts(M, N, K))
         if dtype == torch.bfloat16 and self.gemm_norms_whole(M, N, K):
             return NormPlan(True, 0)
@@ -317,7 +326,7 @@ class HipKernels(Kernels):
 
     def gemm_defers_norm(self, M: int, N: int, K: int, dtype: torch.dtype = torch.bfloat16) -> bool:
         """Whether the product of M rows with an [N, K] weight takes `NormedRows` as its rows and, adding
-        into the stream, leaves a `NextNorm` (that: for fewer than 16384 features)."""
+        into the stream, leaves a `NextNorm` (that: for a multiple of 4 and fewer than 16384 features)."""
         asked = self.lib.llmrs_gemm_defers_norm if dtype == torch.bfloat16 else self.lib.llmrs_gemm_f32_defers_norm
         return self.allow_mfma and bool(asked(int(M), int(N), int(K)))
 
@@ -576,7 +585,7 @@ class HipKernels(Kernels):
             assert epilogue == EPI_ACCUM_F32 and tuple(leave.y.shape) == (M, N) and leave.y.stride(1) == 1
             assert leave.y.dtype == a.dtype and leave.weight.dtype == torch.float32 and leave.weight.shape[0] == N
             if not whole:
-                assert N < 16384 and leave.sumsq.dtype == torch.float32 and leave.sumsq.is_contiguous()
+                assert self.lib.llmrs_gemm_leaves_norm(N) and leave.sumsq.dtype == torch.float32 and leave.sumsq.is_contiguous()
                 assert tuple(leave.sumsq.shape) == (M, self.gemm_next_parts(M, N, K))
         if whole:
             assert a.dtype == torch.bfloat16 and scale is None and self.gemm_norms_whole(M, N, K) and workspace is not None
@@ -628,7 +637,7 @@ class HipKernels(Kernels):
         if isinstance(x, NormedRows):
             scale, x = x, x.y
             assert scale.sumsq.dtype == torch.float32 and scale.sumsq.is_contiguous() and scale.sumsq.shape[0] == x.shape[0]
-            assert self.gemm_defers_norm(x.shape[0], w.shape[0], x.shape[1], x.dtype)
+            assert self.qkv_product_norms_its_rows(x.shape[0], w.shape[0], x.shape[1], x.dtype, head_dim, rotary_dim)
         assert x.stride(1) == 1 and qkv.stride(1) == 1 and w.is_contiguous() and x.dtype == w.dtype == qkv.dtype
         assert rotary_dim == 0 or (inv_freq.dtype == torch.float32 and inv_freq.shape[0] == rotary_dim // 2)
         if write_kv:

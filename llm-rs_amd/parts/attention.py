@@ -420,8 +420,8 @@ class Attention(KeyedBySplitChunk, Mixer):
         if self.prepared:
             return False
         # the q/k/v product norms its rows itself where it is the fused kernel: a rotation it applies (or none)
-        fused = self.position is None or self.position.rotary() is not None
-        return fused and kernels().product_norms_its_rows(rows, self.w_qkv.shape[0], self.hidden, self.dtype)
+        rotary = (None, 0) if self.position is None else self.position.rotary()
+        return rotary is not None and kernels().qkv_product_norms_its_rows(rows, self.w_qkv.shape[0], self.hidden, self.dtype, self.head_dim, rotary[1])
 
     def forward(self, ctx, x, h, cache, sums=None):
         if self.prepared:

@@ -34,7 +34,19 @@ def random_config(seed: int) -> dict:
 
 @pytest.mark.parametrize("seed", [1, 2, 3, 5, 8, 13, 21, 34, 55, 89, 144, 233, 377, 610, 987, 4, 6, 7, 9, 10, 11, 12, 14, 15])
 def test_a_random_configuration(seed):
-    d = random_config(seed)
+    compare(random_config(seed), seed)
+
+
+# Sizes that four features at a time do not divide: heads of 10 (the q/k/v product cannot store them by fours) and a width of 98
+# (nor a product the rows that the next norm reads), between products whose rows are whole 32-bit k-blocks.
+@pytest.mark.parametrize("hidden,heads,kv,head_dim,inter", [(160, 16, 4, 10, 320), (98, 4, 2, 16, 96), (102, 8, 1, 20, 128)])
+def test_sizes_that_are_no_multiple_of_four(hidden, heads, kv, head_dim, inter):
+    compare(dict(architectures=["LlamaForCausalLM"], num_hidden_layers=3, hidden_size=hidden, num_attention_heads=heads, num_key_value_heads=kv,
+                 head_dim=head_dim, intermediate_size=inter, vocab_size=390, rope_theta=10000.0, max_position_embeddings=2048, rms_norm_eps=1e-5,
+                 tie_word_embeddings=False), 17)
+
+
+def compare(d, seed):
     cfg = LlamaConfig.from_dict(d)
     rnd = random.Random(seed + 1000)
     lens = [rnd.choice([1, 2, 16, 17, 64, 65, 129, 300])] + [rnd.randint(3, 260) for _ in range(5)]
