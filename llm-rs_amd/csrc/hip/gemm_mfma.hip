@@ -2,8 +2,8 @@
 //
 // Two kernels, chosen by M (the number of tokens in the step); up to 16 rows go to gemm_few.hip:
 //   M <= 64  many requests decoding.  K % 64 == 0: gemm_ring.h.  Other K "skinny": every
-//            weight is read once, straight from memory into MFMA operands; a block owns 32 or
-//            64 output features and its waves split K.
+//            weight is read once, straight from memory into MFMA operands; a block owns 16 to
+//            112 output features and its waves split K.
 //   M  > 64  "tiled": prompts.  Tiles of 128x128, 256x128, 256x192 or 256x256 outputs, K
 //            in steps of 64 through double-buffered LDS, v_mfma_f32_32x32x16_bf16; when
 //            K % 64 == 0 the tiles are loaded straight into LDS (global_load_lds), or, by
@@ -69,17 +69,23 @@ __device__ __forceinline__ float gated_act_fast(const GatedAct& a, float g, floa
 // where blocks of 64 features are needed to keep the tokens' rows from being
 // read too often, and would otherwise be too few to fill the device.
 // (For rows that are no whole k-blocks; gemm_ring.h takes the others.)
+// LAST < 16: the last of a block's feature tiles has only LAST features (a block of 24 features is a tile and a
+// half): the rows beyond are never asked for (their lanes load nothing and multiply zeros), so a weight whose
+// 32-feature blocks would be an uneven number of rounds of the device can be shared out evenly.
 // ---------------------------------------------------------------------------
-template <int MT, int NT, int NW, int U>
+template <int MT, int NT, int NW, int U, int LAST = 16>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __restrict__ A, int lda,
                                                               const bf16* __restrict__ W, void* __restrict__ out,
                                                               int ldc, int M, int N, int K, int epi,
-                                                              float* __restrict__ partial, QkvEpilogue qe) {
+                                                              float* __restrict__ partial, QkvEpilogue qe, int rot_feats) {
     extern __shared__ __attribute__((aligned(16))) unsigned char skinny_smem[];
     float* red = (float*)skinny_smem;          // [NW][MT][NT][4][64]
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int row = lane & 15, g = lane >> 4;
-    int n0 = blockIdx.x * NT * 16;
+    constexpr int BF = (NT - 1) * 16 + LAST;       // features of a block
+    static_assert(LAST == 16 || LAST == 8, "a whole last tile, or half of one");
+    int n0 = blockIdx.x * BF;
+    const bool last_asks = LAST == 16 || row < LAST;   // whether this lane's row of the last tile exists
     const bf16* wp[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) wp[nt] = W + (size_t)min(n0 + nt * 16 + row, N - 1) * K;
@@ -98,6 +104,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
     int lo = blockIdx.y * per;
     int kb_hi = min(nkb, lo + per);                        // this block's k-blocks: [lo, kb_hi)
     int cnt = max(min(full, kb_hi) - lo, 0);               // the full ones among them
+    // The block walks its full k-blocks starting at `rot` and wraps round: with rot_feats > 0,
+    // neighbouring groups of rot_feats features are at different places of their rows at any
+    // moment.  Rows are a multiple of the memory channels' interleave apart, so blocks in step
+    // would all ask the same few channels at once.  The start depends on the features alone
+    // (a block's features lie within one group), not on how many of them a block takes.
+    int rot = (cnt > 0 && rot_feats > 0) ? (n0 / rot_feats) % cnt : 0;
+    auto turn = [&](int j) { int x = j + rot; return lo + (x >= cnt ? x - cnt : x); };
     // out += sum: the old values of the tile this wave will finish are asked for now, so that
     // their trip to memory runs beside the weights' instead of after the sums are ready
     float old[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -114,9 +127,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
         bf16x8 w[U][NT][2], x[U][MT][2];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            int k = (lo + j + u * NW) * 64 + g * 8;
+            int k = turn(j + u * NW) * 64 + g * 8;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) { w[u][nt][0] = load8(wp[nt] + k); w[u][nt][1] = load8(wp[nt] + k + 32); }
+            for (int nt = 0; nt < NT; ++nt) {
+                if (LAST == 16 || nt < NT - 1 || last_asks) { w[u][nt][0] = load8(wp[nt] + k); w[u][nt][1] = load8(wp[nt] + k + 32); }
+                else { w[u][nt][0] = zero8(); w[u][nt][1] = zero8(); }
+            }
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) { x[u][mt][0] = load8(xp[mt] + k); x[u][mt][1] = load8(xp[mt] + k + 32); }
         }
@@ -135,13 +151,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
     for (;; j += NW) {
         bool partial_turn = j == cnt && kb_hi > lo + cnt;   // one k-block past the full ones, cut by K
         if (j >= cnt && !partial_turn) break;
-        int k = (lo + j) * 64 + g * 8;
+        int k = (partial_turn ? lo + cnt : turn(j)) * 64 + g * 8;
         bool v0 = k < K, v1 = k + 32 < K;
         bf16x8 w0[NT], w1[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            w0[nt] = v0 ? load8(wp[nt] + k) : zero8();
-            w1[nt] = v1 ? load8(wp[nt] + k + 32) : zero8();
+            bool asks = LAST == 16 || nt < NT - 1 || last_asks;
+            w0[nt] = v0 && asks ? load8(wp[nt] + k) : zero8();
+            w1[nt] = v1 && asks ? load8(wp[nt] + k + 32) : zero8();
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -175,6 +192,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16* __rest
         int m = mt * 16 + row;
         int n = n0 + nt * 16 + 4 * g;
         if (m >= M) continue;
+        if (LAST < 16 && nt == NT - 1 && 4 * g >= LAST) continue;     // the half of the last tile that is the next block's
         if (partial != nullptr) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -275,17 +293,18 @@ static void launch_splitk_finish(hipStream_t stream, const float* partial, int s
     gemm_splitk_finish_kernel<<<ceil_div(pairs, 256), 256, 0, stream>>>(partial, splits, out, ldc, M, N, epi);
 }
 
-template <int MT, int NT, int NW, int U>
+template <int MT, int NT, int NW, int U, int LAST = 16>
 static void launch_skinny(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc,
-                          int M, int N, int K, int epi, const QkvEpilogue* qkv, int splits = 1, float* partial = nullptr, const NextNorm* next = nullptr) {
+                          int M, int N, int K, int epi, const QkvEpilogue* qkv, int splits = 1, float* partial = nullptr, int rot_feats = 0,
+                          const NextNorm* next = nullptr) {
     size_t bytes = (size_t)NW * MT * NT * 4 * 64 * sizeof(float);
     static bool configured = false;
     if (!configured) {
-        (void)hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, NT, NW, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        (void)hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, NT, NW, U, LAST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         configured = true;
     }
-    gemm_skinny_kernel<MT, NT, NW, U><<<dim3(ceil_div(N, NT * 16), splits), NW * 64, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi,
-                                                                                                    splits > 1 ? partial : nullptr, qkv ? *qkv : QkvEpilogue{});
+    gemm_skinny_kernel<MT, NT, NW, U, LAST><<<dim3(ceil_div(N, (NT - 1) * 16 + LAST), splits), NW * 64, bytes, stream>>>(
+        A, lda, W, out, ldc, M, N, K, epi, splits > 1 ? partial : nullptr, qkv ? *qkv : QkvEpilogue{}, rot_feats);
     if (splits > 1) launch_splitk_finish(stream, partial, splits, out, ldc, M, N, epi, next);
 }
 
@@ -1360,9 +1379,21 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         auto rows_of = [&](auto tiles) {
             constexpr int MT = decltype(tiles)::value;
             if (K % 64) {
-                if (split) launch_skinny<MT, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, next);
-                else if (wide) launch_skinny<MT, 4, 4, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv);
-                else launch_skinny<MT, 2, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv);
+                // Eight waves where rows are long, and the more k-blocks on their way the fewer features and tokens a block has; a walk
+                // along k that begins at a place of the block's own for wide weights and long rows (17 rows 8192 x 8224: 32.8 us,
+                // in step 49.8; 28672 x 4128: 49.8, in step and in blocks of four tiles 61.9; 64 rows 3072 x 96: 3.4, with eight waves 4.0).
+                const int rot = wide ? 16 * (evenness(7) >= evenness(4) ? 7 : 4) : (K >= 8192 ? 64 : 0);
+                const bool eight = K >= 2048;
+#define SKINNY(NT, NW, U, LAST) launch_skinny<MT, NT, NW, U, LAST>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, rot)
+                if (split) launch_skinny<MT, 4, 8, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, nullptr, splits, (float*)workspace, 0, next);
+                else if (wide) { if (evenness(7) >= evenness(4)) SKINNY(7, 4, 1, 16); else SKINNY(4, 4, 2, 16); }
+                else if (N > 4096) {
+                    if (eight && llmrs_half_tile_blocks(N, 32, cus)) SKINNY(2, 8, (MT == 2 ? 2 : 1), 8);
+                    else if (eight) SKINNY(2, 8, (MT == 2 ? 2 : 1), 16);
+                    else SKINNY(2, 4, 2, 16);
+                }
+                else { if (eight) SKINNY(1, 8, (MT == 2 ? 4 : 2), 16); else SKINNY(1, 4, (MT == 2 ? 4 : 2), 16); }
+#undef SKINNY
                 return;
             }
 #define RING(NT, LAST, KSUB, ROT) launch_ring<MT, NT, LAST, KSUB>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, 1, nullptr, ROT)

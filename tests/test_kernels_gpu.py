@@ -621,6 +621,14 @@ def test_gemm_ring_of_k_blocks(M, N, K):
             assert (err <= out_tol(ref, out.dtype, floor)).all(), (epi, room, float(err.max()))
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 40, 72), (33, 1000, 200), (64, 3000, 1096), (20, 2040, 2056), (48, 4090, 2120), (49, 8200, 328), (32, 6136, 2056),
+                                   (64, 6136, 2120), (24, 8200, 2088), (40, 8200, 8232), (31, 16400, 200), (64, 16500, 1032), (17, 28672, 72), (48, 28650, 328)])
+def test_gemm_rows_that_are_no_whole_k_blocks(M, N, K):
+    """17 to 64 rows of weights whose K is no multiple of 64, operands straight from memory: blocks of 16, 24, 32, 64 and 112 features
+    cut by N, four and eight waves, a walk that begins at a place of its own and wraps round; the ring's epilogues and bounds."""
+    test_gemm_ring_of_k_blocks(M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 4096, 1024), (600, 4100, 1088), (1030, 2048, 2048), (530, 1000, 4160), (512, 130, 8256), (2032, 3072, 192),
                                    (700, 16, 1024)])
 def test_gemm_tall_tiles_split_over_k(M, N, K):
@@ -715,6 +723,18 @@ def test_gemm_tall_tiles_only_where_they_are_faster(N, K, epi, limit):
         calls.append(lambda a=a, out=out, room=room: [k.gemm(a, w, out, epi, room) for w in ws])
     times = [replay_time(*calls) for _ in range(3)]
     assert min(b / a for a, b in times) <= limit, times
+
+
+def test_gemm_long_rows_that_are_no_whole_k_blocks_begin_their_walks_apart():
+    """17 rows of 8192 x 8224 in bfloat16 (K no multiple of 64) take less time than 8192 x 8256 takes through the ring: 0.74 of it with blocks that begin
+    their walks along k at places of their own, 1.14 with blocks in step."""
+    k, calls = kernels(), []
+    for K in (8224, 8256):
+        a, ws = rnd((17, K), torch.bfloat16, 3), [rnd((8192, K), torch.bfloat16, i, 0.1) for i in range(2)]
+        out = torch.zeros((17, 8192), dtype=torch.bfloat16, device=DEV)
+        calls.append(lambda a=a, ws=ws, out=out: [k.gemm(a, w, out, EPI_STORE) for w in ws])
+    times = [replay_time(*calls) for _ in range(3)]
+    assert min(a / b for a, b in times) <= 0.95, times
 
 
 @pytest.mark.parametrize("rows,width,groups,mixed", [(300, 8192, 8, True), (1000, 8192, 1, True), (64, 256, 1, False), (4, 2048, 4, True), (1000, 2048, 4, True)])
