@@ -68,7 +68,7 @@ __device__ __forceinline__ float gated_act_fast(const GatedAct& a, float g, floa
 // the epilogue.  That is for weights with few rows and many tokens (17..64),
 // where blocks of 64 features are needed to keep the tokens' rows from being
 // read too often, and would otherwise be too few to fill the device.
-// (For rows that are no whole k-blocks; gemm_ring.h takes the others.)
+// (For rows that are no whole k-blocks, and few short ones; gemm_ring.h takes the others.)
 // LAST < 16: the last of a block's feature tiles has only LAST features (a block of 24 features is a tile and a
 // half): the rows beyond are never asked for (their lanes load nothing and multiply zeros), so a weight whose
 // 32-feature blocks would be an uneven number of rounds of the device can be shared out evenly.
@@ -1378,7 +1378,9 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         auto evenness = [&](int nt) { int b = ceil_div(N, 16 * nt); return (double)b / ((double)ceil_div(b, cus) * cus); };
         auto rows_of = [&](auto tiles) {
             constexpr int MT = decltype(tiles)::value;
-            if (K % 64) {
+            // (and, adding to the stream, the shortest rows of narrow weights with up to 32 tokens, which come to a few k-blocks a wave and no
+            // steady state of the ring: 17 rows 512 x 512 4.0 us, in the ring 4.4, 1024 x 256 3.45 and 3.7; 40 rows are better off there)
+            if (K % 64 || (MT == 2 && N <= 4096 && K <= 512 && epi == LLMRS_EPI_ACCUM_F32)) {
                 // Eight waves where rows are long, and the more k-blocks on their way the fewer features and tokens a block has; a walk
                 // along k that begins at a place of the block's own for wide weights and long rows (17 rows 8192 x 8224: 32.8 us,
                 // in step 49.8; 28672 x 4128: 49.8, in step and in blocks of four tiles 61.9; 64 rows 3072 x 96: 3.4, with eight waves 4.0).

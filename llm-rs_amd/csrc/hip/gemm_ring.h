@@ -65,6 +65,17 @@ __global__ __launch_bounds__(64 * ring_waves<MT>()) void gemm_ring_kernel(const 
     f32x4 acc[TPW];
 #pragma unroll
     for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // a lane holds token lane % 16 of the wave's tile and features 4 (lane / 16) + r of each of its tiles; out += sum: the old values are
+    // asked for ahead of the weights (asked for after them they were a trip to memory more: 1 to 2 % of the products of up to 4096 x 1024)
+    const int m = mt * 16 + row;
+    const bool adds = partial == nullptr && epi == LLMRS_EPI_ACCUM_F32;
+    float old[TPW][4];
+    if (adds) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) old[t][r] = ((const float*)out)[(size_t)min(m, M - 1) * ldc + min(n0 + (wn + t * WN) * 16 + 4 * g + r, N - 1)];
+    }
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
         if (s < steps) issue(s);
@@ -93,17 +104,7 @@ __global__ __launch_bounds__(64 * ring_waves<MT>()) void gemm_ring_kernel(const 
             }
         }
     }
-    // a lane holds token lane % 16 of the wave's tile and features 4 (lane / 16) + r of each of its tiles
-    const int m = mt * 16 + row;
     if (m >= M) return;
-    const bool adds = partial == nullptr && epi == LLMRS_EPI_ACCUM_F32;
-    float old[TPW][4];
-    if (adds) {
-#pragma unroll
-        for (int t = 0; t < TPW; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) old[t][r] = ((const float*)out)[(size_t)m * ldc + min(n0 + (wn + t * WN) * 16 + 4 * g + r, N - 1)];
-    }
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
         const int nt = wn + t * WN, n = n0 + nt * 16 + 4 * g;
