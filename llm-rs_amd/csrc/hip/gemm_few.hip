@@ -15,9 +15,9 @@
 //   k-block, and of its 16 x 16 results the two 8 x 8 blocks on the diagonal are the halves' sums.
 //   9 to 16 tokens: an operand is 16 features, or 16 tokens, of one half of a k-block, and the two halves have sums of their own;
 //   17 to 32: the same with TT = 2 tiles of tokens.
-// Either way an output is the sum, in wave order, of each wave's (first halves' sum + second halves' sum): in bfloat16 its
+// Either way an output is the sum of each wave's (first halves' sum + second halves' sum), in bfloat16 in wave order: its
 // bits depend on K and on the weight's shape, which choose NW and where a block's walk along k begins, never on M.
-// (In 32-bit they differ between up to 8 and more rows by rounding.)
+// (In 32-bit the waves' sums are added pairwise, and bits differ by rounding between up to 2, up to 8, up to 16 and more rows.)
 // Measured, 16 features an operand and operands from memory -> as here (MI355X, weights from memory, us): bfloat16 at 1 row
 // 2048 x 8192 12.3 -> 8.6, 2048 x 2048 5.7 -> 4.3, 128256 x 2048 90 -> 83 (6.3 TB/s); at 8 rows 4096 x 4096 11.4 -> 8.6, 4096 x 14336
 // 28.5 -> 23.2, 28672 x 4096 44.2 -> 42.0; at 16 rows 4096 x 4096 13.3 -> 8.5, 4096 x 14336 35 -> 24.7, 10240 x 8192 49.5 -> 34.6;
@@ -28,8 +28,9 @@ template <class T> struct Few;
 template <> struct Few<bf16> { typedef bf16x8 Piece; typedef bf16x4 Four; };
 template <> struct Few<float> { typedef f32x4 Piece; typedef f32x4 Four; };
 
-// The sums of a tile: a 32-bit piece is four MFMAs, whose products go to SUMS sums of their own, added pairwise at the end
-// (a quarter of the products one after the other in a sum, and an error against 64 bits to match).
+// The sums of a tile: a 32-bit piece is four MFMAs, whose products go to SUMS sums of their own (eight: those of every other k-block
+// to the second four), added pairwise at the end: a quarter or an eighth of the products one after the other in a sum, and an error
+// against 64 bits to match.
 template <class T, int SUMS>
 struct FewSums {
     f32x4 s[SUMS];
@@ -37,15 +38,17 @@ struct FewSums {
 #pragma unroll
         for (int i = 0; i < SUMS; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    template <int HALF>
     __device__ __forceinline__ void add(const typename Few<T>::Piece& w, const typename Few<T>::Piece& x) {
         if constexpr (sizeof(T) == 2) s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, s[0], 0, 0, 0);
         else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s[j % SUMS] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], s[j % SUMS], 0, 0, 0);
+            for (int j = 0; j < 4; ++j) s[(4 * HALF + j) % SUMS] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], s[(4 * HALF + j) % SUMS], 0, 0, 0);
         }
     }
     __device__ __forceinline__ f32x4 total() const {
-        if constexpr (SUMS == 4) return (s[0] + s[1]) + (s[2] + s[3]);
+        if constexpr (SUMS == 8) return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+        else if constexpr (SUMS == 4) return (s[0] + s[1]) + (s[2] + s[3]);
         else if constexpr (SUMS == 2) return s[0] + s[1];
         else return s[0];
     }
@@ -158,12 +161,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
         at += NW;
         put = put + 1 == R ? 0 : put + 1;
     };
-    auto products = [&](const Piece (&w)[WL], const Piece (&x)[XL]) {
+    auto products = [&](auto half, const Piece (&w)[WL], const Piece (&x)[XL]) {
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-            for (int i = 0; i < WL; ++i) acc[tt][i].add(w[i], x[FOLD ? 0 : 2 * tt + (i & 1)]);
+            for (int i = 0; i < WL; ++i) acc[tt][i].template add<decltype(half)::value>(w[i], x[FOLD ? 0 : 2 * tt + (i & 1)]);
     };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
 #pragma unroll
     for (int i = 0; i < R - 1; ++i)
         if (i < mine) ask();
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
                 w[2 * t + 1] = *(const Piece*)(b + t * 2048 + half + off1);
             }
         }
-        products(w, x);
+        if (SUMS == 8 && (i & 1)) products(odd, w, x); else products(even, w, x);
     }
     if (K % KB != 0 && wave == full % NW) {      // the k-block that K cuts, straight from memory
         const int k = full * KB, first = (FOLD ? (row >> 3) * 4 + g : g) * PER;
@@ -208,7 +213,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
             const int from = k + first + (i & 1) * (KB / 2);
             x[i] = from < K ? *(const Piece*)(A + (size_t)min(FOLD ? f : i / 2 * 16 + row, M - 1) * lda + from) : Piece{};
         }
-        products(w, x);
+        products(even, w, x);
     }
     if (scaled) {
         float ss = 0.0f;
@@ -254,9 +259,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     for (int which = wave; which < TILES * TT; which += NW) {
         const int tile = which % TILES, tt = which / TILES, m = tt * 16 + row;
         if (m >= M || 2 * tile + (g >> 1) >= NG) continue;         // (the half of the last tile is the next block's)
-        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 of[NW];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) s += red[(((w * TT + tt) * NG + 2 * tile) * 2 + g) * TOK + row];
+        for (int w = 0; w < NW; ++w) of[w] = red[(((w * TT + tt) * NG + 2 * tile) * 2 + g) * TOK + row];
+        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (sizeof(T) == 2) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) s += of[w];
+        } else {
+            // pairwise: up to 8 rows of K = 2048 are 1.22e-7 off the 64-bit result, in wave order 1.26e-7
+#pragma unroll
+            for (int step = 1; step < NW; step *= 2)
+#pragma unroll
+                for (int w = 0; w < NW; w += 2 * step) of[w] += of[w + step];
+            s = of[0];
+        }
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = s[r] * inv;
@@ -354,7 +371,8 @@ static int wide_tiles(int N, int cus) {
     return evenness(7) >= evenness(4) ? 7 : 4;
 }
 extern "C" int llmrs_gemm_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 8 == 0; }
-extern "C" int llmrs_gemm_f32_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 32 == 0; }
+// (one row on the widest weights: the norm's kernel and gemm_rows_kernel together are faster, 128256 x 2048 175.6 against 180.0 us; 2 rows 182 and 179.5)
+extern "C" int llmrs_gemm_f32_defers_norm(int M, int N, int K) { return M >= 1 && M <= 16 && N >= 1 && K % 32 == 0 && !(M == 1 && N >= 65536); }
 extern "C" int llmrs_gemm_leaves_norm(int N) { return N < 16384 && N % 4 == 0; }
 extern "C" int llmrs_qkv_by_fours(int head_dim, int rotary_dim) { return head_dim % 4 == 0 && rotary_dim % 4 == 0; }
 extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
@@ -363,7 +381,7 @@ extern "C" int llmrs_gemm_next_parts(int M, int N, int K) {
 
 // Up to 8 rows: blocks of 8 NG features, rings of R k-blocks, in 32-bit four sums a tile; 9 to 16 rows: of 8 NG16, R16, one sum: the
 // error of the 32-bit products against 64 bits is then no larger than it was with one sum for whole k-blocks (K = 2048: 1.25e-7
-// up to 8 rows, 2.1e-7 from 9 on, against 2.9e-7; one and two rows as in gemm_rows_kernel, 1.2e-7).
+// up to 8 rows, 2.1e-7 from 9 on, against 2.9e-7).
 template <class T, int NW, int ROT, int NG, int R, int NG16, int R16>
 static void launch_few_by_rows(const FewCall& c) {
     if (c.M <= 8) launch_few<T, true, NG, NW, R, ROT, sizeof(T) == 4 ? 4 : 1>(c);
@@ -385,17 +403,28 @@ static void few_rows_two_tiles(const FewCall& c) {
     else if (half_blocks_for_narrow(c.N, c.K)) launch_few<float, false, 1, 8, 2, 64, 1, 2>(c);
     else launch_few<float, false, 2, 8, 2, 0, 1, 2>(c);
 }
+// One and two rows in 32-bit: eight waves and eight sums a tile whatever the shape.  gemm_rows_kernel, which takes such products too (see
+// llmrs_gemm), adds up few numbers one after the other, and the error here is to be no larger: K = 1024 0.9e-7 against 1.0e-7, 2048 1.02
+// and 1.23, 4096 1.27 and 1.59 (with four waves and four sums 1.2, 1.57 and 2.1); with a norm left to the product, against the norm's kernel and
+// gemm_rows_kernel, 320 1.0e-7 both, 2048 1.18 and 1.33.
+static void few_rows_one_or_two(const FewCall& c) {
+    const int N = c.N, K = c.K, cus = llmrs_compute_units();
+    if (N >= 16384) launch_few<float, true, 2, 8, 3, 64, 8>(c);
+    else if (K >= 16384 && N >= 8192) launch_few<float, true, 4, 8, 2, 64, 8>(c);
+    else if (half_blocks_for_narrow(N, K)) launch_few<float, true, 1, 8, 5, 64, 8>(c);
+    else if (c.next.y == nullptr && K >= 2048 && llmrs_half_tile_blocks(N, 16, cus)) launch_few<float, true, 3, 8, 3, 96, 8>(c);
+    else launch_few<float, true, 2, 8, 3, 64, 8>(c);
+}
 template <class T>
 static void few_rows(const FewCall& c) {
     const int N = c.N, K = c.K, cus = llmrs_compute_units();
     if (sizeof(T) == 4 && c.M > 16) { few_rows_two_tiles(c); return; }
+    if (sizeof(T) == 4 && c.M <= 2) { few_rows_one_or_two(c); return; }
     if (N >= 16384) {
         // (28672 x 4096 bfloat16 at 8 rows: blocks of 16 features 42.0 us, of 56 43.7, of 112 47; at 16 rows of 56 41.8, of 112 42.4)
         if (wide_tiles(N, cus) == 7) launch_few_by_rows<T, 4, 112, 2, 4, 7, 3>(c);
         // (at 16 rows 16384 x 2048: blocks of 64 features 14.5, of 16 15.1; in 32-bit, where a k-block is more MFMAs, 27.4 and 26.0)
         else if (c.M > 8 && sizeof(T) == 2) launch_few<T, false, 8, 4, 3, 64>(c);
-        // (one and two rows in 32-bit: eight waves, and so sums half as long: the error of gemm_rows_kernel's)
-        else if (c.M <= 2 && sizeof(T) == 4) launch_few<T, true, 2, 8, 3, 64, 4>(c);
         // (deeper rings let fewer blocks share a unit: 16384 x 2048 at 8 rows 14.3 with three, 14.9 with five; 128256 x 2048 93.2 and 90.9)
         else if (N < 32768) launch_few_by_rows<T, 4, 64, 2, 3, 2, 4>(c);
         else launch_few_by_rows<T, 4, 64, 2, 5, 2, 4>(c);

@@ -428,11 +428,17 @@ extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda,
         if (took != 0) return took < 0 ? -1 : 0;
     }
     const bool f32_cores = dtype == LLMRS_F32 && allow_mfma && K % 32 == 0 && lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
-    // (one or two tokens on the widest weights are better off with the walk below: 128256 x 2048 173 against 177 us)
+    const bool plain = scale_sumsq == nullptr && next_y == nullptr;
+    // One or two tokens: the walk below, whose error is the smaller one for K over 128 and under 1024 and which is at least as fast, but for
+    // longer rows of narrow weights and of wide ones and the longest rows of those between (1 row, walk / few rows' kernel, us: 512 x 1536 4.8 /
+    // 5.4, 2048 x 2048 7.8 / 6.1, 2048 x 8192 23 / 14.6, 4096 x 4096 14.6 / 14.5, 4608 x 1536 7.5 / 10.2, 6144 x 4096 20.0 / 22.1, 9216 x 5120
+    // 38.3 / 39.8, 13824 x 5120 56.7 / 52.2; from 65536 on no difference.  2 rows: 1024 x 1024 5.5 / 4.7, 9216 x 5120 41.6 / 40.8, 11008 x 128
+    // 4.7 / 3.8, 11008 x 3584 33.9 / 30.1).
+    const bool walk = plain && M <= 2 && (N >= 65536 || (N <= 4096 ? K < 1024 || (M == 1 && N <= 1536 && K < 2048)
+                                                        : N > 10240 ? K < 2048 : K < 5120 || (M == 1 && N > 8192))) && !(M == 2 && K <= 128 && N < 65536);
     // (17 to 32 on wide weights with the shortest rows with gemm_f32_skinny_kernel: 65536 x 128 16.1 against 19.8 us; from rows of 256 on there is
     // no difference, and the longer ones gain)
-    const bool plain = scale_sumsq == nullptr && next_y == nullptr;
-    if (f32_cores && M <= 32 && !(plain && M <= 2 && N >= 65536) && !(plain && M > 16 && N >= 16384 && K < 256)) {
+    if (f32_cores && M <= 32 && !walk && !(plain && M > 16 && N >= 16384 && K < 256)) {
         LLMRS_REQUIRE(plain || M <= 16, "gemm: a deferred norm needs the matrix-core kernels for few rows (M=%d N=%d K=%d)", M, N, K);
         RowScale rs{scale_sumsq, scale_parts, scale_eps};
         NextNorm nn{next_sumsq, next_y, next_ldy, next_weight, 0.0f};
