@@ -420,14 +420,26 @@ static void few_rows(const FewCall& c) {
     const int N = c.N, K = c.K, cus = llmrs_compute_units();
     if (sizeof(T) == 4 && c.M > 16) { few_rows_two_tiles(c); return; }
     if (sizeof(T) == 4 && c.M <= 2) { few_rows_one_or_two(c); return; }
-    if (N >= 16384) {
+    const int kblocks = ceil_div(K * (int)sizeof(T), 128);
+    // Short rows, and more than two blocks of 16 features a unit: what fills the time is the other blocks, not a deep ring, which a wave has not
+    // the k-blocks to fill and which keeps blocks off the unit (us, rings of three to five in blocks of 16 to 64 features -> as here: 32-bit at 8
+    // rows 65536 x 256 22.9 -> 15.9, 100000 x 128 27 -> 14.6, 13824 x 256 6.7 -> 5.6, at 16 rows 32000 x 256 12.8 -> 9.6; bfloat16 at 8 rows
+    // 65536 x 512 20 -> 14.8, at 16 50304 x 256 13 -> 8.9).  From 32 k-blocks on the rings gain (bfloat16 at 1 row 32000 x 2560 30.7, as here 31.3).
+    if (kblocks <= 16 && ceil_div(N, 16) > 2 * cus) {
+        // (the shortest of them, many features: two waves a block.  32-bit 100000 x 128 at 16 rows 17.6 with four, 15.7 with two; bfloat16 65536 x 512
+        // at 12 rows 16.1 and 15.6, 32000 x 256 6.6 and 5.8; 13824 x 128 at 8 rows 4.4 and 5.1)
+        if (kblocks <= (sizeof(T) == 2 ? 8 : 4) && N >= 24576) launch_few_by_rows<T, 2, 64, 4, 2, 4, 2>(c);
+        else launch_few_by_rows<T, 4, 0, 2, 2, 2, 2>(c);
+    }
+    else if (N >= 16384) {
         // (28672 x 4096 bfloat16 at 8 rows: blocks of 16 features 42.0 us, of 56 43.7, of 112 47; at 16 rows of 56 41.8, of 112 42.4)
         if (wide_tiles(N, cus) == 7) launch_few_by_rows<T, 4, 112, 2, 4, 7, 3>(c);
-        // (at 16 rows 16384 x 2048: blocks of 64 features 14.5, of 16 15.1; in 32-bit, where a k-block is more MFMAs, 27.4 and 26.0)
-        else if (c.M > 8 && sizeof(T) == 2) launch_few<T, false, 8, 4, 3, 64>(c);
+        // (at 16 rows 16384 x 2048: blocks of 64 features 14.5, of 16 15.1; in 32-bit, where a k-block is more MFMAs, of 32 25.8, of 16 27.2, 32000 x 2560
+        // 62.5 and 70.5, 128256 x 2048 181 and 200)
+        else if (c.M > 8) { if (sizeof(T) == 2) launch_few<T, false, 8, 4, 3, 64>(c); else launch_few<T, false, 4, 4, 2, 64>(c); }
         // (deeper rings let fewer blocks share a unit: 16384 x 2048 at 8 rows 14.3 with three, 14.9 with five; 128256 x 2048 93.2 and 90.9)
-        else if (N < 32768) launch_few_by_rows<T, 4, 64, 2, 3, 2, 4>(c);
-        else launch_few_by_rows<T, 4, 64, 2, 5, 2, 4>(c);
+        else if (N < 32768) launch_few<T, true, 2, 4, 3, 64, sizeof(T) == 4 ? 4 : 1>(c);
+        else launch_few<T, true, 2, 4, 5, 64, sizeof(T) == 4 ? 4 : 1>(c);
     }
     else if (K < 2048) launch_few_by_rows<T, 4, 0, 2, 4, 2, 4>(c);
     else if (K >= 16384 && N >= 8192) launch_few_by_rows<T, 8, 64, 4, 2, 4, 2>(c);      // 8192 x 28672 at 16 rows: 80.8 us, in blocks of 16 features 89.9

@@ -570,10 +570,11 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(1, 40, 64), (8, 24, 96), (9, 250, 544), (16, 1990, 2048), (7, 2040, 2080), (16, 2048, 2592), (8, 3000, 2304), (13, 3080, 2176),
-                                   (8, 6136, 2112), (16, 6150, 2048), (3, 16390, 288), (10, 16400, 2048), (8, 33000, 160), (5, 28650, 352), (11, 28672, 64), (8, 8200, 16448)])
+                                   (8, 6136, 2112), (16, 6150, 2048), (3, 16390, 288), (10, 16400, 2048), (8, 33000, 160), (5, 28650, 352), (11, 28672, 64), (8, 8200, 16448),
+                                   (8, 8200, 512), (9, 13830, 416), (3, 24580, 96), (16, 24570, 128), (1, 33000, 520), (12, 32010, 1056)])
 def test_gemm_few_rows_and_their_rings(dtype, M, N, K):
     """Up to 16 rows: waves with no k-block, fewer than their ring has places, as many and more; blocks of 8, 16, 24, 32, 56 and 64
-    features cut by N, a k-block cut by K; both sides of 8 rows; every epilogue, rows with a stride."""
+    features cut by N (both sides of where short rows take shallow rings and two waves), a k-block cut by K; both sides of 8 rows; every epilogue, rows with a stride."""
     k = kernels()
     a, w = rnd((M, K + 24), dtype, 3)[:, :K], rnd((N, K), dtype, 4, 0.1)
     acc = a.double().cpu() @ w.double().cpu().T
@@ -759,6 +760,18 @@ def test_gemm_tall_tiles_only_where_they_are_faster(N, K, epi, limit):
         calls.append(lambda a=a, out=out, room=room: [k.gemm(a, w, out, epi, room) for w in ws])
     times = [replay_time(*calls) for _ in range(3)]
     assert min(b / a for a, b in times) <= limit, times
+
+
+@pytest.mark.parametrize("dtype,M,N,K", [(torch.float32, 8, 100000, 128), (torch.float32, 16, 65536, 256), (torch.bfloat16, 8, 65536, 256)])
+def test_gemm_short_rows_of_many_features_take_no_deep_ring(dtype, M, N, K):
+    """The same number of weights in half as many rows of twice the length: the shorter rows take 1.07 to 1.25 times the time.  With rings
+    that the rows do not fill it was 2.0, 1.45 and 1.9 times."""
+    k, calls = kernels(), []
+    for n, kk in ((N, K), (N // 4, 4 * K)):
+        a, ws, out = rnd((M, kk), dtype, 3), [rnd((n, kk), dtype, i, 0.1) for i in range(4)], torch.zeros((M, n), dtype=dtype, device=DEV)
+        calls.append(lambda a=a, ws=ws, out=out: [k.gemm(a, w, out, EPI_STORE) for w in ws])
+    times = [replay_time(*calls) for _ in range(3)]
+    assert min(a / b for a, b in times) <= 1.35, times
 
 
 def test_gemm_long_rows_that_are_no_whole_k_blocks_begin_their_walks_apart():
