@@ -444,8 +444,17 @@ static void few_rows(const FewCall& c) {
     else if (K < 2048) launch_few_by_rows<T, 4, 0, 2, 4, 2, 4>(c);
     else if (K >= 16384 && N >= 8192) launch_few_by_rows<T, 8, 64, 4, 2, 4, 2>(c);      // 8192 x 28672 at 16 rows: 80.8 us, in blocks of 16 features 89.9
     else if (half_blocks_for_narrow(N, K)) launch_few_by_rows<T, 8, 64, 1, 5, 1, 4>(c);
-    // (nothing is to be left for a norm, which counts its sums by 16 features; 6144 x 4096 at 8 rows 11.6 us, in blocks of 16 13.5)
-    else if (c.next.y == nullptr && (llmrs_half_tile_blocks(N, 16, cus) || ceil_div(N, 16) > 2 * cus)) launch_few_by_rows<T, 8, 96, 3, 3, 3, 3>(c);
+    // Blocks of 24 features where they share the weight out more evenly (6144 x 4096 at 8 rows 11.6 us, in blocks of 16 13.5), and from 9 rows on where
+    // there are more than two blocks of 16 a unit (10240 x 4096 at 16 rows 20.3, of 16 21.7; at 8 rows 18.8 and 18.1, 14336 x 2048 16.4 and
+    // 13.4) -- but not if something is left for a norm, which counts its sums by 16 features.  In bfloat16 the walk along k begins by groups of 48
+    // features in all of these: a row's bits depend neither on what is left nor on how many rows there are.  (32-bit, whose bits do
+    // differ, keeps groups of 64 and 96: those of 48 cost it 5 % of 5120 x 8192.)
+    else if (llmrs_half_tile_blocks(N, 16, cus) || ceil_div(N, 16) > 2 * cus) {
+        constexpr int BY16 = sizeof(T) == 2 ? 48 : 64, BY24 = sizeof(T) == 2 ? 48 : 96;
+        if (c.next.y != nullptr) launch_few_by_rows<T, 8, BY16, 2, 3, 2, 3>(c);
+        else if (ceil_div(N, 16) > 2 * cus && c.M <= 8) launch_few<T, true, 2, 8, 3, BY16, sizeof(T) == 4 ? 4 : 1>(c);
+        else launch_few_by_rows<T, 8, BY24, 3, 3, 3, 3>(c);
+    }
     else launch_few_by_rows<T, 8, 64, 2, 3, 2, 3>(c);
 }
 

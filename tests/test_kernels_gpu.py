@@ -1542,7 +1542,9 @@ def test_gemm_finishes_a_norm_left_to_it(M, N, K, epi):
 
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (8, 4096, 14336), (16, 4096, 4096), (5, 200, 328), (3, 8192, 28672), (12, 100, 64),
                                    # narrow weights with long rows: blocks of 8 features, a partial sum for each
-                                   (1, 2048, 8192), (8, 2048, 2048), (16, 1024, 4096), (3, 2040, 2048)])
+                                   (1, 2048, 8192), (8, 2048, 2048), (16, 1024, 4096), (3, 2040, 2048),
+                                   # blocks of 24 features but for what is left, in one round of the units and in more, and short rows of many features
+                                   (8, 5120, 4096), (16, 6144, 2048), (2, 9216, 5120), (12, 12288, 2112), (16, 9000, 512)])
 def test_residual_product_leaves_what_the_next_norm_needs(M, N, K):
     from llm_rs_amd.kernels import NextNorm
     k = kernels()
@@ -1567,6 +1569,20 @@ def test_residual_product_leaves_what_the_next_norm_needs(M, N, K):
     want = (padded * padded).view(M, parts, per).sum(-1)
     assert float((sums.double().cpu() - want).abs().max()) <= 1e-5 * float(want.abs().max())
     assert float((h.double().cpu() - want_h).abs().max()) <= 1e-5 * math.sqrt(K) + 1e-5 * float(want_h.abs().max())
+
+
+@pytest.mark.parametrize("N,K", [(5120, 4096), (6144, 2048), (9216, 5120), (13824, 2112), (9000, 512), (28672, 2048), (24600, 256), (32000, 1024), (2048, 8192),
+                                 (33000, 2048)])
+def test_a_rows_bits_do_not_depend_on_how_many_rows_there_are(N, K):
+    """bfloat16, up to 16 rows: the first row's result is the same bits beside 0, 1, 7, 8 and 15 others, whatever blocks that means."""
+    k = kernels()
+    a, w = rnd((16, K), torch.bfloat16, 3), rnd((N, K), torch.bfloat16, 4, 0.1)
+    rows = []
+    for M in (1, 2, 8, 9, 16):
+        out = torch.zeros((M, N), device=DEV)
+        k.gemm(a[:M], w, out, EPI_STORE_F32)
+        rows.append(out[0])
+    assert all(torch.equal(r, rows[0]) for r in rows)
 
 
 @pytest.mark.parametrize("M,hidden,inter", [(1, 2048, 8192), (8, 2048, 8192), (16, 1024, 2048), (5, 4096, 14336), (3, 4096, 4096)])
