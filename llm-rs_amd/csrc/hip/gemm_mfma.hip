@@ -1273,8 +1273,13 @@ static bool few_rows_take_tiles(int M, int N, int K) {
 }
 // Of those the products with short rows that store their results or gate them are better off with the ring (tiles with their finish -> ring, us:
 // 17 rows 8192 x 2048 15.3 -> 11.3, 10240 x 4096 27.8 -> 22.0; over 4608 to 16000 features a ratio of 0.67 at K = 1024 whatever
-// the rows, 0.81-0.96 at 2048 to 4096 and up to 48 rows; with more rows or longer ones some gain and some lose up to 22 %).
-static bool ring_stores_faster(int M, int K) { return K <= (M <= 48 ? 4096 : 1024); }
+// the rows, 0.76-0.98 at 2048 to 4096 and up to 32 rows; with more rows or longer ones some gain and some lose up to 22 %).
+// 33 to 48 rows read theirs often enough for the tiles to win over many features with rows of 2048 to 4096 (ring / tiles, 48 rows 14336 x 2560
+// 1.12, 13824 x 3584 1.09, 9216 x 2560 1.05; 40 rows 14336 x 2560 1.04, 12288 x 2560 0.98; at K = 2048 0.92-0.98, at 4096 0.80-1.0).
+static bool ring_stores_faster(int M, int N, int K) {
+    const bool tiles_between = M > 32 && N > (M <= 40 ? 12288 : 8192) && K > 2048 && K < 4096;
+    return K <= (M <= 48 ? 4096 : 1024) && !tiles_between;
+}
 // Room (in floats) for the partial sums of a product that would be split: what the caller should bring.
 extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
     if (M > 16 && M <= 64) {
@@ -1359,7 +1364,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         return 1;
     }
     bool tiles_for_few = false;
-    if (epi != LLMRS_EPI_QKV && few_rows_take_tiles(M, N, K) && (epi == LLMRS_EPI_ACCUM_F32 || !ring_stores_faster(M, K))) {
+    if (epi != LLMRS_EPI_QKV && few_rows_take_tiles(M, N, K) && (epi == LLMRS_EPI_ACCUM_F32 || !ring_stores_faster(M, N, K))) {
         int splits = tiled_splits(M, N, K);
         tiles_for_few = workspace != nullptr && workspace_bytes >= (size_t)splits * M * N * sizeof(float);
     }
