@@ -92,7 +92,7 @@ __device__ __forceinline__ void epilogue_store(int epi, void* out, int ldc, int 
     else if (epi == LLMRS_EPI_ACCUM_F32) ((float*)out)[(size_t)m * ldc + n] += v;
 }
 
-// Up to 16 rows (gemm_few.hip): 16-byte aligned rows, K % 8 == 0 (32-bit: K % 32 == 0), the caller's to check.  1, 0 where the q/k/v
+// Up to 16 rows, in 32-bit up to 32 (gemm_few.hip; scale, next and the q/k/v epilogue for up to 16): 16-byte aligned rows, K % 8 == 0 (32-bit: K % 32 == 0), the caller's to check.  1, 0 where the q/k/v
 // epilogue's shape or alignment is not the kernel's, -1 on error (a deferred norm that cannot be taken); a launch's own
 // error is the caller's to ask for.
 int llmrs_gemm_few_bf16(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi,

@@ -1,4 +1,4 @@
-// Products of up to 16 rows (decoding), in 32-bit up to 32, bfloat16 and 32-bit, on the matrix cores with 32-bit sums.
+// Products of up to 16 rows (decoding), in 32-bit up to 32 (some of one and two rows go to gemm_rows_kernel), bfloat16 and 32-bit, on the matrix cores with 32-bit sums.
 //
 // What bounds them: the weight's bytes, each read once, how many of them are on their way at a time, and the address unit in
 // front of the vector cache, which takes a line a clock.  A block owns 8 NG output features; its NW waves take the k-blocks
@@ -348,8 +348,8 @@ static void launch_few(const FewCall& c) {
         gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS, TT><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
             (const T*)c.A, (const T*)c.W, c.out, c.lda, c.ldc, c.M, c.N, c.K, c.epi, inv_full, extra);
     };
-    if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
-    else if constexpr (TT > 1) launch(FewPlain{});        // (no norm is left to a product of more than 16 rows)
+    if constexpr (TT > 1) launch(FewPlain{});             // (more than 16 rows: no norm is left to them, and no rotation)
+    else if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
     else if (c.next.y != nullptr) launch(FewNext{c.scale, c.next});
     else if (c.scale.sumsq != nullptr) launch(FewScaled{c.scale});
     else launch(FewPlain{});
@@ -468,7 +468,7 @@ static int gemm_few(hipStream_t stream, const T* A, int lda, const T* W, void* o
                                        next->weight != nullptr && next->ldy >= N && next->ldy % 4 == 0 && (uintptr_t)next->y % FOUR == 0));
         if (!ok) { llmrs_fail("gemm: a deferred norm is taken for up to 16 rows (what is left for the next one: with the += epilogue, a multiple of 4 and under 16384 features), got M=%d N=%d K=%d epilogue %d", M, N, K, epi); return -1; }
     }
-    if (epi == LLMRS_EPI_QKV && (qkv == nullptr || !llmrs_qkv_by_fours(qkv->head_dim, qkv->rotary_dim) || ldc % 4 || (uintptr_t)out % FOUR || (uintptr_t)qkv->k_cache % FOUR))
+    if (epi == LLMRS_EPI_QKV && (M > 16 || qkv == nullptr || !llmrs_qkv_by_fours(qkv->head_dim, qkv->rotary_dim) || ldc % 4 || (uintptr_t)out % FOUR || (uintptr_t)qkv->k_cache % FOUR))
         return 0;
     few_rows<T>(FewCall{stream, A, lda, W, out, ldc, M, N, K, epi, qkv ? *qkv : QkvEpilogue{}, scale ? *scale : RowScale{}, next ? *next : NextNorm{}});
     return 1;

@@ -237,7 +237,8 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const T* __restrict__ A,
     }
 }
 
-// 17 tokens and more in 32-bit on the matrix cores (up to 16: gemm_few.hip): v_mfma_f32_16x16x4_f32 multiplies and adds in
+// 33 tokens and more in 32-bit on the matrix cores (up to 32: gemm_few.hip, but for 17 to 32 on wide weights with the shortest rows, which
+// come here): v_mfma_f32_16x16x4_f32 multiplies and adds in
 // 32-bit (no reduced-precision mode).  The weight's rows are the A operand, read once for every 16 MT tokens, 16 bytes a
 // lane (lane l: feature l % 16 of a tile, the four k-values 4 (l / 16) .. + 3 of a group of 16); the tokens' rows are the B
 // operand, read the same way once for all of a block's NT feature tiles.  An MFMA contracts the four k-values that the
@@ -350,8 +351,7 @@ static bool launch_f32_few_rows(hipStream_t stream, const float* a, int lda, con
     const int cus = llmrs_compute_units();
     // Blocks of 32 tokens with the fewest features that still make one round of the compute units.  Where even
     // 64 features to a block make more, the tiles take over, but for up to 32 tokens, whose weights are read once here.
-    // (us, this kernel / tiles: 64 rows 3072 x 2048 19 / 45,
-    // 16384 x 2048 66 / 48; 100 rows 2048 x 2048 19 / 45; 200 rows 2048 x 2048 29 / 45, 3072 x 2048 58 / 46)
+    // (us, this kernel / tiles: 64 rows 3072 x 2048 19 / 45, 16384 x 2048 66 / 48; 100 rows 2048 x 2048 19 / 45; 200 rows 2048 x 2048 29 / 45, 3072 x 2048 58 / 46)
     const long rows = ceil_div(M, 32);
     if (rows * ceil_div(N, 16) <= cus) launch_f32_skinny<2, 1, 4, 4>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
     else if (rows * ceil_div(N, 32) <= cus) launch_f32_skinny<2, 2, 4, 2>(stream, a, lda, w, out, ldc, M, N, K, epi, 64);
