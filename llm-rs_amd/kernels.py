@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 import sys
 from ctypes import c_char_p, c_float, c_int, c_size_t, c_void_p
@@ -301,6 +302,12 @@ class HipKernels(Kernels):
         lib.llmrs_attention_split_chunk.argtypes = [ctypes.c_long, I, I, I, ctypes.c_long]
         lib.llmrs_gemm_workspace_floats.restype = ctypes.c_long
         lib.llmrs_gemm_workspace_floats.argtypes = [I, I, I]
+        # The hand-over of norms is asked about several times a layer, and a step that is not recorded is bound by the host: the library's
+        # answers, which depend on sizes alone, are kept by them.
+        kept = functools.lru_cache(maxsize=4096)
+        self._defers_norm = kept(lambda bf16, M, N, K: bool((lib.llmrs_gemm_defers_norm if bf16 else lib.llmrs_gemm_f32_defers_norm)(M, N, K)))
+        self._stored_by_fours = kept(lambda head_dim, rotary_dim: bool(lib.llmrs_qkv_by_fours(head_dim, rotary_dim)))
+        self._norm_plan = kept(self._ask_norm_plan)
 
     def gemm_workspace_floats(self, M: int, N: int, K: int) -> int:
         """Room that lets a product with too few blocks split K over blocks (the kernels' own rule)."""
@@ -310,14 +317,17 @@ class HipKernels(Kernels):
         return self.gemm_defers_norm(M, N, K, dtype)
 
     def qkv_product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype, head_dim: int, rotary_dim: int) -> bool:
-        return bool(self.lib.llmrs_qkv_by_fours(int(head_dim), int(rotary_dim))) and self.gemm_defers_norm(M, N, K, dtype)
+        return self._stored_by_fours(head_dim, rotary_dim) and self.gemm_defers_norm(M, N, K, dtype)
 
     def norm_left_by_product(self, M: int, N: int, K: int, dtype: torch.dtype) -> Optional[NormPlan]:
+        return self._norm_plan(dtype == torch.bfloat16, M, N, K) if self.allow_mfma else None
+
+    def _ask_norm_plan(self, bf16: bool, M: int, N: int, K: int) -> Optional[NormPlan]:
         # up to a few rows: partial sums of squares, for the next product to finish (the kernels keep at most 1024
         # of them a row); more rows: a product that is split over blocks finishes the norm where its parts are added up
-        if self.lib.llmrs_gemm_leaves_norm(int(N)) and self.gemm_defers_norm(M, N, K, dtype):
+        if self.lib.llmrs_gemm_leaves_norm(N) and self._defers_norm(bf16, M, N, K):
             return NormPlan(False, self.gemm_next_parts(M, N, K))
-        if dtype == torch.bfloat16 and self.gemm_norms_whole(M, N, K):
+        if bf16 and self.lib.llmrs_gemm_norms_whole(M, N, K):
             return NormPlan(True, 0)
         return None
 
@@ -327,8 +337,7 @@ class HipKernels(Kernels):
     def gemm_defers_norm(self, M: int, N: int, K: int, dtype: torch.dtype = torch.bfloat16) -> bool:
         """Whether the product of M rows with an [N, K] weight takes `NormedRows` as its rows and, adding
         into the stream, leaves a `NextNorm` (that: for a multiple of 4 and fewer than 16384 features)."""
-        asked = self.lib.llmrs_gemm_defers_norm if dtype == torch.bfloat16 else self.lib.llmrs_gemm_f32_defers_norm
-        return self.allow_mfma and bool(asked(int(M), int(N), int(K)))
+        return self.allow_mfma and self._defers_norm(dtype == torch.bfloat16, M, N, K)
 
     def gemm_next_parts(self, M: int, N: int, K: int) -> int:
         """Partial sums of squares per row that a product leaving a `NextNorm` writes (one per 16 features, for some

