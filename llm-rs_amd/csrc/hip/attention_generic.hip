@@ -342,9 +342,11 @@ __global__ __launch_bounds__(64) void attention_generic_group_kernel(
 // the maxima and sums of up to 64 chunks, a lane each, and the rows of the first chunks, of both maps, asked for before
 // the length is known (they lie within the scratch; what is beyond the entry's chunks is not used).  Further rows come as many at a time.
 // (32-bit, 8 requests of 200 to 1800 keys, heads of 64: 6.6 us with lengths, maxima and rows one after the other, rows four at
-// a time; now 4.9.  Of up to 1000 keys, two maps and values of 128: 11.3, now 6.0.)  With more than 1024 waves (four to a compute unit)
+// a time; now 4.9.  Of up to 1000 keys, two maps and values of 128: 11.3, now 6.0.)  With more than 512 waves (two to a compute unit)
 // it is bound by what it reads and no longer by the trips, and a recorded step's table may be far wider than its keys: then
-// the length comes first (64 requests of 200 keys, 32 heads of 128, a table for 8192: the call 1.14 times that of a table for 256 otherwise).
+// the length comes first (32 heads, a table as wide as the keys / for 8192, us a call, rows first -> lengths first: 128 requests of 200 keys, heads
+// of 128, 59.2 / 83.4 -> 59.2 / 70.7; 32 of 1000 keys 73.4 / 76.3 -> 73.3 / 73.8; 32 of 200 keys, heads of 64, 13.1 / 22.8 -> 13.1 / 21.7; 16 of 200 keys
+// 9.9 / 20.0 -> 10.0 / 19.3; 8 of 3000 keys 31.0 / 33.7 -> 31.8 / 34.1).
 template <class T, int MAPS, int VALS>
 __global__ __launch_bounds__(64) void attention_generic_merge_kernel(
     const float* __restrict__ partial, T* __restrict__ out, const int* __restrict__ q_starts,
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(64) void attention_generic_merge_kernel(
     const size_t stride = hd + 2;
     int t = q_starts[e], next = q_starts[e + 1], pos = seq_lens[e] - 1;
     float m_first[MAPS], l_first[MAPS], rows[MAPS][AHEAD][VALS];
-    const bool length_first = gridDim.x * gridDim.y > 1024;
+    const bool length_first = gridDim.x * gridDim.y > 512;
     auto ask = [&](float (&v)[AHEAD][VALS], const float* pp, int first, int n) {       // rows first .. of n
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u)
