@@ -19,6 +19,11 @@ def rnd(shape, dtype, seed, scale=1.0):
     return (torch.randn(shape, generator=g) * scale).to(dtype).to(DEV)
 
 
+def product64(a, w):
+    """a w^T of the exact values in 64 bits, by the library's product on the device (on the host the widest took seconds each)."""
+    return (a.double() @ w.double().T).cpu()
+
+
 def out_tol(ref, dtype, floor):
     """Allowed error per element: half an ulp of the output type and then some, or a floor
     for sums that cancel (tests/ops.rs:142-145 uses |e|/64 and a floor for bfloat16 output)."""
@@ -94,7 +99,7 @@ def test_gemm(dtype, M, N, K, epi):
     a_full = rnd((M, K + pad), dtype, 3)
     a = a_full[:, :K]                       # rows with a stride, as q inside qkv has
     w = rnd((N, K), dtype, 4, 0.1)
-    acc = a.double().cpu() @ w.double().cpu().T
+    acc = product64(a, w)
     floor = 2e-6 * math.sqrt(K) if dtype == torch.float32 else 1e-5 * math.sqrt(K)
     if epi == EPI_STORE:
         out = torch.zeros((M, N), dtype=dtype, device=DEV)
@@ -277,8 +282,9 @@ class PagedCase:
                 continue
             qq = torch.zeros((n, self.n_heads, self.hd), dtype=torch.float64)
             qq[-1] = q[i].double()
-            o = plain_attention(qq, self.k[r][:n].double(), self.v[r][:n].double(), scale, window)
-            outs.append(o[-1])
+            # (the plain function on tensors of the device: the table of all rows' scores takes the host a second of each of the longest)
+            o = plain_attention(qq.to(DEV), self.k[r][:n].double().to(DEV), self.v[r][:n].double().to(DEV), scale, window)
+            outs.append(o[-1].cpu())
         return torch.stack(outs)
 
 
@@ -501,7 +507,7 @@ def test_gemm_float32_few_rows_on_the_matrix_cores(M, N, K):
     a_full = rnd((M, K + 24), torch.float32, 3)
     a = a_full[:, :K]
     w = rnd((N, K), torch.float32, 4, 0.1)
-    acc = a.double().cpu() @ w.double().cpu().T
+    acc = product64(a, w)
     k = kernels()
     for epi in (EPI_STORE, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU):
         outs = []
@@ -542,7 +548,7 @@ def test_gemm_float32_forms_by_shape(M, N, K):
     a_full = rnd((M, K + 8), torch.float32, 3)
     a = a_full[:, :K]
     w = rnd((N, K), torch.float32, 4, 0.1)
-    acc = a.double().cpu() @ w.double().cpu().T
+    acc = product64(a, w)
     for epi in (EPI_STORE, EPI_ACCUM_F32, EPI_SWIGLU):
         out = rnd((M, N), torch.float32, 5) if epi == EPI_ACCUM_F32 else torch.zeros((M, N // 2 if epi == EPI_SWIGLU else N), dtype=torch.float32, device=DEV)
         ref = out.double().cpu() + acc if epi == EPI_ACCUM_F32 else plain_silu(acc[:, 0::2]) * acc[:, 1::2] if epi == EPI_SWIGLU else acc
@@ -558,7 +564,7 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
     """Grids of large tiles with more rows than an XCD takes at a time, numbers of tiles that eight does not divide, and 256 x 192
     tiles cut by N: every tile of the output is written, once (a += shows a tile written twice)."""
     a, w = rnd((M, K), torch.bfloat16, 3), rnd((N, K), torch.bfloat16, 4, 0.1)
-    acc = a.double().cpu() @ w.double().cpu().T
+    acc = product64(a, w)
     for epi in (EPI_STORE_F32, EPI_ACCUM_F32):
         out = torch.zeros((M, N), dtype=torch.float32, device=DEV) if epi == EPI_STORE_F32 else rnd((M, N), torch.float32, 5)
         ref = acc if epi == EPI_STORE_F32 else out.double().cpu() + acc
@@ -577,7 +583,7 @@ def test_gemm_few_rows_and_their_rings(dtype, M, N, K):
     features cut by N (both sides of where short rows take shallow rings and two waves), a k-block cut by K; both sides of 8 rows; every epilogue, rows with a stride."""
     k = kernels()
     a, w = rnd((M, K + 24), dtype, 3)[:, :K], rnd((N, K), dtype, 4, 0.1)
-    acc = a.double().cpu() @ w.double().cpu().T
+    acc = product64(a, w)
     for epi in (EPI_STORE, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU):
         if epi == EPI_SWIGLU:
             out, ref = torch.zeros((M, N // 2), dtype=dtype, device=DEV), plain_silu(acc[:, 0::2]) * acc[:, 1::2]
@@ -642,7 +648,7 @@ def test_gemm_ring_of_k_blocks(M, N, K):
     stage holds two, unequal shares of a split k, blocks of 16, 24, 32, 64 and 112 features cut by N; every epilogue, rows with a stride."""
     k = kernels()
     a, w = rnd((M, K + 16), torch.bfloat16, 3)[:, :K], rnd((N, K), torch.bfloat16, 4, 0.1)
-    acc = a.double().cpu() @ w.double().cpu().T
+    acc = product64(a, w)
     n_ws = k.gemm_workspace_floats(M, N, K)
     for epi in (EPI_STORE, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU):
         if epi == EPI_SWIGLU:
@@ -674,7 +680,7 @@ def test_gemm_tall_tiles_split_over_k(M, N, K):
     from llm_rs_amd.kernels import NextNorm
     k = kernels()
     a, w, h = rnd((M, K), torch.bfloat16, 3), rnd((N, K), torch.bfloat16, 4, 0.1), rnd((M, N), torch.float32, 5)
-    ref = h.double().cpu() + a.double().cpu() @ w.double().cpu().T
+    ref = h.double().cpu() + product64(a, w)
     n_ws = k.gemm_workspace_floats(M, N, K)
     tol = out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))
     for room in ([True, False] if n_ws else [False]):
@@ -1367,7 +1373,7 @@ def test_qkv_rope_cache(dtype, M, n_heads, n_kv, hd, rot, K):
     vc = torch.zeros((num_pages, n_kv, hd, page_size), dtype=dtype, device=DEV)
     kernels().qkv_rope_cache(x, w, qkv[:, :N], positions, slots, inv_freq, rot, kc, vc, n_heads, n_kv, hd,
                              page_size, num_pages, True)
-    acc = x.double().cpu() @ w.double().cpu().T
+    acc = product64(x, w)
     q = acc[:, :n_heads * hd].view(M, n_heads, hd)
     k = acc[:, n_heads * hd:(n_heads + n_kv) * hd].view(M, n_kv, hd)
     v = acc[:, (n_heads + n_kv) * hd:].view(M, n_kv, hd)
@@ -1417,7 +1423,7 @@ def test_qkv_rope_cache_adds_up_a_split_product(M, n_heads, n_kv, hd, rot, K):
     vc = torch.zeros((num_pages, n_kv, hd, page_size), dtype=torch.bfloat16, device=DEV)
     ws = torch.empty(n_ws, dtype=torch.float32, device=DEV)
     k.qkv_rope_cache(x, w, qkv[:, :N], positions, slots, inv_freq, rot, kc, vc, n_heads, n_kv, hd, page_size, num_pages, True, ws)
-    acc = x.double().cpu() @ w.double().cpu().T
+    acc = product64(x, w)
     q = plain_rope(acc[:, :n_heads * hd].view(M, n_heads, hd), positions.cpu(), inv_freq.cpu(), "interleaved")
     kk = plain_rope(acc[:, n_heads * hd:(n_heads + n_kv) * hd].view(M, n_kv, hd), positions.cpu(), inv_freq.cpu(), "interleaved")
     v = acc[:, (n_heads + n_kv) * hd:].view(M, n_kv, hd)
@@ -1528,8 +1534,8 @@ def test_gemm_finishes_a_norm_left_to_it(M, N, K, epi):
     h, y, sums = _left_for_norm(M, K, 40, nw)
     w = rnd((N, K), torch.bfloat16, 42, 0.1)
     inv = 1.0 / torch.sqrt((h.double().cpu() ** 2).sum(-1, keepdim=True) / K + eps)
-    acc = (y.double().cpu() @ w.double().cpu().T) * inv
-    other = plain_rmsnorm(h.double().cpu(), nw.double().cpu(), eps).bfloat16().double() @ w.double().cpu().T
+    acc = product64(y, w) * inv
+    other = product64(plain_rmsnorm(h.double().cpu(), nw.double().cpu(), eps).bfloat16().to(DEV), w)
     floor = 1e-5 * math.sqrt(K)
     if epi == EPI_STORE:
         out, ref, odt = torch.zeros((M, N), dtype=torch.bfloat16, device=DEV), acc, torch.bfloat16
@@ -1571,7 +1577,7 @@ def test_residual_product_leaves_what_the_next_norm_needs(M, N, K):
     w = rnd((N, K), torch.bfloat16, 51, 0.1)
     h = rnd((M, N), torch.float32, 52, 2.0)
     nw = rnd((N,), torch.float32, 53) * 0.1 + 1
-    want_h = h.double().cpu() + a.double().cpu() @ w.double().cpu().T
+    want_h = h.double().cpu() + product64(a, w)
     sums = torch.full((M, parts), -1.0, dtype=torch.float32, device=DEV)
     y = torch.full((M, N + 4), 7.0, dtype=torch.bfloat16, device=DEV)
     plain = h.clone()
@@ -1682,7 +1688,7 @@ def test_split_residual_product_finishes_the_next_norm(M, N, K):
     assert (y[:, N:] == 7.0).all(), "padding touched"
     want_h = rnd((M, N), torch.float32, 72, 2.0).double().cpu()
     want_h[M // 2] *= 30.0
-    want_h += a.double().cpu() @ w.double().cpu().T
+    want_h += product64(a, w)
     assert float((h.double().cpu() - want_h).abs().max()) <= 1e-5 * math.sqrt(K) + 1e-5 * float(want_h.abs().max())
     normed = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
     k.rmsnorm(normed, h, nw, eps)

@@ -14,6 +14,7 @@ from typing import Dict, List
 import torch
 
 from llm_rs_amd import VivisunConfig, random_model_tensors, write_model_folder
+from kept_results import kept
 from plain_vivisun import bf16_rounding, plain_vivisun_logits
 
 
@@ -91,6 +92,7 @@ def make_folder(tmp_path, cfg: dict, seed: int = 0, change=None, name: str = "mo
     return folder
 
 
+@kept
 def reference(cfg: dict, tensors, requests: Dict[str, List[int]], rnd=None):
     kw = {} if rnd is None else {"rnd": rnd}
     return {rid: plain_vivisun_logits(cfg, tensors, toks, **kw) for rid, toks in requests.items()}
