@@ -138,12 +138,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     const int full = (unsigned)K / KB;
     // A block's walk along k begins at a k-block of its own and wraps round: rows are a multiple of the memory channels'
     // interleave apart, so blocks in step would all ask the same few channels at once.  The start depends on the group of ROT
-    // features alone that the block's lie in, not on how many it takes: STEP times the group's number, modulo the k-blocks
+    // features alone that the block's lie in, not on how many it takes: `step` times the group's number, modulo the k-blocks
     // (by a product with `inv_full`, 2^32 / full rounded up: exact for what fits in 16 bits, and any start will do).
     int rot = 0;
     if constexpr (ROT > 0) {
-        constexpr unsigned STEP = ROT == 112 && sizeof(T) == 2 ? 1u : 37u;      // (28672 x 4096 bfloat16 at 1 row: 40.3 us with 1, 46.5 with 37; 6144 x 4096 13.9 and 12.6)
-        unsigned start = (unsigned)n0 / ROT * STEP & 0xffffu;
+        // (Of groups of 112 features, rows that are no multiple of 16 KB want neighbours a k-block apart: with 1 in place of 37, up to 8 rows of 18944 to
+        // 57344 x 4096 in bfloat16 and x 2048 in 32-bit take 0.86-0.91 of the time, 37888 x 2048 or 28672 x 3072 the same; rows of 16 KB 1.08-1.16
+        // of it.  Smaller groups of rows of 16 KB: 4096 x 8192 in bfloat16 1.11, in 32-bit 1.24; of 8 KB 0.97-1.02.)
+        const unsigned step = ROT == 112 && (unsigned)K % (16384 / sizeof(T)) != 0 ? 1u : 37u;
+        unsigned start = (unsigned)n0 / ROT * step & 0xffffu;
         rot = full > 1 ? (int)(start - __umulhi(start, inv_full) * (unsigned)full) : 0;
     }
     // This wave's k-blocks, the wave + NW i'th of the walk, through a ring of R places of its own: R - 1 of them on their way.

@@ -781,6 +781,17 @@ def test_gemm_short_rows_of_many_features_take_no_deep_ring(dtype, M, N, K):
     assert min(a / b for a, b in times) <= 1.35, times
 
 
+def test_gemm_rows_of_16_kb_ask_all_channels():
+    """8 rows of a wide bfloat16 weight whose rows are 16 KB: no longer than with rows a k-block shorter (0.96 of the time; with walks along k
+    that began a k-block apart 1.14)."""
+    k, calls = kernels(), []
+    for K in (8192, 8128):
+        a, ws, out = rnd((8, K), torch.bfloat16, 3), [rnd((24576, K), torch.bfloat16, i, 0.1) for i in range(3)], torch.zeros((8, 24576), dtype=torch.bfloat16, device=DEV)
+        calls.append(lambda a=a, ws=ws, out=out: [k.gemm(a, w, out, EPI_STORE) for w in ws])
+    times = [replay_time(*calls) for _ in range(3)]
+    assert min(a / b for a, b in times) <= 1.05, times
+
+
 @pytest.mark.parametrize("N,K", [(14336, 3584), (13824, 2560)])
 def test_gemm_48_rows_of_many_features_take_the_tiles(N, K):
     """48 rows may go to the ring in LDS or to tiles with k split, 64 of such weights go to the tiles: 48 take no longer than 64, with
