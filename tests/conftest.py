@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -21,6 +22,13 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+def pytest_collection_finish(session):
+    """What importing and collecting left is no garbage to come: a recording of a step collects garbage first, a twentieth of a second
+    each time with all of that to look through, and the tests make thousands of recordings."""
+    gc.collect()
+    gc.freeze()
 
 
 def pytest_terminal_summary(terminalreporter):
