@@ -892,85 +892,80 @@ static int launch_pingpong(hipStream_t stream, const bf16* A, int lda, const bf1
 // tiled, four waves: for K % 64 == 0, tiles of 256 x 256, 256 x 192 and 256 x 128.
 // One wave per SIMD with a tile of 128 x 128 outputs, all of them in the accumulation registers (256 of them):
 // a third fewer LDS reads per MFMA than the eight-wave tiles, and nothing shares the SIMD with the wave, so the
-// loop is written so that the wave itself always has work in flight.  A k-tile of 64 is four steps of 16; each
-// step asks LDS for the operands of the next step, moves a quarter of the next k-tile from registers into the
-// other LDS buffer, asks memory for the same quarter of the k-tile after that, and multiplies the operands the
-// step before it asked for.  Loads from memory pass through registers here, two k-tiles ahead of their use (the
+// loop is written so that the wave itself always has work in flight.  A k-tile of 64 is four steps, half of its k times half of the
+// wave's tokens each; a step asks LDS for operands of the next one, moves a quarter of the next k-tile from registers into the
+// other LDS buffer, asks memory for the same quarter of the k-tile after that, and multiplies the operands
+// asked for before.  Loads from memory pass through registers here, two k-tiles ahead of their use (the
 // loads straight into LDS of the loops above hold a wave that has no partner on its SIMD up while the memory
 // pipeline takes them).  The barrier between k-tiles stands before the last step's products, which run on
-// registers read before it: the matrix cores work across the barrier.  Same LDS layout and order of sums as the
-// loops above: bitwise the same results.  The epilogue is a template argument: with all of them in one kernel the
+// registers read before it: the matrix cores work across it.  Same LDS layout as the loops above, and a sum's products are added in
+// the order of k as there: bitwise the same results.  The epilogue is a template argument: with all of them in one kernel the
 // compiler keeps a tile's 256 sums and every epilogue's temporaries alive together and spills.
-// (Measured on MI355X, 2048 x 4096 times 24576 features with the gate/up epilogue: 320 us, 1.29 PFLOP/s; the
-// eight waves in two groups 372-376.  The clock follows the power that the matrix cores draw: their MFMAs alone, on
-// random operands, would take 241.)
+// What bounds it: the clock, which follows the power that the matrix cores and LDS draw.  v_mfma_f32_16x16x32_bf16 with features as its rows (a lane
+// then ends with four consecutive features of a token, so gated pairs need no neighbour and results go out by whole lines)
+// against v_mfma_f32_32x32x16_bf16 with results stored from where they lay, us: 2048 rows 57344 x 8192 gated 1381 -> 1338 (1.44
+// PFLOP/s), 8192 x 28672 added to 723 -> 697, 4096 x 14336 213 -> 206, 4096 x 4096 69.7 -> 64.8, 6144 x 4096 85.7 -> 82.1; 2032 rows
+// 16384 x 2048 gated 113.5 -> 106.3; 571 rows 18112 x 128 added to 29.4 -> 19.3.  The one shape found slower: 1360 rows 3040 x 9152 gated, 144 blocks, 96 -> 101.
 // ---------------------------------------------------------------------------
-// What a wave of the four-wave tile does with its sums: one band of 32 rows at a time.  16-bit results go through
-// the wave's own part of LDS and leave as whole rows of the band, 16 bytes a lane; the 32-bit epilogues read and
-// write memory directly (a lane half holds 32 consecutive columns of a row: whole lines).
+// What a wave of the four-wave tile does with its sums.  acc[i][j] are 16 tokens x 16 features, and a lane holds four consecutive
+// features of one token: a gated pair lies in one lane.  32-bit results leave by bands_to_f32; 16-bit ones likewise, a band of 32 tokens
+// at a time, as whole rows of the band, 16 bytes a lane.
 // epi: the epilogue's number as the caller gave it (EPI with its slot, where it has one)
 template <int BM, int BN, int EPI>
-__device__ __forceinline__ void band_epilogue(f32x16 (&acc)[BM / 64][BN / 64], unsigned char* smem, void* __restrict__ out,
+__device__ __forceinline__ void band_epilogue(f32x4 (&acc)[BM / 32][BN / 32], unsigned char* smem, void* __restrict__ out,
                                               int ldc, int M, int N, int m0, int n0, int epi) {
-    constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 32, FN = TN / 32;
+    constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int wm = wave / 2, wn = wave % 2;
-    int c = lane & 31, hh = lane >> 5;
     if constexpr (EPI == LLMRS_EPI_ACCUM_F32 || EPI == LLMRS_EPI_STORE_F32) {
-        float* o = (float*)out;
-        static_for<0, FM * FN>([&](auto idx) {
-            constexpr int i = decltype(idx)::value / FN, j = decltype(idx)::value % FN;
-            int n = n0 + wn * TN + j * 32 + c;
-            float old[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int m = m0 + wm * TM + i * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                old[r] = EPI == LLMRS_EPI_ACCUM_F32 ? o[(size_t)min(m, M - 1) * ldc + min(n, N - 1)] : 0.0f;
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int m = m0 + wm * TM + i * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                if (m < M && n < N) o[(size_t)m * ldc + n] = old[r] + acc[i][j][r];
-            }
-            __builtin_amdgcn_sched_barrier(0);       // one part of the tile at a time: its old values are not asked for earlier
-        });
+        bands_to_f32<FM, FN, false>(smem + wave * (16 * (TN * 4 + 16)), (float*)out, ldc, M, N, m0 + wm * TM, n0 + wn * TN, EPI == LLMRS_EPI_ACCUM_F32,
+                                    [&](auto ic, auto jc) { return acc[decltype(ic)::value][decltype(jc)::value]; });
     } else {
+        int token = lane & 15, four = (lane >> 4) * 4;
         constexpr bool glu = EPI == LLMRS_EPI_SWIGLU || EPI == LLMRS_EPI_GLU_CLAMP;
         const GatedAct ga = gated_act_of(EPI == LLMRS_EPI_GLU_CLAMP ? epi : EPI);
         constexpr int cols = glu ? TN / 2 : TN;      // columns of the wave's band as stored
-        constexpr int row_bytes = cols * 2;
-        unsigned char* mine = smem + wave * (32 * TN * 2);
-        constexpr int pieces_per_row = cols / 8;     // 16-byte pieces in a row of the band
+        constexpr int row_bytes = cols * 2 + 16;
+        unsigned char* mine = smem + wave * (32 * row_bytes);
+        constexpr int pieces_per_row = cols / 8, PIECES = 32 * pieces_per_row / 64;     // 16-byte pieces: in a row of the band, of a lane
+        static_assert(32 * pieces_per_row % 64 == 0, "a band is the same number of pieces for every lane");
         int n_first = glu ? (n0 + wn * TN) / 2 : n0 + wn * TN, n_lim = glu ? N / 2 : N;
-        const bool odd = lane & 1;
-        static_for<0, FM>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            static_for<0, FN>([&](auto jc) {
-                constexpr int j = decltype(jc)::value;
-                int cc = j * 32 + c;
+        auto write = [&](auto bandc) {
+            static_for<0, 2 * FN>([&](auto jc) {
+                constexpr int half = decltype(jc)::value / FN, j = decltype(jc)::value % FN;
+                f32x4 v = acc[2 * decltype(bandc)::value + half][j];
+                unsigned char* at = mine + (half * 16 + token) * row_bytes;
+                if constexpr (glu) {
+                    bf16x2 two;
+                    two[0] = (bf16)gated_act_fast(ga, v[0], v[1]);
+                    two[1] = (bf16)gated_act_fast(ga, v[2], v[3]);
+                    *(bf16x2*)(at + j * 16 + four) = two;
+                } else {
+                    bf16x4 o4;
 #pragma unroll
-                for (int r = 0; r < 16; r += 2) {                 // (pairs of lanes trade values as in tile_epilogue)
-                    int row = 8 * (r >> 2) + 4 * hh + (r & 3) + (odd ? 1 : 0);
-                    float v0 = acc[i][j][r], v1 = acc[i][j][r + 1];
-                    float got = swap_neighbours(odd ? v0 : v1);
-                    float left = odd ? got : v0, right = odd ? v1 : got;
-                    if (glu) *(bf16*)(mine + row * row_bytes + (cc / 2) * 2) = (bf16)gated_act_fast(ga, left, right);
-                    else {
-                        bf16x2 two;
-                        two[0] = (bf16)left;
-                        two[1] = (bf16)right;
-                        *(bf16x2*)(mine + row * row_bytes + (cc & ~1) * 2) = two;
-                    }
+                    for (int r = 0; r < 4; ++r) o4[r] = (bf16)v[r];
+                    *(bf16x4*)(at + (j * 16 + four) * 2) = o4;
                 }
             });
-            __builtin_amdgcn_s_waitcnt(0xc07f);                   // lgkmcnt(0): the wave's own LDS writes are done
-            for (int piece = lane; piece < 32 * pieces_per_row; piece += 64) {
-                int row = piece / pieces_per_row, lc = (piece % pieces_per_row) * 8;
-                int m = m0 + wm * TM + i * 32 + row;
-                if (m < M && n_first + lc < n_lim)                // (n_lim is a multiple of 8: a lane's 8 columns are in or out together)
-                    *(bf16x8*)((bf16*)out + (size_t)m * ldc + n_first + lc) = *(const bf16x8*)(mine + row * row_bytes + lc * 2);
+        };
+        write(std::integral_constant<int, 0>{});
+        static_for<0, FM / 2>([&](auto ic) {
+            constexpr int band = decltype(ic)::value;
+            bf16x8 v[PIECES];
+            asm volatile("" ::: "memory");           // (a wave's LDS accesses are carried out in the order it asks for them)
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) {
+                int piece = p * 64 + lane;
+                v[p] = *(const bf16x8*)(mine + piece / pieces_per_row * row_bytes + piece % pieces_per_row * 16);
             }
-            __builtin_amdgcn_s_waitcnt(0xc07f);                   // the band's rows are read before the next band overwrites them
+            asm volatile("" ::: "memory");
+            if constexpr (band + 1 < FM / 2) write(std::integral_constant<int, band + 1>{});
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) {
+                int piece = p * 64 + lane, m = m0 + wm * TM + band * 32 + piece / pieces_per_row, lc = piece % pieces_per_row * 8;
+                if (m < M && n_first + lc < n_lim)                // (n_lim is a multiple of 8: a lane's 8 columns are in or out together)
+                    *(bf16x8*)((bf16*)out + (size_t)m * ldc + n_first + lc) = v[p];
+            }
             __builtin_amdgcn_sched_barrier(0);
         });
     }
@@ -982,35 +977,16 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int first_of(int groups, int q) { return q * groups / 4; }
 constexpr int quarter_of(int groups, int q) { return first_of(groups, q + 1) - first_of(groups, q); }
 
-// Which tile of the output a block works on.  Blocks go to the eight XCDs in turn; here an XCD gets a stretch of the tiles
-// that lie one after the other, eight rows of tiles at a time, column after column, so that the 32 blocks its units run at
-// once are eight rows of four columns: each brings its rows of the weight into one L2, once, and shares them with seven
-// others.  (Column after column over all XCDs, a grid of 224 columns gave an XCD 28 of them at once, each for one
-// block: 2048 x 8192 times 57344 features 1773 -> 1473 us, 24576 x 4096 the same.)
-// With rows shorter than 1024 the weight's bytes are few beside the results', and those are written faster as the grid counts its
-// tiles (8192 x 128 times 28672 gated features 157 -> 145 us, 8192 x 256 added to 4096 100 -> 94; 8192 x 512
-// times 8192 88 -> 83; with k of 128 and 16-bit results 1 % slower).
-__device__ __forceinline__ void tile_of_block(int K, int& row, int& column) {
-    row = blockIdx.y;
-    column = blockIdx.x;
-    if (K < 1024) return;
-    int columns = gridDim.x, rows = gridDim.y, id = blockIdx.y * columns + blockIdx.x, share = columns * rows / 8;
-    if (id < 8 * share) id = (id & 7) * share + (id >> 3);         // (what is left over when they do not divide by eight: as it comes)
-    int band = id / (8 * columns), within = id - band * 8 * columns, high = min(8, rows - 8 * band);
-    row = 8 * band + within % high;
-    column = within / high;
-}
-
 template <int BM, int BN, int EPI>
 __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
                                                             void* __restrict__ out, int ldc, int M, int N, int K, int epi) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char fw_smem[];
     constexpr int WAVES = 4;
-    constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 32, FN = TN / 32;
+    constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16, FNH = (FN + 1) / 2;
     constexpr int STAGE_BYTES = (BM + BN) * 128;
     constexpr int A_GROUPS = BM / 8 / WAVES, W_GROUPS = BN / 8 / WAVES;   // 8-row groups per wave
-    static_assert(BM == 256 && BN % 64 == 0 && FM * FN <= 16, "a wave's sums fill at most the 256 accumulation registers");
-    static_assert(32 * TN * 2 * WAVES <= 2 * STAGE_BYTES, "the waves' bands must fit in the tile buffers");
+    static_assert(BM == 256 && BN % 32 == 0 && FM * FN <= 64, "a wave's sums fill at most the 256 accumulation registers");
+    static_assert(32 * (TN * 2 + 16) * WAVES <= 2 * STAGE_BYTES && 16 * (TN * 4 + 16) * WAVES <= 2 * STAGE_BYTES, "the waves' bands must fit in the tile buffers");
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int wm = wave / 2, wn = wave % 2;
     int tile_row, tile_column;
@@ -1067,97 +1043,108 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
 #pragma unroll
         for (int i = first_of(W_GROUPS, q); i < first_of(W_GROUPS, q + 1); ++i) *(u32x4*)(st + BM * 128 + (wave * W_GROUPS + i) * 1024 + lane * 16) = sw_[i];
     };
-    f32x16 acc[FM][FN];
+    f32x4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    int frow = lane & 31, h = lane >> 5;
+        for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int frow = lane & 15, h = lane >> 4;
     int sw = (frow >> 1) & 7;
-    // LDS offsets of this lane's chunk for each of a tile's four k-steps (row tiles lie 4 KB apart)
-    unsigned offa[4], offb[4];
+    // LDS offsets of this lane's chunk for each half of a k-tile, 32 k long (row tiles lie 2 KB apart)
+    unsigned offa[2], offb[2];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        unsigned chunk = (unsigned)(((ks * 2 + h) ^ sw) * 16);
+    for (int ks = 0; ks < 2; ++ks) {
+        unsigned chunk = (unsigned)(((ks * 4 + h) ^ sw) * 16);
         offa[ks] = (wm * TM + frow) * 128 + chunk;
         offb[ks] = BM * 128 + (wn * TN + frow) * 128 + chunk;
     }
-    bf16x8 fa[2][FM], fb[2][FN];
-    auto read = [&](int kt, auto ksc, auto bufc) {
-        constexpr int ks = decltype(ksc)::value, buf = decltype(bufc)::value;
+    bf16x8 fa[FM], fb[2][FN];
+    auto read_a = [&](int kt, auto ksc, auto halfc) {
+        constexpr int ks = decltype(ksc)::value, half = decltype(halfc)::value;
         const unsigned char* st = fw_smem + (kt & 1) * STAGE_BYTES;
 #pragma unroll
-        for (int i = 0; i < FM; ++i) fa[buf][i] = *(const bf16x8*)(st + offa[ks] + i * 32 * 128);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) fb[buf][j] = *(const bf16x8*)(st + offb[ks] + j * 32 * 128);
+        for (int i = half * FM / 2; i < (half + 1) * FM / 2; ++i) fa[i] = *(const bf16x8*)(st + offa[ks] + i * 16 * 128);
     };
-    auto mult = [&](auto bufc) {
-        constexpr int buf = decltype(bufc)::value;
+    auto read_b = [&](int kt, auto ksc, auto halfc) {
+        constexpr int ks = decltype(ksc)::value, half = decltype(halfc)::value;
+        const unsigned char* st = fw_smem + (kt & 1) * STAGE_BYTES;
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int j = half * FNH; j < (half ? FN : FNH); ++j) fb[ks][j] = *(const bf16x8*)(st + offb[ks] + j * 16 * 128);
+    };
+    auto mult = [&](auto ksc, auto halfc) {
+        constexpr int ks = decltype(ksc)::value, half = decltype(halfc)::value;
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[buf][i], fb[buf][j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int i = half * FM / 2; i < (half + 1) * FM / 2; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[ks][j], fa[i], acc[i][j], 0, 0, 0);
     };
     // The order within a step.  A SIMD has this one wave only, so whatever keeps it from issuing its next MFMA leaves the matrix
-    // cores idle: four loads asked for back to back wait for each other and the other waves' at the address unit (16 cycles
-    // each, 16 of them between the four waves) while an MFMA takes 32.  So LDS reads go out in pairs, and every LDS write
-    // and every load from memory by itself, with an MFMA after each.  Measured (2048 rows, back to back, before: all reads, 4
-    // MFMAs, all writes, 4 MFMAs, all loads): 24576 x 4096 350 -> 320 us, 4096 x 14336 232 -> 212, 4096 x 4096 77 -> 70;
-    // reads singly 331, in fours 324, writes and loads of a quarter as groups 331, loads first 357.
-    auto order = [](auto qc) {
-        constexpr int q = decltype(qc)::value, LOADS = quarter_of(A_GROUPS, q) + quarter_of(W_GROUPS, q);
-        static_for<0, (FM + FN) / 2>([](auto) {
+    // cores idle: loads asked for back to back wait for each other and the other waves' at the address unit (16 cycles
+    // each, 16 of them between the four waves), and an MFMA takes 16.  So LDS reads go out in pairs, and every LDS write
+    // and every load from memory by itself, with MFMAs after each.  A step's reads are half of the tokens' operands and half of the
+    // features', the same number in every step: with all of the tokens' in one step of two LDS is asked for more than it gives in that step.  (57344 x
+    // 8192: other numbers of MFMAs after a read, a write and a load within 2 %; reads singly or in fours 1-3 % slower.)
+    auto order = [](auto qc, auto readsc, auto multsc) {
+        constexpr int q = decltype(qc)::value, LOADS = quarter_of(A_GROUPS, q) + quarter_of(W_GROUPS, q), READS = decltype(readsc)::value, MULTS = decltype(multsc)::value;
+        constexpr int after = MULTS >= READS + 3 * LOADS ? 2 : 1;
+        static_for<0, READS / 2>([](auto) {
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, after, 0);
         });
         static_for<0, LOADS>([](auto) {
             __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
         });
-        __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);
-    };
-    // One step (a quarter of a k-tile).  While k-tile kt is multiplied, k-tile kt + 1 goes from registers into the
-    // other LDS buffer and k-tile kt + 2 is asked for into the registers that frees.  A quarter written now was
-    // asked for a k-tile ago; loads complete in order, so it is there when all but the three other quarters, asked for
-    // since, have completed.
-    auto step = [&](int kt, auto ksc, auto qc, auto rbuf, auto mbuf, auto multiply) {
-        read(kt, ksc, rbuf);
-        constexpr int q = decltype(qc)::value, others = A_GROUPS + W_GROUPS - quarter_of(A_GROUPS, q) - quarter_of(W_GROUPS, q);
-        wait_vmcnt<others>();
-        put(kt + 1, qc);
-        ask(kt + 2, qc);
-        if constexpr (decltype(multiply)::value) mult(mbuf);
-        order(qc);
-        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_group_barrier(0x008, MULTS, 0);
     };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
     using I3 = std::integral_constant<int, 3>;
+    // One step (a quarter of a k-tile: half of its k times half of the wave's tokens).  While k-tile kt is multiplied, k-tile kt + 1 goes
+    // from registers into the other LDS buffer and k-tile kt + 2 is asked for into the registers that frees.  A quarter written now was
+    // asked for a k-tile ago; loads complete in order, so it is there when all but the three other quarters, asked for
+    // since, have completed.
+    auto step = [&](int kt, auto qc, auto multiply) {
+        constexpr int q = decltype(qc)::value;
+        using KS = std::integral_constant<int, q / 2>;
+        using Odd = std::integral_constant<int, q % 2>;
+        if constexpr (q % 2 == 0) read_a(kt, KS{}, I0{});
+        read_b(kt, KS{}, Odd{});
+        if constexpr (q % 2 == 1) read_a(kt, KS{}, I1{});
+        constexpr int others = A_GROUPS + W_GROUPS - quarter_of(A_GROUPS, q) - quarter_of(W_GROUPS, q);
+        wait_vmcnt<others>();
+        put(kt + 1, qc);
+        ask(kt + 2, qc);
+        if constexpr (decltype(multiply)::value) {
+            using MK = std::integral_constant<int, q == 0 ? 1 : (q - 1) / 2>;
+            mult(MK{}, std::integral_constant<int, 1 - q % 2>{});
+        }
+        order(qc, std::integral_constant<int, FM / 2 + (q & 1 ? FN - FNH : FNH)>{}, std::integral_constant<int, FM / 2 * FN>{});
+        __builtin_amdgcn_sched_barrier(0);
+    };
     // k-tile 0 into LDS, k-tile 1 into registers
     ask(0, I0{}); ask(0, I1{}); ask(0, I2{}); ask(0, I3{});
     wait_vmcnt<0>();
     put(0, I0{}); put(0, I1{}); put(0, I2{}); put(0, I3{});
     ask(1, I0{}); ask(1, I1{}); ask(1, I2{}); ask(1, I3{});
     __syncthreads();               // (waits for the loads of k-tile 1 as well: once)
-    // A step multiplies the operands that the step before it read; the last step's products of a k-tile run in the
+    // A step multiplies the operands that the steps before it read, and the second half of the features' that it reads itself; the last step's products of a k-tile run in the
     // first step of the next, on operands read before the barrier: the matrix cores work across it.
     auto k_tile = [&](int kt, auto not_first) {
-        step(kt, I0{}, I0{}, I0{}, I1{}, not_first);
-        step(kt, I1{}, I1{}, I1{}, I0{}, std::true_type{});
-        step(kt, I2{}, I2{}, I0{}, I1{}, std::true_type{});
-        step(kt, I3{}, I3{}, I1{}, I0{}, std::true_type{});
+        step(kt, I0{}, not_first);
+        step(kt, I1{}, std::true_type{});
+        step(kt, I2{}, std::true_type{});
+        step(kt, I3{}, std::true_type{});
         block_sync_lds();          // this wave's LDS reads and writes are done, and everybody's
         __builtin_amdgcn_sched_barrier(0);
     };
     k_tile(0, std::false_type{});
     for (int kt = 1; kt < nk; ++kt) k_tile(kt, std::true_type{});
-    mult(I1{});
+    mult(I1{}, I1{});
     wait_vmcnt<0>();
     __syncthreads();
     band_epilogue<BM, BN, EPI>(acc, fw_smem, out, ldc, M, N, m0, n0, epi);

@@ -574,6 +574,27 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
         assert (err <= out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))).all(), (epi, float(err.max()))
 
 
+@pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 2050, 4098, 64), (torch.bfloat16, 700, 6145, 128), (torch.bfloat16, 2048, 6148, 64),
+                                         (torch.float32, 300, 2050, 64), (torch.float32, 1030, 8196, 32), (torch.float32, 257, 1023, 96)])
+@pytest.mark.parametrize("pad,first", [(0, 0), (4, 4), (2, 2), (1, 1)])
+def test_gemm_tiles_write_32bit_rows_of_any_alignment(dtype, M, N, K, pad, first):
+    """32-bit results leave the tiles 16, 8 or 4 bytes a lane, as the rows' length, their stride and where the first one begins allow; added to
+    and stored, nothing beside them touched.  (Bound: sums of K products of 0.1, as in `test_gemm`.)"""
+    a, w = rnd((M, K), dtype, 3), rnd((N, K), dtype, 4, 0.1)
+    acc = product64(a, w)
+    floor = (2e-6 if dtype == torch.float32 else 1e-5) * math.sqrt(K)
+    for epi in (EPI_STORE_F32, EPI_ACCUM_F32):
+        flat = rnd((M * (N + pad) + 8,), torch.float32, 5)
+        before = flat.clone()
+        out = flat[first:first + M * (N + pad)].view(M, N + pad)[:, :N]
+        ref = acc + (out.double().cpu() if epi == EPI_ACCUM_F32 else 0.0)
+        kernels().gemm(a, w, out, epi)
+        err = (out.double().cpu() - ref).abs()
+        assert (err <= out_tol(ref, torch.float32, floor)).all(), float(err.max())
+        out.copy_(before[first:first + M * (N + pad)].view(M, N + pad)[:, :N])
+        assert torch.equal(flat, before)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(1, 40, 64), (8, 24, 96), (9, 250, 544), (16, 1990, 2048), (7, 2040, 2080), (16, 2048, 2592), (8, 3000, 2304), (13, 3080, 2176),
                                    (8, 6136, 2112), (16, 6150, 2048), (3, 16390, 288), (10, 16400, 2048), (8, 33000, 160), (5, 28650, 352), (11, 28672, 64), (8, 8200, 16448),
