@@ -977,16 +977,35 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int first_of(int groups, int q) { return q * groups / 4; }
 constexpr int quarter_of(int groups, int q) { return first_of(groups, q + 1) - first_of(groups, q); }
 
-template <int BM, int BN, int EPI>
+// TAIL: the `over` rows, up to 16, that follow the M whole tiles' rows.  A column of tiles has their 16 features of a wave's B operands in LDS
+// anyway, so its waves share those features out: a wave multiplies 16 more features by 16 more tokens, one MFMA for 64,
+// with the tokens straight from memory in the operand's layout, a k-tile ahead.  (A launch of their own reads the whole weight again:
+// 2064 rows 57344 x 8192 gated 1548 -> 1400 us, 2048 rows 1346; 8192 x 28672 added to 789 -> 698, 8192 x 8192 252 -> 210; 8208 rows 28672 x 4096
+// gated 1428 -> 1366.)
+template <int EPI>
+__device__ __forceinline__ void tail_epilogue(f32x4 v, void* __restrict__ out, int ldc, int N, int m, int n, int epi) {
+    if constexpr (EPI == LLMRS_EPI_SWIGLU || EPI == LLMRS_EPI_GLU_CLAMP) {
+        const GatedAct ga = gated_act_of(EPI == LLMRS_EPI_GLU_CLAMP ? epi : EPI);
+        bf16* o = (bf16*)out + (size_t)m * ldc + n / 2;
+        if (n + 1 < N) o[0] = (bf16)gated_act_fast(ga, v[0], v[1]);
+        if (n + 3 < N) o[1] = (bf16)gated_act_fast(ga, v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (n + r < N) epilogue_store<bf16>(EPI, out, ldc, m, n + r, v[r]);
+    }
+}
+
+template <int BM, int BN, int EPI, int TAIL>
 __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
-                                                            void* __restrict__ out, int ldc, int M, int N, int K, int epi) {
+                                                            void* __restrict__ out, int ldc, int M, int N, int K, int epi, int over) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char fw_smem[];
     constexpr int WAVES = 4;
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16, FNH = (FN + 1) / 2;
     constexpr int STAGE_BYTES = (BM + BN) * 128;
     constexpr int A_GROUPS = BM / 8 / WAVES, W_GROUPS = BN / 8 / WAVES;   // 8-row groups per wave
     static_assert(BM == 256 && BN % 32 == 0 && FM * FN <= 64, "a wave's sums fill at most the 256 accumulation registers");
-    static_assert(32 * (TN * 2 + 16) * WAVES <= 2 * STAGE_BYTES && 16 * (TN * 4 + 16) * WAVES <= 2 * STAGE_BYTES, "the waves' bands must fit in the tile buffers");
+    static_assert(32 * (TN * 2 + 16) * WAVES <= STAGE_BYTES && 16 * (TN * 4 + 16) * WAVES <= STAGE_BYTES, "the waves' bands must fit in one of the tile buffers");
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int wm = wave / 2, wn = wave % 2;
     int tile_row, tile_column;
@@ -1019,7 +1038,7 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         for (int i = 0; i < W_GROUPS; ++i) ow[i] += k_first * 128;
     }
 #if defined(__HIP_DEVICE_COMPILE__)
-    __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)min((size_t)M * lda * 2, (size_t)0xffffffffu), 0x00020000);
+    __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)min((size_t)(M + (TAIL != 0 ? over : 0)) * lda * 2, (size_t)0xffffffffu), 0x00020000);
     __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)min((size_t)N * K * 2, (size_t)0xffffffffu), 0x00020000);
 #endif
     u32x4 sa[A_GROUPS], sw_[W_GROUPS];          // the k-tile on its way, in registers
@@ -1079,6 +1098,42 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
             for (int i = half * FM / 2; i < (half + 1) * FM / 2; ++i)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[ks][j], fa[i], acc[i][j], 0, 0, 0);
     };
+    // The tail's features of this wave: the 16 from 16 * part on.  TAIL == 1 (a column has at least FN tiles): every tile takes a part of each
+    // of its halves, and the two waves of a half take a half of every k-tile each.  TAIL == 2 (at least FN / 2): a wave takes a part
+    // and all of k.  Tiles past the last part multiply it once more and store nothing.
+    constexpr int TK = TAIL == 2 ? 2 : 1;
+    const int my_part = TAIL == 2 ? 2 * tile_row + wm : tile_row, part = min(my_part, FN - 1);
+    unsigned offt = 0, offp = 0;
+    u32x4 ta[TK];
+    bf16x8 tb[TK];
+    f32x4 tails[TK];
+#pragma unroll
+    for (int ks = 0; ks < TK; ++ks) tails[ks] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (TAIL != 0) {
+        offt = (unsigned)(((size_t)(M + min(frow, over - 1)) * lda + h * 8) * 2 + (TAIL == 1 ? wm * 64 : 0));
+        offp = (TAIL == 1 && wm ? offb[1] : offb[0]) + part * 16 * 128;
+    }
+    auto ask_tail = [&](int kt) {
+        kt = min(kt, nk - 1);
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+        for (int ks = 0; ks < TK; ++ks) ta[ks] = __builtin_amdgcn_raw_buffer_load_b128(ra, offt + ks * 64, kt * 128, 0);
+#endif
+    };
+    auto read_tail = [&](int kt) {
+        const unsigned char* st = fw_smem + (kt & 1) * STAGE_BYTES;
+#pragma unroll
+        for (int ks = 0; ks < TK; ++ks) tb[ks] = *(const bf16x8*)(st + (offp ^ (ks * 64)));     // (the other half of k: its chunk's bit 2 the other way)
+    };
+    // (The tile's sums fill the accumulation registers; left to the compiler the tail's would push some of them out and in again in every
+    // k-tile, with waits for their MFMAs: 57344 x 8192 gated at 2064 rows 1446 us against 1400.  Written out they stay in ordinary registers.  The next
+    // that reads a result is a k-tile, or at the end a half of one, later: no wait states of its own are owed.)
+    auto mult_tail = [&]() {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+        for (int ks = 0; ks < TK; ++ks) asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(tails[ks]) : "v"(tb[ks]), "v"(ta[ks]));
+#endif
+    };
     // The order within a step.  A SIMD has this one wave only, so whatever keeps it from issuing its next MFMA leaves the matrix
     // cores idle: loads asked for back to back wait for each other and the other waves' at the address unit (16 cycles
     // each, 16 of them between the four waves), and an MFMA takes 16.  So LDS reads go out in pairs, and every LDS write
@@ -1091,6 +1146,10 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         static_for<0, READS / 2>([](auto) {
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, after, 0);
+        });
+        if constexpr (TAIL != 0 && q == 2) static_for<0, TK>([](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
         });
         static_for<0, LOADS>([](auto) {
             __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
@@ -1115,6 +1174,8 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         if constexpr (q % 2 == 0) read_a(kt, KS{}, I0{});
         read_b(kt, KS{}, Odd{});
         if constexpr (q % 2 == 1) read_a(kt, KS{}, I1{});
+        if constexpr (TAIL != 0 && q == 1) read_tail(kt);
+        if constexpr (TAIL != 0 && q == 2) { mult_tail(); ask_tail(kt + 1); }
         constexpr int others = A_GROUPS + W_GROUPS - quarter_of(A_GROUPS, q) - quarter_of(W_GROUPS, q);
         wait_vmcnt<others>();
         put(kt + 1, qc);
@@ -1123,7 +1184,8 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
             using MK = std::integral_constant<int, q == 0 ? 1 : (q - 1) / 2>;
             mult(MK{}, std::integral_constant<int, 1 - q % 2>{});
         }
-        order(qc, std::integral_constant<int, FM / 2 + (q & 1 ? FN - FNH : FNH)>{}, std::integral_constant<int, FM / 2 * FN>{});
+        order(qc, std::integral_constant<int, FM / 2 + (q & 1 ? FN - FNH : FNH) + (TAIL != 0 && q == 1 ? TK : 0)>{},
+              std::integral_constant<int, FM / 2 * FN>{});
         __builtin_amdgcn_sched_barrier(0);
     };
     // k-tile 0 into LDS, k-tile 1 into registers
@@ -1131,6 +1193,7 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
     wait_vmcnt<0>();
     put(0, I0{}); put(0, I1{}); put(0, I2{}); put(0, I3{});
     ask(1, I0{}); ask(1, I1{}); ask(1, I2{}); ask(1, I3{});
+    if constexpr (TAIL != 0) ask_tail(0);
     __syncthreads();               // (waits for the loads of k-tile 1 as well: once)
     // A step multiplies the operands that the steps before it read, and the second half of the features' that it reads itself; the last step's products of a k-tile run in the
     // first step of the next, on operands read before the barrier: the matrix cores work across it.
@@ -1148,6 +1211,18 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
     wait_vmcnt<0>();
     __syncthreads();
     band_epilogue<BM, BN, EPI>(acc, fw_smem, out, ldc, M, N, m0, n0, epi);
+    if constexpr (TAIL != 0) {
+        f32x4 tail = tails[0];
+        if constexpr (TAIL == 2) tail += tails[TK - 1];
+        if constexpr (TAIL == 1) {             // the halves of k together, through LDS behind what the bands used
+            f32x4* halves = (f32x4*)(fw_smem + STAGE_BYTES) + wn * 64 + lane;
+            if (wm == 1) *halves = tail;
+            __syncthreads();
+            if (wm == 0) tail += *halves;
+        }
+        if (my_part < FN && (TAIL == 2 || wm == 0) && frow < over)
+            tail_epilogue<EPI>(tail, out, ldc, N, M + frow, n0 + wn * TN + part * 16 + h * 4, epi);
+    }
 }
 
 // Whether the four-wave tiles can finish this product: the epilogues it has, 16-bit results as whole 16-byte pieces.
@@ -1157,30 +1232,38 @@ static bool fourwave_takes(int epi, const void* out, int ldc, int N) {
     if (epi_gated(epi)) return ldc % 8 == 0 && ((uintptr_t)out & 15) == 0 && N % 16 == 0;
     return false;
 }
-template <int BM, int BN, int EPI>
-static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1) {
+// over: rows of A and out beyond the M (whole tiles, at least four) that the tiles take along; 0 or, without splits, up to 16
+template <int BM, int BN, int EPI, int TAIL = 0>
+static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1, int over = 0) {
+    if constexpr (TAIL == 0) {
+        if (over > 0 && M >= BM * (BN / 32)) return launch_fourwave_epi<BM, BN, EPI, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, over);
+        if constexpr (BN > 128)                     // (four tiles are a part for every wave pair of the narrow ones)
+            if (over > 0) return launch_fourwave_epi<BM, BN, EPI, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, over);
+    }
     static bool configured = false;
     size_t bytes = (size_t)2 * (BM + BN) * 128;
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_fourwave_kernel<BM, BN, EPI>,
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_fourwave_kernel<BM, BN, EPI, TAIL>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) return llmrs_fail("gemm: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
         configured = true;
     }
     dim3 grid(ceil_div(N, BN), ceil_div(M, BM), splits);
     if (grid.y > 65535) return llmrs_fail("gemm: M=%d is too large for one launch", M);
-    gemm_fourwave_kernel<BM, BN, EPI><<<grid, 256, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi);
+    if (over > 0 && (over > 16 || splits != 1 || M % BM != 0 || TAIL * (int)grid.y < BN / 32))
+        return llmrs_fail("gemm: the four-wave tiles cannot take %d rows beyond M=%d along", over, M);
+    gemm_fourwave_kernel<BM, BN, EPI, TAIL><<<grid, 256, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, over);
     return 0;
 }
 // (operands under 4 GB each, K % 64 == 0, fourwave_takes(epi, ...): the caller's to check)
 template <int BM, int BN>
-static int launch_fourwave(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi) {
-    if (epi >= LLMRS_EPI_GLU_CLAMP) return launch_fourwave_epi<BM, BN, LLMRS_EPI_GLU_CLAMP>(stream, A, lda, W, out, ldc, M, N, K, epi);
+static int launch_fourwave(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int over = 0) {
+    if (epi >= LLMRS_EPI_GLU_CLAMP) return launch_fourwave_epi<BM, BN, LLMRS_EPI_GLU_CLAMP>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
     switch (epi) {
-        case LLMRS_EPI_STORE: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE>(stream, A, lda, W, out, ldc, M, N, K, epi);
-        case LLMRS_EPI_STORE_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE_F32>(stream, A, lda, W, out, ldc, M, N, K, epi);
-        case LLMRS_EPI_ACCUM_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_ACCUM_F32>(stream, A, lda, W, out, ldc, M, N, K, epi);
-        case LLMRS_EPI_SWIGLU: return launch_fourwave_epi<BM, BN, LLMRS_EPI_SWIGLU>(stream, A, lda, W, out, ldc, M, N, K, epi);
+        case LLMRS_EPI_STORE: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
+        case LLMRS_EPI_STORE_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE_F32>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
+        case LLMRS_EPI_ACCUM_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_ACCUM_F32>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
+        case LLMRS_EPI_SWIGLU: return launch_fourwave_epi<BM, BN, LLMRS_EPI_SWIGLU>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
         default: return llmrs_fail("gemm: the four-wave tiles have no epilogue %d", epi);
     }
 }
@@ -1424,7 +1507,18 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         // would cost another row of tiles in full: they go to the kernel for few rows instead,
         // which reads the weight once more at memory speed.
         int over = M % 256;
-        if (K % 64 == 0 && M >= 1024 && over > 0 && over <= 64 && (m_tiles - 1) * ceil_div(N, 256) >= 160) {
+        // Up to 16 of them go along with the four-wave tiles, where those take the product (2-4 % of the tiles' time, at 1032 to 8208 rows less
+        // than the few-row kernel's 8-14; beyond 256 x 128 tiles of fewer than 160 large ones both come to the same, and the few-row kernel stays).
+        // operands under 4 GB are read through buffer descriptors (32-bit offsets), 1-4 % faster
+        const bool small = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
+        const bool over_beside = K % 64 == 0 && M >= 1024 && over > 0 && over <= 64 && (m_tiles - 1) * ceil_div(N, 256) >= 160;
+        int along = 0;
+        if (over_beside && over <= 16 && small && fourwave_takes(epi, out, ldc, N)) {
+            along = over;
+            M -= over;
+            m_tiles -= 1;
+            big_tiles = m_tiles * ceil_div(N, 256);
+        } else if (over_beside) {
             size_t elt = (epi == LLMRS_EPI_STORE_F32 || epi == LLMRS_EPI_ACCUM_F32) ? sizeof(float) : sizeof(bf16);
             int whole_rows = M - over;
             rc = llmrs_gemm_bf16_mfma(stream, A, lda, W, out, ldc, whole_rows, N, K, epi, workspace, workspace_bytes, qkv);
@@ -1435,8 +1529,6 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         // (up to 128 rows a 256-row tile would be half empty; 257-384 rows are still faster on two rows of
         // large tiles than on three of small ones: the lm head at 300 rows 640 against 750 us)
         if (K % 64 == 0 && big_tiles >= 160 && M > 128) {
-            // operands under 4 GB are read through buffer descriptors (32-bit offsets), 1-4 % faster
-            const bool small = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
             // square tiles: four waves with 128 x 128 outputs each where their epilogues and loads allow, else the
             // eight waves in two groups
             const bool four = small && fourwave_takes(epi, out, ldc, N);
@@ -1451,24 +1543,30 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                 size_t elt = (epi == LLMRS_EPI_STORE_F32 || epi == LLMRS_EPI_ACCUM_F32) ? sizeof(float) : sizeof(bf16);
                 void* out_rest = (char*)out + (size_t)(epi_gated(epi) ? n_split / 2 : n_split) * elt;
                 rc = four && fourwave_takes(epi, out, ldc, n_split)
-                         ? launch_fourwave<256, 256>(stream, A, lda, W, out, ldc, M, n_split, K, epi)
+                         ? launch_fourwave<256, 256>(stream, A, lda, W, out, ldc, M, n_split, K, epi, along)
                      : small ? launch_pingpong<256, 256, 2, 4, true>(stream, A, lda, W, out, ldc, M, n_split, K, epi)
                              : launch_pingpong<256, 256, 2, 4, false>(stream, A, lda, W, out, ldc, M, n_split, K, epi);
                 if (rc == 0) {
                     if (four && fourwave_takes(epi, out_rest, ldc, N - n_split) && mid_tiles(M, N - n_split, K, epi, false).four)
-                        rc = launch_fourwave<256, 128>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
-                    else
+                        rc = launch_fourwave<256, 128>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi, along);
+                    else {
                         rc = launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
+                        if (rc == 0 && along > 0) {
+                            int took = llmrs_gemm_bf16_mfma(stream, A + (size_t)M * lda, lda, W + (size_t)n_split * K,
+                                                            (char*)out_rest + (size_t)M * ldc * elt, ldc, along, N - n_split, K, epi, nullptr, 0);
+                            if (took != 1) return took < 0 ? -1 : (llmrs_fail("gemm: nothing takes the last %d rows of N=%d K=%d", along, N, K), -1);
+                        }
+                    }
                 }
             } else if (long t192 = m_tiles * ceil_div(N, 192); rest > 0 && t192 % cus == 0) {
                 // 256 x 192 tiles where they come to whole rounds of the device and the square ones do not: the
                 // q/k/v product of the 8B shape at 2048 rows is 192 square tiles on 256 units, or 256 of these
                 // (four waves of 128 x 96: 87 us, against 100 for the eight waves of 64 x 96)
-                rc = four ? launch_fourwave<256, 192>(stream, A, lda, W, out, ldc, M, N, K, epi)
+                rc = four ? launch_fourwave<256, 192>(stream, A, lda, W, out, ldc, M, N, K, epi, along)
                    : small ? launch_pingpong<256, 192, 4, 2, true>(stream, A, lda, W, out, ldc, M, N, K, epi)
                            : launch_pingpong<256, 192, 4, 2, false>(stream, A, lda, W, out, ldc, M, N, K, epi);
             } else {
-                rc = four ? launch_fourwave<256, 256>(stream, A, lda, W, out, ldc, M, N, K, epi)
+                rc = four ? launch_fourwave<256, 256>(stream, A, lda, W, out, ldc, M, N, K, epi, along)
                      : small ? launch_pingpong<256, 256, 2, 4, true>(stream, A, lda, W, out, ldc, M, N, K, epi)
                              : launch_pingpong<256, 256, 2, 4, false>(stream, A, lda, W, out, ldc, M, N, K, epi);
             }
@@ -1477,15 +1575,15 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             // tiles that cost them another round of the device, or the split of k that filled it, go to the kernel
             // for few rows (the o and down products of the 8B shape: 2049 rows 526 -> about 350 us, 1025 rows 287 -> 240).
             // By the time of the plans for all rows and for the whole tiles' (us, mid_tiles).
+            auto plan_of = [&](int rows) {
+                MidTiles plan = mid_tiles(rows, N, K, epi);
+                if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < (size_t)plan.splits * rows * N * sizeof(float)))
+                    plan = mid_tiles(rows, N, K, epi, false);
+                return plan;
+            };
             int over128 = M % 128;
             if (M >= 1024 && over128 > 0 && over128 <= 64 && !whole && next == nullptr && scale == nullptr) {
-                auto walk = [&](int rows) {
-                    MidTiles plan = mid_tiles(rows, N, K, epi);
-                    if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < (size_t)plan.splits * rows * N * sizeof(float)))
-                        plan = mid_tiles(rows, N, K, epi, false);
-                    return plan.time;
-                };
-                if (walk(M) - walk(M - over128) >= 30.0) {
+                if (plan_of(M).time - plan_of(M - over128).time >= 30.0) {
                     size_t elt = (epi == LLMRS_EPI_STORE_F32 || epi == LLMRS_EPI_ACCUM_F32) ? sizeof(float) : sizeof(bf16);
                     int whole_rows = M - over128;
                     rc = llmrs_gemm_bf16_mfma(stream, A, lda, W, out, ldc, whole_rows, N, K, epi, workspace, workspace_bytes, qkv);
@@ -1495,15 +1593,12 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                 }
             }
             // (a wider tile brings less into a unit for the same work: a k-step of 256 x 128 48 KB, of two 128 x 128 64 KB)
-            const bool small4 = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
-            MidTiles plan = mid_tiles(M, N, K, epi);
-            if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)))
-                plan = mid_tiles(M, N, K, epi, false);
+            const MidTiles plan = plan_of(M);
             const int splits = plan.splits;
-            if (plan.four && small4 && splits > 1) {
+            if (plan.four && small && splits > 1) {
                 rc = launch_fourwave_epi<256, 128, LLMRS_EPI_STORE_F32>(stream, A, lda, W, workspace, N, M, N, K, LLMRS_EPI_STORE_F32, splits);
                 if (rc == 0) launch_splitk_finish(stream, (const float*)workspace, splits, out, ldc, M, N, epi, next);
-            } else if (plan.four && small4 && !whole && next == nullptr && fourwave_takes(epi, out, ldc, N))
+            } else if (plan.four && small && !whole && next == nullptr && fourwave_takes(epi, out, ldc, N))
                 rc = launch_fourwave<256, 128>(stream, A, lda, W, out, ldc, M, N, K, epi);
             else if (splits > 1)
                 rc = launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, splits, (float*)workspace, next);

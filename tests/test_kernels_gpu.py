@@ -6,7 +6,7 @@ import math
 import pytest
 import torch
 
-from llm_rs_amd.kernels import EPI_ACCUM_F32, EPI_STORE, EPI_STORE_F32, EPI_SWIGLU, KernelError, kernels
+from llm_rs_amd.kernels import EPI_ACCUM_F32, EPI_GLU_CLAMP, EPI_STORE, EPI_STORE_F32, EPI_SWIGLU, KernelError, kernels
 from plain_llama import plain_attention, plain_inv_freq, plain_rmsnorm, plain_rope, plain_silu
 
 pytestmark = pytest.mark.gpu
@@ -572,6 +572,33 @@ def test_gemm_large_tiles_of_many_rows(M, N, K):
         kernels().gemm(a, w, out, epi, torch.empty(n_ws, dtype=torch.float32, device=DEV) if n_ws else None)
         err = (out.double().cpu() - ref).abs()
         assert (err <= out_tol(ref, torch.float32, 1e-5 * math.sqrt(K))).all(), (epi, float(err.max()))
+
+
+@pytest.mark.parametrize("M,N,K", [(2049, 5200, 64), (2064, 6144, 128), (2055, 10240, 192), (1040, 10256, 64), (1025, 12296, 192), (1296, 8240, 128),
+                                   (1552, 6144, 320), (2320, 6160, 64), (4100, 4112, 128), (1808, 13000, 64)])
+def test_gemm_rows_that_go_along_with_large_tiles(M, N, K):
+    """1 to 16 rows beyond whole large tiles, four tiles of rows (a wave takes its part alone), five, eight (the waves of a half share
+    a part's k) and more, square tiles, 256 x 192 and a rest of 256 x 128, cut by N: every row once, and nothing behind the last.
+    (Bounds as in `test_gemm`; the gated forms' also of act(g) u with g and u off by the floor.)"""
+    k = kernels()
+    a = rnd((M, K + 24), torch.bfloat16, 3)[:, :K]
+    w = rnd((N, K), torch.bfloat16, 4, 0.1)
+    acc = product64(a, w)
+    g, u = acc[:, 0::2], acc[:, 1::2]
+    clamped = k.glu_clamp_slot(1.5, 1.702, 0.0, 1.0)
+    floor = 1e-5 * math.sqrt(K)
+    gm, um = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+    for epi, ref in ((EPI_STORE, acc), (EPI_STORE_F32, acc), (EPI_ACCUM_F32, acc), (EPI_SWIGLU, plain_silu(g) * u),
+                     (EPI_GLU_CLAMP, gm / (1 + torch.exp(-1.702 * gm)) * (um + 1.0))):
+        dtype = torch.float32 if epi in (EPI_STORE_F32, EPI_ACCUM_F32) else torch.bfloat16
+        room = rnd((M + 16, ref.shape[1]), dtype, 5)
+        before = room.clone()
+        want = ref + before[:M].double().cpu() if epi == EPI_ACCUM_F32 else ref
+        n_ws = k.gemm_workspace_floats(M, N, K)
+        k.gemm(a, w, room[:M], epi, torch.empty(n_ws, device=DEV) if n_ws else None, **({"glu": clamped} if epi == EPI_GLU_CLAMP else {}))
+        err = (room[:M].double().cpu() - want).abs()
+        assert (err <= out_tol(want, dtype, floor * (1 if ref is acc else 1 + 0.1 * math.sqrt(K) + 2.5))).all(), (epi, float(err.max()))
+        assert torch.equal(room[M:], before[M:])
 
 
 @pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 2050, 4098, 64), (torch.bfloat16, 700, 6145, 128), (torch.bfloat16, 2048, 6148, 64),
