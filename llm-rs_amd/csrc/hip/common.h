@@ -45,15 +45,36 @@ __device__ __forceinline__ void load4(const bf16* p, float (&v)[4]) {
     for (int j = 0; j < 4; ++j) v[j] = (float)t[j];
 }
 
+// The sum and the maximum over a wave, all 64 lanes of which must be active, left in every lane.  The moves between lanes are the
+// vector unit's own (halves and rows of 16 lanes swapped between registers, then moves within a row: once lanes eight apart agree, a
+// turn by four reaches the lane four apart): a few cycles each, where six moves through the LDS crossbar are six trips there, and in
+// kernels of one row a block nothing else runs beside them.  Lanes 32, 16, 8, 4, 2 and 1 apart in that order, as a
+// butterfly through the crossbar adds them: the same bits.
+template <int CTRL, class V>
+__device__ __forceinline__ V lanes_moved(V x) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
+}
+template <class V, class Op>
+__device__ __forceinline__ V wave_fold(V v, Op op) {
+    unsigned u = __builtin_bit_cast(unsigned, v);
+    auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);      // {the low half's, the high half's}
+    v = op(__builtin_bit_cast(V, (unsigned)halves[0]), __builtin_bit_cast(V, (unsigned)halves[1]));
+    u = __builtin_bit_cast(unsigned, v);
+    auto rows = __builtin_amdgcn_permlane16_swap(u, u, false, false);        // {the even row's, the odd row's}
+    v = op(__builtin_bit_cast(V, (unsigned)rows[0]), __builtin_bit_cast(V, (unsigned)rows[1]));
+    v = op(v, lanes_moved<0x128>(v));            // row_ror:8
+    v = op(v, lanes_moved<0x124>(v));            // row_ror:4
+    v = op(v, lanes_moved<0x4E>(v));             // quad_perm [2, 3, 0, 1]
+    return op(v, lanes_moved<0xB1>(v));          // quad_perm [1, 0, 3, 2]
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    return wave_fold(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
+    return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ int wave_min(int v) {
+    return wave_fold(v, [](int a, int b) { return min(a, b); });
 }
 
 // x / (1 + exp(-x)), as the reference writes it (shaders/ops.metal:769)

@@ -40,10 +40,6 @@ struct LinearScanArgs {
 // are the vector unit's own (quads, half rows and rows of 16 lanes mirrored; for 32 lanes the register swap between
 // neighbouring rows of 16): a few cycles each, where a move through the LDS crossbar costs a trip there, and a token's
 // two sums stand in the chain from token to token.
-template <int CTRL>
-__device__ __forceinline__ float lanes_moved(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
-}
 __device__ __forceinline__ float neighbouring_row(float x) {
     unsigned u = __float_as_uint(x);
     auto sw = __builtin_amdgcn_permlane16_swap(u, u, false, false);      // {rows 0, 0, 2, 2 of x; rows 1, 1, 3, 3 of x}

@@ -14,14 +14,13 @@
 
 #define ROUTE_MAX_EXPERTS 1024
 
-// The best of a wave's lanes: the largest value, of equal values the lowest index.
+// The best of a wave's lanes, all of which are active: the largest value, of equal values the lowest index.  (Two folds between
+// registers, one for the value and one for the index among the lanes that hold it: both exchanged through the LDS crossbar at
+// each of six distances were most of the choice, six of which make up a token's routing.)
 __device__ __forceinline__ void wave_best(float& best, int& at) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        float ob = __shfl_xor(best, d, 64);
-        int oa = __shfl_xor(at, d, 64);
-        if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-    }
+    const float most = wave_max(best);
+    at = wave_min(best == most ? at : 0x7fffffff);
+    best = most;
 }
 
 // Takes the experts outside the `keep` best of `groups` groups out of the choice: c[i] (what the choice of expert lane +
@@ -136,14 +135,10 @@ __global__ __launch_bounds__(64) void route_topk_sigmoid_kernel(const float* __r
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             if (c[i] > best) { best = c[i]; best_s = s[i]; at = lane + 64 * i; }
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            float ob = __shfl_xor(best, d, 64), os = __shfl_xor(best_s, d, 64);
-            int oa = __shfl_xor(at, d, 64);
-            if (ob > best || (ob == best && oa < at)) { best = ob; best_s = os; at = oa; }
-        }
+        const int own = at;
+        wave_best(best, at);
         if (at == 0x7fffffff) break;
-        chosen_sum += best_s;
+        chosen_sum += wave_sum(own == at ? best_s : 0.0f);         // (one lane's: the others add nothing)
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             if (lane + 64 * i == at) { keep[i] = s[i]; c[i] = -INFINITY; }

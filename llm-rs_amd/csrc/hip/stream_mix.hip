@@ -148,12 +148,25 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
                                                                  const float* __restrict__ mix, const float* __restrict__ w_out, const float* y, int slots) {
     constexpr int SMAX = 4;
     extern __shared__ __attribute__((aligned(16))) float row[];          // [D]
-    __shared__ float partial[HELD * 32];             // a sum of squares for every 64 slots of every group (D / 64 at most)
+    __shared__ __attribute__((aligned(16))) float partial[HELD * 32];             // a sum of squares for every 64 slots of every group (D / 64 at most)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int n4 = D / 4, gs = D / groups, log_per = slots >= 512 && gs >= 512 ? 3 : 2, per_group = 1 << log_per;      // (min(slots, gs) / 64: 4 or 8)
     const int r = rows ? rows[blockIdx.x] : blockIdx.x;
     float* src = x + (size_t)r * D;
     const bool plain = n_streams == 1 && w_in == nullptr;
+    // Every small weight is asked for before the row is (those past the last stream repeat the last one's and are not used): read
+    // where they are used, between the branches over the streams, each was a trip of its own.
+    float m[SMAX][SMAX], wo[SMAX], wi[SMAX];
+#pragma unroll
+    for (int s = 0; s < SMAX; ++s) {
+        const int from = min(s, n_streams - 1);
+        wi[s] = w_in ? w_in[from] : 1.0f;
+        if (MIX) {
+            wo[s] = w_out[from];
+#pragma unroll
+            for (int to = 0; to < SMAX; ++to) m[s][to] = mix[from * n_streams + min(to, n_streams - 1)];
+        }
+    }
     float v[HELD][SMAX][4], yy[HELD][4], wt[HELD][4], u[HELD][4];
     int first[HELD];                                 // where a piece's group has its sums (a piece lies in one group: their size is a multiple of four)
 #pragma unroll
@@ -184,11 +197,11 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
                 if (to < n_streams) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        float nv = mix[to] * old[0][j];
+                        float nv = m[0][to] * old[0][j];
 #pragma unroll
                         for (int s = 1; s < SMAX; ++s)
-                            if (s < n_streams) nv = fmaf(mix[s * n_streams + to], old[s][j], nv);
-                        v[i][to][j] = fmaf(w_out[to], idx < n4 ? yy[i][j] : 0.0f, nv);
+                            if (s < n_streams) nv = fmaf(m[s][to], old[s][j], nv);
+                        v[i][to][j] = fmaf(wo[to], idx < n4 ? yy[i][j] : 0.0f, nv);
                     }
                     if (idx < n4) store4(src + (size_t)to * stream_stride + 4 * idx, v[i][to]);
                 }
@@ -196,10 +209,10 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            u[i][j] = plain ? v[i][0][j] : (w_in ? w_in[0] : 1.0f) * v[i][0][j];
+            u[i][j] = plain ? v[i][0][j] : wi[0] * v[i][0][j];
 #pragma unroll
             for (int s = 1; s < SMAX; ++s)
-                if (s < n_streams) u[i][j] = fmaf(w_in ? w_in[s] : 1.0f, v[i][s][j], u[i][j]);
+                if (s < n_streams) u[i][j] = fmaf(wi[s], v[i][s][j], u[i][j]);
         }
         if (idx < n4) store4(row + 4 * idx, u[i]);
     }
@@ -213,12 +226,8 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
             if (p < groups * per_group)
                 for (int d = (p & (per_group - 1)) * 64 + lane; d < gs; d += slots) ss[t] = fmaf(group[d], group[d], ss[t]);
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float other[2] = {__shfl_xor(ss[0], off, 64), __shfl_xor(ss[1], off, 64)};
-            ss[0] += other[0];
-            ss[1] += other[1];
-        }
+        ss[0] = wave_sum(ss[0]);
+        ss[1] = wave_sum(ss[1]);
         if (lane == 0) {
             partial[part] = ss[0];
             if (part + waves < groups * per_group) partial[part + waves] = ss[1];
@@ -229,8 +238,11 @@ __global__ __launch_bounds__(512) void group_rmsnorm_held_kernel(T* __restrict__
     for (int i = 0; i < HELD; ++i) {
         const int idx = i * blockDim.x + threadIdx.x;
         if (idx >= n4) continue;
-        float total = 0.0f, o[4], z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int p = 0; p < per_group; ++p) total += partial[first[i] + p];
+        float total, o[4], z[4] = {0.0f, 0.0f, 0.0f, 0.0f}, sums[2][4];
+        load4(partial + first[i], sums[0]);
+        load4(partial + first[i] + (log_per == 3 ? 4 : 0), sums[1]);
+        total = ((sums[0][0] + sums[0][1]) + sums[0][2]) + sums[0][3];
+        if (log_per == 3) total = (((total + sums[1][0]) + sums[1][1]) + sums[1][2]) + sums[1][3];
         const float inv = 1.0f / sqrtf(total / (float)gs + eps);
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = u[i][j] * inv * wt[i][j];

@@ -123,6 +123,23 @@ def test_equal_groups_and_equal_experts_go_by_their_index():
     assert [r.nonzero().flatten().tolist() for r in weights.cpu()] == [[0, 1], [4, 5], [2, 3]]
 
 
+@pytest.mark.parametrize("E", [3, 64, 65, 200])
+@pytest.mark.parametrize("score", ["softmax", "sigmoid"])
+def test_routing_takes_the_lowest_of_equal_experts(E, score):
+    """Scores that tie, within a lane's experts and across lanes, some of them minus infinity: of equal ones the lowest index."""
+    top = min(E, 5)
+    g = torch.Generator().manual_seed(E)
+    logits = torch.randint(0, 3, (7, E), generator=g).float()
+    logits[0] = 1.0
+    logits[1, : E // 2] = float("-inf")
+    weights = torch.empty(7, E, device="cuda")
+    kernels().route_topk(logits.cuda(), weights, top, False, score)
+    for row, got in zip(logits.tolist(), weights.cpu()):
+        chosen = sorted(range(E), key=lambda e: (-row[e], e))[:top]
+        chosen = [e for e in chosen if row[e] > float("-inf")]          # (what has no score may be chosen; it weighs nothing)
+        assert [e for e in range(E) if got[e] > 0] == sorted(chosen)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_the_gated_silu_activation(dtype):
     T, ff, E = 19, 6, 3
