@@ -23,6 +23,7 @@
 // 28.5 -> 23.2, 28672 x 4096 44.2 -> 42.0; at 16 rows 4096 x 4096 13.3 -> 8.5, 4096 x 14336 35 -> 24.7, 10240 x 8192 49.5 -> 34.6;
 // 32-bit at 8 rows 2048 x 8192 26.1 -> 15.5, 2048 x 32768 88 -> 52, 16384 x 2048 28.8 -> 25.9, 128256 x 2048 187 -> 174.
 #include "gemm_tile.h"
+#include "recurrent.h"
 
 template <class T> struct Few;
 template <> struct Few<bf16> { typedef bf16x8 Piece; typedef bf16x4 Four; };
@@ -67,14 +68,37 @@ struct FewPlain {};
 struct FewScaled { RowScale scale; };
 struct FewNext { RowScale scale; NextNorm next; };
 struct FewQkv { RowScale scale; QkvEpilogue qkv; };
+// Products of a recurrent mixer in a step where every request brings one token: what the mixer does with the sums, channel by channel
+// and request by request, is done where they are finished (rows: requests; `slots` their state's rows; states 32-bit).  A kernel of its
+// own for it took 4.8 us for a few KB, three trips to memory one after the other, and 1.3 more between two kernels; here the
+// trips for the state run beside the weight's.  (4 requests, product and kernel -> here, us: convolution, 8192 x 2048, 8.2 + 4.8 ->
+// 8.4; minGRU, 6144 x 2048, 7.0 + 4.7 -> 8.0; scan, 4096 x 128, 4.7 + 4.9 -> 5.5.)
+//   FewConv: features below C are inputs of the causal convolution of four taps (recurrent.hip): silu of it goes to x, the state's three
+//     rows move on; the features above go to `out` in 32-bit.
+//   FewGru: the weight's rows are (gate | candidate | output gate), a third each; a block takes eight channels of all three
+//     (an eight of rows each), advances the state and writes the gated one to `out`.
+//   FewScan: the sums are the step sizes of a selective scan of 16 states: the state's step, the output to `out`.  A thread for each
+//     request and channel of the block.
+struct FewConv { const float* taps; const float* bias; float* state; long state_stride; const int* slots; bf16* x; int ldx, C; };
+struct FewGru { const float* bias_z; const float* bias_c; float* state; long state_stride; const int* slots; };
+struct FewScan {
+    const float* dt_bias; const float* A; const float* D; const float* gate; float* state; long state_stride; const int* slots;
+    const bf16* x; const bf16* b; const bf16* c;       // b, c: row 0's 16 of either, rows ldbc apart
+    int ld_gate, ldx, ldbc;
+};
+constexpr int SCAN_STATES = 16;
+template <class Extra> constexpr bool few_scaled = std::is_same<Extra, FewScaled>::value || std::is_same<Extra, FewNext>::value || std::is_same<Extra, FewQkv>::value;
 template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS, int TT, class Extra>
 __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ W, void* __restrict__ out, int lda,
                                                            int ldc, int M, int N, int K, int epi, unsigned inv_full, Extra extra) {
     constexpr bool NEXT = std::is_same<Extra, FewNext>::value, QKV = std::is_same<Extra, FewQkv>::value;
+    constexpr bool CONV = std::is_same<Extra, FewConv>::value, GRU = std::is_same<Extra, FewGru>::value, SCAN = std::is_same<Extra, FewScan>::value;
+    static_assert(!GRU || NG == 3, "an eight of rows of each of the three projections");
+    static_assert(!SCAN || (NG == 2 && NW == 4), "a thread for each of 16 requests and 16 channels");
     RowScale rs{};
     NextNorm nn{};
     QkvEpilogue qe{};
-    if constexpr (!std::is_same<Extra, FewPlain>::value) rs = extra.scale;
+    if constexpr (few_scaled<Extra>) rs = extra.scale;
     if constexpr (NEXT) nn = extra.next;
     if constexpr (QKV) qe = extra.qkv;
     typedef typename Few<T>::Piece Piece;
@@ -92,12 +116,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * NG * 8;
+    auto weight_row = [&](int group, int r) { return min(GRU ? group * (N / 3) + (int)blockIdx.x * 8 + r : n0 + group * 8 + r, N - 1); };   // row r of a block's eight
     // the rows that this lane's part of a load is of, at the chunk that belongs in the lane's slot
     const T* src[LOADS];
     {
         const int lrow = lane >> 3, chunk = ((lane & 7) ^ lrow) * PER;
 #pragma unroll
-        for (int i = 0; i < NG; ++i) src[i] = W + (size_t)min(n0 + i * 8 + lrow, N - 1) * K + chunk;
+        for (int i = 0; i < NG; ++i) src[i] = W + (size_t)weight_row(i, lrow) * K + chunk;
 #pragma unroll
         for (int i = 0; i < XL; ++i) src[NG + i] = A + (size_t)min(i * 8 + lrow, M - 1) * lda + chunk;
     }
@@ -111,7 +136,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
     // the weights, so that their trip to memory (they were written on other XCDs) costs nothing beside the weights'.
     // (Asked for after the walk along k it was a trip in front of every result: 0.9 us of the product.)
     constexpr int AHEAD = 4;
-    const bool scaled = TT == 1 && !std::is_same<Extra, FewPlain>::value && rs.sumsq != nullptr, by_four = rs.nparts % 16 == 0 && ((uintptr_t)rs.sumsq & 15) == 0;
+    const bool scaled = TT == 1 && few_scaled<Extra> && rs.sumsq != nullptr, by_four = rs.nparts % 16 == 0 && ((uintptr_t)rs.sumsq & 15) == 0;
     const float* sp = rs.sumsq + (size_t)min(row, M - 1) * rs.nparts;
     f32x4 part[AHEAD];
     if (scaled && by_four) {
@@ -133,6 +158,52 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
                 old[r] = ((const float*)out)[(size_t)own_m * ldc + n + r];
                 if (NEXT) next_w[r] = nn.weight[n + r];
             }
+    }
+
+    // a recurrent mixer's step: everything that it reads beside the sums
+    f32x4 was[3] = {}, tap[4] = {}, lane_bias[2] = {};
+    float* state_at = nullptr;
+    if constexpr (CONV) {
+        const int n = n0 + wave * 16 + 4 * g;
+        if (wave < TILES && 2 * wave + (g >> 1) < NG && row < M && n < extra.C) {
+            state_at = extra.state + (size_t)extra.slots[row] * extra.state_stride + n;
+            lane_bias[0] = extra.bias ? *(const f32x4*)(extra.bias + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) tap[r] = *(const f32x4*)(extra.taps + (size_t)(n + r) * 4);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) was[j] = *(const f32x4*)(state_at + (size_t)j * extra.C);
+        }
+    }
+    if constexpr (GRU) {
+        const int c = blockIdx.x * 8 + 4 * g;
+        if (wave == 0 && g < 2 && row < M) {
+            state_at = extra.state + (size_t)extra.slots[row] * extra.state_stride + c;
+            lane_bias[0] = extra.bias_z ? *(const f32x4*)(extra.bias_z + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+            lane_bias[1] = extra.bias_c ? *(const f32x4*)(extra.bias_c + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+            was[0] = *(const f32x4*)state_at;
+        }
+    }
+    float S[SCAN ? SCAN_STATES : 1], Ac[SCAN ? SCAN_STATES : 1], xv = 0.0f, gv = 0.0f, Dc = 0.0f, dt0 = 0.0f;
+    bf16x8 Bn[2], Cn[2];
+    const int sm = threadIdx.x >> 4, sf = threadIdx.x & 15;        // SCAN: this thread's request, and its channel of the block's
+    if constexpr (SCAN) {
+        const int c = n0 + sf;
+        if (sm < M) {
+            state_at = extra.state + (size_t)extra.slots[sm] * extra.state_stride + c;          // state n of the channel: state_at[n N]
+#pragma unroll
+            for (int n = 0; n < SCAN_STATES; ++n) Ac[n] = extra.A[(size_t)n * N + c];
+            Dc = extra.D[c];
+            dt0 = extra.dt_bias ? extra.dt_bias[c] : 0.0f;
+            gv = extra.gate[(size_t)sm * extra.ld_gate + c];
+            xv = to_f32(extra.x[(size_t)sm * extra.ldx + c]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                Bn[h] = *(const bf16x8*)(extra.b + (size_t)sm * extra.ldbc + 8 * h);
+                Cn[h] = *(const bf16x8*)(extra.c + (size_t)sm * extra.ldbc + 8 * h);
+            }
+#pragma unroll
+            for (int n = 0; n < SCAN_STATES; ++n) S[n] = state_at[(size_t)n * N];
+        }
     }
 
     const int full = (unsigned)K / KB;
@@ -208,8 +279,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
         Piece w[WL], x[XL];
 #pragma unroll
         for (int i = 0; i < WL; ++i) {
-            const int n = n0 + (FOLD ? i * 8 + f : (i / 2) * 16 + row), from = k + first + (FOLD ? 0 : (i % 2) * (KB / 2));
-            w[i] = from < K ? *(const Piece*)(W + (size_t)min(n, N - 1) * K + from) : Piece{};
+            const int n = FOLD ? weight_row(i, f) : weight_row(i / 2 * 2 + (row >> 3), f), from = k + first + (FOLD ? 0 : (i % 2) * (KB / 2));
+            w[i] = from < K ? *(const Piece*)(W + (size_t)n * K + from) : Piece{};
         }
 #pragma unroll
         for (int i = 0; i < XL; ++i) {
@@ -250,6 +321,43 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
                 if (2 * t + (g >> 1) < NG) red[(((wave * TT + tt) * NG + 2 * t) * 2 + g) * TOK + row] = acc[tt][2 * t].total() + acc[tt][2 * t + 1].total();
     }
     __syncthreads();
+    if constexpr (GRU) {
+        if (wave > 0 || g > 1 || row >= M) return;
+        f32x4 v[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v[i] += red[((w * NG + i) * 2 + g) * TOK + row];
+        }
+        f32x4 s;
+        Four y;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = mingru_state(was[0][r], sigmoid_f32(v[0][r] + lane_bias[0][r]), v[1][r] + lane_bias[1][r]);
+            y[r] = from_f32<T>(s[r] * silu_f32(v[2][r]));
+        }
+        *(f32x4*)state_at = s;
+        *(Four*)((T*)out + (size_t)row * ldc + blockIdx.x * 8 + 4 * g) = y;
+        return;
+    }
+    if constexpr (SCAN) {
+        if (sm >= M) return;
+        float vdt = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) vdt += ((const float*)red)[(((w * NG + (sf >> 3)) * 2 + (sf >> 2 & 1)) * TOK + sm) * 4 + (sf & 3)];
+        const float step = softplus_f32(vdt + dt0), sx = step * xv;
+        float y = 0.0f;
+#pragma unroll
+        for (int n = 0; n < SCAN_STATES; ++n) {
+            S[n] = fmaf(__builtin_amdgcn_exp2f(step * (Ac[n] * LOG2_E)), S[n], sx * (float)Bn[n / 8][n % 8]);
+            y = fmaf(S[n], (float)Cn[n / 8][n % 8], y);
+            state_at[(size_t)n * N] = S[n];
+        }
+        y = fmaf(Dc, xv, y);
+        ((T*)out)[(size_t)sm * ldc + n0 + sf] = from_f32<T>(y * silu_f32(gv));
+        return;
+    }
     // the tiles are shared out over the waves: lane l finishes token l % 16 and features 4 (l / 16) + r
     if (wave >= TILES * TT || (TT == 1 && row >= M)) return;
     float inv = 1.0f;
@@ -281,6 +389,27 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const T* __restrict__
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = s[r] * inv;
         const int n = n0 + tile * 16 + 4 * g;
+        if constexpr (CONV) {
+            static_assert(TILES <= NW, "a wave finishes the one tile whose state it has asked for");
+            if (n >= N) continue;
+            if (n >= extra.C) {
+                *(f32x4*)((float*)out + (size_t)m * ldc + n) = f32x4{v[0], v[1], v[2], v[3]};
+                continue;
+            }
+            Four y;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float a = lane_bias[0][r];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) a = fmaf(tap[r][j], was[j][r], a);
+                y[r] = from_f32<T>(silu_f32(fmaf(tap[r][3], v[r], a)));
+            }
+            *(f32x4*)state_at = was[1];
+            *(f32x4*)(state_at + extra.C) = was[2];
+            *(f32x4*)(state_at + (size_t)2 * extra.C) = f32x4{v[0], v[1], v[2], v[3]};
+            *(Four*)((T*)extra.x + (size_t)m * extra.ldx + n) = y;
+            continue;
+        }
         if (!NEXT && !QKV && epi_gated(epi)) {
 #pragma unroll
             for (int r = 0; r < 4; r += 2)
@@ -336,8 +465,8 @@ struct FewCall {
     RowScale scale;
     NextNorm next;
 };
-template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS = 1, int TT = 1>
-static void launch_few(const FewCall& c) {
+template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS = 1, int TT = 1, class Launch>
+static void with_few_launcher(const FewCall& c, Launch choose) {
     static_assert(ROT % (NG * 8) == 0, "a block's features lie in one group");
     const unsigned full = c.K * sizeof(T) / 128, inv_full = full > 1 ? (unsigned)(((1ull << 32) + full - 1) / full) : 0;
     constexpr size_t bytes = (size_t)NW * R * (NG + (FOLD ? 1 : 2 * TT)) * 1024 + (size_t)NW * TT * NG * 2 * (FOLD ? 8 : 16) * 16 + NW * 16 * sizeof(float);
@@ -351,11 +480,17 @@ static void launch_few(const FewCall& c) {
         gemm_few_kernel<T, FOLD, NG, NW, R, ROT, SUMS, TT><<<ceil_div(c.N, NG * 8), NW * 64, bytes, c.stream>>>(
             (const T*)c.A, (const T*)c.W, c.out, c.lda, c.ldc, c.M, c.N, c.K, c.epi, inv_full, extra);
     };
-    if constexpr (TT > 1) launch(FewPlain{});             // (more than 16 rows: no norm is left to them, and no rotation)
-    else if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
-    else if (c.next.y != nullptr) launch(FewNext{c.scale, c.next});
-    else if (c.scale.sumsq != nullptr) launch(FewScaled{c.scale});
-    else launch(FewPlain{});
+    choose(launch);
+}
+template <class T, bool FOLD, int NG, int NW, int R, int ROT, int SUMS = 1, int TT = 1>
+static void launch_few(const FewCall& c) {
+    with_few_launcher<T, FOLD, NG, NW, R, ROT, SUMS, TT>(c, [&](auto launch) {
+        if constexpr (TT > 1) launch(FewPlain{});             // (more than 16 rows: no norm is left to them, and no rotation)
+        else if (c.epi == LLMRS_EPI_QKV) launch(FewQkv{c.scale, c.qkv});
+        else if (c.next.y != nullptr) launch(FewNext{c.scale, c.next});
+        else if (c.scale.sumsq != nullptr) launch(FewScaled{c.scale});
+        else launch(FewPlain{});
+    });
 }
 // Whether blocks of 24 features (a tile and a half) share a weight of N features out over the device's units more
 // evenly, by a tenth of a round or more, than blocks of `whole` features (16 or 32) do.
@@ -483,4 +618,62 @@ int llmrs_gemm_few_bf16(hipStream_t stream, const bf16* A, int lda, const bf16* 
 int llmrs_gemm_few_f32(hipStream_t stream, const float* A, int lda, const float* W, void* out, int ldc, int M, int N, int K, int epi,
                        const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next) {
     return gemm_few<float>(stream, A, lda, W, out, ldc, M, N, K, epi, qkv, scale, next);
+}
+
+// ---- products of a recurrent mixer's single tokens, with what the mixer does with their sums (FewConv, FewGru, FewScan) ------------
+// bfloat16, up to 16 requests; the rest is for the product and the kernels of recurrent.hip.
+template <int NG, int NW, int R, int ROT, class Extra>
+static void launch_mixer_step(const FewCall& c, const Extra& extra) {
+    if (c.M <= 8) with_few_launcher<bf16, true, NG, NW, R, ROT>(c, [&](auto launch) { launch(extra); });
+    else with_few_launcher<bf16, false, NG, NW, R, ROT>(c, [&](auto launch) { launch(extra); });
+}
+static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+static bool step_rows_ok(const void* A, int lda, const void* W, int M, int K, const float* state, long state_stride, const int* slots) {
+    return M >= 0 && M <= 16 && K > 0 && K % 8 == 0 && lda >= K && lda % 8 == 0 && aligned16(A) && aligned16(W) && state != nullptr && aligned16(state) &&
+           state_stride % 4 == 0 && slots != nullptr;
+}
+
+// sums = A W^T, of which the first C columns go through the causal convolution of four taps [C, 4] and silu into x (bfloat16) and into the state
+// [slots][3][C], and the others, C to N, to out (32-bit, row stride ldc, its first C columns left as they are).
+extern "C" int llmrs_conv_product_step(hipStream_t stream, const bf16* A, int lda, const bf16* W, int M, int N, int K, float* out, int ldc, const float* taps,
+                                       const float* bias, float* state, long state_stride, const int* slots, int C, bf16* x, int ldx) {
+    LLMRS_REQUIRE(step_rows_ok(A, lda, W, M, K, state, state_stride, slots) && state_stride >= 3L * C, "conv_product_step: bad rows or state, M=%d K=%d", M, K);
+    LLMRS_REQUIRE(C > 0 && C % 4 == 0 && N >= C && N % 4 == 0 && ldc >= N && ldc % 4 == 0 && ldx >= C && ldx % 4 == 0 && aligned16(out) && aligned16(taps) &&
+                  aligned16(bias) && taps != nullptr && ((uintptr_t)x & 7) == 0, "conv_product_step: bad sizes N=%d C=%d", N, C);
+    if (M == 0) return 0;
+    FewCall c{stream, A, lda, W, out, ldc, M, N, K, LLMRS_EPI_STORE_F32, QkvEpilogue{}, RowScale{}, NextNorm{}};
+    FewConv e{taps, bias, state, state_stride, slots, x, ldx, C};
+    // (as the plain product's rule above: few rows of a weight, many, and short ones)
+    if (N >= 16384) launch_mixer_step<2, 4, 3, 64>(c, e);
+    else if (K < 2048) launch_mixer_step<2, 4, 4, 0>(c, e);
+    else if (half_blocks_for_narrow(N, K)) launch_mixer_step<1, 8, 4, 64>(c, e);
+    else launch_mixer_step<2, 8, 3, 64>(c, e);
+    LLMRS_LAUNCH_CHECK("conv_product_step");
+    return 0;
+}
+// W: [3 width, K], the rows of gate, candidate and output gate; out: [M, width] bfloat16; state [slots][width].
+extern "C" int llmrs_mingru_product_step(hipStream_t stream, const bf16* A, int lda, const bf16* W, int M, int width, int K, const float* bias_z, const float* bias_c,
+                                         float* state, long state_stride, const int* slots, bf16* out, int ldo) {
+    LLMRS_REQUIRE(step_rows_ok(A, lda, W, M, K, state, state_stride, slots) && state_stride >= width, "mingru_product_step: bad rows or state, M=%d K=%d", M, K);
+    LLMRS_REQUIRE(width > 0 && width % 8 == 0 && ldo >= width && ldo % 4 == 0 && ((uintptr_t)out & 7) == 0 && aligned16(bias_z) && aligned16(bias_c),
+                  "mingru_product_step: bad sizes, width %d", width);
+    if (M == 0) return 0;
+    launch_mixer_step<3, 8, 3, 48>(FewCall{stream, A, lda, W, out, ldo, M, 3 * width, K, LLMRS_EPI_STORE, QkvEpilogue{}, RowScale{}, NextNorm{}},
+                                   FewGru{bias_z, bias_c, state, state_stride, slots});
+    LLMRS_LAUNCH_CHECK("mingru_product_step");
+    return 0;
+}
+// dt = d Wdt^T (d: [M, K], W: [C, K]), and the selective scan's step of 16 states with it.  x [M, C], b and c [M, 16] (16-byte aligned rows, ldbc apart),
+// out [M, C] bfloat16; A [16, C] negative, D [C], gate [M, C] 32-bit; state [slots][16][C].
+extern "C" int llmrs_scan_product_step(hipStream_t stream, const bf16* d, int ldd, const bf16* W, int M, int C, int K, const float* dt_bias, const float* A,
+                                       const float* D, const float* gate, int ld_gate, float* state, long state_stride, const int* slots, const bf16* x, int ldx,
+                                       const bf16* b, const bf16* c, int ldbc, bf16* out, int ldo) {
+    LLMRS_REQUIRE(step_rows_ok(d, ldd, W, M, K, state, state_stride, slots) && state_stride >= 16L * C, "scan_product_step: bad rows or state, M=%d K=%d", M, K);
+    LLMRS_REQUIRE(C > 0 && C % 16 == 0 && A && D && gate && x && out && ld_gate >= C && ldx >= C && ldo >= C && ldbc >= 16 && ldbc % 8 == 0 && b && c && aligned16(b) &&
+                  aligned16(c), "scan_product_step: bad sizes, C=%d", C);
+    if (M == 0) return 0;
+    launch_mixer_step<2, 4, 4, 0>(FewCall{stream, d, ldd, W, out, ldo, M, C, K, LLMRS_EPI_STORE, QkvEpilogue{}, RowScale{}, NextNorm{}},
+                                  FewScan{dt_bias, A, D, gate, state, state_stride, slots, x, b, c, ld_gate, ldx, ldbc});
+    LLMRS_LAUNCH_CHECK("scan_product_step");
+    return 0;
 }

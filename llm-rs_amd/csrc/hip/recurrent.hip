@@ -15,15 +15,11 @@
 // A chunk's place in the carry buffer is q_start / chunk length + entry + chunk: distinct for distinct chunks and
 // below n_tokens / chunk length + n_entries.  Steps whose entries are all short (decoding) take the final launch
 // alone, straight from and to the request's state.  Cut or not, the sums differ in rounding only.
-#include "common.h"
+#include "recurrent.h"
 
 #define SCAN_CHUNK 64                      // tokens of a chunk, and of the B and C rows that wait in LDS together
 #define SCAN_CHUNK_SHORT 32                // chunks of a step with too few long ones to fill the device
 #define SCAN_LOADS 8                       // tokens whose inputs a thread fetches together
-#define LOG2_E 1.44269504088896341f
-
-__device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float softplus_f32(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 
 // ---- minGRU ---------------------------------------------------------------------------------------------------
 // sums: [T, ld] 32-bit, per token the projections' sums (gate | candidate | output gate), each W wide.
@@ -53,10 +49,8 @@ __global__ __launch_bounds__(64) void mingru_scan_kernel(const float* __restrict
     float s = LOCAL ? 0.0f : (chunk > 0 ? carry[place * 2 * W + c] : *sp), keep = 1.0f;
     float bz = bias_z ? bias_z[c] : 0.0f, bc = bias_c ? bias_c[c] : 0.0f;
     auto one = [&](int t, float vz, float vc, float vg) {
-        float z = sigmoid_f32(vz + bz);
-        float u = vc + bc;
-        float cand = u >= 0.0f ? u + 0.5f : sigmoid_f32(u);
-        s = (1.0f - z) * s + z * cand;
+        const float z = sigmoid_f32(vz + bz);
+        s = mingru_state(s, z, vc + bc);
         if (LOCAL) keep *= 1.0f - z;
         else out[(size_t)t * ldo + c] = from_f32<T>(s * silu_f32(vg));
     };

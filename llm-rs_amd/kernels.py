@@ -179,6 +179,12 @@ class Kernels:
         reads the stream next (`NextNorm`), or None: then a norm kernel runs."""
         return None
 
+    def products_step_mixers(self, n_tokens: int, n_entries: int, longest: int, dtype: torch.dtype, tensors) -> bool:
+        """Whether the products of a recurrent mixer can do what it does with their sums themselves (`conv_product_step`,
+        `mingru_product_step`, `scan_product_step`): every request brings one token, there are few, and what is read in
+        pieces of 16 bytes (`tensors`, None among them) lies so."""
+        return False
+
     def grouped_experts_take(self, hidden: int, ff: int, dtype: torch.dtype) -> bool:
         """Whether `expert_up` and `expert_down` (every expert's product over its own rows in one launch) and `expert_few_up` and
         `expert_few_down` (up to 64 tokens; experts that none of them chose are not read) run experts of these sizes."""
@@ -270,6 +276,9 @@ class HipKernels(Kernels):
             "llmrs_expert_few_down": [V, V, I, I, V, V, I, I, I, I, V, I],
             "llmrs_mingru_scan": [V, I, V, I, V, V, V, ctypes.c_long, V, V, I, I, V, I, I, V],
             "llmrs_causal_conv": [V, I, V, I, V, V, V, V, ctypes.c_long, V, V, V, I, I, I, I, I, V, I, V, I, I],
+            "llmrs_conv_product_step": [V, V, I, V, I, I, I, V, I, V, V, V, ctypes.c_long, V, I, V, I],
+            "llmrs_mingru_product_step": [V, V, I, V, I, I, I, V, V, V, ctypes.c_long, V, V, I],
+            "llmrs_scan_product_step": [V, V, I, V, I, I, I, V, V, V, V, I, V, ctypes.c_long, V, V, I, V, V, I, V, I],
             "llmrs_selective_scan": [V, I, V, I, V, I, I, I, V, I, V, V, V, V, I, V, ctypes.c_long, V, V, V, I, I, I, I, V, I, I, V],
         }
         for name, args in sigs.items():
@@ -318,6 +327,10 @@ class HipKernels(Kernels):
 
     def qkv_product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype, head_dim: int, rotary_dim: int) -> bool:
         return self._stored_by_fours(head_dim, rotary_dim) and self.gemm_defers_norm(M, N, K, dtype)
+
+    def products_step_mixers(self, n_tokens: int, n_entries: int, longest: int, dtype: torch.dtype, tensors) -> bool:
+        return (longest == 1 and n_tokens == n_entries and 1 <= n_tokens <= 16 and dtype == torch.bfloat16 and self.allow_mfma
+                and all(t is None or t.data_ptr() % 16 == 0 for t in tensors))
 
     def norm_left_by_product(self, M: int, N: int, K: int, dtype: torch.dtype) -> Optional[NormPlan]:
         return self._norm_plan(dtype == torch.bfloat16, M, N, K) if self.allow_mfma else None
@@ -1166,6 +1179,45 @@ class HipKernels(Kernels):
                   self.lib.llmrs_selective_scan, self._stream(), _code(x.dtype), _p(x), x.stride(0), _p(bc), bc.stride(0), int(off_b),
                   int(off_c), _p(dt), dt.stride(0), _p(dt_bias), _p(A), _p(D), _p(gate), gate.stride(0), _p(state), state.stride(0),
                   _p(ypart), _p(q_starts), _p(slots), slots.numel(), T, C, N, _p(out), out.stride(0), int(longest), _p(carry))
+
+    def conv_product_step(self, a: torch.Tensor, w: torch.Tensor, sums: torch.Tensor, taps: torch.Tensor, bias, state: torch.Tensor, slots, channels: int,
+                          out: torch.Tensor) -> None:
+        """`gemm(a, w, sums, EPI_STORE_F32)` and `causal_conv` (four taps, silu) of its first `channels` columns into `out`, one token a request
+        (`products_step_mixers`): those columns of `sums` are not written."""
+        M, K = a.shape
+        N = w.shape[0]
+        assert a.dtype == w.dtype == out.dtype == torch.bfloat16 and w.shape[1] == K and w.is_contiguous() and a.stride(1) == sums.stride(1) == out.stride(1) == 1
+        assert sums.dtype == taps.dtype == state.dtype == torch.float32 and sums.shape == (M, N) and tuple(taps.shape) == (channels, 4) and taps.is_contiguous()
+        assert state.stride(-1) == 1 and state.shape[1] >= 3 * channels and out.shape == (M, channels) and slots.dtype == torch.int32 and slots.numel() == M
+        assert bias is None or (bias.dtype == torch.float32 and bias.numel() == channels and bias.is_contiguous())
+        self._run(f"gemm {M}x{N}x{K} conv", (M * K + N * K) * 2 + M * (N * 4 + channels * 22), 2 * M * N * K, a.dtype, self.lib.llmrs_conv_product_step,
+                  self._stream(), _p(a), a.stride(0), _p(w), M, N, K, _p(sums), sums.stride(0), _p(taps), _p(bias), _p(state), state.stride(0), _p(slots),
+                  channels, _p(out), out.stride(0))
+
+    def mingru_product_step(self, a: torch.Tensor, w: torch.Tensor, bias_z, bias_c, state: torch.Tensor, slots, width: int, out: torch.Tensor) -> None:
+        """`gemm` with w [gate | candidate | output gate] and `mingru_scan` of its sums into `out`, one token a request (`products_step_mixers`)."""
+        M, K = a.shape
+        assert a.dtype == w.dtype == out.dtype == torch.bfloat16 and tuple(w.shape) == (3 * width, K) and w.is_contiguous() and a.stride(1) == out.stride(1) == 1
+        assert state.dtype == torch.float32 and state.stride(-1) == 1 and state.shape[1] >= width and out.shape == (M, width)
+        assert slots.dtype == torch.int32 and slots.numel() == M
+        for b in (bias_z, bias_c):
+            assert b is None or (b.dtype == torch.float32 and b.numel() == width and b.is_contiguous())
+        self._run(f"gemm {M}x{3 * width}x{K} mingru", (M * K + 3 * width * K) * 2 + M * width * 10, 6 * M * width * K, a.dtype, self.lib.llmrs_mingru_product_step,
+                  self._stream(), _p(a), a.stride(0), _p(w), M, width, K, _p(bias_z), _p(bias_c), _p(state), state.stride(0), _p(slots), _p(out), out.stride(0))
+
+    def scan_product_step(self, bc: torch.Tensor, rank: int, w: torch.Tensor, x: torch.Tensor, dt_bias, A: torch.Tensor, D: torch.Tensor, gate: torch.Tensor,
+                          state: torch.Tensor, slots, out: torch.Tensor) -> None:
+        """`gemm` of bc's first `rank` columns with w (the step sizes' sums) and `selective_scan` of 16 states with B and C in the next 16 columns
+        and the 16 after those, one token a request (`products_step_mixers`)."""
+        M, C = x.shape
+        assert bc.dtype == w.dtype == x.dtype == out.dtype == torch.bfloat16 and bc.shape == (M, rank + 32) and tuple(w.shape) == (C, rank) and w.is_contiguous()
+        assert bc.stride(1) == x.stride(1) == out.stride(1) == gate.stride(1) == 1 and out.shape == gate.shape == (M, C)
+        assert A.dtype == D.dtype == gate.dtype == state.dtype == torch.float32 and tuple(A.shape) == (16, C) and A.is_contiguous() and D.numel() == C
+        assert state.stride(-1) == 1 and state.shape[1] >= 16 * C and slots.dtype == torch.int32 and slots.numel() == M
+        assert dt_bias is None or (dt_bias.dtype == torch.float32 and dt_bias.numel() == C and dt_bias.is_contiguous())
+        self._run(f"gemm {M}x{C}x{rank} scan", (M + C) * rank * 2 + M * C * (8 + 128) + C * 64, 2 * M * C * (rank + 40), bc.dtype, self.lib.llmrs_scan_product_step,
+                  self._stream(), _p(bc), bc.stride(0), _p(w), M, C, rank, _p(dt_bias), _p(A), _p(D), _p(gate), gate.stride(0), _p(state), state.stride(0), _p(slots),
+                  _p(x), x.stride(0), _p(bc[:, rank:]), _p(bc[:, rank + 16:]), bc.stride(0), _p(out), out.stride(0))
 
     def argmax_rows(self, logits: torch.Tensor, out: torch.Tensor, scratch: Optional[torch.Tensor] = None) -> None:
         """`scratch`: 256 bytes per row let several blocks share a long row."""

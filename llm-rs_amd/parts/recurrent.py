@@ -39,6 +39,7 @@ class MinGRU(Mixer):
         leaves = _leaves({"gate": "z", "gate_bias": "z.b", "candidate": "x", "candidate_bias": "x.b", "out_gate": "g", "out": "o"}, p.get("names"))
         self.names = {k: self.name(v) for k, v in leaves.items()}
         self.w_in = self.w_o = self.bias_z = self.bias_c = None
+        self.step_in_products = self.hidden % 8 == 0 and self.width % 8 == 0          # (rows of whole 16-byte pieces, eights of channels)
 
     def tensors(self):
         n, W, H = self.names, self.width, self.hidden
@@ -65,6 +66,14 @@ class MinGRU(Mixer):
     def forward(self, ctx, x, h, cache):
         k = kernels()
         T = x.shape[0]
+        # (up to 16 requests of one token: the product advances the state itself)
+        if self.step_in_products and k.products_step_mixers(T, ctx.n_entries, ctx.longest, self.dtype,
+                                                                  (x, self.w_in, self.bias_z, self.bias_c, cache.state)):
+            gated = ctx.workspace("mingru.gated", (T, self.width), self.dtype)
+            k.mingru_product_step(x, self.w_in, self.bias_z, self.bias_c, cache.state, ctx.slots, self.width, gated)
+            k.gemm(gated, self.w_o, h, EPI_ACCUM_F32, ctx.gemm_workspace(gated, self.w_o))
+            ctx.note_left(h, None)
+            return
         sums = ctx.workspace("mingru.sums", (T, 3 * self.width), torch.float32)
         k.gemm(x, self.w_in, sums, EPI_STORE_F32, ctx.gemm_workspace(x, self.w_in))
         gated = ctx.workspace("mingru.gated", (T, self.width), self.dtype)
@@ -90,6 +99,8 @@ class Mamba1(Mixer):
         self.names = {k: self.name(v) for k, v in leaves.items()}
         self.w_in = self.w_x = self.w_dt = self.w_o = None
         self.conv = self.conv_bias = self.dt_bias = self.A = self.A_log = self.D = None
+        # (four taps and 16 states, as most have; rows of whole 16-byte pieces, sixteens of channels)
+        self.step_in_products = (self.taps == 4 and self.n_state == 16 and self.hidden % 8 == 0 and self.dt_rank % 8 == 0 and self.inner % 16 == 0)
 
     def tensors(self):
         n, C, H, N, R = self.names, self.inner, self.hidden, self.n_state, self.dt_rank
@@ -124,16 +135,25 @@ class Mamba1(Mixer):
         k = kernels()
         T, C, N, R = x.shape[0], self.inner, self.n_state, self.dt_rank
         sums = ctx.workspace("mamba.sums", (T, 2 * C), torch.float32)
-        k.gemm(x, self.w_in, sums, EPI_STORE_F32, ctx.gemm_workspace(x, self.w_in))
         scan_state, conv_state = cache.state[:, :C * N], cache.state[:, C * N:]
         xc = ctx.workspace("mamba.x", (T, C), self.dtype)
-        k.causal_conv(sums, self.conv, self.conv_bias, conv_state, ctx.q_starts, ctx.slots, ctx.token_entry, C, xc, silu=True, longest=ctx.longest)
         dbc = ctx.workspace("mamba.dbc", (T, R + 2 * N), self.dtype)
+        y = ctx.workspace("mamba.y", (T, C), self.dtype)
+        # (up to 16 requests of one token: the products convolve and advance the state themselves)
+        if self.step_in_products and k.products_step_mixers(T, ctx.n_entries, ctx.longest, self.dtype,
+                                                                  (x, self.w_in, self.conv, self.conv_bias, cache.state, self.w_dt)):
+            k.conv_product_step(x, self.w_in, sums, self.conv, self.conv_bias, conv_state, ctx.slots, C, xc)
+            k.gemm(xc, self.w_x, dbc, EPI_STORE, ctx.gemm_workspace(xc, self.w_x))
+            k.scan_product_step(dbc, R, self.w_dt, xc, self.dt_bias, self.A, self.D, sums[:, C:], scan_state, ctx.slots, y)
+            k.gemm(y, self.w_o, h, EPI_ACCUM_F32, ctx.gemm_workspace(y, self.w_o))
+            ctx.note_left(h, None)
+            return
+        k.gemm(x, self.w_in, sums, EPI_STORE_F32, ctx.gemm_workspace(x, self.w_in))
+        k.causal_conv(sums, self.conv, self.conv_bias, conv_state, ctx.q_starts, ctx.slots, ctx.token_entry, C, xc, silu=True, longest=ctx.longest)
         k.gemm(xc, self.w_x, dbc, EPI_STORE, ctx.gemm_workspace(xc, self.w_x))
         dt = ctx.workspace("mamba.dt", (T, C), torch.float32)
         d = dbc[:, :R]
         k.gemm(d, self.w_dt, dt, EPI_STORE_F32, ctx.gemm_workspace(d, self.w_dt))
-        y = ctx.workspace("mamba.y", (T, C), self.dtype)
         ypart = ctx.workspace("mamba.ypart", (T, C), torch.float32) if N > 64 else None
         need = k.scan_carry_floats(T, ctx.n_entries, ctx.longest, (N + 1) * C)
         carry = ctx.workspace("scan.carry", (need,), torch.float32) if need else None

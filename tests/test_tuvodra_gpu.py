@@ -387,6 +387,51 @@ def test_single_tokens_through_the_scan_equal_the_walk(entries, channels, states
     assert all(torch.equal(a, b) for a, b in zip(*got)) and not torch.equal(got[0][0], before)
 
 
+@pytest.mark.parametrize("entries", [1, 4, 8, 9, 16])
+@pytest.mark.parametrize("channels,hidden,rank", [(16, 8, 8), (48, 72, 24), (512, 2048, 40), (4096, 2048, 128), (8208, 64, 72)])
+def test_products_that_step_their_mixers_equal_the_kernels_behind_plain_ones(channels, hidden, rank, entries):
+    """One token a request: the products with the convolution, minGRU's state and the scan's against the product and the mixer's own
+    kernel.  Both read the same bfloat16 numbers; the products' 32-bit sums may be added in another order (K 2^-24 of the terms' sizes,
+    under 1e-4 of states near 1), and outputs round once more (2^-8 of them)."""
+    from llm_rs_amd.kernels import EPI_STORE_F32, kernels
+    k, g = kernels(), torch.Generator(device="cuda").manual_seed(channels + entries)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    b16 = lambda *shape: rnd(*shape).bfloat16()
+    C, slots = channels, torch.randperm(entries + 2, generator=torch.Generator().manual_seed(entries))[:entries].int().cuda()
+    starts, entry = torch.arange(entries + 1, dtype=torch.int32, device="cuda"), torch.arange(entries, dtype=torch.int32, device="cuda")
+    before = rnd(entries + 2, C * 19 + 4)
+
+    def compare(named, got, want):
+        for name, a, b in zip(named, got, want):
+            tol = dict(rtol=2.0 ** -7, atol=2e-3) if a.dtype == torch.bfloat16 else dict(rtol=1e-4, atol=1e-4)
+            torch.testing.assert_close(a, b, msg=lambda m: f"{name}: {m}", **tol)
+
+    x, w, taps, bias = b16(entries, hidden), (rnd(2 * C + 4, hidden) / hidden ** 0.5).bfloat16(), rnd(C, 4), rnd(C)
+    plain, fused = torch.empty(entries, 2 * C + 4, device="cuda"), torch.empty(entries, 2 * C + 4, device="cuda")
+    states, outs = [before.clone(), before.clone()], [torch.empty(entries, C, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    k.gemm(x, w, plain, EPI_STORE_F32)
+    k.causal_conv(plain, taps, bias, states[0][:, 16 * C:], starts, slots, entry, C, outs[0], silu=True, longest=1)
+    k.conv_product_step(x, w, fused, taps, bias, states[1][:, 16 * C:], slots, C, outs[1])
+    compare(("convolved", "its state", "the gate's sums"), (outs[1], states[1], fused[:, C:]), (outs[0], states[0], plain[:, C:]))
+
+    x, w, bz, bc = b16(entries, hidden), (rnd(3 * C, hidden) / hidden ** 0.5).bfloat16(), rnd(C), rnd(C)
+    sums = torch.empty(entries, 3 * C, device="cuda")
+    states, outs = [before.clone(), before.clone()], [torch.empty(entries, C, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    k.gemm(x, w, sums, EPI_STORE_F32)
+    k.mingru_scan(sums, bz, bc, states[0], starts, slots, C, outs[0], 1)
+    k.mingru_product_step(x, w, bz, bc, states[1], slots, C, outs[1])
+    compare(("minGRU", "its state"), (outs[1], states[1]), (outs[0], states[0]))
+
+    u, dbc, w, gate = b16(entries, C), b16(entries, rank + 32), (rnd(C, rank) / rank ** 0.5).bfloat16(), rnd(entries, C)
+    A, D, bias = -torch.exp(rnd(16, C)), rnd(C), rnd(C) - 2.0
+    dt = torch.empty(entries, C, device="cuda")
+    states, outs = [before.clone(), before.clone()], [torch.empty(entries, C, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    k.gemm(dbc[:, :rank], w, dt, EPI_STORE_F32)
+    k.selective_scan(u, dbc, rank, rank + 16, dt, bias, A, D, gate, states[0], starts, slots, outs[0], longest=1)
+    k.scan_product_step(dbc, rank, w, u, bias, A, D, gate, states[1], slots, outs[1])
+    compare(("scan", "its state"), (outs[1], states[1]), (outs[0], states[0]))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_step_of_more_than_a_thousand_tokens(dtype):
     """Steps this long take the convolution several tokens a block: a long portion beside a short one, both continued
