@@ -354,10 +354,12 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(const bf16* __restrict_
 // (swz: kk for 256-byte rows and longer, kk >> 1 for 128-byte rows): the 16 lanes of an operand
 // read want one chunk of 16 different keys and then hit 16 different bank groups.  Values are
 // [VD][16] per page and are read in lane order; they need no swizzle.
+// SHARES == 2: a block has eight waves, four for each half of its tiles of keys, with rings of their own; the first four make the
+// two results one.  For blocks that have a unit to themselves, where the walk along the keys is a chain (see `launch`).
 // Two maps: wave w holds map w & 1 of the tokens of group w / 2 (tokens of two groups a block instead of four), KW
 // features of the keys from map * KW on enter its products, and the group's even wave makes the two results one.
-template <int KD, int VD, int MAPS, int WAVES = 4>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(VD <= 128 ? 2 : 1))) void attn_tiles_lds_kernel(const bf16* __restrict__ q, bf16* __restrict__ out,
+template <int KD, int VD, int MAPS, int WAVES = 4, int SHARES = 1>
+__global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_per_eu(VD <= 128 ? 2 : 1))) void attn_tiles_lds_kernel(const bf16* __restrict__ q, bf16* __restrict__ out,
                                                              const bf16* __restrict__ kc, const bf16* __restrict__ vc,
                                                              const int* __restrict__ block_table,
                                                              const int* __restrict__ positions,
@@ -376,10 +378,15 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(VD <
     constexpr int HALF_K = SHARE_K / 1024, HALF_V = SHARE_V / 1024;   // load instructions of a wave for its share of a page
     constexpr int SWZ_SHIFT = ROW_BYTES >= 256 ? 0 : 1;
     constexpr int R = (4 * (TILE_K + TILE_V) <= 65536) ? 4 : 2;   // tiles in each of the two rings (keys, values)
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[R * (TILE_K + TILE_V)];
+    constexpr int RINGS = R * (TILE_K + TILE_V);
+    __shared__ __attribute__((aligned(1024))) unsigned char all_rings[SHARES * RINGS];
+    static_assert(SHARES == 1 || (SHARES == 2 && MAPS == 1 && WAVES == 4 && WAVES * 32 * VD * 4 <= RINGS), "the second share's results pass through its rings' place");
     static_assert(MAPS == 1 || GROUPS * 32 * VD * 4 <= R * (TILE_K + TILE_V), "the second maps' results pass through the rings' place at the end");
     int lane = threadIdx.x & 63;
     int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // the same in all lanes: say so
+    const int share = SHARES == 1 ? 0 : wave / WAVES;
+    if (SHARES > 1) wave %= WAVES;
+    unsigned char* lds = all_rings + share * RINGS;
     int c = lane & 31, h = lane >> 5;
     int kvh = blockIdx.x % a.n_kv_heads;
     // Order of work.  A tile's work grows with its place in its entry, so the tiles are handed out
@@ -453,13 +460,16 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(VD <
     // most 32 of them; the kept keys among the window's tiles pass the mask there), then the window's.
     const ScoreBend bend{a.softcap, a.softcap > 0.0f ? a.scale / a.softcap : 0.0f, a.keep_first};
     int ns = (a.keep_first > 0 && t_begin > 0) ? (min(a.keep_first, t_begin) + 31) >> 5 : 0;
-    int n = ns + ((t_end - t_begin + 31) >> 5);
+    const int n_all = ns + ((t_end - t_begin + 31) >> 5);
+    // This share's tiles: n from `first` on, and `last` the last one there is of them (where the second share has none, or one fewer
+    // than the first, it goes through the block's last tile, and that as if it lay behind every query: masked).
+    const int n = SHARES == 1 ? n_all : (n_all + 1) >> 1, first = share * n, last = share ? n_all - 1 : n - 1;
     auto tile_t0 = [&](int tile) { return tile < ns ? 32 * tile : t_begin + 32 * (tile - ns); };
     int lp0 = t_begin >> 4;                          // the first window tile's first logical page
     // The request's page numbers for 64 logical pages at a time, one in each lane.
-    int pv_base = lp0;
-    auto load_pages = [&](int first) {
-        int pg = table[min(first + lane, a.table_width - 1)];
+    int pv_base = lp0 + 2 * max(min(first, last) - ns, 0);
+    auto load_pages = [&](int from) {
+        int pg = table[min(from + lane, a.table_width - 1)];
         return min(max(pg, 0), a.num_pages - 1);
     };
     int pv = load_pages(pv_base);
@@ -495,7 +505,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(VD <
     // same number of loads: where the tile would lie outside [0, n) the nearest real one is
     // loaded once more, into a slot that nobody reads; that costs less than telling the cases apart.
     auto issue = [&](int t, int t_mod) {
-        int tk = min(t + R, n - 1), tv = min(max(t + R - 1, 0), n - 1);
+        int tk = min(first + t + R, last), tv = min(first + max(t + R - 1, 0), last);
         int wk = tk - ns, wv = max(tv - ns, 0);                                // their numbers among the window's tiles
         if (__builtin_expect(wk >= 0 && lp0 + 2 * wk + 1 - pv_base >= 64, 0)) {      // tv <= tk: its pages stay in the window
             pv_base = lp0 + 2 * wv;
@@ -591,14 +601,14 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(VD <
             float alpha;
             bf16x8 pf[2], vf[VF];
             bool moved;
-            if (is_edge(t)) {
+            if (is_edge(first + t)) {
                 S_next = scores((s + 1) % R);         // (nothing real for the last tile: not used then)
                 read_values(s, vf);
-                moved = softmax_tile(S_cur, m, l, tile_t0(t), pos, lo, h, scale_log2e, alpha, true, far, bend);
+                moved = softmax_tile(S_cur, m, l, tile_t0(first + t), pos, lo, h, scale_log2e, alpha, true, far, bend);
             } else {
                 S_next = scores((s + 1) % R);
                 read_values(s, vf);
-                moved = softmax_tile(S_cur, m, l, tile_t0(t), pos, lo, h, scale_log2e, alpha, false, far, bend);
+                moved = softmax_tile(S_cur, m, l, tile_t0(first + t), pos, lo, h, scale_log2e, alpha, false, far, bend);
             }
             to_bf16(S_cur, pf);
             rescale(moved, alpha);
@@ -608,6 +618,32 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(VD <
         }
     }
 
+    if constexpr (SHARES == 2) {
+        // The second share's results meet the first's through the second's rings (every load into them has landed, and a barrier stands
+        // between their last reads and this), a lane's registers in the same lane's places; reference and sum through the first's.
+        wait_vmcnt_all();
+        block_sync();
+        float* meet = (float*)(all_rings + RINGS) + wave * (32 * VD) + lane;
+        float* meet_ml = (float*)all_rings + wave * 128 + lane;
+        if (share == 1) {
+            meet_ml[0] = m;
+            meet_ml[64] = l;
+#pragma unroll
+            for (int dt = 0; dt < VD / 32; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) meet[(dt * 16 + i) * 64] = O[dt][i];
+        }
+        block_sync();
+        if (share == 1) return;
+        const float m2 = meet_ml[0], l2 = meet_ml[64], most = fmaxf(m, m2), base = most == -INFINITY ? 0.0f : most;
+        const float f1 = __builtin_amdgcn_exp2f(m - base), f2 = __builtin_amdgcn_exp2f(m2 - base);
+        l = l * f1 + l2 * f2;
+        m = most;
+#pragma unroll
+        for (int dt = 0; dt < VD / 32; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) O[dt][i] = O[dt][i] * f1 + meet[(dt * 16 + i) * 64] * f2;
+    }
     float inv = 1.0f / (l + attn_sink_term_base2(a, head, m));      // (the sum is complete here: the sink joins it once)
     if constexpr (MAPS == 2) {
         // The odd wave of a pair leaves its map's results where the rings were (every load into them has landed, and the
@@ -777,8 +813,8 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
     const int* table = block_table + (size_t)e * a.table_width;
     bf16x8 qf[KD / 32];
     int token, pos_t, lo_t, t_begin, pv = 0;
-    auto load_pages = [&](int first) {
-        int pg = table[min(first + lane, a.table_width - 1)];
+    auto load_pages = [&](int from) {
+        int pg = table[min(from + lane, a.table_width - 1)];
         return min(max(pg, 0), a.num_pages - 1);
     };
     if (plain) {
@@ -1286,14 +1322,31 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
             // blocks' lengths then differ too much for one block to a unit).
             bool wide = false;
             if constexpr (KD == 128 && VD == 128) wide = max_seq_len >= ATTN_WIDE_FROM_KEYS;     // (head size 256 has no registers for two waves a SIMD)
-            if (wide) {
+            // Blocks that have a unit to themselves, over more than a few tiles of keys: two shares of the keys a block.  (Alone on its unit
+            // a block takes 1.17 us a tile, two shares 1.4 for two; in a full grid of short ones, two to a unit, their starts and
+            // ends hide behind each other and the shares lose.  us, four waves and shares, 32 heads on 8: 512 tokens over
+            // 8512 keys 257 and 172, of 64 features 211 and 140; 128 over 4128 128 and 89; eight portions of 64 over 3064 100 and 71;
+            // a prompt of 1024 41 and 34, of 130 15.3 and 15.5, of 17 9.4 and 12.2, eight of 250 22.6 and 33.5, twelve of 600 98 and 133;
+            // one of 2048, 512 blocks, 79 and 75, but with a window of 300 29 and 39.)  Beside single tokens, whose waves want LDS too,
+            // blocks for up to half of the units (64 heads on 8, 100 tokens over 2148 keys beside 16 single tokens 120 and 80).
+            bool shared_out = false;
+            const int btiles = a.n_tokens / (4 / MAPS * heads_tpt) + n_entries;
+            if constexpr (MAPS == 1 && KD <= 128 && VD <= 128) {
+                const int cus = llmrs_compute_units(), singles = split ? std::max(n_single, 0) : 0;
+                const long blocks = (long)btiles * a.n_kv_heads, busy = ((long)(a.n_tokens - singles) / (4 * heads_tpt) + n_entries - singles) * a.n_kv_heads;
+                shared_out = (split ? busy <= cus / 2 && blocks <= 2 * cus : blocks <= cus + 2 * a.n_kv_heads) && max_seq_len >= 256 &&
+                             (attn_reach(a) == 0 || attn_reach(a) >= 256);
+                if (shared_out)
+                    attn_tiles_lds_kernel<KD, VD, MAPS, 4, 2><<<btiles * a.n_kv_heads, 512, 0, stream>>>(q, out, kc, vc, table, positions, q_starts,
+                                                                                        n_entries, a, G / MAPS, heads_tpt, split, 0);
+            }
+            if (!shared_out && wide) {
                 if constexpr (KD == 128 && VD == 128) {
-                    int btiles = a.n_tokens / (8 / MAPS * heads_tpt) + n_entries;
-                    attn_tiles_lds_kernel<KD, VD, MAPS, 8><<<btiles * a.n_kv_heads, 512, 0, stream>>>(q, out, kc, vc, table, positions, q_starts,
+                    const int wide_btiles = a.n_tokens / (8 / MAPS * heads_tpt) + n_entries;
+                    attn_tiles_lds_kernel<KD, VD, MAPS, 8><<<wide_btiles * a.n_kv_heads, 512, 0, stream>>>(q, out, kc, vc, table, positions, q_starts,
                                                                                         n_entries, a, G / MAPS, heads_tpt, split, 0);
                 }
-            } else {
-                int btiles = a.n_tokens / (4 / MAPS * heads_tpt) + n_entries;
+            } else if (!shared_out) {
                 attn_tiles_lds_kernel<KD, VD, MAPS><<<btiles * a.n_kv_heads, 256, 0, stream>>>(q, out, kc, vc, table, positions, q_starts,
                                                                                      n_entries, a, G / MAPS, heads_tpt, split, llmrs_compute_units());
             }

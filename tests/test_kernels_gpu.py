@@ -388,6 +388,34 @@ def test_attention_at_131008_keys():
         assert (got[0].float() - ref).abs().max() <= 4e-3 + 2e-2 * float(ref.abs().max()), f"random query {i}"
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,window", [(8, 2, 128, 0), (6, 2, 64, 0), (16, 2, 64, 256), (4, 4, 128, 300), (5, 1, 64, 0)])
+def test_attention_of_few_portions_shares_their_keys_out(n_heads, n_kv, hd, window):
+    """Portions whose blocks have a unit to themselves go through their keys in two shares: one tile of keys (the second share has none),
+    two, an odd number, the second share's keys all behind some queries, windows that begin inside a share, a block's worth of
+    tokens and ragged ends."""
+    spans = [(0, 5), (0, 33), (31, 33), (60, 65), (64, 97), (0, 130), (290, 300), (511, 700), (640, 643), (1, 1023)]
+    case = PagedCase(torch.bfloat16, [hi for _, hi in spans], n_heads, n_kv, hd, 16, seed=hd + window)
+    g = torch.Generator().manual_seed(n_heads)
+    q_pos = [list(range(lo, hi)) for lo, hi in spans]
+    qs = [torch.randn((len(p), n_heads, hd), generator=g).to(torch.bfloat16) * 2 for p in q_pos]
+    got, at = case.run(qs, q_pos, window=window, n_single=0, bound=1024), 0
+    for r, p in enumerate(q_pos):
+        rows = got[at:at + len(p)].float()
+        at += len(p)
+        for i in sorted({0, 1, 17, 31, 32, 33, len(p) // 2, len(p) - 2, len(p) - 1} & set(range(len(p)))):
+            ref = case.reference(r, qs[r][i:i + 1], [p[i]], window=window)[0].float()
+            assert (rows[i] - ref).abs().max() <= 4e-3 + 2e-2 * float(ref.abs().max()), (r, i)
+
+
+def test_attention_of_many_portions_is_the_same_in_wide_blocks():
+    """Portions of more blocks than there are units, over a bound that gives blocks of four waves and one that gives eight: the same bits."""
+    case = PagedCase(torch.bfloat16, [40 + i % 30 for i in range(140)], 8, 2, 128, 16, seed=5)
+    q_pos = [list(range(n - 3 - n % 3, n)) for n in case.lens]
+    qs = [torch.randn((len(p), 8, 128), generator=torch.Generator().manual_seed(i)).to(torch.bfloat16) for i, p in enumerate(q_pos)]
+    four, eight = (case.run(qs, q_pos, n_single=0, bound=bound) for bound in (300, 32768))
+    assert torch.equal(four, eight)
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,window", [(8, 2, 128, 0), (6, 2, 128, 20000), (16, 2, 128, 0)])
 def test_attention_prompt_portions_over_long_caches(n_heads, n_kv, hd, window):
     """Prompt portions against caches of 33,000 and 40,000 keys in bfloat16: from 32,768 keys on the tiles' blocks
