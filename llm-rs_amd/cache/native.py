@@ -66,8 +66,9 @@ def _i32(a) -> np.ndarray:
     return np.ascontiguousarray(a, dtype=np.int32)
 
 
-def _ptr(a: np.ndarray):
-    return a.ctypes.data_as(c_void_p)
+def _ptr(a: np.ndarray) -> int:
+    # (`a.ctypes.data_as(c_void_p)` costs as much as the call that the address is for)
+    return a.__array_interface__["data"][0]
 
 
 class BatchOffsets:
@@ -101,6 +102,11 @@ class HostCore:
         self.groups = [tuple(int(x) for x in g) for g in groups]
         self.max_requests = max_requests
         self._n_off = self._lib.llmrs_batch_num_offsets(self._h)
+        # where the plan, its sources, a batch's offsets and what a commit finished come back, call after call
+        self._planned = np.zeros((4, max(max_requests, 1)), dtype=np.int32)
+        self._sources, self._finished = np.zeros(max(max_requests, 1), dtype=np.int32), np.zeros(max(max_requests, 1), dtype=np.int32)
+        self._offsets = np.zeros(self._n_off, dtype=np.int32)
+        self._plan_args = [_ptr(row) for row in self._planned]
 
     def __del__(self):
         if getattr(self, "_h", None):
@@ -182,16 +188,14 @@ class HostCore:
 
     def plan(self):
         """[(slot, start, count, samples)] of the next step."""
-        cap = self.max_requests
-        a = [np.zeros(cap, dtype=np.int32) for _ in range(4)]
-        n = self._check(self._lib.llmrs_sched_plan(self._h, *(_ptr(x) for x in a), cap))
-        return [(int(a[0][i]), int(a[1][i]), int(a[2][i]), bool(a[3][i])) for i in range(n)]
+        n = self._check(self._lib.llmrs_sched_plan(self._h, *self._plan_args, self.max_requests))
+        slots, starts, counts, samples = self._planned[:, :n].tolist()
+        return [(slot, start, count, bool(sample)) for slot, start, count, sample in zip(slots, starts, counts, samples)]
 
     def plan_sources(self) -> List[int]:
         """For each entry of the plan: the row of the step in flight whose sample is the entry's one token, or -1."""
-        src = np.zeros(self.max_requests, dtype=np.int32)
-        n = self._check(self._lib.llmrs_sched_plan_sources(self._h, _ptr(src), src.size))
-        return src[:n].tolist()
+        n = self._check(self._lib.llmrs_sched_plan_sources(self._h, _ptr(self._sources), self.max_requests))
+        return self._sources[:n].tolist()
 
     def launch(self) -> None:
         """The planned step has been started: `plan()` may be called for the step after it, before `commit()`
@@ -207,7 +211,7 @@ class HostCore:
 
     def build_planned(self, words: np.ndarray, fixed_widths=None):
         """Flatten the planned step; returns (offsets, n_tokens, n_sampling_rows)."""
-        off = np.zeros(self._n_off, dtype=np.int32)
+        off = self._offsets
         nt, nw = c_int32(0), c_int32(0)
         fw = _i32(fixed_widths) if fixed_widths is not None else None
         n = self._check(self._lib.llmrs_sched_build(self._h, _ptr(fw) if fw is not None else None, _ptr(words),
@@ -216,9 +220,8 @@ class HostCore:
 
     def commit(self, sampled) -> List[int]:
         sampled = _i32(sampled)
-        fin = np.zeros(self.max_requests, dtype=np.int32)
-        n = self._check(self._lib.llmrs_sched_commit(self._h, _ptr(sampled), len(sampled), _ptr(fin), fin.size))
-        return fin[:n].tolist()
+        n = self._check(self._lib.llmrs_sched_commit(self._h, _ptr(sampled), len(sampled), _ptr(self._finished), self.max_requests))
+        return self._finished[:n].tolist()
 
     def request_info(self, slot: int) -> dict:
         info = np.zeros(6, dtype=np.int32)

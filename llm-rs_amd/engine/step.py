@@ -193,6 +193,7 @@ class StepRunner:
     def __init__(self, model, cache: CacheManager, device, words_capacity: int = 1 << 16):
         self.model, self.cache, self.device = model, cache, torch.device(device)
         self._buffers: Dict[str, torch.Tensor] = {}
+        self._views: Dict[str, tuple] = {}      # name -> (shape, dtype, the view of its buffer handed out last)
         self._pinned = self.device.type == "cuda"
         self._host = [self._new_host(words_capacity) for _ in range(2)]
         self._events = [None, None]
@@ -219,6 +220,10 @@ class StepRunner:
         return torch.zeros(n, dtype=torch.int32, pin_memory=self._pinned)
 
     def workspace(self, name: str, shape, dtype: torch.dtype) -> torch.Tensor:
+        # A step asks for the same room layer after layer, and making a view costs as much host time as a launch.
+        last = self._views.get(name)
+        if last is not None and last[0] == shape and last[1] == dtype:
+            return last[2]
         n = 1
         for s in shape:
             n *= int(s)
@@ -235,7 +240,9 @@ class StepRunner:
             buf = torch.empty(cap, dtype=torch.uint8, device=self.device)
             self._buffers[name] = buf
             self._drop_graphs()         # recorded graphs hold the old addresses
-        return buf[:nbytes].view(dtype).view(*shape)
+        view = buf[:nbytes].view(dtype).view(*shape)
+        self._views[name] = (tuple(shape), dtype, view)       # (the one it replaces is of the old buffer where that has grown)
+        return view
 
     def _drop_graphs(self) -> None:
         """Forgets every recorded graph.  Destroying a graph frees device objects, so never during a recording."""

@@ -317,10 +317,12 @@ class HipKernels(Kernels):
         self._defers_norm = kept(lambda bf16, M, N, K: bool((lib.llmrs_gemm_defers_norm if bf16 else lib.llmrs_gemm_f32_defers_norm)(M, N, K)))
         self._stored_by_fours = kept(lambda head_dim, rotary_dim: bool(lib.llmrs_qkv_by_fours(head_dim, rotary_dim)))
         self._norm_plan = kept(self._ask_norm_plan)
+        self._workspace_floats = kept(lambda M, N, K: int(lib.llmrs_gemm_workspace_floats(int(M), int(N), int(K))))
+        self._next_parts = kept(lambda M, N, K: int(lib.llmrs_gemm_next_parts(int(M), int(N), int(K))))
 
     def gemm_workspace_floats(self, M: int, N: int, K: int) -> int:
         """Room that lets a product with too few blocks split K over blocks (the kernels' own rule)."""
-        return int(self.lib.llmrs_gemm_workspace_floats(int(M), int(N), int(K)))
+        return self._workspace_floats(M, N, K)
 
     def product_norms_its_rows(self, M: int, N: int, K: int, dtype: torch.dtype) -> bool:
         return self.gemm_defers_norm(M, N, K, dtype)
@@ -355,7 +357,7 @@ class HipKernels(Kernels):
     def gemm_next_parts(self, M: int, N: int, K: int) -> int:
         """Partial sums of squares per row that a product leaving a `NextNorm` writes (one per 16 features, for some
         shapes per 8): the second dimension of `NextNorm.sumsq`."""
-        return int(self.lib.llmrs_gemm_next_parts(int(M), int(N), int(K)))
+        return self._next_parts(M, N, K)
 
     def gemm_norms_whole(self, M: int, N: int, K: int) -> bool:
         """Whether the bfloat16 product of M rows with an [N, K] weight, adding into the stream with the workspace
@@ -433,7 +435,7 @@ class HipKernels(Kernels):
         n = out.shape[0]
         assert out.shape[1] == x.shape[1] == weight.shape[0]
         assert (rows is None and n == x.shape[0]) or (rows is not None and rows.dtype == torch.int32 and rows.shape[0] == n)
-        self._run(f"rmsnorm {n}x{x.shape[1]}", n * x.shape[1] * (4 + out.element_size()) + x.shape[1] * 4, 5 * n * x.shape[1], None,
+        self._run("" if self.times is None else f"rmsnorm {n}x{x.shape[1]}", n * x.shape[1] * (4 + out.element_size()) + x.shape[1] * 4, 5 * n * x.shape[1], None,
                   self.lib.llmrs_rmsnorm, self._stream(), _code(out.dtype), _p(out), _p(x), _p(weight), _p(rows),
                   n, x.shape[1], eps)
 
@@ -615,8 +617,10 @@ class HipKernels(Kernels):
             assert self.gemm_defers_norm(M, N, K, a.dtype)
         want = torch.float32 if epilogue in (EPI_STORE_F32, EPI_ACCUM_F32) else a.dtype
         assert out.dtype == want and out.shape[0] == M and out.shape[1] == (N // 2 if epilogue in _EPI_GATED else N)
-        moved = (M * K + N * K) * a.element_size() + out.numel() * out.element_size() * (2 if epilogue == EPI_ACCUM_F32 else 1)
-        label = f"gemm {M}x{N}x{K} {'norm+' if scale is not None else ''}{_EPI_NAMES[epilogue]}{('+norm' if whole else '+next') if leave is not None else ''}"
+        moved, label = 0, ""
+        if self.times is not None:
+            moved = (M * K + N * K) * a.element_size() + out.numel() * out.element_size() * (2 if epilogue == EPI_ACCUM_F32 else 1)
+            label = f"gemm {M}x{N}x{K} {'norm+' if scale is not None else ''}{_EPI_NAMES[epilogue]}{('+norm' if whole else '+next') if leave is not None else ''}"
         self._run(label, moved, 2 * M * N * K, a.dtype,
                   self.lib.llmrs_gemm, self._stream(), _code(a.dtype), _p(a), a.stride(0), _p(w), _p(out), out.stride(0),
                   M, N, K, epilogue + (glu or 0), _p(workspace),
@@ -666,7 +670,7 @@ class HipKernels(Kernels):
             assert k_cache.dtype == x.dtype and k_cache.is_contiguous() and v_cache.is_contiguous()
             assert k_cache.numel() == num_pages * n_kv_heads * page_size * head_dim == v_cache.numel()
         M, K, N = x.shape[0], x.shape[1], w.shape[0]
-        self._run(f"gemm {M}x{N}x{K} {'norm+' if scale is not None else ''}qkv+rope+cache", (M * K + N * K + M * N) * x.element_size(), 2 * M * N * K, x.dtype,
+        self._run("" if self.times is None else f"gemm {M}x{N}x{K} {'norm+' if scale is not None else ''}qkv+rope+cache", (M * K + N * K + M * N) * x.element_size(), 2 * M * N * K, x.dtype,
                   self.lib.llmrs_qkv_rope_cache,
                   self._stream(), _code(x.dtype), _p(x), x.stride(0), _p(w), _p(qkv), qkv.stride(0), x.shape[0], x.shape[1],
                   _p(positions), _p(slot_map), _p(inv_freq), rotary_dim, _p(k_cache), _p(v_cache), n_heads, n_kv_heads,
