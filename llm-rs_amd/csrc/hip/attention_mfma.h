@@ -354,11 +354,11 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(const bf16* __restrict_
 // (swz: kk for 256-byte rows and longer, kk >> 1 for 128-byte rows): the 16 lanes of an operand
 // read want one chunk of 16 different keys and then hit 16 different bank groups.  Values are
 // [VD][16] per page and are read in lane order; they need no swizzle.
-// SHARES == 2: a block has eight waves, four for each half of its tiles of keys, with rings of their own; the first four make the
-// two results one.  For blocks that have a unit to themselves, where the walk along the keys is a chain (see `launch`).
+// SHARES == 2: a block's waves own two groups of tokens, twice: two waves for each half of its tiles of keys, with rings of their own of RING
+// tiles; the first two make the results one.  For few blocks, where the walk along the keys is a chain (see `launch`).
 // Two maps: wave w holds map w & 1 of the tokens of group w / 2 (tokens of two groups a block instead of four), KW
 // features of the keys from map * KW on enter its products, and the group's even wave makes the two results one.
-template <int KD, int VD, int MAPS, int WAVES = 4, int SHARES = 1>
+template <int KD, int VD, int MAPS, int WAVES = 4, int SHARES = 1, int RING = 4>
 __global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_per_eu(VD <= 128 ? 2 : 1))) void attn_tiles_lds_kernel(const bf16* __restrict__ q, bf16* __restrict__ out,
                                                              const bf16* __restrict__ kc, const bf16* __restrict__ vc,
                                                              const int* __restrict__ block_table,
@@ -372,15 +372,15 @@ __global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_pe
     constexpr int PAGE_K = 16 * ROW_BYTES, PAGE_V = 16 * VD * 2;      // a page of one kv head: keys [16][KD], values [VD][16]
     constexpr int TILE_K = 2 * PAGE_K, TILE_V = 2 * PAGE_V;           // a tile's keys, its values: two pages
     constexpr int GROUPS = WAVES / MAPS;            // groups of tpt tokens in a block
-    static_assert(WAVES == 4 || WAVES == 8, "four waves, or eight for long caches");
+    static_assert(WAVES == 4 || WAVES == 8 || (WAVES == 2 && SHARES == 2), "four waves, eight for long caches, or two for each share");
     constexpr int SHARE_K = PAGE_K / (WAVES / 2), SHARE_V = PAGE_V / (WAVES / 2); // bytes of a page that one wave brings: two pages, WAVES / 2 waves each
     static_assert(SHARE_K >= 1024 && SHARE_K % 1024 == 0 && SHARE_V >= 1024 && SHARE_V % 1024 == 0, "a load instruction of a wave brings 1 KB");
     constexpr int HALF_K = SHARE_K / 1024, HALF_V = SHARE_V / 1024;   // load instructions of a wave for its share of a page
     constexpr int SWZ_SHIFT = ROW_BYTES >= 256 ? 0 : 1;
-    constexpr int R = (4 * (TILE_K + TILE_V) <= 65536) ? 4 : 2;   // tiles in each of the two rings (keys, values)
+    constexpr int R = (RING * (TILE_K + TILE_V) <= 65536) ? RING : 2;   // tiles in each of the two rings (keys, values)
     constexpr int RINGS = R * (TILE_K + TILE_V);
     __shared__ __attribute__((aligned(1024))) unsigned char all_rings[SHARES * RINGS];
-    static_assert(SHARES == 1 || (SHARES == 2 && MAPS == 1 && WAVES == 4 && WAVES * 32 * VD * 4 <= RINGS), "the second share's results pass through its rings' place");
+    static_assert(SHARES == 1 || (SHARES == 2 && MAPS == 1 && WAVES * 32 * VD * 4 <= RINGS), "the second share's results pass through its rings' place");
     static_assert(MAPS == 1 || GROUPS * 32 * VD * 4 <= R * (TILE_K + TILE_V), "the second maps' results pass through the rings' place at the end");
     int lane = threadIdx.x & 63;
     int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // the same in all lanes: say so
@@ -1322,24 +1322,34 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
             // blocks' lengths then differ too much for one block to a unit).
             bool wide = false;
             if constexpr (KD == 128 && VD == 128) wide = max_seq_len >= ATTN_WIDE_FROM_KEYS;     // (head size 256 has no registers for two waves a SIMD)
-            // Blocks that have a unit to themselves, over more than a few tiles of keys: two shares of the keys a block.  (Alone on its unit
-            // a block takes 1.17 us a tile, two shares 1.4 for two; in a full grid of short ones, two to a unit, their starts and
-            // ends hide behind each other and the shares lose.  us, four waves and shares, 32 heads on 8: 512 tokens over
-            // 8512 keys 257 and 172, of 64 features 211 and 140; 128 over 4128 128 and 89; eight portions of 64 over 3064 100 and 71;
-            // a prompt of 1024 41 and 34, of 130 15.3 and 15.5, of 17 9.4 and 12.2, eight of 250 22.6 and 33.5, twelve of 600 98 and 133;
-            // one of 2048, 512 blocks, 79 and 75, but with a window of 300 29 and 39.)  Beside single tokens, whose waves want LDS too,
-            // blocks for up to half of the units (64 heads on 8, 100 tokens over 2148 keys beside 16 single tokens 120 and 80).
+            // Where there are few blocks the walk of a block along its keys is what takes the time (alone on its unit four waves take 1.17 us a
+            // tile of 32 keys, and two shares 1.4 for two): blocks of half as many tokens, in two shares of their keys.  Fuller grids hide one
+            // block's waits behind another's, and there the second pass over the keys costs more.  us, blocks of four groups and shares, 32 heads on 8:
+            // 512 tokens over 8512 keys 257 and 139, of 64 features 209 and 117; 128 over 4128 128 and 71; a prompt of 512 24.4 and 18.3, of 1024
+            // 41 and 30, of 64 features 32 and 21.5; eight of 250 21 and 30, 2048 tokens with a window of 300 31 and 41.
+            // With more blocks the longest walk still decides where there are up to 24 blocks for every tile of its keys and little lies before the step's
+            // tokens (32 heads on 8, 1536 tokens 60 and 49, 1800 from position 100 93 and 60, 2048 78 and 70, of 64 features 60 and 49, prompts of
+            // 1200 and 300 61 and 36, of 1500 and 500 58 and 50; 40 heads on 5, 1333 tokens 57 and 34; but 64 heads on 8, 1024 tokens
+            // 46 and 50, twelve prompts of 600 98 and 133, 2048 tokens over 4096 keys 154 and 161).
+            // Beside single tokens, whose waves want the units' LDS too, blocks for as many units as their keys leave (64 heads on 8, 200 tokens
+            // over 2248 keys beside 4 of 300 115 and 56; 100 over 2148 beside 16 of 4000 120 and 81; 300 beside 20 of 8000 153 and 168).
             bool shared_out = false;
-            const int btiles = a.n_tokens / (4 / MAPS * heads_tpt) + n_entries;
             if constexpr (MAPS == 1 && KD <= 128 && VD <= 128) {
-                const int cus = llmrs_compute_units(), singles = split ? std::max(n_single, 0) : 0;
-                const long blocks = (long)btiles * a.n_kv_heads, busy = ((long)(a.n_tokens - singles) / (4 * heads_tpt) + n_entries - singles) * a.n_kv_heads;
-                shared_out = (split ? busy <= cus / 2 && blocks <= 2 * cus : blocks <= cus + 2 * a.n_kv_heads) && max_seq_len >= 256 &&
-                             (attn_reach(a) == 0 || attn_reach(a) >= 256);
+                const long cus = llmrs_compute_units(), share_btiles = a.n_tokens / (2 * heads_tpt) + n_entries, blocks = share_btiles * a.n_kv_heads;
+                if (split) {
+                    const long singles = std::max(n_single, 0), busy = ((a.n_tokens - singles) / (2 * heads_tpt) + n_entries - singles) * a.n_kv_heads;
+                    const long read = (single_keys > 0 ? single_keys : std::max(singles, 1L) * max_seq_len) * a.n_kv_heads * KD;
+                    shared_out = blocks <= 4 * cus && busy <= (read <= 1L << 25 ? cus : read <= 68L << 20 ? cus / 2 : 0);
+                } else {
+                    shared_out = blocks <= 2 * cus + 2 * a.n_kv_heads || (blocks <= 4 * cus + 2 * a.n_kv_heads && max_seq_len <= a.n_tokens + a.n_tokens / 4 &&
+                                                                          blocks <= 24L * ((max_seq_len + 31) / 32));
+                }
+                shared_out = shared_out && max_seq_len >= 256 && (attn_reach(a) == 0 || (attn_reach(a) >= 768 && blocks <= 2 * cus + 2 * a.n_kv_heads));
                 if (shared_out)
-                    attn_tiles_lds_kernel<KD, VD, MAPS, 4, 2><<<btiles * a.n_kv_heads, 512, 0, stream>>>(q, out, kc, vc, table, positions, q_starts,
-                                                                                        n_entries, a, G / MAPS, heads_tpt, split, 0);
+                    attn_tiles_lds_kernel<KD, VD, MAPS, 2, 2, KD == 64 && VD == 64 ? 4 : 2><<<blocks, 256, 0, stream>>>(
+                        q, out, kc, vc, table, positions, q_starts, n_entries, a, G / MAPS, heads_tpt, split, blocks > 2 * cus ? (int)cus : 0);
             }
+            const int btiles = a.n_tokens / (4 / MAPS * heads_tpt) + n_entries;
             if (!shared_out && wide) {
                 if constexpr (KD == 128 && VD == 128) {
                     const int wide_btiles = a.n_tokens / (8 / MAPS * heads_tpt) + n_entries;
