@@ -34,10 +34,11 @@ __device__ __forceinline__ void position_wave(float pos, float rate, float rate_
     s = fmaf(rest, c0, s0);
     c = fmaf(-rest, s0, c0);
 }
-template <class T, bool ADD, bool WAVES>
+// COPIES: the same rows into `copies` streams, `copy_stride` numbers apart.
+template <class T, bool ADD, bool WAVES, bool COPIES = false>
 __global__ void embed_rows_kernel(float* __restrict__ out, const T* __restrict__ table,
                                   const int* __restrict__ tokens, int D, int V, float scale,
-                                  const int* __restrict__ positions, const float* __restrict__ rates) {
+                                  const int* __restrict__ positions, const float* __restrict__ rates, int copies = 1, size_t copy_stride = 0) {
     int t = blockIdx.x;
     const float pos = WAVES ? (float)positions[t] : 0.0f;
     const int n_rates = (D + 1) / 2;
@@ -65,6 +66,8 @@ __global__ void embed_rows_kernel(float* __restrict__ out, const T* __restrict__
                     }
                 }
                 store8(dst + d, v);
+                if constexpr (COPIES)
+                    for (int c = 1; c < copies; ++c) store8(dst + c * copy_stride + d, v);
             }
             return;
         }
@@ -77,6 +80,8 @@ __global__ void embed_rows_kernel(float* __restrict__ out, const T* __restrict__
             v += (d & 1) ? c : s;
         }
         dst[d] = v;
+        if constexpr (COPIES)
+            for (int c = 1; c < copies; ++c) dst[c * copy_stride + d] = v;
     }
 }
 
@@ -176,6 +181,19 @@ static int embed_rows(hipStream_t stream, int dtype, float* out, const void* tab
 extern "C" int llmrs_embed_rows(hipStream_t stream, int dtype, float* out, const void* table, const int* tokens,
                                 int n_tokens, int D, int V, float scale) {
     return embed_rows<false, false>(stream, dtype, out, table, tokens, n_tokens, D, V, scale);
+}
+// The same rows into each of n_streams streams of [n_tokens, D].  (4 rows of 2048 into four streams, us: rows and then copies of the first
+// stream 3.2 + 2.4, and 1.3 between them; here 3.3.)
+extern "C" int llmrs_embed_streams(hipStream_t stream, int dtype, float* out, int n_streams, const void* table, const int* tokens,
+                                   int n_tokens, int D, int V, float scale) {
+    LLMRS_REQUIRE(n_streams >= 1 && n_tokens >= 0 && D > 0 && V > 0, "embed_streams: bad sizes T=%d D=%d V=%d streams=%d", n_tokens, D, V, n_streams);
+    LLMRS_REQUIRE(dtype == LLMRS_F32 || dtype == LLMRS_BF16, "embed_streams: unknown dtype %d", dtype);
+    if (n_tokens == 0) return 0;
+    const size_t stride = (size_t)n_tokens * D;
+    if (dtype == LLMRS_F32) embed_rows_kernel<float, false, false, true><<<n_tokens, 256, 0, stream>>>(out, (const float*)table, tokens, D, V, scale, nullptr, nullptr, n_streams, stride);
+    else embed_rows_kernel<bf16, false, false, true><<<n_tokens, 256, 0, stream>>>(out, (const bf16*)table, tokens, D, V, scale, nullptr, nullptr, n_streams, stride);
+    LLMRS_LAUNCH_CHECK("embed_streams");
+    return 0;
 }
 // out[t, :] += float(table[tokens[t], :]) * scale
 extern "C" int llmrs_embed_rows_add(hipStream_t stream, int dtype, float* out, const void* table, const int* tokens,

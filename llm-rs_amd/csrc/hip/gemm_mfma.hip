@@ -7,7 +7,8 @@
 //   M  > 64  "tiled": prompts.  Tiles of 128x128, 256x128, 256x192 or 256x256 outputs, K
 //            in steps of 64 through double-buffered LDS, v_mfma_f32_32x32x16_bf16; when
 //            K % 64 == 0 the tiles are loaded straight into LDS (global_load_lds), or, by
-//            the four waves of the large ones, through registers between the MFMAs.
+//            the four waves of the large ones, through registers between their MFMAs
+//            (v_mfma_f32_16x16x32_bf16).
 // Both need K % 8 == 0 and 16-byte aligned rows (16-byte loads); otherwise the
 // caller falls back to the plain kernel.
 //

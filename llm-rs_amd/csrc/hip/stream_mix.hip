@@ -277,14 +277,6 @@ __global__ void streams_mix_kernel(float* __restrict__ x, size_t stream_stride, 
     }
 }
 
-// Every stream starts as a copy of the first.
-__global__ void streams_copy_first_kernel(float* __restrict__ x, size_t stream_stride, int n_streams, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float v = x[i];
-    for (int s = 1; s < n_streams; ++s) x[(size_t)s * stream_stride + i] = v;
-}
-
 // out[i, :] = weight * groupnorm(sum_s w_in[s] x[s][rows[i] or i, :]) in the type `dtype` says.
 // zero: if given, [n_rows, D] 32-bit that is cleared on the way (room for a sublayer to add its result into);
 // combined: if given, [n_rows, D] 32-bit that gets the combined rows before the norm.
@@ -344,13 +336,5 @@ extern "C" int llmrs_streams_mix(hipStream_t stream, float* x, long stream_strid
     if (n == 0) return 0;
     streams_mix_kernel<<<ceil_div(n, 256), 256, 0, stream>>>(x, (size_t)stream_stride, n_streams, mix, w_out, y, (size_t)n);
     LLMRS_LAUNCH_CHECK("streams_mix");
-    return 0;
-}
-
-extern "C" int llmrs_streams_copy_first(hipStream_t stream, float* x, long stream_stride, int n_streams, long n) {
-    LLMRS_REQUIRE(n_streams >= 1 && n >= 0 && stream_stride >= n, "streams_copy_first: bad sizes");
-    if (n == 0 || n_streams == 1) return 0;
-    streams_copy_first_kernel<<<ceil_div(n, 256), 256, 0, stream>>>(x, (size_t)stream_stride, n_streams, (size_t)n);
-    LLMRS_LAUNCH_CHECK("streams_copy_first");
     return 0;
 }

@@ -147,8 +147,7 @@ class Model:
         if self.streamed:
             # [streams, T, hidden]: every copy starts as the embedding; blocks read and write all of them
             h = ctx.workspace("model.h", (self.streams, T, self.spec.hidden_size), torch.float32)
-            k.embed_rows(h[0], self.embedding, ctx.tokens, self.spec.embedding_scale)
-            k.streams_copy_first(h)
+            k.embed_streams(h, self.embedding, ctx.tokens, self.spec.embedding_scale)
         elif self.pairs is not None:
             h = ctx.workspace("model.h", (T, self.spec.hidden_size), torch.float32)
             table = self.spec.pair_table

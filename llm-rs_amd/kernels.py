@@ -179,6 +179,12 @@ class Kernels:
         reads the stream next (`NextNorm`), or None: then a norm kernel runs."""
         return None
 
+    def embed_streams(self, x: torch.Tensor, table: torch.Tensor, tokens: torch.Tensor, scale: float = 1.0) -> None:
+        """`embed_rows` into every stream of x [streams, T, hidden]."""
+        self.embed_rows(x[0], table, tokens, scale)
+        for stream in x[1:]:
+            stream.copy_(x[0])
+
     def products_step_mixers(self, n_tokens: int, n_entries: int, longest: int, dtype: torch.dtype, tensors) -> bool:
         """Whether the products of a recurrent mixer can do what it does with their sums themselves (`conv_product_step`,
         `mingru_product_step`, `scan_product_step`): every request brings one token, there are few, and what is read in
@@ -255,7 +261,7 @@ class HipKernels(Kernels):
             "llmrs_attention_ext": [V, I, V, I, V, I, V, V, V, I, V, V, V, V, I, I, I, I, I, I, I, I, F, V, c_size_t, I, I, ctypes.c_long, I, I, V, V, F, I, V, V, I, I, I, I, F, F, F],
             "llmrs_group_rmsnorm": [V, I, V, V, ctypes.c_long, I, V, V, V, I, I, I, F, V, V, V, V, V],
             "llmrs_streams_mix": [V, V, ctypes.c_long, I, V, V, V, ctypes.c_long],
-            "llmrs_streams_copy_first": [V, V, ctypes.c_long, I, ctypes.c_long],
+            "llmrs_embed_streams": [V, I, V, I, V, V, I, I, I, F],
             "llmrs_qkv_finish": [V, I, V, I, V, V, I, V, V, V, I, I, I, I, I, I, I, I, F, V, V, I, V, V, F, V, I, V, ctypes.c_long, V, V, V, I, I, I, F, I],
             "llmrs_linear_scan": [V, V, I, V, I, V, I, V, I, V, V, I, V, ctypes.c_long, V, V, I, I, I, I, I, I, V, I, V, V, I, I, I, V],
             "llmrs_silu_columns": [V, V, I, I, I, I],
@@ -799,10 +805,11 @@ class HipKernels(Kernels):
                   self.lib.llmrs_streams_mix, self._stream(), _p(x), x.stride(0), S, _p(mix), _p(w_out), _p(y), y.numel())
 
     # x[s] = x[0] for every s
-    def streams_copy_first(self, x: torch.Tensor) -> None:
-        assert x.dim() == 3 and x.dtype == torch.float32 and x.is_contiguous()
-        self._run("streams_copy_first", (x.shape[0] + 1) * x[0].numel() * 4, 0, None,
-                  self.lib.llmrs_streams_copy_first, self._stream(), _p(x), x.stride(0), x.shape[0], x[0].numel())
+    def embed_streams(self, x: torch.Tensor, table: torch.Tensor, tokens: torch.Tensor, scale: float = 1.0) -> None:
+        assert x.dim() == 3 and x.dtype == torch.float32 and x.is_contiguous() and tokens.dtype == torch.int32 and table.is_contiguous()
+        assert tuple(x.shape[1:]) == (tokens.shape[0], table.shape[1])
+        self._run("embed streams", x.numel() * 4 + x[0].numel() * table.element_size(), 0, None, self.lib.llmrs_embed_streams, self._stream(),
+                  _code(table.dtype), _p(x), x.shape[0], _p(table), _p(tokens), tokens.shape[0], table.shape[1], table.shape[0], float(scale))
 
     def qkv_finish(self, sums: torch.Tensor, bias: Optional[torch.Tensor], q: torch.Tensor, slot_map, k_cache, v_cache,
                    n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, page_size: int, num_pages: int, write_kv: bool,

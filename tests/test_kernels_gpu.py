@@ -407,6 +407,36 @@ def test_attention_of_few_portions_shares_their_keys_out(n_heads, n_kv, hd, wind
             assert (rows[i] - ref).abs().max() <= 4e-3 + 2e-2 * float(ref.abs().max()), (r, i)
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("more", [{}, {"keep_first": 40}, {"softcap": 15.0}, {"sink": True}, {"distance": True}, {"gate": True}])
+def test_attention_in_shares_with_what_bends_scores(hd, more):
+    """A portion alone (its keys in two shares) and the same portion eighty times (blocks of four groups), under a window, with kept first keys, a
+    soft cap, a sink, a distance penalty and a gate: the same but for the order of 32-bit sums and one rounding to bfloat16."""
+    heads, kv, n, count, window = 8, 2, 1500, 61, 900
+    pages = -(-n // 16)
+    g = torch.Generator(device=DEV).manual_seed(hd)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=DEV)
+    kc, vc, q = rnd(pages, kv, 16, hd).bfloat16(), rnd(pages, kv, hd, 16).bfloat16(), rnd(count, heads * hd).bfloat16() * 2
+    extra = {"keep_first": 40, "softcap": 15.0} if more.get("sink") else {}
+    extra.update({k: v for k, v in more.items() if v is not True})
+    if more.get("sink"):
+        extra["sink"] = rnd(heads)
+    if more.get("distance"):
+        extra["distance"] = (rnd(heads).abs() * 0.01, None)
+    gate = rnd(count, heads * hd) if more.get("gate") else None
+    rows = []
+    for times in (1, 80):
+        table = torch.randperm(pages, generator=torch.Generator().manual_seed(3)).int().repeat(times, 1).to(DEV)
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+        out = torch.empty(times * count, heads * hd, dtype=torch.bfloat16, device=DEV)
+        kernels().attention(q.repeat(times, 1), out, kc, vc, table, i32(list(range(times))).repeat_interleave(count), i32(list(range(n - count, n)) * times),
+                            i32([count * t for t in range(times + 1)]), i32([n] * times), heads, kv, hd, 16, pages, window, hd ** -0.5, None, n, 0,
+                            **extra, **({} if gate is None else {"gate": gate.repeat(times, 1)}))
+        rows.append(out[:count].float())
+    assert torch.isfinite(rows[0]).all()
+    torch.testing.assert_close(rows[0], rows[1], rtol=2.0 ** -7, atol=2.0 ** -7 * float(rows[1].abs().max()))
+
+
 def test_attention_of_many_portions_is_the_same_in_wide_blocks():
     """Portions of more blocks than there are units, over a bound that gives blocks of four waves and one that gives eight: the same bits."""
     case = PagedCase(torch.bfloat16, [40 + i % 30 for i in range(140)], 8, 2, 128, 16, seed=5)

@@ -387,6 +387,18 @@ def test_single_tokens_through_the_scan_equal_the_walk(entries, channels, states
     assert all(torch.equal(a, b) for a, b in zip(*got)) and not torch.equal(got[0][0], before)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("streams,tokens,width", [(1, 3, 8), (4, 1, 2048), (3, 17, 97), (16, 5, 1000)])
+def test_embeddings_into_every_stream(streams, tokens, width, dtype):
+    """The rows times the scale in 32-bit, the same bits in every stream."""
+    from llm_rs_amd.kernels import kernels
+    g = torch.Generator().manual_seed(width)
+    table, ids = torch.randn(50, width, generator=g).to(dtype), torch.randint(0, 50, (tokens,), generator=g).int()
+    out = torch.full((streams, tokens, width), float("nan"), device="cuda")
+    kernels().embed_streams(out, table.cuda(), ids.cuda(), 3.5)
+    assert torch.equal(out.cpu(), (table[ids.long()].float() * 3.5).expand(streams, tokens, width))
+
+
 @pytest.mark.parametrize("entries", [1, 4, 8, 9, 16])
 @pytest.mark.parametrize("channels,hidden,rank", [(16, 8, 8), (48, 72, 24), (512, 2048, 40), (4096, 2048, 128), (8208, 64, 72)])
 def test_products_that_step_their_mixers_equal_the_kernels_behind_plain_ones(channels, hidden, rank, entries):
