@@ -363,7 +363,8 @@ class StepRunner:
         off = core.build_batch(slots, starts, counts, tokens, want_rows, words, fixed_widths=widths)
         dev = self._upload(off.words)
         ctx = self._bind(dev, off, T, R, len(want_rows), list(zip(slots, starts, counts)), want_rows == list(range(T)))
-        return self._execute(ctx, widths)
+        logits = self._execute(ctx, widths)
+        return None if logits is None else logits[:]       # (a tensor of the caller's own over the same memory: the runner keeps its view)
 
     def run_planned(self, samples_in_flight: Optional[torch.Tensor] = None):
         """Runs the step the scheduler planned; returns (logits or None, rows that sample, the plan).
