@@ -1127,12 +1127,20 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         for (int ks = 0; ks < TK; ++ks) tb[ks] = *(const bf16x8*)(st + (offp ^ (ks * 64)));     // (the other half of k: its chunk's bit 2 the other way)
     };
     // (The tile's sums fill the accumulation registers; left to the compiler the tail's would push some of them out and in again in every
-    // k-tile, with waits for their MFMAs: 57344 x 8192 gated at 2064 rows 1446 us against 1400.  Written out they stay in ordinary registers.  The next
-    // that reads a result is a k-tile, or at the end a half of one, later: no wait states of its own are owed.)
+    // k-tile, with waits for their MFMAs: 57344 x 8192 gated at 2064 rows 1446 us against 1400.  Written out they stay in ordinary registers.  The
+    // waits that the compiler sees to for its own MFMAs are owed here: a vector instruction's write of a source, the zeroing of the sums
+    // for one, lies two wait states before the MFMA, which stand in front of it; and what reads a result does so seven or more after its MFMA,
+    // which the next k-tile's is, and `settle_tail` sees to at the end.)
     auto mult_tail = [&]() {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-        for (int ks = 0; ks < TK; ++ks) asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(tails[ks]) : "v"(tb[ks]), "v"(ta[ks]));
+        for (int ks = 0; ks < TK; ++ks) asm("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(tails[ks]) : "v"(tb[ks]), "v"(ta[ks]));
+#endif
+    };
+    auto settle_tail = [&]() {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+        for (int ks = 0; ks < TK; ++ks) asm volatile("s_nop 7" : "+v"(tails[ks]));
 #endif
     };
     // The order within a step.  A SIMD has this one wave only, so whatever keeps it from issuing its next MFMA leaves the matrix
@@ -1213,6 +1221,7 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
     __syncthreads();
     band_epilogue<BM, BN, EPI>(acc, fw_smem, out, ldc, M, N, m0, n0, epi);
     if constexpr (TAIL != 0) {
+        settle_tail();
         f32x4 tail = tails[0];
         if constexpr (TAIL == 2) tail += tails[TK - 1];
         if constexpr (TAIL == 1) {             // the halves of k together, through LDS behind what the bands used
