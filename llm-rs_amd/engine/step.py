@@ -224,6 +224,10 @@ class StepRunner:
         last = self._views.get(name)
         if last is not None and last[0] == shape and last[1] == dtype:
             return last[2]
+        if torch.is_inference_mode_enabled():
+            # (what is made in that mode could not be written by torch's operations in a step outside of it)
+            with torch.inference_mode(False):
+                return self.workspace(name, shape, dtype)
         n = 1
         for s in shape:
             n *= int(s)
