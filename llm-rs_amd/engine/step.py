@@ -400,7 +400,8 @@ class StepRunner:
             from ..kernels import kernels
             kernels().place_ids(ctx.tokens, dev[off.words:off.words + n], dev[off.words + n:off.words + 2 * n],
                                 samples_in_flight, self.model.spec.vocab_size)
-        return self._execute(ctx, widths), n_want, plan
+        logits = self._execute(ctx, widths)
+        return None if logits is None else logits[:], n_want, plan       # (as `run` does)
 
     def _execute(self, ctx: StepContext, graph_widths=None) -> Optional[torch.Tensor]:
         fresh = [slot for slot, start, _ in ctx.entries if start == 0]

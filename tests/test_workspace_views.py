@@ -31,3 +31,20 @@ def test_steps_inside_and_outside_of_inference_mode(engine):
     engine.runner.workspace("new", (3, 2), torch.float32).add_(1.0)
     engine.runner.workspace("new", (2, 2), torch.float32).add_(1.0)
     assert torch.equal(engine.step([StepEntry(slot, 0, [5, 6, 7], [2])]), want)
+
+
+@pytest.mark.parametrize("planned", [False, True])
+def test_a_callers_logits_may_be_reshaped_in_place(engine, planned):
+    core, runner = engine.cache.core, engine.runner
+    slot = core.add_request([5, 6, 7], 8)
+    assert slot >= 0
+    for step in range(3):
+        if planned:
+            logits, n, plan = runner.run_planned()
+            assert n == 1 and len(plan) == 1
+        else:
+            logits = engine.step([StepEntry(slot, 0, [5, 6, 7], [0, 1])])
+        assert tuple(logits.shape) == (1 if planned else 2, runner.model.spec.vocab_size)
+        if planned:
+            core.commit([int(logits[0].argmax())])
+        logits.t_()
