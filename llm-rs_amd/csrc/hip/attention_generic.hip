@@ -521,7 +521,8 @@ static int launch_generic(hipStream_t stream, const T* q, T* out, const T* k_cac
 // n_single: how many entries bring one token, if the host knows (-1: it does not); n_single == n_entries is the
 // caller's word that every entry brings exactly one token (then token t is entry t, and q_starts is not read);
 // single_keys: how many keys those entries see together (windows counted), if the host knows (0: it does not):
-// the matrix-core kernels choose the keys per wave by it.
+// the matrix-core kernels choose the keys per wave by it; portion_keys: how many keys the tokens of all other entries see together,
+// or 0: the same kernels choose by it whether the two kinds of entries run side by side.
 // v_dim: the width of a value (the cache's values are [page][kv_head][v_dim][slot], `out` has v_dim per head);
 // dist_r1, dist_r2: [n_heads] 32-bit, the distance penalty of AttnArgs (dist_r2 null: with the distance itself), or both null.
 // softcap, keep_first: the soft cap of the scores and the first keys that a window keeps (AttnArgs), or 0.
@@ -535,7 +536,7 @@ extern "C" int llmrs_attention_ext(hipStream_t stream, int dtype, const void* q,
                                    const int* token_entry, const int* positions, const int* q_starts,
                                    const int* seq_lens, int n_entries, int n_tokens, int n_heads, int n_kv_heads,
                                    int head_dim, int page_size, int num_pages, int window, float scale,
-                                   void* scratch, size_t scratch_bytes, int max_seq_len, int n_single, long single_keys,
+                                   void* scratch, size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, long portion_keys,
                                    int allow_mfma, int v_dim, const float* dist_r1, const float* dist_r2, float softcap,
                                    int keep_first, const float* sink, const float* gate, int gate_stride, int gate_per, int mask_chunk,
                                    int maps, float diff_lambda, float diff_eps, float diff_scale) {
@@ -563,7 +564,7 @@ extern "C" int llmrs_attention_ext(hipStream_t stream, int dtype, const void* q,
     if (dtype == LLMRS_BF16 && allow_mfma) {
         int took = llmrs_attention_bf16_mfma(stream, (const bf16*)q, (bf16*)out, (const bf16*)k_cache, (const bf16*)v_cache,
                                              block_table, token_entry, positions, q_starts, seq_lens, n_entries,
-                                             (float*)scratch, scratch_bytes, max_seq_len, n_single, single_keys, a);
+                                             (float*)scratch, scratch_bytes, max_seq_len, n_single, single_keys, portion_keys, a);
         if (took != 0) return took < 0 ? -1 : 0;
     }
     int rc = 0;
@@ -587,10 +588,10 @@ extern "C" int llmrs_attention(hipStream_t stream, int dtype, const void* q, int
                                const int* token_entry, const int* positions, const int* q_starts,
                                const int* seq_lens, int n_entries, int n_tokens, int n_heads, int n_kv_heads,
                                int head_dim, int page_size, int num_pages, int window, float scale,
-                               void* scratch, size_t scratch_bytes, int max_seq_len, int n_single, long single_keys,
+                               void* scratch, size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, long portion_keys,
                                int allow_mfma) {
     return llmrs_attention_ext(stream, dtype, q, q_stride, out, out_stride, k_cache, v_cache, block_table, table_width,
                                token_entry, positions, q_starts, seq_lens, n_entries, n_tokens, n_heads, n_kv_heads,
                                head_dim, page_size, num_pages, window, scale, scratch, scratch_bytes, max_seq_len, n_single,
-                               single_keys, allow_mfma, head_dim, nullptr, nullptr, 0.0f, 0, nullptr, nullptr, 0, 1, 0, 1, 0.0f, 0.0f, 0.0f);
+                               single_keys, portion_keys, allow_mfma, head_dim, nullptr, nullptr, 0.0f, 0, nullptr, nullptr, 0, 1, 0, 1, 0.0f, 0.0f, 0.0f);
 }

@@ -1289,7 +1289,7 @@ SideStream* llmrs_attention_side_stream();
 template <int KD, int VD, int MAPS>
 static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, const bf16* vc, const int* table,
                   const int* positions, const int* q_starts, const int* seq_lens, int n_entries, float* scratch,
-                  size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, const AttnArgs& a) {
+                  size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, long portion_keys, const AttnArgs& a) {
     int G = a.n_heads / a.n_kv_heads * MAPS;          // columns of a kv head
     int tpt = 32 / G;
     int chunk = llmrs_attention_split_chunk(n_single > 0 ? n_single : n_entries, a.n_kv_heads, KD, max_seq_len, single_keys);
@@ -1303,12 +1303,8 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
     // both kinds of work: the single tokens' kernels on the second stream, beside the tiles
     hipStream_t single_stream = stream;
     SideStream* side = nullptr;
-    // More tiles than three to a unit: one kind after the other.  Single tokens' waves that start between two rounds of tiles take the LDS that a
-    // tile's block of the next round waits for (64 heads on 8, 2048 tokens from position 2048 beside 16 single tokens over 4096 keys, 1032
-    // blocks, side by side 389 us, in turn 344; 1300 tokens, 656 blocks, 177 and 183; 32 heads on 8, 2000 tokens, 504 blocks, 228 and 280).
-    const int lone = std::max(n_single, 0);
-    const bool in_turn = ((long)(a.n_tokens - lone) / (4 * tpt) + n_entries - lone) * a.n_kv_heads > 3L * llmrs_compute_units();
-    if (split && !only_single && !in_turn) {
+    // (or one kind after the other, by the rule's answer)
+    if (split && !only_single && !llmrs_attention_in_turn(a.n_tokens, n_entries, n_single, single_keys, portion_keys, a.n_heads, a.n_kv_heads, KD, VD, MAPS)) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) side = llmrs_attention_side_stream();
         else (void)hipGetLastError();

@@ -101,16 +101,36 @@ extern "C" int llmrs_attention_split_chunk(long singles, int n_kv_heads, int hea
     return std::max(pick(keys), least);
 }
 
+// Whether a mixed step's single tokens wait for its tiles instead of running beside them on a stream of their own.  Their waves that start between two
+// rounds of tiles take the LDS that a tile's block of the next round waits for; in turn nothing hides the tiles' last
+// round, and the single tokens' keys come when the matrix cores are idle.  So in turn with more than three and a half blocks of tiles to a unit (two
+// run there at once) if the single tokens' keys, at 5 TB/s, take no more than a fifth of the tiles' time at 0.7 PFLOP/s.  Measured, us, side by
+// side and in turn (64 heads on 8): 2048 tokens from position 2048 beside 16 of 4096 keys, 0.18 of it, 389 and 339; 2940 from 1000 beside 14 of 1300,
+// 0.04, 352 and 327; but 1800 from the start beside 16 of 2000, 0.35, 109 and 122; 1600 from 2048 beside 250 of 2000, 1.9, 595 and 619; 32 on 8, 4096
+// from 2048 beside 37 of 1500, 0.12, 432 and 383; three of 1365 beside 100 of 2200, 2.8, 262 and 298.  Over 252 steps of
+// 1.5 to 8 blocks to a unit, 1 to 256 single tokens and seven shapes of heads what the rule puts in turn takes 0.84 to 1.025 of the time (from
+// three blocks on one step would take 1.07); with heads of 64, which need half of the LDS, in turn is 0.92 to 1.48 of it, and the gains are small.
+// portion_keys: how many keys the other entries' tokens see together; 0, unknown: as if every such entry began at position 0.
+extern "C" int llmrs_attention_in_turn(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
+                                       int v_dim, int maps) {
+    const int per_tile = 4 * (32 / std::max(n_heads / std::max(n_kv_heads, 1), 1)), portions = n_entries - n_single;
+    if (head_dim != 128 || v_dim != 128 || maps != 1 || n_single <= 0 || portions <= 0 || single_keys <= 0 || per_tile == 0) return 0;
+    const double tokens = n_tokens - n_single;
+    if (((n_tokens - n_single) / per_tile + portions) * (double)n_kv_heads <= 3.5 * llmrs_compute_units()) return 0;
+    const double seen = portion_keys > 0 ? (double)portion_keys : tokens * tokens / (2.0 * portions);
+    return (double)single_keys * n_kv_heads * (4.0 * head_dim) / 5e6 <= 0.2 * (seen * n_heads * (4.0 * head_dim) / 0.7e9);
+}
+
 // Heads of two maps (attention_mfma_maps.hip).
 int llmrs_attention_bf16_mfma_maps(hipStream_t stream, const bf16* q, bf16* out, const bf16* k_cache, const bf16* v_cache,
                                    const int* block_table, const int* positions, const int* q_starts, const int* seq_lens,
                                    int n_entries, float* scratch, size_t scratch_bytes, int max_seq_len, int n_single,
-                                   long single_keys, const AttnArgs& a);
+                                   long single_keys, long portion_keys, const AttnArgs& a);
 
 int llmrs_attention_bf16_mfma(hipStream_t stream, const bf16* q, bf16* out, const bf16* k_cache, const bf16* v_cache,
                               const int* block_table, const int* token_entry, const int* positions,
                               const int* q_starts, const int* seq_lens, int n_entries, float* scratch,
-                              size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, const AttnArgs& a) {
+                              size_t scratch_bytes, int max_seq_len, int n_single, long single_keys, long portion_keys, const AttnArgs& a) {
     (void)token_entry;
     int G = a.n_heads / a.n_kv_heads * a.maps;
     // (a distance penalty is these kernels' too)
@@ -123,10 +143,10 @@ int llmrs_attention_bf16_mfma(hipStream_t stream, const bf16* q, bf16* out, cons
     int rc;
     if (a.maps == 2) {
         rc = llmrs_attention_bf16_mfma_maps(stream, q, out, k_cache, v_cache, block_table, positions, q_starts, seq_lens, n_entries,
-                                            scratch, scratch_bytes, max_seq_len, n_single, single_keys, a);
+                                            scratch, scratch_bytes, max_seq_len, n_single, single_keys, portion_keys, a);
         if (rc <= 0) return rc;
     } else switch (a.head_dim) {
-#define CASE(HD) case HD: rc = launch<HD, HD, 1>(stream, q, out, k_cache, v_cache, block_table, positions, q_starts, seq_lens, n_entries, scratch, scratch_bytes, max_seq_len, n_single, single_keys, a); break;
+#define CASE(HD) case HD: rc = launch<HD, HD, 1>(stream, q, out, k_cache, v_cache, block_table, positions, q_starts, seq_lens, n_entries, scratch, scratch_bytes, max_seq_len, n_single, single_keys, portion_keys, a); break;
         CASE(32) CASE(64) CASE(96) CASE(128) CASE(192) CASE(256)
 #undef CASE
         default: return 0;

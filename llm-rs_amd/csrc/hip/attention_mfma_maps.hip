@@ -6,8 +6,8 @@
 int llmrs_attention_bf16_mfma_maps(hipStream_t stream, const bf16* q, bf16* out, const bf16* k_cache, const bf16* v_cache,
                                    const int* block_table, const int* positions, const int* q_starts, const int* seq_lens,
                                    int n_entries, float* scratch, size_t scratch_bytes, int max_seq_len, int n_single,
-                                   long single_keys, const AttnArgs& a) {
-#define RUN(KD, VD) return launch<KD, VD, 2>(stream, q, out, k_cache, v_cache, block_table, positions, q_starts, seq_lens, n_entries, scratch, scratch_bytes, max_seq_len, n_single, single_keys, a)
+                                   long single_keys, long portion_keys, const AttnArgs& a) {
+#define RUN(KD, VD) return launch<KD, VD, 2>(stream, q, out, k_cache, v_cache, block_table, positions, q_starts, seq_lens, n_entries, scratch, scratch_bytes, max_seq_len, n_single, single_keys, portion_keys, a)
     const bool both = a.v_dim == a.head_dim, one = 2 * a.v_dim == a.head_dim;
     switch (a.head_dim) {
         case 32: if (both) RUN(32, 32); break;

@@ -146,6 +146,19 @@ class StepContext:
             self._keys_seen[(window, mask_chunk)] = got
         return got
 
+    def portion_keys(self, window: int = 0, mask_chunk: int = 0) -> int:
+        """How many keys the tokens of all other entries see together (in chunks of positions: at most)."""
+        key = ("portions", window, mask_chunk)
+        got = self._keys_seen.get(key)
+        if got is None:
+            reach, got = window or mask_chunk or self.max_seq_len, 0
+            for _, start, count in self.entries:
+                if count > 1:
+                    rising = min(max(reach - start, 0), count)        # tokens that see everything before them
+                    got += rising * start + rising * (rising + 1) // 2 + (count - rising) * reach
+            self._keys_seen[key] = got
+        return got
+
     def room_for_next_norm(self, h: torch.Tensor, w: torch.Tensor):
         """For a part about to add a product with weight `w` into the stream `h`: a `kernels.NextNorm` for that
         product to fill (`kernels().gemm(..., leave=...)`; then `note_left(h, it)`), or None when the norm that

@@ -185,6 +185,9 @@ class Kernels:
         for stream in x[1:]:
             stream.copy_(x[0])
 
+    # Whether `attention` takes `portion_keys` (`engine/step.py`) in steps that mix single tokens and portions.
+    weighs_portions = False
+
     def products_step_mixers(self, n_tokens: int, n_entries: int, longest: int, dtype: torch.dtype, tensors) -> bool:
         """Whether the products of a recurrent mixer can do what it does with their sums themselves (`conv_product_step`,
         `mingru_product_step`, `scan_product_step`): every request brings one token, there are few, and what is read in
@@ -214,6 +217,8 @@ class Kernels:
 
 class HipKernels(Kernels):
     """Launches on the current torch stream of the tensors' device."""
+
+    weighs_portions = True
 
     def __init__(self):
         from .csrc.build import load_hip
@@ -253,12 +258,12 @@ class HipKernels(Kernels):
             "llmrs_gemm_norms_whole": [I, I, I],
             "llmrs_gemm_next_parts": [I, I, I],
             "llmrs_rope_kv_write": [V, I, V, I, V, V, V, I, I, V, V, I, I, I, I, I, I, I],
-            "llmrs_attention": [V, I, V, I, V, I, V, V, V, I, V, V, V, V, I, I, I, I, I, I, I, I, F, V, c_size_t, I, I, ctypes.c_long, I],
+            "llmrs_attention": [V, I, V, I, V, I, V, V, V, I, V, V, V, V, I, I, I, I, I, I, I, I, F, V, c_size_t, I, I, ctypes.c_long, ctypes.c_long, I],
             "llmrs_qkv_rope_cache": [V, I, V, I, V, V, I, I, I, V, V, V, I, V, V, I, I, I, I, I, I, V, c_size_t, I, V, I, F],
             "llmrs_argmax_rows": [V, V, I, I, I, V, V, c_size_t],
             "llmrs_sample_rows": [V, V, I, I, I, V, V],
             "llmrs_place_ids": [V, V, I, V, V, V, I, I, I],
-            "llmrs_attention_ext": [V, I, V, I, V, I, V, V, V, I, V, V, V, V, I, I, I, I, I, I, I, I, F, V, c_size_t, I, I, ctypes.c_long, I, I, V, V, F, I, V, V, I, I, I, I, F, F, F],
+            "llmrs_attention_ext": [V, I, V, I, V, I, V, V, V, I, V, V, V, V, I, I, I, I, I, I, I, I, F, V, c_size_t, I, I, ctypes.c_long, ctypes.c_long, I, I, V, V, F, I, V, V, I, I, I, I, F, F, F],
             "llmrs_group_rmsnorm": [V, I, V, V, ctypes.c_long, I, V, V, V, I, I, I, F, V, V, V, V, V],
             "llmrs_streams_mix": [V, V, ctypes.c_long, I, V, V, V, ctypes.c_long],
             "llmrs_embed_streams": [V, I, V, I, V, V, I, I, I, F],
@@ -694,7 +699,7 @@ class HipKernels(Kernels):
     def attention(self, q, out, k_cache, v_cache, block_table, token_entry, positions, q_starts, seq_lens,
                   n_heads, n_kv_heads, head_dim, page_size, num_pages, window, scale, scratch=None, max_seq_len=0, n_single=-1,
                   single_keys=0, value_dim=0, distance=None, softcap=0.0, keep_first=0, sink=None, gate=None, gate_per=1,
-                  mask_chunk=0, difference=None) -> None:
+                  mask_chunk=0, difference=None, portion_keys=0) -> None:
         """mask_chunk: > 0 (window 0): positions lie in chunks of so many, and a query sees its own chunk's keys only.
         difference = (lambda, eps, scale): differential attention: a head's head_dim features of q and of a key are two
         halves, each an attention of its own over the same values; with their results a1 and a2 the head's is
@@ -702,7 +707,8 @@ class HipKernels(Kernels):
         gate: float32 [T, n_heads * value_dim / gate_per] or None: every gate_per consecutive output features of a token
         are multiplied by the sigmoid of their number (32-bit, before the one rounding).
         sink: float32 [n_heads] or None: the softmax's denominator of head h also holds exp(sink[h]), once for every
-        query (a key without a value; not scaled).  single_keys: how many keys the single-token entries see together (windows counted), 0 if unknown.
+        query (a key without a value; not scaled).  single_keys: how many keys the single-token entries see together (windows counted), 0 if unknown;
+        portion_keys: how many the tokens of all other entries see (`weighs_portions`).
         value_dim: the width of a value where it is not a key's (0: the same).  distance: (r1, r2), float32 [n_heads]
         each: r1[h] * ln(1 + r2[h] * (i - j)) is taken off the scaled score of query i and key j; with r2 None r1[h] * (i - j).  softcap > 0: the
         scaled score s becomes softcap * tanh(s / softcap).  keep_first: with a window, the request's first so many
@@ -715,7 +721,7 @@ class HipKernels(Kernels):
                 or mask_chunk > 0 or difference is not None:
             return self._attention_ext(q, out, k_cache, v_cache, block_table, token_entry, positions, q_starts, seq_lens, n_heads,
                                        n_kv_heads, head_dim, page_size, num_pages, window, scale, scratch, max_seq_len, n_single,
-                                       single_keys, v_dim, distance, softcap, keep_first, sink, gate, gate_per, mask_chunk, difference)
+                                       single_keys, v_dim, distance, softcap, keep_first, sink, gate, gate_per, mask_chunk, difference, portion_keys)
         T = q.shape[0]
         assert token_entry.shape[0] == T and positions.shape[0] == T and out.shape[0] == T
         moved = flops = 0
@@ -730,11 +736,11 @@ class HipKernels(Kernels):
                   _p(block_table), block_table.shape[1], _p(token_entry), _p(positions), _p(q_starts), _p(seq_lens),
                   block_table.shape[0], T, n_heads, n_kv_heads, head_dim, page_size, num_pages, window, scale,
                   _p(scratch), 0 if scratch is None else scratch.numel() * scratch.element_size(), int(max_seq_len),
-                  int(n_single), int(single_keys), int(self.allow_mfma))
+                  int(n_single), int(single_keys), int(portion_keys), int(self.allow_mfma))
 
     def _attention_ext(self, q, out, k_cache, v_cache, block_table, token_entry, positions, q_starts, seq_lens, n_heads,
                        n_kv_heads, head_dim, page_size, num_pages, window, scale, scratch, max_seq_len, n_single, single_keys,
-                       v_dim, distance, softcap=0.0, keep_first=0, sink=None, gate=None, gate_per=1, mask_chunk=0, difference=None) -> None:
+                       v_dim, distance, softcap=0.0, keep_first=0, sink=None, gate=None, gate_per=1, mask_chunk=0, difference=None, portion_keys=0) -> None:
         T = q.shape[0]
         maps = 1 if difference is None else 2
         lam, diff_eps, diff_scale = (0.0, 0.0, 0.0) if difference is None else difference
@@ -765,7 +771,7 @@ class HipKernels(Kernels):
                   _p(block_table), block_table.shape[1], _p(token_entry), _p(positions), _p(q_starts), _p(seq_lens),
                   block_table.shape[0], T, n_heads, n_kv_heads, head_dim, page_size, num_pages, window, scale,
                   _p(scratch), 0 if scratch is None else scratch.numel() * scratch.element_size(), int(max_seq_len),
-                  int(n_single), int(single_keys), int(self.allow_mfma), v_dim, _p(r1), _p(r2), float(softcap), int(keep_first), _p(sink),
+                  int(n_single), int(single_keys), int(portion_keys), int(self.allow_mfma), v_dim, _p(r1), _p(r2), float(softcap), int(keep_first), _p(sink),
                   _p(gate), 0 if gate is None else gate.stride(0), int(gate_per), int(mask_chunk), maps, float(lam), float(diff_eps), float(diff_scale))
 
     # out[i, :] = weight * groupnorm(sum_s w_in[s] * x[s][rows[i] or i, :]); x: [T, D] or [S, T, D] float32

@@ -93,6 +93,12 @@ class KeyedBySplitChunk:
             return now[1]
         return ctx.single_keys(*self.recording_signature[3:])
 
+    def _portions(self, ctx) -> dict:
+        """What `attention` is told about entries with several tokens beside single ones."""
+        if not kernels().weighs_portions or not 0 < ctx.n_single < ctx.n_entries:
+            return {}
+        return {"portion_keys": ctx.portion_keys(*self.recording_signature[3:])}
+
 
 class Attention(KeyedBySplitChunk, Mixer):
     graph_safe = True
@@ -410,7 +416,7 @@ class Attention(KeyedBySplitChunk, Mixer):
                     distance=None if self.distance is None else (self.r1, self.r2), softcap=self.softcap, keep_first=self.keep_first, sink=self.sink,
                     gate=sums[:, self.qkv_width:] if self.gate is not None else None, gate_per=1 if self.gate == "feature" else self.value_dim,
                     **({} if self.mask_chunk == 0 else {"mask_chunk": self.mask_chunk}),
-                    **({} if self.maps == 1 else {"difference": (self.diff_lambda, self.diff_eps, 1.0 - self.diff_base)}))
+                    **({} if self.maps == 1 else {"difference": (self.diff_lambda, self.diff_eps, 1.0 - self.diff_base)}), **self._portions(ctx))
         k.gemm(o, self.w_o, h, EPI_ACCUM_F32, ctx.gemm_workspace(o, self.w_o))
         if self.has_o_bias and not self.output_bias_left_to_holder:
             k.add_bias_rows(h, self.o_bias)
@@ -453,7 +459,7 @@ class Attention(KeyedBySplitChunk, Mixer):
         k.attention(qkv[:, :self.q_size], o, cache.k, cache.v, ctx.block_tables[g], ctx.token_entry, ctx.positions,
                     ctx.q_starts, ctx.seq_lens, self.heads, self.kv_heads, self.head_dim, cache.page_size,
                     cache.num_pages, self.window, self.scale, scratch, ctx.max_seq_len, ctx.n_single,
-                    self._keys_for_the_split(ctx))
+                    self._keys_for_the_split(ctx), **self._portions(ctx))
         leave = ctx.room_for_next_norm(h, self.w_o) if not self.has_o_bias else None
         k.gemm(o, self.w_o, h, EPI_ACCUM_F32, ctx.gemm_workspace(o, self.w_o), **({} if leave is None else {"leave": leave}))
         if self.has_o_bias and not self.output_bias_left_to_holder:

@@ -1,6 +1,7 @@
 """Each kernel alone against the plain reference of its part, at sizes other than
 the tiny models': widths and vocabularies that are no power of two, head sizes in
 steps of 16, any number of heads and groups."""
+import ctypes
 import math
 
 import pytest
@@ -248,7 +249,7 @@ class PagedCase:
                 self.kc[page, :, :hi - lo, :] = self.k[r][lo:hi].permute(1, 0, 2)
                 self.vc[page, :, :, :hi - lo] = self.v[r][lo:hi].permute(1, 2, 0)
 
-    def run(self, q_list, q_pos_list, window=0, scale=None, scratch_floats=1 << 22, bound=None, n_single=-1, single_keys=0):
+    def run(self, q_list, q_pos_list, window=0, scale=None, scratch_floats=1 << 22, bound=None, n_single=-1, single_keys=0, **more):
         """q_list[r]: [n_r, heads, hd] queries of request r at positions q_pos_list[r]."""
         scale = 1.0 / math.sqrt(self.hd) if scale is None else scale
         q = torch.cat(q_list).reshape(-1, self.n_heads * self.hd).to(DEV)
@@ -263,7 +264,7 @@ class PagedCase:
         scratch = torch.empty(scratch_floats, dtype=torch.float32, device=DEV)
         kernels().attention(q, out, self.kc.to(DEV), self.vc.to(DEV), self.tables.to(DEV), entry, pos, q_starts, seq_lens,
                             self.n_heads, self.n_kv, self.hd, self.ps, self.num_pages, window, scale, scratch,
-                            max(lens_now) if bound is None else bound, n_single, single_keys)
+                            max(lens_now) if bound is None else bound, n_single, single_keys, **more)
         return out.cpu().view(T, self.n_heads, self.hd)
 
     def reference(self, r, q, positions, window=0, scale=None):
@@ -435,6 +436,39 @@ def test_attention_in_shares_with_what_bends_scores(hd, more):
         rows.append(out[:count].float())
     assert torch.isfinite(rows[0]).all()
     torch.testing.assert_close(rows[0], rows[1], rtol=2.0 ** -7, atol=2.0 ** -7 * float(rows[1].abs().max()))
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,portions,singles,window,in_turn", [
+    (64, 8, 128, [(2048, 200)], [300, 17, 255, 300], 0, False),           # blocks of half as many tokens, in two shares of their keys
+    (32, 8, 64, [(1000, 300)], [2000] * 6, 0, False), (6, 2, 64, [(290, 33), (5, 2)], [31, 700, 32], 0, False), (16, 2, 128, [(1500, 90)], [1, 1600, 900], 800, False),
+    (64, 8, 128, [(0, 1800)], [2000 - i for i in range(16)], 0, False),   # more than three blocks to a unit, side by side
+    (64, 8, 128, [(2048, 2048)], [4095 - 7 * i for i in range(16)], 0, True), (32, 8, 128, [(1500, 2100), (1000, 1999)], [1, 16, 17, 900], 0, True)])
+def test_attention_of_portions_beside_single_tokens(n_heads, n_kv, hd, portions, singles, window, in_turn):
+    """Portions between single tokens, on both sides of the rules that choose blocks and order (shares of the keys; in turn or side by
+    side): rows of every portion and every single token against the formula in 64 bits.  (Bound as for portions alone.)"""
+    half = len(singles) // 2
+    spans = [(n - 1, 1) for n in singles[:half]] + portions[:1] + [(n - 1, 1) for n in singles[half:]] + portions[1:]
+    case = PagedCase(torch.bfloat16, [start + count for start, count in spans], n_heads, n_kv, hd, 16, seed=len(singles))
+    g = torch.Generator().manual_seed(n_heads)
+    pos = [list(range(start, start + count)) for start, count in spans]
+    qs = [torch.randn((len(p), n_heads, hd), generator=g).to(torch.bfloat16) * 2 for p in pos]
+    sees = lambda p: min(p + 1, window or p + 1)
+    keys, seen = sum(sees(n - 1) for n in singles), sum(sees(p) for ps in pos if len(ps) > 1 for p in ps)
+    longest = max(start + count for start, count in spans)
+    k = kernels()
+    assert bool(k.lib.llmrs_attention_in_turn(sum(map(len, pos)), len(pos), len(singles), ctypes.c_long(keys), ctypes.c_long(seen), n_heads, n_kv, hd, hd, 1)) == in_turn
+    got, at = case.run(qs, pos, window=window, scratch_floats=k.attention_scratch_floats(len(pos), n_heads, hd, longest, n_kv, len(singles)),
+                       n_single=len(singles), single_keys=keys, portion_keys=seen), 0
+    for r, places in enumerate(pos):
+        rows, q = got[at:at + len(places)].to(DEV).double(), qs[r].to(DEV).double()
+        at += len(places)
+        K, V = case.k[r].to(DEV).double(), case.v[r].to(DEV).double()
+        for i in sorted({0, 1, 15, 16, 31, 32, len(places) // 2, len(places) - 2, len(places) - 1} & set(range(len(places)))):
+            lo, hi = places[i] + 1 - sees(places[i]), places[i] + 1
+            for h in range(n_heads):
+                kv = h // (n_heads // n_kv)
+                ref = torch.softmax((K[lo:hi, kv] @ q[i, h]) * hd ** -0.5, 0) @ V[lo:hi, kv]
+                assert (rows[i, h] - ref).abs().max() <= 4e-3 + 2e-2 * float(ref.abs().max()), (r, i, h)
 
 
 def test_attention_of_many_portions_is_the_same_in_wide_blocks():
