@@ -152,6 +152,8 @@ int llmrs_attention_bf16_mfma(hipStream_t stream, const bf16* q, bf16* out, cons
 // that see single_keys keys together (0: unknown; 1 gives the smallest chunk any number of keys can give for these
 // entries and this bound, which is what the scratch is sized by).
 extern "C" int llmrs_attention_split_chunk(long singles, int n_kv_heads, int head_dim, int max_seq_len, long single_keys);
+extern "C" int llmrs_attention_in_shares(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
+                                         int reach, int max_seq_len);
 extern "C" int llmrs_attention_in_turn(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
                                        int v_dim, int maps);
 

@@ -1323,32 +1323,14 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
             // blocks' lengths then differ too much for one block to a unit).
             bool wide = false;
             if constexpr (KD == 128 && VD == 128) wide = max_seq_len >= ATTN_WIDE_FROM_KEYS;     // (head size 256 has no registers for two waves a SIMD)
-            // Where there are few blocks the walk of a block along its keys is what takes the time (alone on its unit four waves take 1.17 us a
-            // tile of 32 keys, and two shares 1.4 for two): blocks of half as many tokens, in two shares of their keys.  Fuller grids hide one
-            // block's waits behind another's, and there the second pass over the keys costs more.  us, blocks of four groups and shares, 32 heads on 8:
-            // 512 tokens over 8512 keys 257 and 139, of 64 features 209 and 117; 128 over 4128 128 and 71; a prompt of 512 24.4 and 18.3, of 1024
-            // 41 and 30, of 64 features 32 and 21.5; eight of 250 21 and 30, 2048 tokens with a window of 300 31 and 41.
-            // With more blocks the longest walk still decides where there are up to 24 blocks for every tile of its keys and little lies before the step's
-            // tokens (32 heads on 8, 1536 tokens 60 and 49, 1800 from position 100 93 and 60, 2048 78 and 70, of 64 features 60 and 49, prompts of
-            // 1200 and 300 61 and 36, of 1500 and 500 58 and 50; 40 heads on 5, 1333 tokens 57 and 34; but 64 heads on 8, 1024 tokens
-            // 46 and 50, twelve prompts of 600 98 and 133, 2048 tokens over 4096 keys 154 and 161).
-            // Beside single tokens, whose waves want the units' LDS too, blocks for as many units as their keys leave (64 heads on 8, 200 tokens
-            // over 2248 keys beside 4 of 300 115 and 56; 100 over 2148 beside 16 of 4000 120 and 81; 300 beside 20 of 8000 153 and 168).
+            // Blocks of half as many tokens, in two shares of their keys, where the rule says so.
             bool shared_out = false;
             if constexpr (MAPS == 1 && KD <= 128 && VD <= 128) {
-                const long cus = llmrs_compute_units(), share_btiles = a.n_tokens / (2 * heads_tpt) + n_entries, blocks = share_btiles * a.n_kv_heads;
-                if (split) {
-                    const long singles = std::max(n_single, 0), busy = ((a.n_tokens - singles) / (2 * heads_tpt) + n_entries - singles) * a.n_kv_heads;
-                    const long read = (single_keys > 0 ? single_keys : std::max(singles, 1L) * max_seq_len) * a.n_kv_heads * KD;
-                    shared_out = blocks <= 4 * cus && busy <= (read <= 1L << 25 ? cus : read <= 68L << 20 ? cus / 2 : 0);
-                } else {
-                    shared_out = blocks <= 2 * cus + 2 * a.n_kv_heads || (blocks <= 4 * cus + 2 * a.n_kv_heads && max_seq_len <= a.n_tokens + a.n_tokens / 4 &&
-                                                                          blocks <= 24L * ((max_seq_len + 31) / 32));
-                }
-                shared_out = shared_out && max_seq_len >= 256 && (attn_reach(a) == 0 || (attn_reach(a) >= 768 && blocks <= 2 * cus + 2 * a.n_kv_heads));
+                const int cus = llmrs_compute_units(), blocks = (a.n_tokens / (2 * heads_tpt) + n_entries) * a.n_kv_heads;
+                shared_out = llmrs_attention_in_shares(a.n_tokens, n_entries, split ? std::max(n_single, 1) : 0, single_keys, portion_keys, a.n_heads, a.n_kv_heads, KD, attn_reach(a), max_seq_len);
                 if (shared_out)
                     attn_tiles_lds_kernel<KD, VD, MAPS, 2, 2, KD == 64 && VD == 64 ? 4 : 2><<<blocks, 256, 0, stream>>>(
-                        q, out, kc, vc, table, positions, q_starts, n_entries, a, G / MAPS, heads_tpt, split, blocks > 2 * cus ? (int)cus : 0);
+                        q, out, kc, vc, table, positions, q_starts, n_entries, a, G / MAPS, heads_tpt, split, blocks > 2 * cus ? cus : 0);
             }
             const int btiles = a.n_tokens / (4 / MAPS * heads_tpt) + n_entries;
             if (!shared_out && wide) {

@@ -101,23 +101,62 @@ extern "C" int llmrs_attention_split_chunk(long singles, int n_kv_heads, int hea
     return std::max(pick(keys), least);
 }
 
+// How many keys the tokens of entries with several tokens see together: what the caller says (portion_keys), or, where that is 0, as if
+// every such entry began at position 0.
+static double keys_of_portions(int n_tokens, int n_entries, int n_single, long portion_keys) {
+    const double tokens = n_tokens - n_single;
+    return portion_keys > 0 ? (double)portion_keys : tokens * tokens / (2.0 * std::max(n_entries - n_single, 1));
+}
+
+// Whether the tiles' blocks are of half as many tokens, in two shares of their keys (attn_tiles_lds_kernel with two shares; one map, heads of up to 128).
+// Where there are few blocks the walk of a block along its keys is what takes the time (alone on its unit four waves take 1.17 us a
+// tile of 32 keys, and two shares 1.4 for two).  Fuller grids hide one
+// block's waits behind another's, and there the second pass over the keys costs more.  us, blocks of four groups and shares, 32 heads on 8:
+// 512 tokens over 8512 keys 257 and 139, of 64 features 209 and 117; 128 over 4128 128 and 71; a prompt of 512 24.4 and 18.3, of 1024
+// 41 and 30, of 64 features 32 and 21.5; eight of 250 21 and 30; under windows, 400 tokens from 3000 on 44 and 24 (768), 55 and 28 (1024), 1000 tokens 45 and
+// 32 (768), 84 and 49 (2048, of 64 features), but 2048 tokens under one of 300 31 and 41; windows in between were not measured.
+// With more blocks the longest walk still decides where there are up to 24 blocks for every tile of its keys and little lies before the step's
+// tokens (32 heads on 8, 1536 tokens 60 and 49, 1800 from position 100 93 and 60, 2048 78 and 70, of 64 features 60 and 49, prompts of
+// 1200 and 300 61 and 36, of 1500 and 500 58 and 50; 40 heads on 5, 1333 tokens 57 and 34; but 64 heads on 8, 1024 tokens
+// 46 and 50, twelve prompts of 600 98 and 133, 2048 tokens over 4096 keys 154 and 161).  (blocks: as many as the tokens could make; a prompt or two of 2048
+// tokens in all are within the slack of two.)
+// Beside single tokens (n_single > 0), whose waves want the units' LDS too, blocks for as many units as their keys leave: all up to 2^25 keys times
+// kv heads and features, half up to 68 * 2^20 (64 heads on 8, 200 tokens over 2248 keys beside 4 of 300 115 and 56; 100 over 2148 beside 16 of 4000 120
+// and 81; 300 beside 20 of 8000 153 and 168), and a walk that is not over before theirs is, nor within what a step on two streams takes anyway: 25 us and four
+// fifths of their keys' time at 5 TB/s.  The walk is taken for the portions' mean place and half their length.  (32 heads on 8, two of 109 tokens from 300 on
+// beside 10 of 3200 69.7 and 73.4; 64 on 8, 94 from 300 beside 25 of 2600 72.9 and 77.2; heads of 64, 506 from 300 beside 15 44.0 and 47.9; 230 such steps with
+// shares 0.44 to 1.2 of the time, of which the walk's rule leaves 119, 0.44 to 1.05, and four of the others would gain more than 5 %.)
+extern "C" int llmrs_attention_in_shares(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
+                                         int reach, int max_seq_len) {
+    const long cus = llmrs_compute_units(), per_block = 2L * std::max(32 / std::max(n_heads / std::max(n_kv_heads, 1), 1), 1);
+    const long blocks = (n_tokens / per_block + n_entries) * n_kv_heads, few = 2 * cus + 2 * n_kv_heads;
+    if (max_seq_len < 256 || (reach > 0 && (reach < 768 || blocks > few))) return 0;
+    if (n_single <= 0)
+        return blocks <= few || (blocks <= 4 * cus + 2 * n_kv_heads && max_seq_len <= n_tokens + n_tokens / 4 && blocks <= 24L * ((max_seq_len + 31) / 32));
+    const int tokens = n_tokens - n_single, portions = n_entries - n_single;
+    if (tokens <= 0 || portions <= 0 || blocks > 4 * cus) return 0;
+    const long busy = (tokens / per_block + portions) * n_kv_heads;
+    const long read = (single_keys > 0 ? single_keys : (long)n_single * max_seq_len) * n_kv_heads * head_dim;
+    const double walk = keys_of_portions(n_tokens, n_entries, n_single, portion_keys) / tokens + tokens / (2.0 * portions);
+    const double walk_us = walk / 32.0 * (head_dim >= 128 ? 1.17 : 0.79), single_us = (double)read * 4.0 / 5e6;
+    return busy <= (read <= 1L << 25 ? cus : read <= 68L << 20 ? cus / 2 : 0) && walk_us >= std::max(25.0, 0.8 * single_us);
+}
+
 // Whether a mixed step's single tokens wait for its tiles instead of running beside them on a stream of their own.  Their waves that start between two
 // rounds of tiles take the LDS that a tile's block of the next round waits for; in turn nothing hides the tiles' last
-// round, and the single tokens' keys come when the matrix cores are idle.  So in turn with more than three and a half blocks of tiles to a unit (two
-// run there at once) if the single tokens' keys, at 5 TB/s, take no more than a fifth of the tiles' time at 0.7 PFLOP/s.  Measured, us, side by
+// round, and the single tokens' keys come when the matrix cores are idle.  So in turn with more than three and three quarters of a block of tiles to a unit (two
+// run there at once; 1800 tokens from the start beside 16 of 300, 3.5 of them, 104 and 108) if the single tokens' keys, at 5 TB/s, take no more than a fifth of the tiles' time at 0.7 PFLOP/s.  Measured, us, side by
 // side and in turn (64 heads on 8): 2048 tokens from position 2048 beside 16 of 4096 keys, 0.18 of it, 389 and 339; 2940 from 1000 beside 14 of 1300,
 // 0.04, 352 and 327; but 1800 from the start beside 16 of 2000, 0.35, 109 and 122; 1600 from 2048 beside 250 of 2000, 1.9, 595 and 619; 32 on 8, 4096
 // from 2048 beside 37 of 1500, 0.12, 432 and 383; three of 1365 beside 100 of 2200, 2.8, 262 and 298.  Over 252 steps of
 // 1.5 to 8 blocks to a unit, 1 to 256 single tokens and seven shapes of heads what the rule puts in turn takes 0.84 to 1.025 of the time (from
 // three blocks on one step would take 1.07); with heads of 64, which need half of the LDS, in turn is 0.92 to 1.48 of it, and the gains are small.
-// portion_keys: how many keys the other entries' tokens see together; 0, unknown: as if every such entry began at position 0.
 extern "C" int llmrs_attention_in_turn(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
                                        int v_dim, int maps) {
     const int per_tile = 4 * (32 / std::max(n_heads / std::max(n_kv_heads, 1), 1)), portions = n_entries - n_single;
     if (head_dim != 128 || v_dim != 128 || maps != 1 || n_single <= 0 || portions <= 0 || single_keys <= 0 || per_tile == 0) return 0;
-    const double tokens = n_tokens - n_single;
-    if (((n_tokens - n_single) / per_tile + portions) * (double)n_kv_heads <= 3.5 * llmrs_compute_units()) return 0;
-    const double seen = portion_keys > 0 ? (double)portion_keys : tokens * tokens / (2.0 * portions);
+    if (((n_tokens - n_single) / per_tile + portions) * (double)n_kv_heads <= 3.75 * llmrs_compute_units()) return 0;
+    const double seen = keys_of_portions(n_tokens, n_entries, n_single, portion_keys);
     return (double)single_keys * n_kv_heads * (4.0 * head_dim) / 5e6 <= 0.2 * (seen * n_heads * (4.0 * head_dim) / 0.7e9);
 }
 

@@ -438,12 +438,13 @@ def test_attention_in_shares_with_what_bends_scores(hd, more):
     torch.testing.assert_close(rows[0], rows[1], rtol=2.0 ** -7, atol=2.0 ** -7 * float(rows[1].abs().max()))
 
 
-@pytest.mark.parametrize("n_heads,n_kv,hd,portions,singles,window,in_turn", [
-    (64, 8, 128, [(2048, 200)], [300, 17, 255, 300], 0, False),           # blocks of half as many tokens, in two shares of their keys
-    (32, 8, 64, [(1000, 300)], [2000] * 6, 0, False), (6, 2, 64, [(290, 33), (5, 2)], [31, 700, 32], 0, False), (16, 2, 128, [(1500, 90)], [1, 1600, 900], 800, False),
-    (64, 8, 128, [(0, 1800)], [2000 - i for i in range(16)], 0, False),   # more than three blocks to a unit, side by side
-    (64, 8, 128, [(2048, 2048)], [4095 - 7 * i for i in range(16)], 0, True), (32, 8, 128, [(1500, 2100), (1000, 1999)], [1, 16, 17, 900], 0, True)])
-def test_attention_of_portions_beside_single_tokens(n_heads, n_kv, hd, portions, singles, window, in_turn):
+@pytest.mark.parametrize("n_heads,n_kv,hd,portions,singles,window,in_turn,shares", [
+    (64, 8, 128, [(2048, 200)], [300, 17, 255, 300], 0, False, True), (32, 8, 64, [(1000, 300)], [2000] * 6, 0, False, True),
+    (16, 2, 128, [(1500, 90)], [1, 1600, 900], 800, False, True), (6, 2, 64, [(290, 33), (5, 2)], [31, 700, 32], 0, False, False),
+    (32, 8, 128, [(300, 109), (300, 109)], [3220] * 10, 0, False, False),      # the walk is over before the single tokens' is
+    (64, 8, 128, [(0, 1800)], [2000 - i for i in range(16)], 0, False, False),   # three and a half blocks to a unit, side by side
+    (64, 8, 128, [(2048, 2048)], [4095 - 7 * i for i in range(16)], 0, True, False), (32, 8, 128, [(1500, 2100), (1000, 1999)], [1, 16, 17, 900], 0, True, False)])
+def test_attention_of_portions_beside_single_tokens(n_heads, n_kv, hd, portions, singles, window, in_turn, shares):
     """Portions between single tokens, on both sides of the rules that choose blocks and order (shares of the keys; in turn or side by
     side): rows of every portion and every single token against the formula in 64 bits.  (Bound as for portions alone.)"""
     half = len(singles) // 2
@@ -456,7 +457,8 @@ def test_attention_of_portions_beside_single_tokens(n_heads, n_kv, hd, portions,
     keys, seen = sum(sees(n - 1) for n in singles), sum(sees(p) for ps in pos if len(ps) > 1 for p in ps)
     longest = max(start + count for start, count in spans)
     k = kernels()
-    assert bool(k.lib.llmrs_attention_in_turn(sum(map(len, pos)), len(pos), len(singles), ctypes.c_long(keys), ctypes.c_long(seen), n_heads, n_kv, hd, hd, 1)) == in_turn
+    sizes = (sum(map(len, pos)), len(pos), len(singles), ctypes.c_long(keys), ctypes.c_long(seen), n_heads, n_kv, hd)
+    assert bool(k.lib.llmrs_attention_in_turn(*sizes, hd, 1)) == in_turn and bool(k.lib.llmrs_attention_in_shares(*sizes, window, longest)) == shares
     got, at = case.run(qs, pos, window=window, scratch_floats=k.attention_scratch_floats(len(pos), n_heads, hd, longest, n_kv, len(singles)),
                        n_single=len(singles), single_keys=keys, portion_keys=seen), 0
     for r, places in enumerate(pos):
