@@ -4,8 +4,8 @@ full vocabulary, random weights, in float32 and bfloat16.
 First the four ways of cutting (whole; the last 32 tokens one by one; portions of changing size; mixed
 with reused pages) on four short requests, every row compared with the plain implementation.  Then the
 steps the benchmark runs, which no small model reaches: a prompt of 2,049 tokens and one of 1,025 in one
-step each (whole rounds of the large tiles and one row more) and cut at 1,024, and a portion of 2,048
-tokens beside sixteen requests that decode, as one step.
+step each (whole rounds of the large tiles and one row more) and cut at 1,024, 1,041 and 1,088, and a portion of
+2,048 tokens beside sixteen requests that decode, as one step.
 
 The engine makes its weights on the device from the seed; the plain implementation makes the same
 tensors on the host, one layer at a time, from the same seed (the fill is the same function of seed and
@@ -134,9 +134,10 @@ def test_the_1b_shape_at_full_depth_in_every_cut(case_1b, dtype):
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_the_steps_the_benchmark_runs(case, dtype):
-    """Steps of 2,049, 1,025 and 2,048 + 16 rows through all 32 layers: the large tiles with their rows beyond whole
-    tiles handed to the few-row kernel, the prompt attention over 128 pages, the rotation kernel of many rows, the
-    second stream for the decoding requests' attention, workspaces grown to such steps."""
+    """Steps of 2,049, 1,025, 1,041, 1,088 and 2,048 + 16 rows through all 32 layers: the large tiles with up to 16 rows beyond
+    whole ones multiplied along (in bfloat16, where four waves take the product), 17 to 64 handed to the kernels for few rows, the prompt
+    attention over 128 pages, the rotation kernel of many rows, the second stream for the decoding requests' attention,
+    workspaces grown to such steps."""
     cfg, _, long, reference, by_rounding = case
     allowed = allowed_for(dtype, by_rounding, long)
     engine = Engine.from_random(cfg, SEED, dtype=dtype, device="cuda", page_size=16, num_pages=360, max_requests=32)
@@ -164,6 +165,8 @@ def test_the_steps_the_benchmark_runs(case, dtype):
 
     run_cut("2049 whole", "a", [2049])
     run_cut("2049 as 1024 + 1025", "a", [1024, 1025])
+    run_cut("2049 as 1041 + 1008", "a", [1041, 1008])
+    run_cut("2049 as 1088 + 961", "a", [1088, 961])
     run_cut("1025 whole", "b", [1025])
     run_cut("1025 as 1024 + 1", "b", [1024, 1])
     # sixteen requests up to their last token but one (as one step of sixteen portions), then one step:
