@@ -906,7 +906,9 @@ static int launch_pingpong(hipStream_t stream, const bf16* A, int lda, const bf1
 // then ends with four consecutive features of a token, so gated pairs need no neighbour and results go out by whole lines)
 // against v_mfma_f32_32x32x16_bf16 with results stored from where they lay, us: 2048 rows 57344 x 8192 gated 1381 -> 1338 (1.44
 // PFLOP/s), 8192 x 28672 added to 723 -> 697, 4096 x 14336 213 -> 206, 4096 x 4096 69.7 -> 64.8, 6144 x 4096 85.7 -> 82.1; 2032 rows
-// 16384 x 2048 gated 113.5 -> 106.3; 571 rows 18112 x 128 added to 29.4 -> 19.3.  The one shape found slower: 1360 rows 3040 x 9152 gated, 144 blocks, 96 -> 101.
+// 16384 x 2048 gated 113.5 -> 106.3; 571 rows 18112 x 128 added to 29.4 -> 19.3.  Found slower: grids of 6 x 24 tiles of 256 x 128
+// with long rows that store or gate (1360 rows 3040 x 9152 gated 89.4 -> 93.4, 3040 x 4096 42.9 -> 45.1, 1536 rows 3072 x 9152 stored 90.8 -> 93.9), which
+// neither their neighbours do (5 x 24 0.94-0.97 of the time, 6 x 26 and 6 x 28 0.98-1.0) nor the same grids adding to the stream (0.94-0.98).
 // ---------------------------------------------------------------------------
 // What a wave of the four-wave tile does with its sums.  acc[i][j] are 16 tokens x 16 features, and a lane holds four consecutive
 // features of one token: a gated pair lies in one lane.  32-bit results leave by bands_to_f32; 16-bit ones likewise, a band of 32 tokens
