@@ -658,8 +658,19 @@ extern "C" int llmrs_mingru_product_step(hipStream_t stream, const bf16* A, int 
     LLMRS_REQUIRE(width > 0 && width % 8 == 0 && ldo >= width && ldo % 4 == 0 && ((uintptr_t)out & 7) == 0 && aligned16(bias_z) && aligned16(bias_c),
                   "mingru_product_step: bad sizes, width %d", width);
     if (M == 0) return 0;
-    launch_mixer_step<3, 8, 3, 48>(FewCall{stream, A, lda, W, out, ldo, M, 3 * width, K, LLMRS_EPI_STORE, QkvEpilogue{}, RowScale{}, NextNorm{}},
-                                   FewGru{bias_z, bias_c, state, state_stride, slots});
+    // A unit's LDS holds one block of eight waves with rings of three.  With more blocks than units, blocks of four waves share a unit: two with rings of
+    // four, three with rings of three (from 9 rows on, and where three a unit are one round of a weight whose rows are short) or two (rows of less than 2048,
+    // which fill no deeper one).  (Product and kernel, eight waves, four, us: 4 rows 2560 x 2560 12.2, 14.4, 12.3; 4096 x 4096 21.8, 22.4, 20.0; 5632 x
+    // 5632 39.6, 38.7, 35.1; 5120 x 2560 18.5, 21.8, 17.7, with rings of four 19.0; 8192 x 1024 14.1, -, 13.0, with rings of four 14.7; 16 rows 2560 x 2560
+    // 15.2, 15.5, 13.5; up to 256 blocks 4 rows 2048 x 2048 9.5, 7.9, 8.0.  Product and kernel stay ahead for two to six rows of 5120 x 5120, 31.2 and
+    // 32.3, and for widths of twenty rows' length, 10240 x 512 11.1 and 11.9.)
+    const FewCall call{stream, A, lda, W, out, ldo, M, 3 * width, K, LLMRS_EPI_STORE, QkvEpilogue{}, RowScale{}, NextNorm{}};
+    const FewGru step{bias_z, bias_c, state, state_stride, slots};
+    const int blocks = width / 8, cus = llmrs_compute_units();
+    if (blocks <= cus) launch_mixer_step<3, 8, 3, 48>(call, step);
+    else if (blocks > 2 * cus && K < 2048) launch_mixer_step<3, 4, 2, 48>(call, step);
+    else if (M <= 8 && !(blocks > 2 * cus && blocks <= 3 * cus && K < 4096)) launch_mixer_step<3, 4, 4, 48>(call, step);
+    else launch_mixer_step<3, 4, 3, 48>(call, step);
     LLMRS_LAUNCH_CHECK("mingru_product_step");
     return 0;
 }
