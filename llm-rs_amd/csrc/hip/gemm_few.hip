@@ -643,8 +643,16 @@ extern "C" int llmrs_conv_product_step(hipStream_t stream, const bf16* A, int ld
     if (M == 0) return 0;
     FewCall c{stream, A, lda, W, out, ldc, M, N, K, LLMRS_EPI_STORE_F32, QkvEpilogue{}, RowScale{}, NextNorm{}};
     FewConv e{taps, bias, state, state_stride, slots, x, ldx, C};
-    // (as the plain product's rule above: few rows of a weight, many, and short ones)
-    if (N >= 16384) launch_mixer_step<2, 4, 3, 64>(c, e);
+    // (as the plain product's rule above: few rows of a weight, many, and short ones.  The widest, product and kernel -> here, us: up to 8 rows rings of
+    // four where the plain product takes seven tiles, of three elsewhere (8 rows 20480 x 5120 41.7 -> 40.0, with three 43.3; 16384 x 4096 27.8 -> 24.9,
+    // with four 26.2); a few rows more rings of four (11 rows 18432 x 4608 42.8 -> 34.4, in blocks of 32
+    // features 37.4), and beyond, or over the very widest, blocks of twice as many features, which read the rows half as often (16 rows 24576 x 6144
+    // 58.8 -> 56.8, 62.0 in blocks of 16; 32768 x 8192 96.3 -> 92.6 and 103; 12 rows 24576 x 6144 in blocks of 16 59.3).)
+    if (N >= 16384) {
+        if (M <= 8 && wide_tiles(N, llmrs_compute_units()) != 7) launch_mixer_step<2, 4, 3, 64>(c, e);
+        else if (M <= (N >= 32768 ? 8 : N >= 22528 ? 10 : 12)) launch_mixer_step<2, 4, 4, 64>(c, e);
+        else launch_mixer_step<4, 4, 3, 64>(c, e);
+    }
     else if (K < 2048) launch_mixer_step<2, 4, 4, 0>(c, e);
     else if (half_blocks_for_narrow(N, K)) launch_mixer_step<1, 8, 4, 64>(c, e);
     else launch_mixer_step<2, 8, 3, 64>(c, e);
