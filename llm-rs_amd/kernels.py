@@ -194,6 +194,10 @@ class Kernels:
         pieces of 16 bytes (`tensors`, None among them) lies so."""
         return False
 
+    def product_steps_scan(self, n_tokens: int, channels: int) -> bool:
+        """Whether, of the products that may step their mixers, the scan's is the faster one (else a plain product and `selective_scan`)."""
+        return True
+
     def grouped_experts_take(self, hidden: int, ff: int, dtype: torch.dtype) -> bool:
         """Whether `expert_up` and `expert_down` (every expert's product over its own rows in one launch) and `expert_few_up` and
         `expert_few_down` (up to 64 tokens; experts that none of them chose are not read) run experts of these sizes."""
@@ -344,6 +348,12 @@ class HipKernels(Kernels):
     def products_step_mixers(self, n_tokens: int, n_entries: int, longest: int, dtype: torch.dtype, tensors) -> bool:
         return (longest == 1 and n_tokens == n_entries and 1 <= n_tokens <= 16 and dtype == torch.bfloat16 and self.allow_mfma
                 and all(t is None or t.data_ptr() % 16 == 0 for t in tensors))
+
+    def product_steps_scan(self, n_tokens: int, channels: int) -> bool:
+        # Beyond so many states the walk over them is what takes the time, and the scan's own kernel has more waves for it (product and kernel
+        # -> product that steps, us: 9 tokens of 12288 channels 9.5 -> 9.2, 14 of 8192 8.8 -> 8.6, 12 of 9216 9.1 -> 9.2; 16 of 8192 9.1 -> 9.3,
+        # 12 of 12288 10.4 -> 10.6, 16 of 12288 11.0 -> 12.3, of 16384 13.3 -> 15.1).
+        return n_tokens * channels <= 7 << 14
 
     def norm_left_by_product(self, M: int, N: int, K: int, dtype: torch.dtype) -> Optional[NormPlan]:
         return self._norm_plan(dtype == torch.bfloat16, M, N, K) if self.allow_mfma else None

@@ -139,26 +139,26 @@ class Mamba1(Mixer):
         xc = ctx.workspace("mamba.x", (T, C), self.dtype)
         dbc = ctx.workspace("mamba.dbc", (T, R + 2 * N), self.dtype)
         y = ctx.workspace("mamba.y", (T, C), self.dtype)
-        # (up to 16 requests of one token: the products convolve and advance the state themselves)
-        if self.step_in_products and k.products_step_mixers(T, ctx.n_entries, ctx.longest, self.dtype,
-                                                                  (x, self.w_in, self.conv, self.conv_bias, cache.state, self.w_dt)):
+        # (up to 16 requests of one token: the products convolve and, of few states, advance the state themselves)
+        in_products = self.step_in_products and k.products_step_mixers(T, ctx.n_entries, ctx.longest, self.dtype,
+                                                                        (x, self.w_in, self.conv, self.conv_bias, cache.state, self.w_dt))
+        if in_products:
             k.conv_product_step(x, self.w_in, sums, self.conv, self.conv_bias, conv_state, ctx.slots, C, xc)
-            k.gemm(xc, self.w_x, dbc, EPI_STORE, ctx.gemm_workspace(xc, self.w_x))
-            k.scan_product_step(dbc, R, self.w_dt, xc, self.dt_bias, self.A, self.D, sums[:, C:], scan_state, ctx.slots, y)
-            k.gemm(y, self.w_o, h, EPI_ACCUM_F32, ctx.gemm_workspace(y, self.w_o))
-            ctx.note_left(h, None)
-            return
-        k.gemm(x, self.w_in, sums, EPI_STORE_F32, ctx.gemm_workspace(x, self.w_in))
-        k.causal_conv(sums, self.conv, self.conv_bias, conv_state, ctx.q_starts, ctx.slots, ctx.token_entry, C, xc, silu=True, longest=ctx.longest)
+        else:
+            k.gemm(x, self.w_in, sums, EPI_STORE_F32, ctx.gemm_workspace(x, self.w_in))
+            k.causal_conv(sums, self.conv, self.conv_bias, conv_state, ctx.q_starts, ctx.slots, ctx.token_entry, C, xc, silu=True, longest=ctx.longest)
         k.gemm(xc, self.w_x, dbc, EPI_STORE, ctx.gemm_workspace(xc, self.w_x))
-        dt = ctx.workspace("mamba.dt", (T, C), torch.float32)
-        d = dbc[:, :R]
-        k.gemm(d, self.w_dt, dt, EPI_STORE_F32, ctx.gemm_workspace(d, self.w_dt))
-        ypart = ctx.workspace("mamba.ypart", (T, C), torch.float32) if N > 64 else None
-        need = k.scan_carry_floats(T, ctx.n_entries, ctx.longest, (N + 1) * C)
-        carry = ctx.workspace("scan.carry", (need,), torch.float32) if need else None
-        k.selective_scan(xc, dbc, R, R + N, dt, self.dt_bias, self.A, self.D, sums[:, C:], scan_state, ctx.q_starts, ctx.slots, y, ypart,
-                         ctx.longest, carry)
+        if in_products and k.product_steps_scan(T, C):
+            k.scan_product_step(dbc, R, self.w_dt, xc, self.dt_bias, self.A, self.D, sums[:, C:], scan_state, ctx.slots, y)
+        else:
+            dt = ctx.workspace("mamba.dt", (T, C), torch.float32)
+            d = dbc[:, :R]
+            k.gemm(d, self.w_dt, dt, EPI_STORE_F32, ctx.gemm_workspace(d, self.w_dt))
+            ypart = ctx.workspace("mamba.ypart", (T, C), torch.float32) if N > 64 else None
+            need = k.scan_carry_floats(T, ctx.n_entries, ctx.longest, (N + 1) * C)
+            carry = ctx.workspace("scan.carry", (need,), torch.float32) if need else None
+            k.selective_scan(xc, dbc, R, R + N, dt, self.dt_bias, self.A, self.D, sums[:, C:], scan_state, ctx.q_starts, ctx.slots, y, ypart,
+                             ctx.longest, carry)
         k.gemm(y, self.w_o, h, EPI_ACCUM_F32, ctx.gemm_workspace(y, self.w_o))
         ctx.note_left(h, None)
 
