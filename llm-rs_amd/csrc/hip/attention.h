@@ -156,6 +156,11 @@ extern "C" int llmrs_attention_in_shares(int n_tokens, int n_entries, int n_sing
                                          int reach, int max_seq_len);
 extern "C" int llmrs_attention_in_turn(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
                                        int v_dim, int maps);
+// How tiles and single tokens go into one grid: the bits say what it does.
+#define ATTN_TOGETHER_SHARES 1
+#define ATTN_TOGETHER_SINGLES_FIRST 2
+extern "C" int llmrs_attention_together(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
+                                        int reach, int max_seq_len);
 
 // 32-bit tiles on the matrix cores for entries with several tokens (attention_f32_mfma.hip); skip_single: entries
 // with one token are left to the caller.  Return 1 when it took them, 0 when the shape is not its own, -1 on error.

@@ -358,14 +358,14 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(const bf16* __restrict_
 // tiles; the first two make the results one.  For few blocks, where the walk along the keys is a chain (see `launch`).
 // Two maps: wave w holds map w & 1 of the tokens of group w / 2 (tokens of two groups a block instead of four), KW
 // features of the keys from map * KW on enter its products, and the group's even wave makes the two results one.
-template <int KD, int VD, int MAPS, int WAVES = 4, int SHARES = 1, int RING = 4>
-__global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_per_eu(VD <= 128 ? 2 : 1))) void attn_tiles_lds_kernel(const bf16* __restrict__ q, bf16* __restrict__ out,
-                                                             const bf16* __restrict__ kc, const bf16* __restrict__ vc,
-                                                             const int* __restrict__ block_table,
-                                                             const int* __restrict__ positions,
-                                                             const int* __restrict__ q_starts, int n_entries,
-                                                             AttnArgs a, int G, int tpt, int skip_single,
-                                                             int round_blocks) {
+constexpr int tiles_ring(int kd, int vd, int ring) { return ring * (kd + vd) * 64 <= 65536 ? ring : 2; }       // tiles in each of the two rings (keys, values)
+constexpr int tiles_lds_bytes(int kd, int vd, int shares, int ring) { return shares * tiles_ring(kd, vd, ring) * (kd + vd) * 64; }
+template <int KD, int VD, int MAPS, int WAVES, int SHARES, int RING>
+__device__ __forceinline__ void attend_tiles_lds(unsigned char* all_rings, const int block, const bf16* __restrict__ q, bf16* __restrict__ out,
+                                                 const bf16* __restrict__ kc, const bf16* __restrict__ vc,
+                                                 const int* __restrict__ block_table, const int* __restrict__ positions,
+                                                 const int* __restrict__ q_starts, int n_entries, const AttnArgs& a, int G, int tpt, int skip_single,
+                                                 int round_blocks) {
     constexpr int CHUNKS = KD / 8;                  // 16-byte chunks in a key's row
     constexpr int ROW_BYTES = KD * 2;
     constexpr int KW = KD / MAPS;                   // features of a key that a wave's products run over
@@ -377,9 +377,9 @@ __global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_pe
     static_assert(SHARE_K >= 1024 && SHARE_K % 1024 == 0 && SHARE_V >= 1024 && SHARE_V % 1024 == 0, "a load instruction of a wave brings 1 KB");
     constexpr int HALF_K = SHARE_K / 1024, HALF_V = SHARE_V / 1024;   // load instructions of a wave for its share of a page
     constexpr int SWZ_SHIFT = ROW_BYTES >= 256 ? 0 : 1;
-    constexpr int R = (RING * (TILE_K + TILE_V) <= 65536) ? RING : 2;   // tiles in each of the two rings (keys, values)
+    constexpr int R = tiles_ring(KD, VD, RING);
     constexpr int RINGS = R * (TILE_K + TILE_V);
-    __shared__ __attribute__((aligned(1024))) unsigned char all_rings[SHARES * RINGS];
+    static_assert(SHARES * RINGS == tiles_lds_bytes(KD, VD, SHARES, RING), "what the kernels set aside");
     static_assert(SHARES == 1 || (SHARES == 2 && MAPS == 1 && WAVES * 32 * VD * 4 <= RINGS), "the second share's results pass through its rings' place");
     static_assert(MAPS == 1 || GROUPS * 32 * VD * 4 <= R * (TILE_K + TILE_V), "the second maps' results pass through the rings' place at the end");
     int lane = threadIdx.x & 63;
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_pe
     if (SHARES > 1) wave %= WAVES;
     unsigned char* lds = all_rings + share * RINGS;
     int c = lane & 31, h = lane >> 5;
-    int kvh = blockIdx.x % a.n_kv_heads;
+    int kvh = block % a.n_kv_heads;
     // Order of work.  A tile's work grows with its place in its entry, so the tiles are handed out
     // from the last to the first: the longest start first, they decide when the grid ends.  All
     // blocks of the first two rounds (a round: as many blocks as the device holds at once in one
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_pe
     // units, so the second round runs in the opposite order and puts the shortest beside the longest
     // (`round_blocks` 0, for blocks that have a unit to themselves: from the last to the first throughout).
     int n_btiles = count_tiles(q_starts, n_entries, GROUPS * tpt, skip_single);      // (every wave for itself: the same figures)
-    int g = blockIdx.x / a.n_kv_heads;
+    int g = block / a.n_kv_heads;
     if (g >= n_btiles) return;                       // the grid is sized for the most tiles the tokens could make
     int gr = round_blocks / a.n_kv_heads;
     if (g >= gr && g < 2 * gr) g = gr + (min(2 * gr, n_btiles) - 1 - g);
@@ -683,6 +683,17 @@ __global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_pe
             *(bf16x4*)(op + o_feature(dt, i4 * 4, h)) = v;
         }
 }
+template <int KD, int VD, int MAPS, int WAVES = 4, int SHARES = 1, int RING = 4>
+__global__ __launch_bounds__(WAVES * SHARES * 64) __attribute__((amdgpu_waves_per_eu(VD <= 128 ? 2 : 1))) void attn_tiles_lds_kernel(const bf16* __restrict__ q, bf16* __restrict__ out,
+                                                             const bf16* __restrict__ kc, const bf16* __restrict__ vc,
+                                                             const int* __restrict__ block_table,
+                                                             const int* __restrict__ positions,
+                                                             const int* __restrict__ q_starts, int n_entries,
+                                                             AttnArgs a, int G, int tpt, int skip_single,
+                                                             int round_blocks) {
+    __shared__ __attribute__((aligned(1024))) unsigned char all_rings[tiles_lds_bytes(KD, VD, SHARES, RING)];
+    attend_tiles_lds<KD, VD, MAPS, WAVES, SHARES, RING>(all_rings, blockIdx.x, q, out, kc, vc, block_table, positions, q_starts, n_entries, a, G, tpt, skip_single, round_blocks);
+}
 
 // ---- entries with one token: a wave for each (entry, kv head, chunk of keys) --
 // partial: [(entry * columns + column) * max_chunks + chunk][VD + 2] = m, l, O (not yet divided); a column is a head, or with
@@ -794,19 +805,14 @@ __device__ __forceinline__ float across_groups_sum(float x) {
     return x + other_half(x);
 }
 
-template <int KD, int VD, int MAPS>
-__global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict__ q, float* __restrict__ partial,
-                                                          const bf16* __restrict__ kc, const bf16* __restrict__ vc,
-                                                          const int* __restrict__ block_table,
-                                                          const int* __restrict__ seq_lens,
-                                                          const int* __restrict__ q_starts, AttnArgs a, int G,
-                                                          int max_chunks, int chunk, int plain, int entry_first) {
+template <int KD, int VD, int MAPS, int RING>        // RING: steps in LDS (0: operands straight from memory)
+__device__ __forceinline__ void attend_single16(unsigned char* smem, const int kvh, const int e, const int ch, const bf16* __restrict__ q,
+                                                float* __restrict__ partial, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
+                                                const int* __restrict__ block_table, const int* __restrict__ seq_lens,
+                                                const int* __restrict__ q_starts, const AttnArgs& a, int G, int max_chunks, int chunk, int plain) {
     static_assert(KD % 32 == 0 && VD % 16 == 0, "the score products take 32 features at a time");
-    constexpr int RING = split16_ring(KD, VD);      // steps in LDS (0: operands straight from memory)
     constexpr int PAGE_K = KD * 32, PAGE_V = VD * 32, STEP = 2 * (PAGE_K + PAGE_V), LOADS = STEP / 1024;
     static_assert(RING * STEP <= SPLIT16_LDS_BYTES, "the steps lie in what a block asks for");
-    extern __shared__ __attribute__((aligned(1024))) unsigned char split16_smem[];
-    int kvh = entry_first ? blockIdx.y : blockIdx.x, e = entry_first ? blockIdx.x : blockIdx.y, ch = blockIdx.z;      // (see `launch`)
     int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     bool cvalid = c < G;
     int column = kvh * G + min(c, G - 1), head = column / MAPS, map = column % MAPS;
@@ -882,7 +888,7 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
     auto bring = [&](int t0, int place) {
         int a0, a1;
         pages_of(t0, a0, a1);
-        unsigned char* to = split16_smem + place * STEP;
+        unsigned char* to = smem + place * STEP;
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             const bf16* kp = kc + ((size_t)(p ? a1 : a0) * a.n_kv_heads + kvh) * (16 * KD);
@@ -930,7 +936,7 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
             if (t0 + 32 * (RING - 2) < t_end) wait_vmcnt_n<(RING - 2) * LOADS>(); else wait_vmcnt_all();
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (t0 + 32 * (RING - 1) < t_end) { bring(t0 + 32 * (RING - 1), put); put = put + 1 == RING ? 0 : put + 1; }
-            const unsigned char* from = split16_smem + get * STEP;
+            const unsigned char* from = smem + get * STEP;
             get = get + 1 == RING ? 0 : get + 1;
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -1026,6 +1032,43 @@ __global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict
     for (int dt = 0; dt < VD / 16; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) pp[2 + dt * 16 + 4 * g + r] = O[dt][r];
+}
+template <int KD, int VD, int MAPS>
+__global__ __launch_bounds__(64) void attn_split16_kernel(const bf16* __restrict__ q, float* __restrict__ partial,
+                                                          const bf16* __restrict__ kc, const bf16* __restrict__ vc,
+                                                          const int* __restrict__ block_table,
+                                                          const int* __restrict__ seq_lens,
+                                                          const int* __restrict__ q_starts, AttnArgs a, int G,
+                                                          int max_chunks, int chunk, int plain, int entry_first) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char split16_smem[];
+    int kvh = entry_first ? blockIdx.y : blockIdx.x, e = entry_first ? blockIdx.x : blockIdx.y, ch = blockIdx.z;      // (see `launch`)
+    attend_single16<KD, VD, MAPS, split16_ring(KD, VD)>(split16_smem, kvh, e, ch, q, partial, kc, vc, block_table, seq_lens, q_starts, a, G, max_chunks, chunk, plain);
+}
+
+// ---- both kinds in one grid --
+// Blocks of four waves: the first `single_first` of them, and those from single_first + tile_blocks on, are four (kv head, entry, chunk) of the
+// single tokens, a wave each; the ones between are tiles.  Single tokens are bound by memory and tiles by the matrix cores and their own chain, so a unit that holds
+// one of each does both at once; the tiles' registers leave a SIMD two waves, so a unit holds two blocks of either kind.  (On two streams, as before, the fork and the
+// join alone are 28 us of a call: 4 requests of 60 to 300 keys beside 100 tokens 51 -> 16 us, 64 of 300 to 3000 beside 512 tokens, heads of 64, 72 -> 58,
+// 160 of 128 to 4096 beside three portions of 331 to 927 173 -> 160, heads of 128 298 -> 280; 220 such steps of eight shapes of heads 0.53 of the time.  A wave's
+// operands come straight from memory here: through two or three steps' places in LDS, of heads of 64, the 160 take 161 and 162; with registers for three blocks to
+// a unit the tiles spill, 158 to 164.)
+template <int KD, int VD, int WAVES, int SHARES, int RING>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_mixed_kernel(
+        const bf16* __restrict__ q, bf16* __restrict__ out, float* __restrict__ partial, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
+        const int* __restrict__ block_table, const int* __restrict__ positions, const int* __restrict__ q_starts, const int* __restrict__ seq_lens,
+        int n_entries, AttnArgs a, int G, int tpt, int round_blocks, int tile_blocks, int single_first, int max_chunks, int chunk, int entry_first) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char mixed_smem[];
+    int b = blockIdx.x;
+    if (b >= single_first && b < single_first + tile_blocks) {
+        attend_tiles_lds<KD, VD, 1, WAVES, SHARES, RING>(mixed_smem, b - single_first, q, out, kc, vc, block_table, positions, q_starts, n_entries, a, G, tpt, 1, round_blocks);
+        return;
+    }
+    if (b >= single_first) b -= tile_blocks;
+    const int task = b * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), inner = entry_first ? n_entries : a.n_kv_heads, per_chunk = n_entries * a.n_kv_heads;
+    const int ch = task / per_chunk, rest = task - ch * per_chunk, y = rest / inner, x = rest - y * inner;
+    if (ch >= max_chunks) return;
+    attend_single16<KD, VD, 1, 0>(mixed_smem, entry_first ? y : x, entry_first ? x : y, ch, q, partial, kc, vc, block_table, seq_lens, q_starts, a, G, max_chunks, chunk, 0);
 }
 
 #define MERGE_MAX_CHUNKS 1024
@@ -1275,7 +1318,7 @@ static __global__ __launch_bounds__(MERGE_GROUP_THREADS) void attn_merge_maps_ke
 
 // A step with a prompt portion beside decoding requests has two kinds of attention work that do not depend on
 // each other: tiles of many tokens, bound by the matrix cores, and single tokens over their whole caches, bound by
-// memory.  They run side by side: the single tokens' kernels go to a second stream of this library's own (default
+// memory.  They run side by side: in one grid where a kernel holds both (attn_mixed_kernel), else the single tokens' kernels go to a second stream of this library's own (default
 // priority), which waits for everything the caller's stream held when the call came and which the caller's stream
 // waits for before it goes on.  One such stream and pair of events per device, made at first use.  While the
 // caller's stream is being captured into a graph nothing is forked: the two kinds follow each other as before.
@@ -1300,11 +1343,45 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
     // every entry brings one token, on the caller's word (n_single == n_entries): no tile work.  It is not read off
     // n_tokens == n_entries, which entries of two tokens and of none would satisfy as well.
     int only_single = split && n_single == n_entries && a.n_tokens == n_entries;
+    // Blocks go to the eight XCDs in turn, so the grid's first dimension is one that all entries share alike: with the
+    // entries there, each XCD had every eighth entry whole, and one with a longer cache than the others kept its XCD busy
+    // alone (24 requests of 800 to 8000 keys: 106 -> 102 us, 160 of 128 to 4096, heads of 64, in chunks of 1024: 165 -> 147).
+    // The chunk comes last: a recorded step's grid is as wide as its block table, and an entry's last chunk may hold a
+    // few keys, so with the chunks before the entries, whole, short and empty ones alternated, and the units that got
+    // the short ones first were left without work (64 requests of 2060 keys under a bound of 4096: 105 us, 132 that way;
+    // 256: 406, 506; without empty chunks the same either way).
+    // With a grid of many more chunks than there are keys (one long cache under the same bound as many short ones) the entry
+    // comes first after all: a first dimension of a few blocks hands thousands of empty ones out more slowly (bound 4096, 32
+    // requests of 60 keys, heads of 64: 9.1 against 10.4 us; bound 32,768, 200 of 600: 66 against 74; of 13 to 14 times the
+    // keys neither is faster); and with no more than three waves to a unit, where nothing waits for a longer entry and the merge,
+    // whose blocks also go by entry, finds the parts in its XCD's L2 (8 requests of 600 keys: 10.4 against 10.9 us, 64 heads
+    // 11.0 against 11.7).
+    const int entry_first = single_keys <= 0 || (double)n_entries * max_chunks * chunk > 8.0 * single_keys ||
+                            (double)single_keys * a.n_kv_heads <= 3.0 * llmrs_compute_units() * chunk;
     // both kinds of work: the single tokens' kernels on the second stream, beside the tiles
     hipStream_t single_stream = stream;
     SideStream* side = nullptr;
-    // (or one kind after the other, by the rule's answer)
-    if (split && !only_single && !llmrs_attention_in_turn(a.n_tokens, n_entries, n_single, single_keys, portion_keys, a.n_heads, a.n_kv_heads, KD, VD, MAPS)) {
+    // (or one kind after the other, by the rule's answer; or both in one grid, where a kernel of both is built)
+    const bool in_turn = split && !only_single && llmrs_attention_in_turn(a.n_tokens, n_entries, n_single, single_keys, portion_keys, a.n_heads, a.n_kv_heads, KD, VD, MAPS);
+    bool together = false;
+    if constexpr (MAPS == 1 && KD == VD && (KD == 64 || KD == 128)) {
+        const double tasks = (double)n_entries * a.n_kv_heads * max_chunks;
+        together = split && !only_single && !in_turn && G <= 16 && max_seq_len < ATTN_WIDE_FROM_KEYS && tasks < (1 << 28);
+        if (together) {
+            constexpr int SHARE_RING = KD == 64 ? 4 : 2;
+            const int how = llmrs_attention_together(a.n_tokens, n_entries, n_single, single_keys, portion_keys, a.n_heads, a.n_kv_heads, KD, attn_reach(a), max_seq_len);
+            const bool shared_out = how & ATTN_TOGETHER_SHARES;
+            const int cus = llmrs_compute_units(), single_blocks = ((int)tasks + 3) / 4, tile_blocks = (a.n_tokens / ((shared_out ? 2 : 4) * tpt) + n_entries) * a.n_kv_heads;
+            const int single_first = (how & ATTN_TOGETHER_SINGLES_FIRST) ? std::min(single_blocks, 2 * cus) : 0;
+            if (shared_out)
+                attn_mixed_kernel<KD, VD, 2, 2, SHARE_RING><<<tile_blocks + single_blocks, 256, tiles_lds_bytes(KD, VD, 2, SHARE_RING), stream>>>(
+                    q, out, scratch, kc, vc, table, positions, q_starts, seq_lens, n_entries, a, G, tpt, tile_blocks > 2 * cus ? cus : 0, tile_blocks, single_first, max_chunks, chunk, entry_first);
+            else
+                attn_mixed_kernel<KD, VD, 4, 1, 4><<<tile_blocks + single_blocks, 256, tiles_lds_bytes(KD, VD, 1, 4), stream>>>(
+                    q, out, scratch, kc, vc, table, positions, q_starts, seq_lens, n_entries, a, G, tpt, cus, tile_blocks, single_first, max_chunks, chunk, entry_first);
+        }
+    }
+    if (split && !only_single && !together && !in_turn) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) side = llmrs_attention_side_stream();
         else (void)hipGetLastError();
@@ -1314,7 +1391,7 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
             else { (void)hipGetLastError(); side = nullptr; }
         }
     }
-    if (!only_single) {
+    if (!only_single && !together) {
         if constexpr ((KD == 64 || KD == 128 || KD == 256) && VD >= 64) {
             const int heads_tpt = 32 / (G / MAPS);        // (a wave's columns are heads here, all of one map)
             // Over long caches blocks of eight waves, one to a unit: every tile of keys and values comes in for
@@ -1350,24 +1427,11 @@ static int launch(hipStream_t stream, const bf16* q, bf16* out, const bf16* kc, 
         }
     }
     if (split) {
-        // Blocks go to the eight XCDs in turn, so the grid's first dimension is one that all entries share alike: with the
-        // entries there, each XCD had every eighth entry whole, and one with a longer cache than the others kept its XCD busy
-        // alone (24 requests of 800 to 8000 keys: 106 -> 102 us, 160 of 128 to 4096, heads of 64, in chunks of 1024: 165 -> 147).
-        // The chunk comes last: a recorded step's grid is as wide as its block table, and an entry's last chunk may hold a
-        // few keys, so with the chunks before the entries, whole, short and empty ones alternated, and the units that got
-        // the short ones first were left without work (64 requests of 2060 keys under a bound of 4096: 105 us, 132 that way;
-        // 256: 406, 506; without empty chunks the same either way).
-        // With a grid of many more chunks than there are keys (one long cache under the same bound as many short ones) the entry
-        // comes first after all: a first dimension of a few blocks hands thousands of empty ones out more slowly (bound 4096, 32
-        // requests of 60 keys, heads of 64: 9.1 against 10.4 us; bound 32,768, 200 of 600: 66 against 74; of 13 to 14 times the
-        // keys neither is faster); and with no more than three waves to a unit, where nothing waits for a longer entry and the merge,
-        // whose blocks also go by entry, finds the parts in its XCD's L2 (8 requests of 600 keys: 10.4 against 10.9 us, 64 heads
-        // 11.0 against 11.7).
-        const int entry_first = single_keys <= 0 || (double)n_entries * max_chunks * chunk > 8.0 * single_keys ||
-                                (double)single_keys * a.n_kv_heads <= 3.0 * llmrs_compute_units() * chunk;
         dim3 grid(entry_first ? n_entries : a.n_kv_heads, entry_first ? a.n_kv_heads : n_entries, max_chunks);
         int plain = only_single && attn_reach(a) == 0;
-        if (G <= 16)
+        if (together) {
+            // (their keys have been walked)
+        } else if (G <= 16)
             attn_split16_kernel<KD, VD, MAPS><<<grid, 64, SPLIT16_LDS_BYTES, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain, entry_first);
         else
             attn_split_kernel<KD, VD, MAPS><<<grid, 64, 0, single_stream>>>(q, scratch, kc, vc, table, seq_lens, q_starts, a, G, max_chunks, chunk, plain, entry_first);

@@ -160,6 +160,26 @@ extern "C" int llmrs_attention_in_turn(int n_tokens, int n_entries, int n_single
     return (double)single_keys * n_kv_heads * (4.0 * head_dim) / 5e6 <= 0.2 * (seen * n_heads * (4.0 * head_dim) / 0.7e9);
 }
 
+// How both kinds of work of a step go into one grid (attn_mixed_kernel): ATTN_TOGETHER_SHARES, the tiles' keys in two shares, where no more than four of their
+// blocks come to a unit and their walk is not over well before the single tokens' keys have come (at 5 TB/s); ATTN_TOGETHER_SINGLES_FIRST, the single tokens' first 512
+// blocks before the tiles, where their keys take more than 20 us and longer than the tiles' walk.  Of 220 steps (1 to 160 single tokens, one to four
+// portions of 2 to 2000 tokens, eight shapes of heads) the time with what the two choose is 1.017 of the best of both choices' six combinations in the mean, and 0.53
+// of that on two streams.  Shares, without and with: 32 heads on 8 of 64 features, 23 requests of 445 keys beside a prompt of 1284 58.7 and 38.6; 64 heads on 8,
+// 10 of 2300 beside portions of 355 and 453 38.5 and 46.9 (the walk says no), 40 on 8, 4 beside four of 470 45.2 and 52.1 (five blocks to a unit).  Tiles first and single tokens first:
+// 64 heads on 8, 68 of 1030 to 1533 beside 1232 tokens 143 and 102; 12 heads of 64, 75 of 1200 beside 98 tokens over 3000 keys (the longer walk) 79 and 98.
+extern "C" int llmrs_attention_together(int n_tokens, int n_entries, int n_single, long single_keys, long portion_keys, int n_heads, int n_kv_heads, int head_dim,
+                                        int reach, int max_seq_len) {
+    const int singles = std::max(n_single, 0), tokens = n_tokens - singles, portions = n_entries - singles;
+    if (tokens <= 0 || portions <= 0) return 0;
+    const long cus = llmrs_compute_units(), per_block = 2L * std::max(32 / std::max(n_heads / std::max(n_kv_heads, 1), 1), 1);
+    const double read = (single_keys > 0 ? (double)single_keys : (double)singles * max_seq_len) * n_kv_heads * head_dim, single_us = read * 4.0 / 5e6;
+    double walk = keys_of_portions(n_tokens, n_entries, singles, portion_keys) / tokens + tokens / (2.0 * portions);
+    if (reach > 0) walk = std::min(walk, (double)reach);
+    const double walk_us = walk / 32.0 * (head_dim >= 128 ? 1.17 : 0.79);
+    const bool shares = max_seq_len >= 256 && (reach <= 0 || reach >= 768) && (tokens / per_block + portions) * n_kv_heads <= 4 * cus && walk_us >= 0.25 * single_us;
+    return (shares ? ATTN_TOGETHER_SHARES : 0) | (single_us > 20.0 && single_us > walk_us ? ATTN_TOGETHER_SINGLES_FIRST : 0);
+}
+
 // Heads of two maps (attention_mfma_maps.hip).
 int llmrs_attention_bf16_mfma_maps(hipStream_t stream, const bf16* q, bf16* out, const bf16* k_cache, const bf16* v_cache,
                                    const int* block_table, const int* positions, const int* q_starts, const int* seq_lens,

@@ -438,6 +438,54 @@ def test_attention_in_shares_with_what_bends_scores(hd, more):
     torch.testing.assert_close(rows[0], rows[1], rtol=2.0 ** -7, atol=2.0 ** -7 * float(rows[1].abs().max()))
 
 
+@pytest.mark.parametrize("heads,kv,hd,spans,singles,how,more", [
+    (8, 2, 64, [(0, 2), (250, 33)], [1, 300, 16, 17], 1, {}), (8, 2, 128, [(700, 61)], [1000, 33, 999], 1, {"window": 800, "keep_first": 40}),
+    (16, 1, 64, [(3, 7), (0, 5), (90, 2)], [31, 32, 33, 64, 100], 0, {"softcap": 15.0, "sink": True}), (5, 5, 128, [(0, 40)], [257], 1, {"gate": True}),
+    (32, 8, 64, [(0, 50), (12, 35)], [2500 - 9 * i for i in range(45)], 2, {}), (8, 8, 128, [(2, 130)], [4000] * 12, 2, {"distance": True}),
+    (64, 8, 128, [(0, 700), (5, 700), (0, 2)], [2, 600, 5], 0, {}), (9, 3, 64, [(1400, 300)], [1900 + i for i in range(300)], 3, {"window": 1300})])
+def test_attention_of_both_kinds_in_one_grid(heads, kv, hd, spans, singles, how, more):
+    """Portions and single tokens in one call, the rows of q apart by more than they are long, against the same rows in calls of one kind
+    each: single tokens bit for bit (the same chunks in the same order), portions but for one rounding to bfloat16 (their keys may be shared out otherwise)."""
+    entries = [s for pair in zip(singles, spans) for s in ((pair[0] - 1, 1), pair[1])] + [(n - 1, 1) for n in singles[len(spans):]] + spans[len(singles):]
+    seq, counts = [a + c for a, c in entries], [c for _, c in entries]
+    longest, width, pages = max(seq), -(-max(seq) // 16), 300
+    g = torch.Generator(device=DEV).manual_seed(hd + heads)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    kc, vc, T = rnd(pages, kv, 16, hd).bfloat16(), rnd(pages, kv, hd, 16).bfloat16(), sum(counts)
+    wide = rnd(T, heads * hd + 24).bfloat16() * 2
+    table = torch.randint(0, pages, (len(entries), width), generator=torch.Generator().manual_seed(1)).int().to(DEV)
+    extra, window = {k: v for k, v in more.items() if v is not True and k != "window"}, more.get("window", 0)
+    if more.get("sink"):
+        extra["sink"] = rnd(heads)
+    if more.get("distance"):
+        extra["distance"] = (rnd(heads).abs() * 0.01, None)
+    gates = rnd(T, heads * hd) if more.get("gate") else None
+    sees = lambda p: min(p + 1, window or p + 1)
+    keys, k = sum(sees(n - 1) for n in singles), kernels()
+    seen = sum(sees(a + i) for a, c in entries if c > 1 for i in range(c))
+    ask = k.lib.llmrs_attention_together
+    assert ask(T, len(entries), len(singles), ctypes.c_long(keys), ctypes.c_long(seen), heads, kv, hd, window, longest) == how
+    assert not k.lib.llmrs_attention_in_turn(T, len(entries), len(singles), ctypes.c_long(keys), ctypes.c_long(seen), heads, kv, hd, hd, 1)
+
+    def run(which, n_single):
+        rows = torch.cat([torch.arange(sum(counts[:e]), sum(counts[:e + 1])) for e in which]).to(DEV)
+        n = [counts[e] for e in which]
+        q, out = wide[rows][:, :heads * hd], torch.full((len(rows), heads * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        at = [entries[e][0] + i for e in which for i in range(counts[e])]
+        scratch = torch.empty(k.attention_scratch_floats(len(which), heads, hd, longest, kv, n_single), device=DEV)
+        k.attention(q, out, kc, vc, table[which].contiguous(), i32([j for j, c in enumerate(n) for _ in range(c)]), i32(at), i32([sum(n[:j]) for j in range(len(n) + 1)]),
+                    i32([seq[e] for e in which]), heads, kv, hd, 16, pages, window, hd ** -0.5, scratch, longest, n_single, keys if n_single else 0,
+                    portion_keys=seen if len(which) > n_single else 0, **extra, **({} if gates is None else {"gate": gates[rows]}))
+        return rows, out
+
+    both = run(list(range(len(entries))), len(singles))[1]
+    rows, alone = run([e for e, c in enumerate(counts) if c == 1], len(singles))
+    assert torch.isfinite(both.float()).all() and torch.equal(both[rows], alone)
+    rows, alone = run([e for e, c in enumerate(counts) if c > 1], 0)
+    torch.testing.assert_close(both[rows].float(), alone.float(), rtol=2.0 ** -7, atol=2.0 ** -7 * float(alone.float().abs().max()))
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,portions,singles,window,in_turn,shares", [
     (64, 8, 128, [(2048, 200)], [300, 17, 255, 300], 0, False, True), (32, 8, 64, [(1000, 300)], [2000] * 6, 0, False, True),
     (16, 2, 128, [(1500, 90)], [1, 1600, 900], 800, False, True), (6, 2, 64, [(290, 33), (5, 2)], [31, 700, 32], 0, False, False),
