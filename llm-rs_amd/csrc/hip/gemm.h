@@ -127,6 +127,8 @@ extern "C" int llmrs_gemm_leaves_norm(int N);
 extern "C" int llmrs_qkv_by_fours(int head_dim, int rotary_dim);
 // The parts per row of the sums of squares that such a product leaves (NextNorm): what the caller sizes sumsq by.
 extern "C" int llmrs_gemm_next_parts(int M, int N, int K);
+// Which tiles a product of more than 64 rows takes that is too small for the square large ones (gemm_mfma.hip).
+extern "C" int llmrs_gemm_mid_plan(int M, int N, int K, int epi);
 // Whether the bfloat16 product of this shape, adding into the stream and given the workspace that
-// llmrs_gemm_workspace_floats asks for, is split over blocks so that it can finish the following norm (NextNorm with eps).
+// llmrs_gemm_workspace_floats asks for, can finish the following norm (NextNorm with eps): where its sums are added up, or in a launch of its own.
 extern "C" int llmrs_gemm_norms_whole(int M, int N, int K);

@@ -6,9 +6,9 @@
 //            112 output features and its waves split K.
 //   M  > 64  "tiled": prompts.  Tiles of 128x128, 256x128, 256x192 or 256x256 outputs, K
 //            in steps of 64 through double-buffered LDS, v_mfma_f32_32x32x16_bf16; when
-//            K % 64 == 0 the tiles are loaded straight into LDS (global_load_lds), or, by
-//            the four waves of the large ones, through registers between their MFMAs
-//            (v_mfma_f32_16x16x32_bf16).
+//            K % 64 == 0 the tiles are loaded straight into LDS (by waves that do nothing
+//            else), or, by the four waves of the largest, through registers between their
+//            MFMAs (v_mfma_f32_16x16x32_bf16).
 // Both need K % 8 == 0 and 16-byte aligned rows (16-byte loads); otherwise the
 // caller falls back to the plain kernel.
 //
@@ -242,6 +242,7 @@ __global__ void gemm_splitk_finish_kernel(const float* __restrict__ partial, int
 // The same for a product that adds into the 32-bit stream and is followed by a norm x / rms(x) * weight: a block
 // for each row adds the parts in the same order, writes the stream's new row, and, having the whole row, the
 // normed row as well (NextNorm with eps): no norm kernel runs.  Up to 16384 features (16 per thread), a multiple of 4.
+// With no parts (splits 0) the stream's rows are whole already and only the norm is left to do.
 __global__ __launch_bounds__(1024) void gemm_splitk_finish_norm_kernel(const float* __restrict__ partial, int splits,
                                                                         float* __restrict__ out, int ldc, int M, int N,
                                                                         NextNorm nn) {
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(1024) void gemm_splitk_finish_norm_kernel(const flo
             f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int s = 0; s < splits; ++s) v += *(const f32x4*)(p0 + (size_t)s * M * N + n);
             h[i] = *(const f32x4*)(o + n) + v;
-            *(f32x4*)(o + n) = h[i];
+            if (splits > 0) *(f32x4*)(o + n) = h[i];
 #pragma unroll
             for (int r = 0; r < 4; ++r) ss = fmaf(h[i][r], h[i][r], ss);
         }
@@ -1028,18 +1029,7 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
         int row = (wave * W_GROUPS + i) * 8 + lrow;
         ow[i] = (unsigned)(((size_t)min(n0 + row, N - 1) * K + ((lslot ^ ((row >> 1) & 7)) * 8)) * 2);
     }
-    // With gridDim.z > 1 (the epilogue then is STORE_F32, `out` the partial sums [gridDim.z][M][N]) a block takes its share of
-    // the k-tiles, a contiguous range; no share is empty (the launcher sees to it).
-    int nk = K / 64;
-    if (gridDim.z > 1) {
-        const int share = (nk + gridDim.z - 1) / gridDim.z, k_first = blockIdx.z * share;
-        nk = min(share, nk - k_first);
-        out = (float*)out + (size_t)blockIdx.z * M * N;
-#pragma unroll
-        for (int i = 0; i < A_GROUPS; ++i) oa[i] += k_first * 128;
-#pragma unroll
-        for (int i = 0; i < W_GROUPS; ++i) ow[i] += k_first * 128;
-    }
+    const int nk = K / 64;
 #if defined(__HIP_DEVICE_COMPILE__)
     __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)min((size_t)(M + (TAIL != 0 ? over : 0)) * lda * 2, (size_t)0xffffffffu), 0x00020000);
     __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)min((size_t)N * K * 2, (size_t)0xffffffffu), 0x00020000);
@@ -1237,6 +1227,209 @@ __global__ __launch_bounds__(256) void gemm_fourwave_kernel(const bf16* __restri
     }
 }
 
+// Tiles of 256 x 128 and 128 x 128 whose four multiplying waves have four more beside them, one to a SIMD, that do nothing but bring the operands
+// straight into LDS (three k-tiles' places of 48 KB, four of 32).  A wave that multiplies then issues LDS reads and MFMAs alone, its registers hold no operands
+// on their way, and half of LDS's work at a k-tile, the writes from registers, goes: 64 MFMAs of a 256 x 128 k-tile take 1024 cycles of a
+// SIMD, its reads 768 of LDS and the loads into it 384.  Past the last k-tile the loading waves bring the old values
+// that the sums are added to.  Same layout in LDS and same order of k as the kernel above: bitwise the same results.
+// What bounds it: the clock under power for long rows (1.15-1.2 PFLOP/s), for short ones the way in and out.  256 x 128 tiles, waves bringing their own -> these, us: 2048 rows
+// 4096 x 4096 added to 64.7 -> 57.0 (61.0 without the old values ahead), 4096 x 14336 209.5 -> 202, 2032 rows 3072 x 2048 31.5 -> 28.0, 777 rows 6144 x 4096 49.6 -> 43.3.  128 x 128,
+// one block of these to a unit against two of four waves there: 2032 rows 2048 x 2048 added to 36.9 -> 22.7, 2048 x 8192 104 -> 60.
+// (The order of reads and MFMAs, two and two, by ones, two and four or reads first, and a raised priority of the multiplying waves: all within 2 %.)
+constexpr int fed_stages(int bm) { return bm == 256 ? 3 : 4; }
+// The += epilogue with the old values in LDS: piece (band i, wave w, p) is 1 KB, 64 lanes of 16 bytes, number (4 i + w) * 4 + p.  As many bands' as
+// two k-tiles' places hold (all of 128 rows, six of eight of 256) lie in `first` and `second`, the others' are read from memory.
+template <int BM>
+__device__ __forceinline__ void fed_add_epilogue(f32x4 (&acc)[BM / 32][4], unsigned char* mine, const unsigned char* first, const unsigned char* second,
+                                                 float* __restrict__ o, int ldc, int M, int N, int m_first, int n_first) {
+    constexpr int FM = BM / 32, PER = 4, IN_STAGE = (BM + 128) * 128 / 1024, IN_LDS = 2 * IN_STAGE / 16 < FM ? 2 * IN_STAGE / 16 : FM;      // IN_LDS: bands
+    constexpr int ROW_BYTES = 64 * 4 + 16;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), token = lane & 15, g = lane >> 4;
+    auto write = [&](auto ic) {
+        static_for<0, 4>([&](auto jc) { *(f32x4*)(mine + token * ROW_BYTES + (decltype(jc)::value * 16 + g * 4) * 4) = acc[decltype(ic)::value][decltype(jc)::value]; });
+    };
+    const int n = n_first + (lane & 15) * 4;
+    f32x4 late[FM > IN_LDS ? FM - IN_LDS : 1][PER];          // old values that are still to come
+    static_for<IN_LDS, FM>([&](auto ic) {
+#pragma unroll
+        for (int p = 0; p < PER; ++p) late[decltype(ic)::value - IN_LDS][p] = *(const f32x4*)(o + (size_t)min(m_first + decltype(ic)::value * 16 + p * 4 + g, M - 1) * ldc + min(n, N - 4));
+    });
+    write(std::integral_constant<int, 0>{});
+    static_for<0, FM>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        f32x4 v[PER], old[PER];
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            v[p] = *(const f32x4*)(mine + (p * 4 + g) * ROW_BYTES + (lane & 15) * 16);
+            if constexpr (i < IN_LDS) {
+                const int piece = (i * 4 + wave) * 4 + p;
+                old[p] = *(const f32x4*)((piece < IN_STAGE ? first + piece * 1024 : second + (piece - IN_STAGE) * 1024) + lane * 16);
+            } else old[p] = late[i - IN_LDS][p];
+        }
+        asm volatile("" ::: "memory");
+        if constexpr (i + 1 < FM) write(std::integral_constant<int, i + 1>{});
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            const int m = m_first + i * 16 + p * 4 + g;
+            if (m < M && n < N) *(f32x4*)(o + (size_t)m * ldc + n) = old[p] + v[p];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+template <int BM, int EPI>
+__global__ __launch_bounds__(512) void gemm_fed_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
+                                                       void* __restrict__ out, int ldc, int M, int N, int K, int epi, int old_ahead) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char fed_smem[];
+    constexpr int BN = 128, STAGES = fed_stages(BM), STAGE_BYTES = (BM + BN) * 128;
+    constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
+    constexpr int A_GROUPS = BM / 8 / 4, W_GROUPS = BN / 8 / 4, LOADS = A_GROUPS + W_GROUPS;      // 8-row groups of a loading wave
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int tile_row, tile_column;
+    tile_of_block(K, tile_row, tile_column);
+    const int m0 = tile_row * BM, n0 = tile_column * BN;
+    // With gridDim.z > 1 (the epilogue then is STORE_F32, `out` the partial sums [gridDim.z][M][N]) a block takes its share of
+    // the k-tiles, a contiguous range; no share is empty (the launcher sees to it).
+    int nk = K / 64, k_first = 0;
+    if (gridDim.z > 1) {
+        const int share = (nk + gridDim.z - 1) / gridDim.z;
+        k_first = blockIdx.z * share;
+        nk = min(share, nk - k_first);
+        out = (float*)out + (size_t)blockIdx.z * M * N;
+    }
+    if (wave >= 4) {
+        const int w = wave - 4, lrow = lane >> 3, lslot = lane & 7;
+        unsigned oa[A_GROUPS], ow[W_GROUPS];
+#pragma unroll
+        for (int i = 0; i < A_GROUPS; ++i) {
+            int row = (w * A_GROUPS + i) * 8 + lrow;
+            oa[i] = (unsigned)(((size_t)min(m0 + row, M - 1) * lda + ((lslot ^ ((row >> 1) & 7)) * 8)) * 2);
+        }
+#pragma unroll
+        for (int i = 0; i < W_GROUPS; ++i) {
+            int row = (w * W_GROUPS + i) * 8 + lrow;
+            ow[i] = (unsigned)(((size_t)min(n0 + row, N - 1) * K + ((lslot ^ ((row >> 1) & 7)) * 8)) * 2);
+        }
+#if defined(__HIP_DEVICE_COMPILE__)
+        __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)min((size_t)M * lda * 2, (size_t)0xffffffffu), 0x00020000);
+        __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)min((size_t)N * K * 2, (size_t)0xffffffffu), 0x00020000);
+#endif
+        // k-tile kt into its place; past the end the old values that the sums are added to (fed_add_epilogue), two places' worth of them
+        auto bring = [&](int kt, int place) {
+#if defined(__HIP_DEVICE_COMPILE__)
+            if (kt < nk) {
+                const unsigned base = __builtin_amdgcn_readfirstlane(place * STAGE_BYTES + w * A_GROUPS * 1024);
+                const unsigned wbase = __builtin_amdgcn_readfirstlane(place * STAGE_BYTES + BM * 128 + w * W_GROUPS * 1024);
+                const int at = (k_first + kt) * 128;
+#pragma unroll
+                for (int i = 0; i < A_GROUPS; ++i)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(fed_smem + base + i * 1024), 16, oa[i], at, 0, 0);
+#pragma unroll
+                for (int i = 0; i < W_GROUPS; ++i)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)(fed_smem + wbase + i * 1024), 16, ow[i], at, 0, 0);
+            } else if (EPI == LLMRS_EPI_ACCUM_F32 && old_ahead && kt < nk + 2) {
+                __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)min((size_t)M * ldc * 4, (size_t)0xffffffffu), 0x00020000);
+#pragma unroll
+                for (int i = 0; i < LOADS; ++i) {
+                    const int piece = (kt - nk) * (4 * LOADS) + w * LOADS + i, band = piece >> 4, cw = (piece >> 2) & 3, p = piece & 3;      // the band is of compute wave cw
+                    const int m = min(m0 + (cw >> 1) * (BM / 2) + band * 16 + p * 4 + (lane >> 4), M - 1), n = min(n0 + (cw & 1) * (BN / 2) + (lane & 15) * 4, N - 4);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(ro, (__attribute__((address_space(3))) void*)(fed_smem + __builtin_amdgcn_readfirstlane(place * STAGE_BYTES + (w * LOADS + i) * 1024)),
+                                                             16, (unsigned)(((size_t)m * ldc + n) * 4), 0, 0, 0);
+                }
+            }
+#endif
+        };
+#pragma unroll
+        for (int kt = 0; kt < STAGES; ++kt) bring(kt, kt);
+        const int last = nk + (EPI == LLMRS_EPI_ACCUM_F32 && old_ahead ? 2 : 0);
+        if (STAGES <= last) wait_vmcnt<(STAGES - 1) * LOADS>(); else wait_vmcnt<0>();
+        block_sync_lds();
+        int place = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            // k-tile kt + 1 is there when all but what has been started since have landed
+            if (kt + 1 < nk) {
+                if (kt + STAGES - 1 < last) wait_vmcnt<(STAGES - 2) * LOADS>();
+                else if (STAGES > 3 && kt + 2 < last) wait_vmcnt<LOADS>();
+                else wait_vmcnt<0>();
+            }
+            block_sync_lds();                        // and k-tile kt has been read
+            bring(kt + STAGES, place);
+            place = place == STAGES - 1 ? 0 : place + 1;
+        }
+        wait_vmcnt<0>();                       // (the bands of the results go through the same LDS)
+        block_sync_lds();
+        return;
+    }
+    const int wm = wave / 2, wn = wave % 2;
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int frow = lane & 15, h = lane >> 4, sw = (frow >> 1) & 7;
+    unsigned offa[2], offb[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        unsigned chunk = (unsigned)(((ks * 4 + h) ^ sw) * 16);
+        offa[ks] = (wm * TM + frow) * 128 + chunk;
+        offb[ks] = BM * 128 + (wn * TN + frow) * 128 + chunk;
+    }
+    bf16x8 fa[FM], fb[2][FN];
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    auto step = [&](const unsigned char* st, auto qc, auto multiply) {
+        constexpr int q = decltype(qc)::value, ks = q / 2, odd = q % 2;
+#pragma unroll
+        for (int j = odd * FN / 2; j < (odd + 1) * FN / 2; ++j) fb[ks][j] = *(const bf16x8*)(st + offb[ks] + j * 16 * 128);
+#pragma unroll
+        for (int i = odd * FM / 2; i < (odd + 1) * FM / 2; ++i) fa[i] = *(const bf16x8*)(st + offa[ks] + i * 16 * 128);
+        if constexpr (decltype(multiply)::value) {
+            constexpr int mk = q == 0 ? 1 : (q - 1) / 2, half = 1 - odd;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int i = half * FM / 2; i < (half + 1) * FM / 2; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[mk][j], fa[i], acc[i][j], 0, 0, 0);
+        }
+        static_for<0, (FM + FN) / 4>([](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        });
+        __builtin_amdgcn_sched_group_barrier(0x008, FM / 2 * FN, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto k_tile = [&](const unsigned char* st, auto not_first) {
+        step(st, I0{}, not_first);
+        step(st, I1{}, std::true_type{});
+        step(st, I2{}, std::true_type{});
+        step(st, I3{}, std::true_type{});
+        block_sync_lds();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    block_sync_lds();                          // k-tile 0 is there
+    const unsigned char* st = fed_smem;
+    k_tile(st, std::false_type{});
+    for (int kt = 1; kt < nk; ++kt) {
+        st = st == fed_smem + (STAGES - 1) * STAGE_BYTES ? fed_smem : st + STAGE_BYTES;
+        k_tile(st, std::true_type{});
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int i = FM / 2; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[i], acc[i][j], 0, 0, 0);
+    block_sync_lds();
+    if constexpr (EPI == LLMRS_EPI_ACCUM_F32) {
+        if (old_ahead) {
+            auto place = [&](int kt) { return fed_smem + kt % STAGES * STAGE_BYTES; };
+            fed_add_epilogue<BM>(acc, place(nk + 2) + wave * (16 * (TN * 4 + 16)), place(nk), place(nk + 1), (float*)out, ldc, M, N, m0 + wm * TM, n0 + wn * TN);
+            return;
+        }
+    }
+    band_epilogue<BM, BN, EPI>(acc, fed_smem, out, ldc, M, N, m0, n0, epi);
+}
+
 // Whether the four-wave tiles can finish this product: the epilogues it has, 16-bit results as whole 16-byte pieces.
 static bool fourwave_takes(int epi, const void* out, int ldc, int N) {
     if (epi == LLMRS_EPI_ACCUM_F32 || epi == LLMRS_EPI_STORE_F32) return true;
@@ -1244,13 +1437,41 @@ static bool fourwave_takes(int epi, const void* out, int ldc, int N) {
     if (epi_gated(epi)) return ldc % 8 == 0 && ((uintptr_t)out & 15) == 0 && N % 16 == 0;
     return false;
 }
-// over: rows of A and out beyond the M (whole tiles, at least four) that the tiles take along; 0 or, without splits, up to 16
+template <int BM, int EPI>
+static int launch_fed_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1) {
+    constexpr int BN = 128;
+    static bool configured = false;
+    const size_t bytes = (size_t)fed_stages(BM) * (BM + BN) * 128;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_fed_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (e != hipSuccess) return llmrs_fail("gemm: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+        configured = true;
+    }
+    dim3 grid(ceil_div(N, BN), ceil_div(M, BM), splits);
+    if (grid.y > 65535) return llmrs_fail("gemm: M=%d is too large for one launch", M);
+    const int old_ahead = EPI == LLMRS_EPI_ACCUM_F32 && splits == 1 && N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)out & 15) == 0 && (size_t)M * ldc * 4 < ((size_t)1 << 32);
+    gemm_fed_kernel<BM, EPI><<<grid, 512, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, old_ahead);
+    return 0;
+}
+// (operands under 4 GB each, K % 64 == 0, fourwave_takes(epi, ...): the caller's to check, and that no share of k is empty)
+template <int BM>
+static int launch_fed(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1) {
+    if (epi >= LLMRS_EPI_GLU_CLAMP) return launch_fed_epi<BM, LLMRS_EPI_GLU_CLAMP>(stream, A, lda, W, out, ldc, M, N, K, epi);
+    switch (epi) {
+        case LLMRS_EPI_STORE: return launch_fed_epi<BM, LLMRS_EPI_STORE>(stream, A, lda, W, out, ldc, M, N, K, epi);
+        case LLMRS_EPI_STORE_F32: return launch_fed_epi<BM, LLMRS_EPI_STORE_F32>(stream, A, lda, W, out, ldc, M, N, K, epi, splits);
+        case LLMRS_EPI_ACCUM_F32: return launch_fed_epi<BM, LLMRS_EPI_ACCUM_F32>(stream, A, lda, W, out, ldc, M, N, K, epi);
+        case LLMRS_EPI_SWIGLU: return launch_fed_epi<BM, LLMRS_EPI_SWIGLU>(stream, A, lda, W, out, ldc, M, N, K, epi);
+        default: return llmrs_fail("gemm: the tiles with waves for the loads have no epilogue %d", epi);
+    }
+}
+// over: rows of A and out beyond the M (whole tiles, at least four) that the tiles take along, up to 16
 template <int BM, int BN, int EPI, int TAIL = 0>
-static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1, int over = 0) {
+static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int over = 0) {
     if constexpr (TAIL == 0) {
-        if (over > 0 && M >= BM * (BN / 32)) return launch_fourwave_epi<BM, BN, EPI, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, over);
+        if (over > 0 && M >= BM * (BN / 32)) return launch_fourwave_epi<BM, BN, EPI, 1>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
         if constexpr (BN > 128)                     // (four tiles are a part for every wave pair of the narrow ones)
-            if (over > 0) return launch_fourwave_epi<BM, BN, EPI, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, over);
+            if (over > 0) return launch_fourwave_epi<BM, BN, EPI, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
     }
     static bool configured = false;
     size_t bytes = (size_t)2 * (BM + BN) * 128;
@@ -1260,9 +1481,9 @@ static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const
         if (e != hipSuccess) return llmrs_fail("gemm: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
         configured = true;
     }
-    dim3 grid(ceil_div(N, BN), ceil_div(M, BM), splits);
+    dim3 grid(ceil_div(N, BN), ceil_div(M, BM));
     if (grid.y > 65535) return llmrs_fail("gemm: M=%d is too large for one launch", M);
-    if (over > 0 && (over > 16 || splits != 1 || M % BM != 0 || TAIL * (int)grid.y < BN / 32))
+    if (over > 0 && (over > 16 || M % BM != 0 || TAIL * (int)grid.y < BN / 32))
         return llmrs_fail("gemm: the four-wave tiles cannot take %d rows beyond M=%d along", over, M);
     gemm_fourwave_kernel<BM, BN, EPI, TAIL><<<grid, 256, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, over);
     return 0;
@@ -1270,12 +1491,14 @@ static int launch_fourwave_epi(hipStream_t stream, const bf16* A, int lda, const
 // (operands under 4 GB each, K % 64 == 0, fourwave_takes(epi, ...): the caller's to check)
 template <int BM, int BN>
 static int launch_fourwave(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int over = 0) {
-    if (epi >= LLMRS_EPI_GLU_CLAMP) return launch_fourwave_epi<BM, BN, LLMRS_EPI_GLU_CLAMP>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
+    constexpr int TAIL = BN == 128 ? 1 : 0;       // (256 x 128 tiles without rows to take along are launch_fed's)
+    if (TAIL == 1 && over == 0) return launch_fed<256>(stream, A, lda, W, out, ldc, M, N, K, epi);
+    if (epi >= LLMRS_EPI_GLU_CLAMP) return launch_fourwave_epi<BM, BN, LLMRS_EPI_GLU_CLAMP, TAIL>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
     switch (epi) {
-        case LLMRS_EPI_STORE: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
-        case LLMRS_EPI_STORE_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE_F32>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
-        case LLMRS_EPI_ACCUM_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_ACCUM_F32>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
-        case LLMRS_EPI_SWIGLU: return launch_fourwave_epi<BM, BN, LLMRS_EPI_SWIGLU>(stream, A, lda, W, out, ldc, M, N, K, epi, 1, over);
+        case LLMRS_EPI_STORE: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE, TAIL>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
+        case LLMRS_EPI_STORE_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_STORE_F32, TAIL>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
+        case LLMRS_EPI_ACCUM_F32: return launch_fourwave_epi<BM, BN, LLMRS_EPI_ACCUM_F32, TAIL>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
+        case LLMRS_EPI_SWIGLU: return launch_fourwave_epi<BM, BN, LLMRS_EPI_SWIGLU, TAIL>(stream, A, lda, W, out, ldc, M, N, K, epi, over);
         default: return llmrs_fail("gemm: the four-wave tiles have no epilogue %d", epi);
     }
 }
@@ -1290,6 +1513,7 @@ static int skinny_splits(int N, int K) {
     while (blocks <= 64 && blocks * splits < 256 && splits < 16 && nkb / (splits * 2) >= 8) splits *= 2;
     return splits;
 }
+// (128 x 128 tiles for 17 to 64 rows, and for operands of 4 GB and more.)
 // Up to 256 rows whose 128 x 128 tiles are no more than the compute units: one block of eight waves per
 // unit with four k-tiles in LDS (three on their way) instead of two blocks of four waves with two
 // k-tiles each.  A tile's loads into LDS take longer than its MFMAs, and with few blocks per unit
@@ -1316,34 +1540,51 @@ static int launch_tiles_128(hipStream_t stream, const bf16* A, int lda, const bf
     if (deep_tiles(M, N, K)) return launch_dma<128, 128, 2, 4, 4>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, partial, next, finish);
     return launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W, out, ldc, M, N, K, epi, splits, partial, next, finish);
 }
-// From 512 rows on, where square large tiles would not fill the device: tiles of 256 x 128 on four waves, a block to a unit, or
-// the 128 x 128 tiles above, two to a unit, by the time either takes: the k-tiles that a unit works through, round after
-// round, times what one takes there (measured, us: 1.0 for a 256 x 128 k-tile of 64, 1.25 for two of 128 x 128, 1.05 for
-// one that is alone), and for a block of the first what its way in and out takes beyond what two blocks of a unit hide from each other:
-// 1.5 where it stores 16-bit results, none where 32-bit ones, 0.8 where gated halves, 6 where it adds to 32-bit ones, and 3.5 where it leaves
-// a part of the sum, 5 of a weight of fewer than 2048 features (each XCD then reads all rows).  Both split k over blocks until
-// the device is full.  Measured, 128 x 128 -> 256 x 128: 2032 rows 2048 x 8192 in 2 parts 81 -> 71 us, 3072 x 2048
-// 35 -> 29; 1024 rows 4096 x 14336 in 2 parts 140 -> 111; 512 rows in 4 parts 78 -> 64; but 600 rows 4096 x 128
-// added to 32-bit 7.5 -> 12 us, 2049 rows 4096 x 1024 40 -> 48, 640 rows 512 x 2048 in 4 parts 15.2 -> 17.7.  (512 to 6000 rows of 160 to 8192
-// features, k from 64 to 4096, every epilogue, against 128 x 128 alone: none slower by more than 3 %.  Both sum in one
-// order.  The two operands' sizes, under 4 GB, are looked at where it is launched.)
+// More than 64 rows, where square large tiles would not fill the device: tiles of 256 x 128 or of 128 x 128 with waves of their own for the loads, a
+// block to a unit, with k split over 1 to 16 blocks, whichever takes the least time (us) by what was measured: a part for every k-tile
+// of a round, a part that follows how full the device is (the clock follows the power), a block's way in and out, the operands' first trip from
+// memory, and for a split product the kernel that adds the parts up, or the norm's own kernel where a product that adds to the stream is not split.
+// (603 products of 65 to 4200 rows, 160 to 28,000 features and k of 64 to 14336, every epilogue, weights from memory: the plans chosen take 1.010 of the
+// best of all nine, and 0.8 of the time of the 128 x 128 and 256 x 128 tiles before, whose waves brought their own operands; those were the
+// faster ones nowhere from 512 rows on.  us, before and now: 2032 rows 2048 x 2048 added to, with the norm 39.0 -> 33.1, 2048 x 8192 87.6 -> 75.5,
+// 3072 x 2048 33.0 -> 29.4; 1024 rows 4096 x 4096 with the norm 51.1 -> 48.2, 900 rows 3072 x 2048 28.5 -> 18.0, 450 rows 6144 x 4096 46.9 -> 33.9, 200 rows 4096 x 14336
+// 48.5 -> 43.7, 96 rows 2048 x 2048 16.0 -> 13.9.  The worst choice: 1047 rows 4096 x 10368, 157 and 113 in two parts.)
+// The two operands' sizes, under 4 GB, are looked at where it is launched.
 struct MidTiles {
-    bool four;
+    int rows;          // of a tile: 256 or 128
     int splits;
     double time;
 };
 static MidTiles mid_tiles(int M, int N, int K, int epi, bool may_split = true) {
-    const int cus = llmrs_compute_units(), nk = K / 64, s = may_split ? tiled_splits(M, N, K) : 1;
-    const long tall = (long)ceil_div(M, 256) * ceil_div(N, 128), small = (long)ceil_div(M, 128) * ceil_div(N, 128) * s;
-    const long last = small % (2L * cus);
-    const double small_time = (1.25 * (double)(small / (2L * cus)) + (last == 0 ? 0.0 : last <= cus ? 1.05 : 1.25)) * ceil_div(nk, s);
-    if (M < 512 || K % 64) return MidTiles{false, s, small_time};
-    int z = 1;
-    while (may_split && tall * z * 2 <= cus && z < 16 && nk / (z * 2) >= 8 && (z * 2 - 1) * ceil_div(nk, z * 2) < nk) z *= 2;
-    const double in_and_out = z > 1 ? (N >= 2048 ? 3.5 : 5.0) : epi == LLMRS_EPI_ACCUM_F32 ? 6.0 : epi == LLMRS_EPI_STORE_F32 ? 0.0 : epi_gated(epi) ? 0.8 : 1.5;
-    const double tall_time = (double)ceil_div(tall * z, (long)cus) * (ceil_div(nk, z) + in_and_out);
-    if (tall_time <= small_time) return MidTiles{true, z, tall_time};
-    return MidTiles{false, s, small_time};
+    const int cus = llmrs_compute_units(), nk = K / 64;
+    MidTiles best{128, 1, 1e30};
+    if (K % 64) return best;
+    const double mn = (double)M * N * 1e-6, mk = (double)M * K * 2e-6, nkb = (double)N * K * 2e-6;
+    const bool adds = epi == LLMRS_EPI_ACCUM_F32;
+    for (int rows = 256; rows >= 128; rows /= 2)
+        for (int z = 1; z == 1 || (may_split && z <= 16 && nk / z >= 8); z *= 2) {
+            const int share = ceil_div(nk, z);
+            if ((z - 1) * share >= nk) continue;                      // (no share may be empty)
+            const long blocks = (long)ceil_div(M, rows) * ceil_div(N, 128) * z;
+            const double rounds = (double)ceil_div(blocks, (long)cus), full = (double)blocks / cus;
+            const bool stores_f32 = epi == LLMRS_EPI_STORE_F32 || z > 1;
+            double t = rows == 256 ? rounds * (3.2 + 0.42 * share + (stores_f32 ? 1.9 : adds ? 3.2 : 0.0)) + 0.28 * share * full + 0.16 * mk + 0.06 * nkb
+                                   : rounds * (2.3 + 0.28 * share + (stores_f32 ? 1.0 : adds ? 1.9 : 0.0)) + 0.18 * share * full + 0.05 * mk + 0.085 * nkb;
+            t += 3.0;
+            if (z > 1) t = 1.06 * (t + 2.5 + 0.2 * mn * (4 * z + (adds ? 8 : epi == LLMRS_EPI_STORE_F32 ? 4 : epi_gated(epi) ? 1 : 2)));
+            else if (adds) t += 2.0 + 1.33 * mn;
+            if (t < best.time) best = MidTiles{rows, z, t};
+        }
+    return best;
+}
+static int launch_mid(hipStream_t stream, int rows, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1) {
+    return rows == 256 ? launch_fed<256>(stream, A, lda, W, out, ldc, M, N, K, epi, splits) : launch_fed<128>(stream, A, lda, W, out, ldc, M, N, K, epi, splits);
+}
+// As parts of its sum, for whatever epilogue follows: the most that any of them asks for (so much room is what a caller brings).
+static int most_splits(int M, int N, int K) {
+    int most = 1;
+    for (int epi : {LLMRS_EPI_STORE, LLMRS_EPI_STORE_F32, LLMRS_EPI_ACCUM_F32, LLMRS_EPI_SWIGLU}) most = std::max(most, mid_tiles(M, N, K, epi).splits);
+    return most;
 }
 // 17..64 rows on a weight of middling width (more than 4096 features, fewer than the wide ones that
 // get blocks of many feature tiles): the 128 x 128 tiles with k split over blocks.  Where they add to the stream their finish also
@@ -1362,7 +1603,16 @@ static bool ring_stores_faster(int M, int N, int K) {
     const bool tiles_between = M > 32 && N > (M <= 40 ? 12288 : 8192) && K > 2048 && K < 4096;
     return K <= (M <= 48 ? 4096 : 1024) && !tiles_between;
 }
-// Room (in floats) for the partial sums of a product that would be split: what the caller should bring.
+// Whether a product of more than 64 rows goes to the tiles of `mid_tiles` (the launcher asks the same).
+static bool mid_takes(int M, int N, int K) { return M > 64 && K % 64 == 0 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160; }
+// What `mid_tiles` says of a product that goes there: 100 times the splits and 1 or 2 for tiles of 128 or 256 rows; 0 where it does not go.
+extern "C" int llmrs_gemm_mid_plan(int M, int N, int K, int epi) {
+    if (!mid_takes(M, N, K)) return 0;
+    const MidTiles plan = mid_tiles(M, N, K, epi);
+    return 100 * plan.splits + plan.rows / 128;
+}
+// Room (in floats) for the partial sums of a product that would be split: what the caller should bring.  (A little of it
+// where none is split but the norm that follows can be finished, which is asked for by bringing some.)
 extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
     if (M > 16 && M <= 64) {
         int s = few_rows_take_tiles(M, N, K) ? tiled_splits(M, N, K) : skinny_splits(N, K);
@@ -1373,8 +1623,8 @@ extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
         return s > 1 ? (long)s * (M % 256) * N : 0;
     }
     if (M > 64 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160) {
-        int s = mid_tiles(M, N, K, LLMRS_EPI_ACCUM_F32).splits;      // (no epilogue's plan has more parts)
-        long own = s > 1 ? (long)s * M * N : 0;
+        int s = most_splits(M, N, K);
+        long own = s > 1 ? (long)s * M * N : mid_takes(M, N, K) ? 64 : 0;
         // a few rows beyond whole 128-row tiles may go to the kernel for few rows, and the whole tiles be split then
         int over128 = M % 128;
         if (M >= 1024 && over128 > 0 && over128 <= 64 && K % 64 == 0)
@@ -1384,13 +1634,11 @@ extern "C" long llmrs_gemm_workspace_floats(int M, int N, int K) {
     return 0;
 }
 
-// 17 rows or more whose sums are split over blocks: the kernel that adds the parts up can finish the following norm.
-// (Beyond 256 rows that is where the 128 x 128 tiles take all rows with k split: a narrow weight whose tiles leave
-// half of the device's places empty, as the o and down products of a small model do beside a prompt portion.)
+// 17 rows or more whose sums are split over blocks: the kernel that adds the parts up can finish the following norm.  So can, in a launch
+// behind the product, every product of more than 64 rows that goes to the tiles of `mid_tiles`, split or not.
 extern "C" int llmrs_gemm_norms_whole(int M, int N, int K) {
     if (!(M > 16 && N >= 4 && N % 4 == 0 && N <= 16384 && K % 8 == 0)) return 0;
-    if (M <= 256) return llmrs_gemm_workspace_floats(M, N, K) > 0;
-    return K % 64 == 0 && (long)ceil_div(M, 256) * ceil_div(N, 256) < 160 && mid_tiles(M, N, K, LLMRS_EPI_ACCUM_F32).splits > 1;
+    return M <= 64 ? llmrs_gemm_workspace_floats(M, N, K) > 0 : mid_takes(M, N, K);
 }
 
 // The product as parts of its sum over k, [parts][M][N] 32-bit in `workspace`, for a caller that adds them up itself
@@ -1400,10 +1648,14 @@ extern "C" int llmrs_gemm_norms_whole(int M, int N, int K) {
 int llmrs_gemm_bf16_split_parts(hipStream_t stream, const bf16* A, int lda, const bf16* W, int M, int N, int K,
                                 void* workspace, size_t workspace_bytes) {
     if (K % 64 || lda % 8 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) || workspace == nullptr || M > 512) return 0;
-    const bool tiles = M > 64 ? !((long)ceil_div(M, 256) * ceil_div(N, 256) >= 160 && M > 128) : few_rows_take_tiles(M, N, K);
-    int splits = tiles ? tiled_splits(M, N, K) : 1;
+    const bool small = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
+    if (M > 64 ? (long)ceil_div(M, 256) * ceil_div(N, 256) >= 160 || !small : !few_rows_take_tiles(M, N, K)) return 0;
+    const MidTiles plan = M > 64 ? mid_tiles(M, N, K, LLMRS_EPI_STORE) : MidTiles{0, tiled_splits(M, N, K), 0.0};
+    const int splits = plan.splits;
     if (splits <= 1 || workspace_bytes < (size_t)splits * M * N * sizeof(float)) return 0;
-    if (launch_tiles_128(stream, A, lda, W, nullptr, N, M, N, K, LLMRS_EPI_STORE, splits, (float*)workspace, nullptr, false) != 0) return -1;
+    const int rc = plan.rows != 0 ? launch_mid(stream, plan.rows, A, lda, W, workspace, N, M, N, K, LLMRS_EPI_STORE_F32, splits)
+                                  : launch_tiles_128(stream, A, lda, W, nullptr, N, M, N, K, LLMRS_EPI_STORE, splits, (float*)workspace, nullptr, false);
+    if (rc != 0) return -1;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { llmrs_fail("gemm (mfma): launch failed: %s", hipGetErrorString(e)); return -1; }
     return splits;
@@ -1503,16 +1755,14 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         else if (M <= 48) rows_of(std::integral_constant<int, 3>{});
         else rows_of(std::integral_constant<int, 4>{});
     } else {
-        // K % 64 == 0: tiles loaded straight into LDS, two k-tiles of 64 there.  Other K: through
+        // K % 64 == 0: tiles whose operands are brought into LDS whole k-tiles of 64 ahead.  Other K: through
         // registers, with zero-filled tails.
-        // 256 x 256 tiles of eight waves in two groups out of step (128 x 64 per wave: one LDS read
-        // per MFMA less than the 64 x 64 per wave of the 128 x 128 tiles) where they fill most of the
-        // device; else 128 x 128
-        // tiles of four waves, two blocks to a compute unit, with the k range split over blocks when
-        // even those are too few (measured on MI355X).
+        // 256 x 256 tiles where they fill most of the device (from 160 of them on; below, the smaller ones take less time, above they
+        // take 1.01 to 1.27 of it at 41 of 43 sizes); else 256 x 128 or 128 x 128, with the k range split over blocks when even
+        // those are too few (mid_tiles).
         // One large tile runs on a compute unit at a time, so a grid of them works in rounds and the
         // last round may be far from full (896 tiles on 256 units: 3.5 rounds cost 4).  Then the large
-        // tiles get the features that make whole rounds and the small tiles, two to a unit, the rest.
+        // tiles get the features that make whole rounds and the smaller ones the rest.
         long m_tiles = ceil_div(M, 256), big_tiles = m_tiles * ceil_div(N, 256);
         int cus = llmrs_compute_units();
         // A few rows beyond whole tiles (a prompt portion of 2048 tokens beside 16 decoded ones)
@@ -1559,10 +1809,12 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                      : small ? launch_pingpong<256, 256, 2, 4, true>(stream, A, lda, W, out, ldc, M, n_split, K, epi)
                              : launch_pingpong<256, 256, 2, 4, false>(stream, A, lda, W, out, ldc, M, n_split, K, epi);
                 if (rc == 0) {
-                    if (four && fourwave_takes(epi, out_rest, ldc, N - n_split) && mid_tiles(M, N - n_split, K, epi, false).four)
+                    const bool fed = four && fourwave_takes(epi, out_rest, ldc, N - n_split);
+                    if (fed && mid_tiles(M, N - n_split, K, epi, false).rows == 256)
                         rc = launch_fourwave<256, 128>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi, along);
                     else {
-                        rc = launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
+                        rc = fed ? launch_fed<128>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi)
+                                 : launch_dma<128, 128, 2, 2, 2>(stream, A, lda, W + (size_t)n_split * K, out_rest, ldc, M, N - n_split, K, epi);
                         if (rc == 0 && along > 0) {
                             int took = llmrs_gemm_bf16_mfma(stream, A + (size_t)M * lda, lda, W + (size_t)n_split * K,
                                                             (char*)out_rest + (size_t)M * ldc * elt, ldc, along, N - n_split, K, epi, nullptr, 0);
@@ -1594,29 +1846,30 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                 return plan;
             };
             int over128 = M % 128;
-            if (M >= 1024 && over128 > 0 && over128 <= 64 && !whole && next == nullptr && scale == nullptr) {
+            if (M >= 1024 && over128 > 0 && over128 <= 64) {
                 if (plan_of(M).time - plan_of(M - over128).time >= 30.0) {
                     size_t elt = (epi == LLMRS_EPI_STORE_F32 || epi == LLMRS_EPI_ACCUM_F32) ? sizeof(float) : sizeof(bf16);
                     int whole_rows = M - over128;
                     rc = llmrs_gemm_bf16_mfma(stream, A, lda, W, out, ldc, whole_rows, N, K, epi, workspace, workspace_bytes, qkv);
                     if (rc != 1) return rc;
-                    return llmrs_gemm_bf16_mfma(stream, A + (size_t)whole_rows * lda, lda, W, (char*)out + (size_t)whole_rows * ldc * elt,
-                                                ldc, over128, N, K, epi, workspace, workspace_bytes, qkv);
+                    rc = llmrs_gemm_bf16_mfma(stream, A + (size_t)whole_rows * lda, lda, W, (char*)out + (size_t)whole_rows * ldc * elt,
+                                              ldc, over128, N, K, epi, workspace, workspace_bytes, qkv);
+                    if (rc == 1 && whole) launch_splitk_finish(stream, nullptr, 0, out, ldc, M, N, epi, next);
+                    return rc;
                 }
             }
-            // (a wider tile brings less into a unit for the same work: a k-step of 256 x 128 48 KB, of two 128 x 128 64 KB)
             const MidTiles plan = plan_of(M);
             const int splits = plan.splits;
-            if (plan.four && small && splits > 1) {
-                rc = launch_fourwave_epi<256, 128, LLMRS_EPI_STORE_F32>(stream, A, lda, W, workspace, N, M, N, K, LLMRS_EPI_STORE_F32, splits);
+            if (small && splits > 1) {
+                rc = launch_mid(stream, plan.rows, A, lda, W, workspace, N, M, N, K, LLMRS_EPI_STORE_F32, splits);
                 if (rc == 0) launch_splitk_finish(stream, (const float*)workspace, splits, out, ldc, M, N, epi, next);
-            } else if (plan.four && small && !whole && next == nullptr && fourwave_takes(epi, out, ldc, N))
-                rc = launch_fourwave<256, 128>(stream, A, lda, W, out, ldc, M, N, K, epi);
-            else if (splits > 1)
+            } else if (splits > 1)
                 rc = launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, splits, (float*)workspace, next);
-            else if (whole) rc = llmrs_fail("gemm: M=%d N=%d K=%d is not split after all: the norm cannot be finished here", M, N, K);
-            else
-                rc = launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, 1, nullptr);
+            else {
+                rc = small && fourwave_takes(epi, out, ldc, N) ? launch_mid(stream, plan.rows, A, lda, W, out, ldc, M, N, K, epi)
+                                                               : launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, 1, nullptr);
+                if (rc == 0 && whole) launch_splitk_finish(stream, nullptr, 0, out, ldc, M, N, epi, next);
+            }
         }
         else rc = launch_tiled<128, 128, 64, 1>(stream, A, lda, W, out, ldc, M, N, K, epi);
     }

@@ -743,6 +743,35 @@ def test_gemm_rows_that_go_along_with_large_tiles(M, N, K):
         assert torch.equal(room[M:], before[M:])
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 130, 64), (66, 16, 128), (129, 128, 192), (300, 1000, 256), (257, 384, 320), (512, 136, 384), (1000, 3000, 64), (640, 2064, 2048),
+                                   (1040, 4096, 832), (130, 28000, 320), (1500, 6150, 448), (2040, 2056, 1088), (600, 8200, 128)])
+def test_gemm_tiles_with_waves_for_the_loads(M, N, K):
+    """Fewer k-tiles than LDS has places for and more, rows and features beyond whole tiles, one block and several rounds of them, split and not,
+    features of a number that four does not divide (their old values are read when they are due): every epilogue, the rows of both operands further apart than they
+    are long, nothing touched behind the last row.  (Bounds as in `test_gemm_rows_that_go_along_with_large_tiles`.)"""
+    k = kernels()
+    a = rnd((M, K + 24), torch.bfloat16, 3)[:, :K]
+    w = rnd((N, K), torch.bfloat16, 4, 0.1)
+    acc = product64(a, w)
+    g, u = acc[:, 0::2], acc[:, 1::2]
+    clamped = k.glu_clamp_slot(1.5, 1.702, 0.0, 1.0)
+    floor, gm, um = 1e-5 * math.sqrt(K), g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+    for epi, ref in ((EPI_STORE, acc), (EPI_STORE_F32, acc), (EPI_ACCUM_F32, acc), (EPI_SWIGLU, plain_silu(g) * u),
+                     (EPI_GLU_CLAMP, gm / (1 + torch.exp(-1.702 * gm)) * (um + 1.0))):
+        assert k.lib.llmrs_gemm_mid_plan(M, N, K, epi) > 0
+        dtype = torch.float32 if epi in (EPI_STORE_F32, EPI_ACCUM_F32) else torch.bfloat16
+        room = rnd((M + 16, ref.shape[1] + 8), dtype, 5)
+        before = room.clone()
+        want = ref + before[:M, :ref.shape[1]].double().cpu() if epi == EPI_ACCUM_F32 else ref
+        n_ws = k.gemm_workspace_floats(M, N, K)
+        for ws in (torch.empty(n_ws, device=DEV) if n_ws else None, None):       # (without room nothing is split)
+            room.copy_(before)
+            k.gemm(a, w, room[:M, :ref.shape[1]], epi, ws, **({"glu": clamped} if epi == EPI_GLU_CLAMP else {}))
+            err = (room[:M, :ref.shape[1]].double().cpu() - want).abs()
+            assert (err <= out_tol(want, dtype, floor * (1 if ref is acc else 1 + 0.1 * math.sqrt(K) + 2.5))).all(), (epi, float(err.max()))
+            assert torch.equal(room[M:], before[M:]) and torch.equal(room[:, ref.shape[1]:], before[:, ref.shape[1]:])
+
+
 @pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 2050, 4098, 64), (torch.bfloat16, 700, 6145, 128), (torch.bfloat16, 2048, 6148, 64),
                                          (torch.float32, 300, 2050, 64), (torch.float32, 1030, 8196, 32), (torch.float32, 257, 1023, 96)])
 @pytest.mark.parametrize("pad,first", [(0, 0), (4, 4), (2, 2), (1, 1)])
