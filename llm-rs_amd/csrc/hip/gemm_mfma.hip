@@ -242,7 +242,6 @@ __global__ void gemm_splitk_finish_kernel(const float* __restrict__ partial, int
 // The same for a product that adds into the 32-bit stream and is followed by a norm x / rms(x) * weight: a block
 // for each row adds the parts in the same order, writes the stream's new row, and, having the whole row, the
 // normed row as well (NextNorm with eps): no norm kernel runs.  Up to 16384 features (16 per thread), a multiple of 4.
-// With no parts (splits 0) the stream's rows are whole already and only the norm is left to do.
 __global__ __launch_bounds__(1024) void gemm_splitk_finish_norm_kernel(const float* __restrict__ partial, int splits,
                                                                         float* __restrict__ out, int ldc, int M, int N,
                                                                         NextNorm nn) {
@@ -260,7 +259,7 @@ __global__ __launch_bounds__(1024) void gemm_splitk_finish_norm_kernel(const flo
             f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int s = 0; s < splits; ++s) v += *(const f32x4*)(p0 + (size_t)s * M * N + n);
             h[i] = *(const f32x4*)(o + n) + v;
-            if (splits > 0) *(f32x4*)(o + n) = h[i];
+            *(f32x4*)(o + n) = h[i];
 #pragma unroll
             for (int r = 0; r < 4; ++r) ss = fmaf(h[i][r], h[i][r], ss);
         }
@@ -282,6 +281,44 @@ __global__ __launch_bounds__(1024) void gemm_splitk_finish_norm_kernel(const flo
             *(bf16x4*)((bf16*)nn.y + (size_t)m * nn.ldy + n) = y;
         }
     }
+}
+// The norm alone, of rows that a product has added to as a whole: bound by reading them (2048 rows of 4096: 50 MB).  A block for each row, four pieces of it
+// and of the weight asked for at once by every thread, 256 threads for 4096 features: 8.8 us, of 2048 features 5.9; the kernel above with no parts,
+// 1024 threads that wait for the row before they ask for the weight, 12.2 and 6.9.  Features as there.
+__global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict__ x, int ldx, int N, NextNorm nn) {
+    __shared__ float red[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+    const float* row = x + (size_t)blockIdx.x * ldx;
+    f32x4 h[4], w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = (i * (int)blockDim.x + tid) * 4;
+        h[i] = n < N ? *(const f32x4*)(row + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+        w[i] = n < N ? *(const f32x4*)(nn.weight + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ss = fmaf(h[i][r], h[i][r], ss);
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    float total = 0.0f;
+    for (int i = 0; i < waves; ++i) total += red[i];
+    const float inv = 1.0f / sqrtf(total / (float)N + nn.eps);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = (i * (int)blockDim.x + tid) * 4;
+        if (n >= N) continue;
+        bf16x4 y;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = (bf16)(h[i][r] * inv * w[i][r]);
+        *(bf16x4*)((bf16*)nn.y + (size_t)blockIdx.x * nn.ldy + n) = y;
+    }
+}
+static void launch_norm_rows(hipStream_t stream, const void* x, int ldx, int M, int N, const NextNorm& next) {
+    norm_rows_kernel<<<M, min(1024, max(64, ceil_div(ceil_div(N, 16), 64) * 64)), 0, stream>>>((const float*)x, ldx, N, next);
 }
 // Adds the parts of a split product up: with the norm that follows where one is to be finished (NextNorm with eps).
 static void launch_splitk_finish(hipStream_t stream, const float* partial, int splits, void* out, int ldc, int M, int N,
@@ -1854,7 +1891,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
                     if (rc != 1) return rc;
                     rc = llmrs_gemm_bf16_mfma(stream, A + (size_t)whole_rows * lda, lda, W, (char*)out + (size_t)whole_rows * ldc * elt,
                                               ldc, over128, N, K, epi, workspace, workspace_bytes, qkv);
-                    if (rc == 1 && whole) launch_splitk_finish(stream, nullptr, 0, out, ldc, M, N, epi, next);
+                    if (rc == 1 && whole) launch_norm_rows(stream, out, ldc, M, N, *next);
                     return rc;
                 }
             }
@@ -1868,7 +1905,7 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
             else {
                 rc = small && fourwave_takes(epi, out, ldc, N) ? launch_mid(stream, plan.rows, A, lda, W, out, ldc, M, N, K, epi)
                                                                : launch_tiles_128(stream, A, lda, W, out, ldc, M, N, K, epi, 1, nullptr);
-                if (rc == 0 && whole) launch_splitk_finish(stream, nullptr, 0, out, ldc, M, N, epi, next);
+                if (rc == 0 && whole) launch_norm_rows(stream, out, ldc, M, N, *next);
             }
         }
         else rc = launch_tiled<128, 128, 64, 1>(stream, A, lda, W, out, ldc, M, N, K, epi);
