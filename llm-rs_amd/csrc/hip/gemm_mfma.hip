@@ -1314,9 +1314,129 @@ __device__ __forceinline__ void fed_add_epilogue(f32x4 (&acc)[BM / 32][4], unsig
         __builtin_amdgcn_sched_barrier(0);
     });
 }
+// The q/k/v epilogue of those tiles: the rotation and the cache writes, which were a kernel of their own behind the product (2047 rows, 32 heads on 8 of 64,
+// k 2048: 43.3 us for the two, 33.0 in one; 8 of 128 and k 4096 at 1023 rows 66.5 and 55; the product alone 30 and 51).  The rows of q and k
+// are also rounded once instead of twice: error against 64 bits 2.34e-3 -> 1.66e-3 of their norm.
+struct NothingMore {};
+template <int EPI>
+using MoreOf = std::conditional_t<EPI == LLMRS_EPI_QKV, QkvEpilogue, NothingMore>;
+
+// The sine and cosine of x, |x| below 2^24: whole turns are taken off by fused multiply-adds with 2 pi in three parts (Cody and Waite's reduction), what
+// is left, within half a turn, goes to the vector unit's own instructions, which take turns.
+__device__ __forceinline__ void sine_cosine(float x, float& sine, float& cosine) {
+    const float n = rintf(x * 0.159154943f);
+    float r = __builtin_fmaf(n, -6.28318548f, x);
+    r = __builtin_fmaf(n, 1.74845553e-07f, r);
+    r = __builtin_fmaf(n, 6.86049956e-15f, r) * 0.159154943f;
+    sine = __builtin_amdgcn_sinf(r);
+    cosine = __builtin_amdgcn_cosf(r);
+}
+// What a lane of a multiplying wave asks for before its products: its tokens' positions (fragment i holds token lane % 16 of 16) and the slots of the
+// rows of q and k that it stores pieces of (row p * 8 + lane / 8 of a band of 32); below 0 where nothing is to be written.
+__device__ __forceinline__ int slot_of_row(const QkvEpilogue& qe, int M, int m) {
+    const int slot = qe.write_kv && m < M ? qe.slot_map[m] : -1;
+    return slot < qe.num_pages * 16 ? slot : -1;
+}
+template <int BM>
+struct QkvRows {
+    static constexpr int FM = BM / 32, BANDS = FM / 2;
+    float place[FM];
+    int slot[BANDS][4];
+};
+template <int BM>
+__device__ __forceinline__ QkvRows<BM> qkv_rows(const QkvEpilogue& qe, int M, int m_first) {
+    const int lane = threadIdx.x & 63;
+    QkvRows<BM> rows;
+#pragma unroll
+    for (int i = 0; i < rows.FM; ++i) rows.place[i] = (float)qe.positions[min(m_first + i * 16 + (lane & 15), M - 1)];
+#pragma unroll
+    for (int b = 0; b < rows.BANDS; ++b)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) rows.slot[b][p] = slot_of_row(qe, M, m_first + b * 32 + p * 8 + (lane >> 3));
+    return rows;
+}
+// A wave's 64 features: pairs turn where they lie, in 32-bit, before their one rounding; the rows go through LDS, `mine` (BM / 2 rows, 16 bytes further
+// apart than they are long), and those of q and k leave 16 bytes a lane, to the output and to the pages' rows.  Pages of 16 slots, heads
+// of a multiple of 8 features.
+constexpr int QKV_ROW_BYTES = 64 * 2 + 16;
+template <int BM>
+__device__ __forceinline__ void qkv_epilogue(f32x4 (&acc)[BM / 32][4], unsigned char* mine, bf16* __restrict__ out, int ldc, int M,
+                                             int m_first, int n_first, const QkvEpilogue& qe, const QkvRows<BM>& rows) {
+    constexpr int FN = 4;
+    const int lane = threadIdx.x & 63, token = lane & 15, four = (lane >> 4) * 4, hd = qe.head_dim;
+    const int keys_from = qe.n_heads * hd, values_from = keys_from + qe.n_kv_heads * hd;
+    float freq[FN][2];
+    unsigned turning = 0;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int n = n_first + j * 16 + four, d = n % hd;
+        const bool turns = n < values_from && d < qe.rotary_dim;
+        turning |= turns ? 1u << j : 0u;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) freq[j][r] = turns ? qe.inv_freq[d / 2 + r] : 0.0f;
+    }
+    // where this lane's pieces of rows go
+    const int n = n_first + (lane & 7) * 8, kvh = (n - keys_from) / hd;
+    bf16* const k_at = (bf16*)qe.k_cache + ((size_t)kvh * 16 * hd + (n - keys_from - kvh * hd));
+    const size_t page_size = (size_t)qe.n_kv_heads * 16 * hd;                     // of all kv heads
+    auto write = [&](auto bandc) {
+        static_for<0, 2 * FN>([&](auto jc) {
+            constexpr int half = decltype(jc)::value / FN, j = decltype(jc)::value % FN, i = 2 * decltype(bandc)::value + half;
+            f32x4 v = acc[i][j];
+            if (turning >> j & 1) {
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    float sn, cs;
+                    sine_cosine(rows.place[i] * freq[j][r / 2], sn, cs);
+                    const float a = v[r], b = v[r + 1];
+                    v[r] = a * cs - b * sn;
+                    v[r + 1] = a * sn + b * cs;
+                }
+            }
+            bf16x4 o4;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o4[r] = (bf16)v[r];
+            *(bf16x4*)(mine + (i * 16 + token) * QKV_ROW_BYTES + (j * 16 + four) * 2) = o4;
+        });
+    };
+    write(std::integral_constant<int, 0>{});
+    static_for<0, QkvRows<BM>::BANDS>([&](auto bc) {
+        constexpr int band = decltype(bc)::value;
+        bf16x8 v[4];
+        asm volatile("" ::: "memory");           // (a wave's LDS accesses are carried out in the order it asks for them)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[p] = *(const bf16x8*)(mine + (band * 32 + p * 8 + (lane >> 3)) * QKV_ROW_BYTES + (lane & 7) * 16);
+        asm volatile("" ::: "memory");
+        if constexpr (band + 1 < QkvRows<BM>::BANDS) write(std::integral_constant<int, band + 1>{});
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int m = m_first + band * 32 + p * 8 + (lane >> 3), slot = rows.slot[band][p];
+            if (n < keys_from) {
+                if (m < M) *(bf16x8*)(out + (size_t)m * ldc + n) = v[p];
+            } else if (n < values_from && slot >= 0) *(bf16x8*)(k_at + (size_t)(slot >> 4) * page_size + (slot & 15) * hd) = v[p];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+// Values, [feature][slot] in a page, two bytes a lane with neighbouring lanes on neighbouring tokens, by all eight waves of a block: those of the
+// rows that multiplying wave `wave` % 4 left in LDS, the first half of them or the second.  (By the four waves that hold them alone they are what the whole grid waits
+// for: 2047 rows of 32 heads on 8 of 64, k 2048, 37.4 us, without the cache writes 30.1.)
+template <int BM>
+__device__ __forceinline__ void qkv_values(const unsigned char* tile, int wave, int M, int N, int m0, int n0, const QkvEpilogue& qe) {
+    constexpr int ROWS = BM / 2, HALF = ROWS / 2, STEP = 64 / HALF;               // a lane: one row and every STEP-th feature
+    const int lane = threadIdx.x & 63, of = wave & 3, row = (wave >> 2) * HALF + lane % HALF, hd = qe.head_dim;
+    const int values_from = (qe.n_heads + qe.n_kv_heads) * hd, n_first = n0 + (of & 1) * 64;
+    const int slot = slot_of_row(qe, M, m0 + (of >> 1) * ROWS + row), from = max(values_from - n_first, 0) + lane / HALF, end = min(N - n_first, 64);
+    if (slot < 0) return;
+    const unsigned char* mine = tile + of * (ROWS * QKV_ROW_BYTES) + row * QKV_ROW_BYTES;
+    // (heads lie one after the other in a page: [kv head][feature][slot])
+    bf16* at = (bf16*)qe.v_cache + (size_t)(slot >> 4) * ((size_t)qe.n_kv_heads * 16 * hd) + (slot & 15);
+#pragma unroll 4
+    for (int lc = from; lc < end; lc += STEP) at[(size_t)(n_first + lc - values_from) * 16] = *(const bf16*)(mine + lc * 2);
+}
 template <int BM, int EPI>
 __global__ __launch_bounds__(512) void gemm_fed_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
-                                                       void* __restrict__ out, int ldc, int M, int N, int K, int epi, int old_ahead) {
+                                                       void* __restrict__ out, int ldc, int M, int N, int K, int epi, int old_ahead, MoreOf<EPI> more) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char fed_smem[];
     constexpr int BN = 128, STAGES = fed_stages(BM), STAGE_BYTES = (BM + BN) * 128;
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
@@ -1395,6 +1515,11 @@ __global__ __launch_bounds__(512) void gemm_fed_kernel(const bf16* __restrict__ 
         }
         wait_vmcnt<0>();                       // (the bands of the results go through the same LDS)
         block_sync_lds();
+        if constexpr (EPI == LLMRS_EPI_QKV)
+            if (more.write_kv && n0 + BN > (more.n_heads + more.n_kv_heads) * more.head_dim) {
+                block_sync_lds();
+                qkv_values<BM>(fed_smem, wave, M, N, m0, n0, more);
+            }
         return;
     }
     const int wm = wave / 2, wn = wave % 2;
@@ -1445,6 +1570,8 @@ __global__ __launch_bounds__(512) void gemm_fed_kernel(const bf16* __restrict__ 
         block_sync_lds();
         __builtin_amdgcn_sched_barrier(0);
     };
+    [[maybe_unused]] std::conditional_t<EPI == LLMRS_EPI_QKV, QkvRows<BM>, NothingMore> rows;
+    if constexpr (EPI == LLMRS_EPI_QKV) rows = qkv_rows<BM>(more, M, m0 + wm * TM);
     block_sync_lds();                          // k-tile 0 is there
     const unsigned char* st = fed_smem;
     k_tile(st, std::false_type{});
@@ -1464,7 +1591,14 @@ __global__ __launch_bounds__(512) void gemm_fed_kernel(const bf16* __restrict__ 
             return;
         }
     }
-    band_epilogue<BM, BN, EPI>(acc, fed_smem, out, ldc, M, N, m0, n0, epi);
+    if constexpr (EPI == LLMRS_EPI_QKV) {
+        static_assert(4 * TM * QKV_ROW_BYTES <= STAGES * STAGE_BYTES && TN == 64, "the whole tile as 16-bit rows lies in LDS");
+        qkv_epilogue<BM>(acc, fed_smem + wave * (TM * QKV_ROW_BYTES), (bf16*)out, ldc, M, m0 + wm * TM, n0 + wn * TN, more, rows);
+        if (more.write_kv && n0 + BN > (more.n_heads + more.n_kv_heads) * more.head_dim) {
+            block_sync_lds();
+            qkv_values<BM>(fed_smem, wave, M, N, m0, n0, more);
+        }
+    } else band_epilogue<BM, BN, EPI>(acc, fed_smem, out, ldc, M, N, m0, n0, epi);
 }
 
 // Whether the four-wave tiles can finish this product: the epilogues it has, 16-bit results as whole 16-byte pieces.
@@ -1475,7 +1609,7 @@ static bool fourwave_takes(int epi, const void* out, int ldc, int N) {
     return false;
 }
 template <int BM, int EPI>
-static int launch_fed_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1) {
+static int launch_fed_epi(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, int epi, int splits = 1, const MoreOf<EPI>& more = {}) {
     constexpr int BN = 128;
     static bool configured = false;
     const size_t bytes = (size_t)fed_stages(BM) * (BM + BN) * 128;
@@ -1487,7 +1621,7 @@ static int launch_fed_epi(hipStream_t stream, const bf16* A, int lda, const bf16
     dim3 grid(ceil_div(N, BN), ceil_div(M, BM), splits);
     if (grid.y > 65535) return llmrs_fail("gemm: M=%d is too large for one launch", M);
     const int old_ahead = EPI == LLMRS_EPI_ACCUM_F32 && splits == 1 && N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)out & 15) == 0 && (size_t)M * ldc * 4 < ((size_t)1 << 32);
-    gemm_fed_kernel<BM, EPI><<<grid, 512, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, old_ahead);
+    gemm_fed_kernel<BM, EPI><<<grid, 512, bytes, stream>>>(A, lda, W, out, ldc, M, N, K, epi, old_ahead, more);
     return 0;
 }
 // (operands under 4 GB each, K % 64 == 0, fourwave_takes(epi, ...): the caller's to check, and that no share of k is empty)
@@ -1698,6 +1832,24 @@ int llmrs_gemm_bf16_split_parts(hipStream_t stream, const bf16* A, int lda, cons
     return splits;
 }
 
+// More than 64 rows of a q/k/v product whose rotation and cache write its tiles do themselves: those of `mid_tiles` that are not
+// split (there the rotation adds the parts up as it reads them).  The four-wave tiles of 256 features that take more rows keep the kernel behind them: with
+// this epilogue they were no faster, 106 us either way at 2048 x 6144 x 4096.  1, 0 where the product goes another way, -1 on error.
+static int qkv_in_tiles(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc, int M, int N, int K, const QkvEpilogue& qkv) {
+    const bool small = (size_t)M * lda * 2 < ((size_t)1 << 32) && (size_t)N * K * 2 < ((size_t)1 << 32);
+    if (!mid_takes(M, N, K) || !small || qkv.page_size != 16 || qkv.head_dim % 8 || ldc % 8 || (((uintptr_t)out | (uintptr_t)qkv.k_cache) & 15)) return 0;
+    const int over = M % 128;
+    const MidTiles plan = mid_tiles(M, N, K, LLMRS_EPI_STORE);
+    // (the rows beyond whole tiles that the launcher below gives to the kernel for few rows go there)
+    if (plan.splits > 1 || (M >= 1024 && over > 0 && over <= 64 && plan.time - mid_tiles(M - over, N, K, LLMRS_EPI_STORE).time >= 30.0)) return 0;
+    const int rc = plan.rows == 256 ? launch_fed_epi<256, LLMRS_EPI_QKV>(stream, A, lda, W, out, ldc, M, N, K, LLMRS_EPI_QKV, 1, qkv)
+                                    : launch_fed_epi<128, LLMRS_EPI_QKV>(stream, A, lda, W, out, ldc, M, N, K, LLMRS_EPI_QKV, 1, qkv);
+    if (rc != 0) return -1;
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) { llmrs_fail("gemm (mfma): launch failed: %s", hipGetErrorString(e)); return -1; }
+    return 1;
+}
+
 int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16* W, void* out, int ldc,
                          int M, int N, int K, int epi, void* workspace, size_t workspace_bytes,
                          const QkvEpilogue* qkv, const RowScale* scale, const NextNorm* next) {
@@ -1716,10 +1868,11 @@ int llmrs_gemm_bf16_mfma(hipStream_t stream, const bf16* A, int lda, const bf16*
         llmrs_fail("gemm: a deferred norm is taken for up to 16 rows, got M=%d N=%d K=%d epilogue %d", M, N, K, epi);
         return -1;
     }
-    if (epi == LLMRS_EPI_QKV) {   // only the skinny kernel fuses it; its 8-byte stores need aligned rows
-        if (M > 64 || qkv == nullptr || !llmrs_qkv_by_fours(qkv->head_dim, qkv->rotary_dim) || ldc % 4 || ((uintptr_t)out & 7) ||
+    if (epi == LLMRS_EPI_QKV) {   // four features of a head at a time: aligned rows
+        if (qkv == nullptr || !llmrs_qkv_by_fours(qkv->head_dim, qkv->rotary_dim) || ldc % 4 || ((uintptr_t)out & 7) ||
             ((uintptr_t)qkv->k_cache & 7))
             return 0;
+        if (M > 64) return scale != nullptr ? 0 : qkv_in_tiles(stream, A, lda, W, out, ldc, M, N, K, *qkv);
         // long rows and many tokens: the tiles with k split over blocks are so much faster that
         // the separate rotation kernel is paid for (10240 x 8192 at 64 rows: 60 us in the ring, 52 + 6; the tiles' parts are added by the rotation)
         // (with rows of 4096 the same route gains nothing: a decode step of the 8B shape at 64 requests 7.60 -> 7.55 ms,

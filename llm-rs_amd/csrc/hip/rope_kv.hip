@@ -246,7 +246,7 @@ extern "C" int llmrs_gemm(hipStream_t stream, int dtype, const void* A, int lda,
 
 // qkv = x W^T for W = [q heads; k heads; v heads], then what llmrs_rope_kv_write does,
 // with pairs (2i, 2i+1): in one kernel when the product is one the rotation fuses into
-// (bfloat16 up to 64 tokens, 32-bit up to 16), else as two.  In the fused case only q is written to
+// (bfloat16 where it is not split over blocks nor shared out between tiles of two kinds, 32-bit up to 16), else as two.  In the fused case only q is written to
 // `qkv`; k and v go to the cache alone.
 extern "C" int llmrs_qkv_rope_cache(hipStream_t stream, int dtype, const void* x, int lda, const void* w, void* qkv,
                                     int row_stride, int M, int K, const int* positions, const int* slot_map,

@@ -1682,6 +1682,48 @@ def test_qkv_rope_cache_adds_up_a_split_product(M, n_heads, n_kv, hd, rot, K):
     assert (kc2.float() - kc.float()).abs().max() <= scale / 64 and (vc2.float() - vc.float()).abs().max() <= scale / 64
 
 
+@pytest.mark.parametrize("M,n_heads,n_kv,hd,rot,K", [(65, 12, 4, 64, 64, 128), (129, 40, 8, 64, 32, 192), (300, 9, 3, 40, 24, 128), (257, 20, 2, 72, 72, 128),
+                                                     (520, 32, 8, 128, 128, 256), (700, 16, 0, 128, 64, 320), (1000, 3, 1, 8, 8, 64), (2047, 32, 8, 64, 64, 128),
+                                                     (300, 24, 8, 24, 0, 64)])
+@pytest.mark.parametrize("write_kv", [True, False])
+def test_qkv_rope_cache_in_the_tiles(M, n_heads, n_kv, hd, rot, K, write_kv):
+    """More than 64 rows of a product that is not split: the tiles rotate their 32-bit sums and write the cache.  Rows and features
+    beyond whole tiles, heads across tiles, queries, keys and values in one tile; slots in order, scattered, none and beyond the last page; positions
+    in the ten thousands.  One rounding to bfloat16 (2^-8 of a value), of sums of K products of 0.1 and of a pair turned by a 32-bit sine and cosine."""
+    page_size, num_pages = 16, -(-M // 16) + 3
+    N = (n_heads + 2 * n_kv) * hd
+    k = kernels()
+    assert k.lib.llmrs_gemm_mid_plan(M, N, K, EPI_STORE) // 100 == 1
+    x = rnd((M, K + 8), torch.bfloat16, 30)[:, :K]
+    w = rnd((N, K), torch.bfloat16, 31, 0.1)
+    g = torch.Generator().manual_seed(32)
+    positions = torch.randint(0, 100000, (M,), generator=g).to(torch.int32)
+    slots = torch.arange(5, 5 + M, dtype=torch.int32)
+    slots[M // 3:M // 2] = slots[M // 3:M // 2][torch.randperm(M // 2 - M // 3, generator=g)]
+    slots[7::11], slots[9::23] = -1, num_pages * page_size
+    inv_freq = plain_inv_freq(rot, 10000.0, None).to(DEV) if rot else None
+    room = rnd((M + 16, N + 8), torch.bfloat16, 34)
+    before = room.clone()
+    kc = torch.zeros((num_pages, n_kv, page_size, hd), dtype=torch.bfloat16, device=DEV)
+    vc = torch.zeros((num_pages, n_kv, hd, page_size), dtype=torch.bfloat16, device=DEV)
+    k.qkv_rope_cache(x, w, room[:M, :N], positions.to(DEV), slots.to(DEV), inv_freq, rot, kc, vc, n_heads, n_kv, hd, page_size, num_pages, write_kv)
+    acc = product64(x, w).view(M, n_heads + 2 * n_kv, hd)
+    turned = plain_rope(acc, positions, inv_freq.cpu(), "interleaved") if rot else acc
+    pair = torch.cat([acc[..., :rot].unflatten(-1, (rot // 2, 2)).norm(dim=-1, keepdim=True).expand(-1, -1, -1, 2).flatten(-2), acc[..., rot:].abs()], -1)
+    to = torch.nonzero((slots >= 0) & (slots < num_pages * page_size)).flatten() if write_kv else torch.zeros(0, dtype=torch.long)
+    page, off = (slots[to] // page_size).long(), (slots[to] % page_size).long()
+    kv, floor = n_heads + n_kv, 1e-5 * math.sqrt(K)
+    for name, got, ref, size in (("q", room[:M, :n_heads * hd].double().cpu().view(M, n_heads, hd), turned[:, :n_heads], pair[:, :n_heads]),
+                                 ("k", kc.double().cpu()[page, :, off, :], turned[to, n_heads:kv], pair[to, n_heads:kv]),
+                                 ("v", vc.double().cpu()[page, :, :, off], acc[to, kv:], acc[to, kv:].abs())):
+        assert ((got - ref).abs() <= ref.abs() * (1.01 / 256) + size * 2.0 ** -18 + floor).all(), (name, float((got - ref).abs().max()))
+    assert torch.equal(room[M:], before[M:]) and torch.equal(room[:, n_heads * hd:], before[:, n_heads * hd:])
+    untouched = torch.ones(num_pages * page_size, dtype=torch.bool)
+    untouched[slots[to].long()] = False
+    assert (kc.cpu().permute(0, 2, 1, 3).reshape(num_pages * page_size, -1)[untouched] == 0).all(), "a slot that no token maps to was written"
+    assert (vc.cpu().permute(0, 3, 1, 2).reshape(num_pages * page_size, -1)[untouched] == 0).all(), "a slot that no token maps to was written"
+
+
 # ---- utilities ----------------------------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", DTYPES)
