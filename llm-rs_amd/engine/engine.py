@@ -19,7 +19,7 @@ from ..config import load_config
 from ..sampling import Sampler, SamplingParams
 from ..weights import RandomTensors, load_tensors, random_tensors
 from .model import Model
-from .step import StepEntry, StepRunner
+from .step import StepEntry, StepRunner, record_event
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32, "f32": torch.float32,
            "fp32": torch.float32, torch.bfloat16: torch.bfloat16, torch.float32: torch.float32}
@@ -107,6 +107,7 @@ class Engine:
         self.overlap = bool(overlap)
         self._flight: Optional[_Flight] = None               # the step in flight (overlap)
         self._ids_host = [None, None]                        # pinned room for samples on their way to the host, in turns
+        self._landed = [None, None]                          # the events behind those copies
         self._ids_turn = 0
         self._steps = 0
         self._step_events: List[tuple] = []                 # (before the first kernel, after sampling) of measured steps
@@ -264,8 +265,7 @@ class Engine:
                     host = self._ids_host[self._ids_turn] = torch.zeros(max(2 * n_want, 256), dtype=torch.int32, pin_memory=True)
                 host = host[:n_want]
                 host.copy_(ids, non_blocking=True)
-                landed = torch.cuda.Event()
-                landed.record()
+                landed = self._landed[self._ids_turn] = record_event(self._landed[self._ids_turn])
             else:
                 host = ids.clone()
         self._steps += 1
@@ -280,11 +280,11 @@ class Engine:
         if flight.host is not None:
             if flight.landed is not None:
                 flight.landed.synchronize()
-            sampled = flight.host.numpy().copy()
+            sampled = flight.host.tolist()
             # A sampler or hand-over fault must not go on as "the request decodes from token 0": fail here.
             vocab = self.model.spec.vocab_size
-            if len(sampled) and (int(sampled.min()) < 0 or int(sampled.max()) >= vocab):
-                raise RuntimeError(f"a step sampled token ids outside [0, {vocab}): {int(sampled.min())}..{int(sampled.max())}")
+            if sampled and (min(sampled) < 0 or max(sampled) >= vocab):
+                raise RuntimeError(f"a step sampled token ids outside [0, {vocab}): {min(sampled)}..{max(sampled)}")
         finished = set(core.commit(sampled))
         out: List[Emitted] = []
         for (slot, request), token in zip(flight.owners, sampled):
@@ -292,11 +292,11 @@ class Engine:
                 continue                    # it ended while this step was in flight (a stop token, a cancel): dropped
             if slot in finished:
                 reason = "stop" if core.request_info(slot)["finish"] == 1 else "length"
-                out.append(Emitted(request, None if reason == "stop" else int(token), reason))
+                out.append(Emitted(request, None if reason == "stop" else token, reason))
                 core.drop_request(slot)
                 self._forget(slot)
             else:
-                out.append(Emitted(request, int(token)))
+                out.append(Emitted(request, token))
         return out
 
     def _advance_overlapped(self) -> List[Emitted]:

@@ -37,6 +37,15 @@ class OutOfPages(RuntimeError):
     pass
 
 
+def record_event(event: Optional["torch.cuda.Event"]) -> "torch.cuda.Event":
+    """Records `event` (None: a new one) on the current stream and returns it.  An event that is kept and a stream asked for by its
+    device's number: 2 us instead of 7."""
+    if event is None:
+        event = torch.cuda.Event()
+    event.record(torch.cuda.current_stream(torch.cuda.current_device()))
+    return event
+
+
 class _GrewWhileRecording(Exception):
     """A buffer would have had to grow in the middle of a recording."""
 
@@ -47,6 +56,10 @@ class StepEntry:
     start: int
     tokens: Sequence[int]
     want: Sequence[int] = ()      # places among `tokens` whose logits are wanted
+
+
+# The views of a step's words that a context hands out (StepContext.lay_out).
+_ARRAYS = frozenset(("tokens", "positions", "token_entry", "q_starts", "seq_lens", "slots", "want_rows", "sampling", "slot_maps", "block_tables"))
 
 
 class StepContext:
@@ -60,10 +73,7 @@ class StepContext:
         self.n_entries = 0
         self.n_want = 0
         self.run_index = -1
-        self.tokens = self.positions = self.token_entry = None
-        self.q_starts = self.seq_lens = self.slots = self.want_rows = self.sampling = None
-        self.slot_maps: List[torch.Tensor] = []
-        self.block_tables: List[torch.Tensor] = []
+        self.lay_out(None, None)
         self.entries: List[Tuple[int, int, int]] = []   # host copy: (slot, start, count)
         self.max_seq_len = 0                            # largest start + count among the entries
         self.longest = 0                                # the most tokens an entry brings
@@ -91,6 +101,32 @@ class StepContext:
         # Where the model wants the stream's rows after the block that runs now, in the activation type (what comes next
         # reads them as they are): a block whose last kernel can write them does and sets this to None.
         self.rows_after_block: Optional[torch.Tensor] = None
+
+    # The step's arrays are views of the one block of words on the device, made when they are first asked for: a replayed
+    # step asks for two of the ten (binding all of them took 16 us a step, 4 now, of the 135 of a small replayed step's host time).
+    def lay_out(self, dev: Optional[torch.Tensor], off) -> None:
+        """From now on the arrays are those at the offsets `off` (a `BatchOffsets`) of `dev`; None: there are none."""
+        for name in _ARRAYS:
+            self.__dict__.pop(name, None)
+        self._dev, self._off = dev, off
+
+    def __getattr__(self, name):
+        if name not in _ARRAYS:
+            raise AttributeError(name)
+        dev, off, T, R, n = self._dev, self._off, self.n_tokens, self.n_entries, self.n_want
+        if name == "slot_maps":
+            got = [] if dev is None else [dev[o:o + T] for o in off.slot_maps]
+        elif name == "block_tables":
+            got = [] if dev is None else [dev[o:o + R * w].view(R, w) for o, w in zip(off.tables, off.widths)]
+        elif dev is None:
+            got = None
+        elif name == "sampling":
+            got = dev[off.sampling:off.sampling + 4 * n].view(n, 4)
+        else:
+            first = getattr(off, name)
+            got = dev[first:first + (T if name in ("tokens", "positions", "token_entry") else n if name == "want_rows" else R + (name == "q_starts"))]
+        self.__dict__[name] = got
+        return got
 
     # A block on several streams leaves its last mix to the norm that reads the streams next (one launch, one pass
     # over the streams less).  Whoever else reads them calls flush_streams() first.
@@ -209,7 +245,8 @@ class StepRunner:
         self._views: Dict[str, tuple] = {}      # name -> (shape, dtype, the view of its buffer handed out last)
         self._pinned = self.device.type == "cuda"
         self._host = [self._new_host(words_capacity) for _ in range(2)]
-        self._events = [None, None]
+        self._copied = [None, None]             # the events behind the copies of `_host`, and whether one is still to be waited for
+        self._copying = [False, False]
         self._turn = 0
         self._dev_words = torch.zeros(words_capacity, dtype=torch.int32, device=self.device)
         self.ctx = StepContext(self)
@@ -279,9 +316,9 @@ class StepRunner:
     def _staging(self, words_needed: int) -> np.ndarray:
         self._turn ^= 1
         i = self._turn
-        if self._events[i] is not None:
-            self._events[i].synchronize()
-            self._events[i] = None
+        if self._copying[i]:
+            self._copied[i].synchronize()
+            self._copying[i] = False
         if self._host[i].numel() < words_needed:
             self._host[i] = self._new_host(max(words_needed, 2 * self._host[i].numel()))
         return self._host[i].numpy()
@@ -294,9 +331,8 @@ class StepRunner:
         dev = self._dev_words[:n_words]
         dev.copy_(self._host[i][:n_words], non_blocking=True)
         if self._pinned:
-            ev = torch.cuda.Event()
-            ev.record()
-            self._events[i] = ev
+            self._copied[i] = record_event(self._copied[i])
+            self._copying[i] = True
         return dev
 
     def _estimate_words(self, T: int, R: int, n_want: int, longest: int, widths=None) -> int:
@@ -334,16 +370,7 @@ class StepRunner:
         c._clean_rooms.clear()
         c.rows_after_block = None
         c.serial += 1
-        c.tokens = dev[off.tokens:off.tokens + T]
-        c.positions = dev[off.positions:off.positions + T]
-        c.token_entry = dev[off.token_entry:off.token_entry + T]
-        c.q_starts = dev[off.q_starts:off.q_starts + R + 1]
-        c.seq_lens = dev[off.seq_lens:off.seq_lens + R]
-        c.slots = dev[off.slots:off.slots + R]
-        c.want_rows = dev[off.want_rows:off.want_rows + n_want]
-        c.sampling = dev[off.sampling:off.sampling + 4 * n_want].view(n_want, 4)
-        c.slot_maps = [dev[o:o + T] for o in off.slot_maps]
-        c.block_tables = [dev[o:o + R * w].view(R, w) for o, w in zip(off.tables, off.widths)]
+        c.lay_out(dev, off)
         return c
 
     # -- the step ------------------------------------------------------------------
