@@ -7,8 +7,12 @@ import torch
 from llm_rs_amd.engine.step import StepContext
 
 
+class Runner:
+    device = torch.device("cpu")
+
+
 def test_arrays_are_those_of_the_step_that_is_bound():
-    runner = types.SimpleNamespace(device=torch.device("cpu"))
+    runner = Runner()
     ctx = StepContext(runner)
     assert ctx.tokens is None and ctx.slot_maps == [] and ctx.block_tables == []
     for T, R, n, widths in ((5, 2, 1, [3]), (1, 1, 1, [64, 2]), (7, 3, 0, [])):
