@@ -12,8 +12,9 @@
 // Both need K % 8 == 0 and 16-byte aligned rows (16-byte loads); otherwise the
 // caller falls back to the plain kernel.
 //
-// The order in which an output's products are summed depends on K, N and the
-// kernel, never on M, the row's place in the batch or the tile it falls in.
+// The order in which an output's products are summed depends on K, N, the
+// kernel and the parts that K is split into, never on the row's place in the
+// batch or the tile it falls in.
 // Replaces the reference's matvec_bf16_simd / gemm_bf16 (shaders/ops.metal:52-159,
 // :1090-1143); unlike gemm_bf16 (:1107) the accumulator is 32-bit.
 #include "gemm_ring.h"
